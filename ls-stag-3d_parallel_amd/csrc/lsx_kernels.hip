@@ -83,7 +83,17 @@ __device__ inline void decode(int i, int N, int M, int* x, int* y, int* z) {
   *x = r - *y * N;
 }
 
-__device__ inline int slot_sub(int npts, int dir) {  // coupling to the previous cell of a line
+// The cell of this thread in the one-cell-per-thread kernels: rows of at least 64 cells by tiles
+// (tile_cell), shorter ones, which would leave most of a tile's lanes idle, in index order.
+__device__ inline bool own_cell(int N, int M, int K, int* x, int* y, int* z) {
+  if (N >= 64) return tile_cell(N, M, x, y, z);
+  const unsigned i = blockIdx.x * 256u + threadIdx.x;
+  if (i >= (unsigned)N * M * K) return false;
+  decode((int)i, N, M, x, y, z);
+  return true;
+}
+
+__host__ __device__ inline int slot_sub(int npts, int dir) {  // coupling to the previous cell of a line
   if (npts == 7) return dir == 0 ? 2 : (dir == 1 ? 1 : 0);
   return dir == 0 ? 12 : (dir == 1 ? 10 : 4);
 }
@@ -95,7 +105,9 @@ __device__ inline int slot_diag(int npts) { return npts == 7 ? 3 : 13; }
 
 // Row i of the operator applied to x, accumulated in ascending column order (the CSR order
 // of the reference matrices: [b,s,w,p,e,n,t] on the fine level, sorted columns on Galerkin
-// levels).  mode: 0 -> acc starts at 0 and adds; 1 -> acc starts at b and subtracts.
+// levels).  acc starts at the given value; subtract: terms are subtracted.  Every load is issued
+// unconditionally (absent neighbours read a present cell) and absent terms leave the sum
+// unchanged, so the loads of a row are in flight together.
 template <int NPTS>
 __device__ inline double row_apply(const double* __restrict__ coef, long n, int i, int x, int y, int z, int N, int M,
                                    int K, const double* __restrict__ xv, double acc, bool subtract) {
@@ -103,25 +115,34 @@ __device__ inline double row_apply(const double* __restrict__ coef, long n, int 
   if (NPTS == 7) {
     const int off[7] = {-NM, -N, -1, 0, 1, N, NM};
     const bool ok[7] = {z > 0, y > 0, x > 0, true, x < N - 1, y < M - 1, z < K - 1};
+    double a[7], v[7];
 #pragma unroll
-    for (int q = 0; q < 7; ++q)
-      if (ok[q]) {
-        const double t = coef[q * n + i] * xv[i + off[q]];
-        acc = subtract ? acc - t : acc + t;
-      }
+    for (int q = 0; q < 7; ++q) {
+      a[q] = coef[q * n + i];
+      v[q] = xv[ok[q] ? i + off[q] : i];
+    }
+#pragma unroll
+    for (int q = 0; q < 7; ++q) {
+      const double t = a[q] * v[q];
+      const double s = subtract ? acc - t : acc + t;
+      acc = ok[q] ? s : acc;
+    }
   } else {
+    const bool okx[3] = {x > 0, true, x < N - 1}, oky[3] = {y > 0, true, y < M - 1}, okz[3] = {z > 0, true, z < K - 1};
+    const int ox[3] = {okx[0] ? -1 : 0, 0, okx[2] ? 1 : 0}, oy[3] = {oky[0] ? -N : 0, 0, oky[2] ? N : 0};
+    const int oz[3] = {okz[0] ? -NM : 0, 0, okz[2] ? NM : 0};
+    double a[27], v[27];
 #pragma unroll
-    for (int dz = -1; dz <= 1; ++dz)
+    for (int q = 0; q < 27; ++q) {
+      a[q] = coef[q * n + i];
+      v[q] = xv[i + ox[q % 3] + oy[q / 3 % 3] + oz[q / 9]];
+    }
 #pragma unroll
-      for (int dy = -1; dy <= 1; ++dy)
-#pragma unroll
-        for (int dx = -1; dx <= 1; ++dx) {
-          const int zz = z + dz, yy = y + dy, xx = x + dx;
-          if (zz < 0 || zz >= K || yy < 0 || yy >= M || xx < 0 || xx >= N) continue;
-          const int q = (dx + 1) + 3 * (dy + 1) + 9 * (dz + 1);
-          const double t = coef[q * n + i] * xv[i + dx + N * dy + NM * dz];
-          acc = subtract ? acc - t : acc + t;
-        }
+    for (int q = 0; q < 27; ++q) {
+      const double t = a[q] * v[q];
+      const double s = subtract ? acc - t : acc + t;
+      acc = okx[q % 3] && oky[q / 3 % 3] && okz[q / 9] ? s : acc;
+    }
   }
   return acc;
 }
@@ -653,39 +674,28 @@ __device__ inline double row_apply_sym_t(const double* __restrict__ s4, long n, 
   return acc;
 }
 
-template <int MODE, int BS>
-__global__ void k_stencil_sym_t(const double* __restrict__ s4, int N, int M, int K, SymExc ex,
-                                const double* __restrict__ x, const double* __restrict__ b, double* __restrict__ y,
-                                double* __restrict__ partial) {
+// y = A x or y -= A x (TR: A^T), one thread per cell
+template <int MODE, bool TR>
+__global__ void __launch_bounds__(256) k_stencil_sym(const double* __restrict__ s4, int N, int M, int K, SymExc ex,
+                                                     const double* __restrict__ x, double* __restrict__ y) {
+  static_assert(MODE == ST_PROD || MODE == ST_SUBR, "the residual with its norm has a kernel of its own");
+  int xx, yy, zz;
+  if (!own_cell(N, M, K, &xx, &yy, &zz)) return;
   const long n = (long)N * M * K;
-  long lo, hi;
-  chunk_of(n, blockIdx.x, gridDim.x, &lo, &hi);
-  double ss = 0.0;
-  for (long li = lo + threadIdx.x; li < hi; li += BS) {
-    const int i = (int)li;
-    int xx, yy, zz;
-    decode(i, N, M, &xx, &yy, &zz);
-    if (MODE == ST_PROD) {
-      y[i] = row_apply_sym_t(s4, n, i, xx, yy, zz, N, M, K, x, 0.0, false, ex);
-    } else if (MODE == ST_RESID) {
-      const double r = row_apply_sym_t(s4, n, i, xx, yy, zz, N, M, K, x, b[i], true, ex);
-      y[i] = r;
-      ss += r * r;
-    } else {
-      const double q = row_apply_sym_t(s4, n, i, xx, yy, zz, N, M, K, x, 0.0, false, ex);
-      y[i] = y[i] - q;
-    }
-  }
-  if (MODE == ST_RESID) {
-    ss = block_sum<BS>(ss);
-    if (threadIdx.x == 0) partial[blockIdx.x] = ss;
-  }
+  const int i = xx + N * (yy + M * zz);
+  double q;
+  if constexpr (TR)
+    q = row_apply_sym_t(s4, n, i, xx, yy, zz, N, M, K, x, 0.0, false, ex);
+  else
+    q = row_apply_sym(s4, n, i, xx, yy, zz, N, M, K, x, 0.0, false, ex);
+  y[i] = MODE == ST_PROD ? q : y[i] - q;
 }
 
-template <int MODE, int BS>
-__global__ void k_stencil_sym(const double* __restrict__ s4, int N, int M, int K, SymExc ex,
-                              const double* __restrict__ x, const double* __restrict__ b, double* __restrict__ y,
-                              double* __restrict__ partial) {
+// y = b - A x (TR: A^T) with the partial sums of y^2 over the reductions' fixed chunks
+template <int BS, bool TR>
+__global__ void k_stencil_sym_resid(const double* __restrict__ s4, int N, int M, int K, SymExc ex,
+                                    const double* __restrict__ x, const double* __restrict__ b, double* __restrict__ y,
+                                    double* __restrict__ partial) {
   const long n = (long)N * M * K;
   long lo, hi;
   chunk_of(n, blockIdx.x, gridDim.x, &lo, &hi);
@@ -694,21 +704,16 @@ __global__ void k_stencil_sym(const double* __restrict__ s4, int N, int M, int K
     const int i = (int)li;
     int xx, yy, zz;
     decode(i, N, M, &xx, &yy, &zz);
-    if (MODE == ST_PROD) {
-      y[i] = row_apply_sym(s4, n, i, xx, yy, zz, N, M, K, x, 0.0, false, ex);
-    } else if (MODE == ST_RESID) {
-      const double r = row_apply_sym(s4, n, i, xx, yy, zz, N, M, K, x, b[i], true, ex);
-      y[i] = r;
-      ss += r * r;
-    } else {
-      const double q = row_apply_sym(s4, n, i, xx, yy, zz, N, M, K, x, 0.0, false, ex);
-      y[i] = y[i] - q;
-    }
+    double r;
+    if constexpr (TR)
+      r = row_apply_sym_t(s4, n, i, xx, yy, zz, N, M, K, x, b[i], true, ex);
+    else
+      r = row_apply_sym(s4, n, i, xx, yy, zz, N, M, K, x, b[i], true, ex);
+    y[i] = r;
+    ss += r * r;
   }
-  if (MODE == ST_RESID) {
-    ss = block_sum<BS>(ss);
-    if (threadIdx.x == 0) partial[blockIdx.x] = ss;
-  }
+  ss = block_sum<BS>(ss);
+  if (threadIdx.x == 0) partial[blockIdx.x] = ss;
 }
 
 // y = A^T x with an FP32 x
@@ -732,9 +737,25 @@ __global__ void k_stencil_sym_f32x(const double* __restrict__ s4, int N, int M, 
 }
 
 // ---- kernels: solve phase ---------------------------------------------------------------------
-template <int NPTS, int MODE, int BS>
-__global__ void k_stencil(const double* __restrict__ coef, int N, int M, int K, const double* __restrict__ x,
-                          const double* __restrict__ b, double* __restrict__ y, double* __restrict__ partial) {
+// y = A x or y -= A x, one thread per cell: what bounds it is the NPTS + 2 planes moved, and on
+// small levels the latency of one row, so no thread takes a second cell (27 points: 4 us at 16^3 and
+// 32^3, 36 us at 96^3; up to four cells a thread, their loads behind branches: 17 us averaged over
+// the levels of 64^3)
+template <int NPTS, int MODE>
+__global__ void __launch_bounds__(256) k_stencil(const double* __restrict__ coef, int N, int M, int K,
+                                                 const double* __restrict__ x, double* __restrict__ y) {
+  static_assert(MODE == ST_PROD || MODE == ST_SUBR, "the residual with its norm has a kernel of its own");
+  int xx, yy, zz;
+  if (!own_cell(N, M, K, &xx, &yy, &zz)) return;
+  const int i = xx + N * (yy + M * zz);
+  const double q = row_apply<NPTS>(coef, (long)N * M * K, i, xx, yy, zz, N, M, K, x, 0.0, false);
+  y[i] = MODE == ST_PROD ? q : y[i] - q;
+}
+
+// y = b - A x with the partial sums of y^2 over the reductions' fixed chunks
+template <int NPTS, int BS>
+__global__ void k_stencil_resid(const double* __restrict__ coef, int N, int M, int K, const double* __restrict__ x,
+                                const double* __restrict__ b, double* __restrict__ y, double* __restrict__ partial) {
   const long n = (long)N * M * K;
   long lo, hi;
   chunk_of(n, blockIdx.x, gridDim.x, &lo, &hi);
@@ -743,21 +764,12 @@ __global__ void k_stencil(const double* __restrict__ coef, int N, int M, int K, 
     const int i = (int)li;
     int xx, yy, zz;
     decode(i, N, M, &xx, &yy, &zz);
-    if (MODE == ST_PROD) {
-      y[i] = row_apply<NPTS>(coef, n, i, xx, yy, zz, N, M, K, x, 0.0, false);
-    } else if (MODE == ST_RESID) {
-      const double r = row_apply<NPTS>(coef, n, i, xx, yy, zz, N, M, K, x, b[i], true);
-      y[i] = r;
-      ss += r * r;
-    } else {
-      const double q = row_apply<NPTS>(coef, n, i, xx, yy, zz, N, M, K, x, 0.0, false);
-      y[i] = y[i] - q;
-    }
+    const double r = row_apply<NPTS>(coef, n, i, xx, yy, zz, N, M, K, x, b[i], true);
+    y[i] = r;
+    ss += r * r;
   }
-  if (MODE == ST_RESID) {
-    ss = block_sum<BS>(ss);
-    if (threadIdx.x == 0) partial[blockIdx.x] = ss;
-  }
+  ss = block_sum<BS>(ss);
+  if (threadIdx.x == 0) partial[blockIdx.x] = ss;
 }
 
 // r_c = R r_f: each coarse cell sums 1/8 of its 8 children (R row order a,b,c,d,aa,bb,cc,dd)
@@ -808,45 +820,188 @@ __global__ void k_prolong(const double* __restrict__ chc, int Nc, int Mc, double
 }
 
 // c = omega * T_dir^{-1} r ; ch += c (smoother_adlj_interface.h:73-82 with the TDMA kernels
-// smoother_adlj_x.h:38-48, smoother_adlj_y.h:36-50).  One thread per line.  For z lines the
-// reference reads the first right-hand-side element at index y*N*K + x (its z call passes
-// N*K where the y kernel expects N*M); z_head_fix = 0 reproduces that read.
-__global__ void k_line_solve(const double* __restrict__ coef, int npts, int N, int M, int K, int dir,
-                             const double* __restrict__ dinv, const double* __restrict__ eu,
-                             const double* __restrict__ r, double* __restrict__ c, double* __restrict__ ch,
-                             double omega, int z_head_fix) {
-  const long n = (long)N * M * K;
-  const int nlines = dir == 0 ? M * K : (dir == 1 ? N * K : N * M);
-  const int t = blockIdx.x * blockDim.x + threadIdx.x;
-  if (t >= nlines) return;
-  int start, stride, len;
-  line_geometry(t, dir, N, M, K, &start, &stride, &len);
-  const double* sb = coef + slot_sub(npts, dir) * n;
-  int head = start;
-  if (dir == 2 && !z_head_fix) {
-    const int x = t % N, y = t / N;
-    head = y * N * K + x;
+// smoother_adlj_x.h:38-48, smoother_adlj_y.h:36-50).  One thread per line, the Thomas steps in the
+// reference's order.  For z lines the reference reads the first right-hand-side element at index
+// y*N*K + x (its z call passes N*K where the y kernel expects N*M); z_head_fix = 0 reproduces
+// that read.
+//
+// A step is three dependent FP64 operations, far shorter than a memory access, so what bounds a line
+// is its loads.  A wavefront takes LT lines and moves them in tiles of LT lines x LW cells: 64 lanes
+// load a tile of every array (16 loads a lane and array, all in flight, the next tile's under way
+// while this one is worked on), post it to LDS, and LT lanes run the Thomas steps on LDS operands.
+// Adjacent lanes load adjacent memory for every direction (LW cells of a row for x lines, LT
+// adjacent x of a row for y and z lines: whole 128-byte pieces).  The forward result y stays in
+// LDS, so r, the factors, the coupling and ch are read once and c and ch written once (56 bytes a
+// cell); a line of at most LW cells waits for memory twice in all.  YG: lines too long for that
+// pass y through c in memory.  Few lines to a wavefront, so that small levels spread over the
+// chip; the LDS accesses of the LT lanes are what a long line then waits for (two values to an
+// access; ch stays in registers).  Measured (x / y / z pass): 192^3 90 / 96 / 99 us (4.0-4.4 TB/s),
+// 128^3 27 / 29 / 28 us, 64^3 11 us; one thread per line with its loads in the loop: 57 us averaged
+// over the levels of 192^3, 111 us over the directions at 127 x 128 x 128.
+constexpr int LT = 16, LW = 64, LB = 8;
+
+template <int DIR, bool YG>
+__global__ void __launch_bounds__(64) k_line_tile(const double* __restrict__ sb, int N, int M, int K,
+                                                  const double* __restrict__ dinv, const double* __restrict__ eu,
+                                                  const double* __restrict__ r, double* c,
+                                                  double* __restrict__ ch, double omega, int z_head_fix) {
+  // tiles of LT rows of LP values: the coupling or eu, dinv, and the r tiles, which y replaces
+  // (one for each LW cells of a line; YG: one for all)
+  constexpr int LP = LW + 2, TILE = LT * LP, E = LT * LW / 64;
+  extern __shared__ __align__(16) double lds_line[];
+  double *tb = lds_line, *tc = tb + TILE, *ty = tc + TILE;
+  const int nlines = DIR == 0 ? M * K : (DIR == 1 ? N * K : N * M);
+  const int len = DIR == 0 ? N : (DIR == 1 ? M : K);
+  const int stride = DIR == 0 ? 1 : (DIR == 1 ? N : N * M);
+  const int lane = threadIdx.x, line0 = blockIdx.x * LT;
+  auto start_of = [&](int t) {
+    if (DIR == 0) return t * N;
+    if (DIR == 1) return t % N + N * M * (t / N);
+    return t;
+  };
+  // the tile elements of this lane: x lines cell `lane` of line j; y and z lines line lane % LT,
+  // cells lane / LT + 4 j
+  auto el = [&](int j, int& l, int& k) {
+    l = DIR == 0 ? j : lane % LT;
+    k = DIR == 0 ? lane : lane / LT + (64 / LT) * j;
+  };
+  const int own = line0 + lane % LT < nlines ? line0 + lane % LT : nlines - 1;
+  const int base = DIR == 0 ? 0 : start_of(own);
+  auto index = [&](int l, int k) {  // past the last line or cell: the last one
+    const int kk = k < len ? k : len - 1;
+    if (DIR == 0) return start_of(line0 + l < nlines ? line0 + l : nlines - 1) + kk;
+    return base + stride * kk;
+  };
+  double a[E], b[E], d[E];
+  auto load = [&](int k0, const double* pa, const double* pb, const double* pd) {
+#pragma unroll
+    for (int j = 0; j < E; ++j) {
+      int l, k;
+      el(j, l, k);
+      const int i = index(l, k0 + k);
+      if (pa) a[j] = pa[i];
+      b[j] = pb[i];
+      d[j] = pd[i];
+    }
+  };
+  // LB consecutive values of this lane's line in a tile, two to an LDS access
+  auto take = [&](const double* t, int u0, double (&v)[LB]) {
+    const double2* q = reinterpret_cast<const double2*>(t + lane * LP + u0);
+#pragma unroll
+    for (int u = 0; u < LB / 2; ++u) {
+      const double2 w = q[u];
+      v[2 * u] = w.x;
+      v[2 * u + 1] = w.y;
+    }
+  };
+  auto put = [&](double* t, int u0, const double (&v)[LB]) {
+    double2* q = reinterpret_cast<double2*>(t + lane * LP + u0);
+#pragma unroll
+    for (int u = 0; u < LB / 2; ++u) q[u] = make_double2(v[2 * u], v[2 * u + 1]);
+  };
+  load(0, r, sb, dinv);
+  if (DIR == 2 && !z_head_fix && lane < LT) a[0] = r[own / N * N * K + own % N];
+  double yprev = 0.0;
+  for (int k0 = 0; k0 < len; k0 += LW) {
+    double* yt = YG ? ty : ty + k0 / LW * TILE;
+#pragma unroll
+    for (int j = 0; j < E; ++j) {
+      int l, k;
+      el(j, l, k);
+      yt[l * LP + k] = a[j];
+      tb[l * LP + k] = k0 + k == 0 ? 0.0 : b[j];  // the first cell couples to none: r - 0 y = r
+      tc[l * LP + k] = d[j];
+    }
+    __syncthreads();
+    if (k0 + LW < len) load(k0 + LW, r, sb, dinv);
+    if (lane < LT) {
+      // the operands of the next LB cells are read before the results of these are written, which
+      // would hold them back
+      const int m = len - k0 < LW ? len - k0 : LW;
+      double ra[LB], rb[LB], rd[LB];
+      take(yt, 0, ra);
+      take(tb, 0, rb);
+      take(tc, 0, rd);
+      for (int u0 = 0; u0 < m; u0 += LB) {
+        double yv[LB];
+#pragma unroll
+        for (int u = 0; u < LB; ++u) {
+          yprev = (ra[u] - rb[u] * yprev) * rd[u];
+          yv[u] = yprev;  // past the line's end: unused
+        }
+        if (u0 + LB < m) {
+          take(yt, u0 + LB, ra);
+          take(tb, u0 + LB, rb);
+          take(tc, u0 + LB, rd);
+        }
+        put(yt, u0, yv);
+      }
+    }
+    __syncthreads();
+    if constexpr (YG) {
+#pragma unroll
+      for (int j = 0; j < E; ++j) {
+        int l, k;
+        el(j, l, k);
+        if (line0 + l < nlines && k0 + k < len) c[index(l, k0 + k)] = ty[l * LP + k];
+      }
+      __threadfence_block();  // read back below by other lanes
+      __syncthreads();
+    }
   }
-  int i = start;
-  double yprev = r[head] * dinv[i];
-  c[i] = yprev;
-  for (int k = 1; k < len; ++k) {
-    i += stride;
-    yprev = (r[i] - sb[i] * yprev) * dinv[i];
-    c[i] = yprev;
-  }
-  // backward: x_k = y_k - e_k x_{k+1}; write omega*x and accumulate into ch
-  double xnext = yprev;
-  double cv = xnext * omega;
-  c[i] = cv;
-  ch[i] = ch[i] + cv;
-  for (int k = len - 2; k >= 0; --k) {
-    i -= stride;
-    const double xv = c[i] - eu[i] * xnext;
-    xnext = xv;
-    cv = xv * omega;
-    c[i] = cv;
-    ch[i] = ch[i] + cv;
+  // backward: x_k = y_k - e_k x_{k+1}; write omega x and accumulate into ch.  Cells past the line's
+  // end have y = e = 0, so that the last cell starts from x = 0 (its own e is 0)
+  const int last = (len - 1) / LW * LW;
+  const double* yg = YG ? c : nullptr;
+  load(last, yg, eu, ch);
+  double xnext = 0.0;
+  for (int k0 = last; k0 >= 0; k0 -= LW) {
+    double* yt = YG ? ty : ty + k0 / LW * TILE;
+    double h[E];  // this tile's ch stays with the lanes that loaded it
+#pragma unroll
+    for (int j = 0; j < E; ++j) {
+      int l, k;
+      el(j, l, k);
+      const bool in = k0 + k < len;
+      if (YG || !in) yt[l * LP + k] = YG && in ? a[j] : 0.0;
+      tb[l * LP + k] = in ? b[j] : 0.0;
+      h[j] = d[j];
+    }
+    __syncthreads();
+    if (k0 >= LW) load(k0 - LW, yg, eu, ch);
+    if (lane < LT) {
+      const int m = len - k0 < LW ? len - k0 : LW;
+      double ra[LB], rb[LB];
+      const int top = (m - 1) / LB * LB;
+      take(yt, top, ra);
+      take(tb, top, rb);
+      for (int u0 = top; u0 >= 0; u0 -= LB) {
+        double cv[LB];
+#pragma unroll
+        for (int u = LB - 1; u >= 0; --u) {
+          xnext = ra[u] - rb[u] * xnext;
+          cv[u] = xnext * omega;
+        }
+        if (u0 >= LB) {
+          take(yt, u0 - LB, ra);
+          take(tb, u0 - LB, rb);
+        }
+        put(yt, u0, cv);
+      }
+    }
+    __syncthreads();
+#pragma unroll
+    for (int j = 0; j < E; ++j) {
+      int l, k;
+      el(j, l, k);
+      if (line0 + l < nlines && k0 + k < len) {
+        const int i = index(l, k0 + k);
+        const double cv = yt[l * LP + k];
+        c[i] = cv;
+        ch[i] = h[j] + cv;
+      }
+    }
+    __syncthreads();
   }
 }
 
@@ -1244,6 +1399,8 @@ int grid_1d(long n, int bs = 256) {
 // ================================================================================================
 // blocks of tile_cell
 static unsigned tile_blocks(Dims d) { return (unsigned)((long)((d.N + 63) / 64) * ((d.M + 3) / 4) * d.K); }
+// blocks of own_cell
+static unsigned cell_blocks(Dims d) { return d.N >= 64 ? tile_blocks(d) : (unsigned)((d.n() + 255) / 256); }
 
 int reduction_blocks(long n) {
   long b = (n + RED_THREADS * 4 - 1) / (RED_THREADS * 4);
@@ -1298,17 +1455,32 @@ void lu_factor(const double* coef27, Dims d, double* scale, int* perm, double* L
 void stencil_apply(const double* coef, int npts, Dims d, const double* x, const double* b, double* y, int mode,
                    double* partial, hipStream_t s) {
   const int nb = reduction_blocks(d.n());
-#define LSX_ST(NP, MD) k_stencil<NP, MD, RED_THREADS><<<nb, RED_THREADS, 0, s>>>(coef, d.N, d.M, d.K, x, b, y, partial)
-  if (npts == 7) {
-    if (mode == ST_PROD) LSX_ST(7, ST_PROD);
-    else if (mode == ST_RESID) LSX_ST(7, ST_RESID);
-    else LSX_ST(7, ST_SUBR);
-  } else {
-    if (mode == ST_PROD) LSX_ST(27, ST_PROD);
-    else if (mode == ST_RESID) LSX_ST(27, ST_RESID);
-    else LSX_ST(27, ST_SUBR);
-  }
+#define LSX_ST(NP)                                                                                          \
+  do {                                                                                                      \
+    if (mode == ST_RESID)                                                                                   \
+      k_stencil_resid<NP, RED_THREADS><<<nb, RED_THREADS, 0, s>>>(coef, d.N, d.M, d.K, x, b, y, partial);   \
+    else if (mode == ST_PROD)                                                                               \
+      k_stencil<NP, ST_PROD><<<cell_blocks(d), 256, 0, s>>>(coef, d.N, d.M, d.K, x, y);                     \
+    else                                                                                                    \
+      k_stencil<NP, ST_SUBR><<<cell_blocks(d), 256, 0, s>>>(coef, d.N, d.M, d.K, x, y);                     \
+  } while (0)
+  if (npts == 7)
+    LSX_ST(7);
+  else
+    LSX_ST(27);
 #undef LSX_ST
+}
+
+template <bool TR>
+static void stencil_sym_any(const double* s4, const SymExc& ex, Dims d, const double* x, const double* b, double* y,
+                            int mode, double* partial, hipStream_t s) {
+  if (mode == ST_RESID)
+    k_stencil_sym_resid<RED_THREADS, TR><<<reduction_blocks(d.n()), RED_THREADS, 0, s>>>(s4, d.N, d.M, d.K, ex, x, b,
+                                                                                         y, partial);
+  else if (mode == ST_PROD)
+    k_stencil_sym<ST_PROD, TR><<<cell_blocks(d), 256, 0, s>>>(s4, d.N, d.M, d.K, ex, x, y);
+  else
+    k_stencil_sym<ST_SUBR, TR><<<cell_blocks(d), 256, 0, s>>>(s4, d.N, d.M, d.K, ex, x, y);
 }
 
 void sym_check(const double* coef7, Dims d, unsigned char* exc, int* asym, hipStream_t s) {
@@ -1321,13 +1493,7 @@ void sym_build(const double* coef7, const unsigned char* exc, Dims d, double* s4
 
 void stencil_apply_sym(const double* s4, const SymExc& ex, Dims d, const double* x, const double* b, double* y,
                        int mode, double* partial, hipStream_t s) {
-  const int nb = reduction_blocks(d.n());
-  if (mode == ST_PROD)
-    k_stencil_sym<ST_PROD, RED_THREADS><<<nb, RED_THREADS, 0, s>>>(s4, d.N, d.M, d.K, ex, x, b, y, partial);
-  else if (mode == ST_RESID)
-    k_stencil_sym<ST_RESID, RED_THREADS><<<nb, RED_THREADS, 0, s>>>(s4, d.N, d.M, d.K, ex, x, b, y, partial);
-  else
-    k_stencil_sym<ST_SUBR, RED_THREADS><<<nb, RED_THREADS, 0, s>>>(s4, d.N, d.M, d.K, ex, x, b, y, partial);
+  stencil_sym_any<false>(s4, ex, d, x, b, y, mode, partial, s);
 }
 
 void restrict_full(const double* rf, Dims df, double* rc, Dims dc, hipStream_t s) {
@@ -1348,9 +1514,25 @@ void prolong_copy(const double* chc, Dims dc, double* chf, double* cf, Dims df, 
 
 void line_solve(const double* coef, int npts, Dims d, int dir, const double* dinv, const double* eu, const double* r,
                 double* c, double* ch, double omega, int z_head_fix, hipStream_t s) {
-  const int nlines = dir == 0 ? d.M * d.K : (dir == 1 ? d.N * d.K : d.N * d.M);
-  k_line_solve<<<div_up(nlines, 64), 64, 0, s>>>(coef, npts, d.N, d.M, d.K, dir, dinv, eu, r, c, ch, omega,
-                                                 z_head_fix);
+  const double* sb = coef + slot_sub(npts, dir) * d.n();
+  const int len = dir == 0 ? d.N : (dir == 1 ? d.M : d.K);
+  const int blocks = div_up(d.n() / len, LT);
+  // y in LDS while two workgroups and more share a CU's (lines of up to 5 LW cells)
+  const size_t tile = LT * (LW + 2) * sizeof(double), tiles = 3 * tile, lds = (2 + (len + LW - 1) / LW) * tile;
+#define LSX_LINE(DIR)                                                                                              \
+  do {                                                                                                             \
+    if (lds <= 65536)                                                                                              \
+      k_line_tile<DIR, false><<<blocks, 64, lds, s>>>(sb, d.N, d.M, d.K, dinv, eu, r, c, ch, omega, z_head_fix);   \
+    else                                                                                                           \
+      k_line_tile<DIR, true><<<blocks, 64, tiles, s>>>(sb, d.N, d.M, d.K, dinv, eu, r, c, ch, omega, z_head_fix);  \
+  } while (0)
+  if (dir == 0)
+    LSX_LINE(0);
+  else if (dir == 1)
+    LSX_LINE(1);
+  else
+    LSX_LINE(2);
+#undef LSX_LINE
 }
 
 void lu_solve(const double* scale, const int* perm, const double* L, const double* U, int n, const double* b,
@@ -1434,13 +1616,7 @@ void cgs_update_scaled(const double* V, long ldv, int cnt, const double* h, cons
 
 void stencil_apply_sym_t(const double* s4, const SymExc& ex, Dims d, const double* x, const double* b, double* y,
                          int mode, double* partial, hipStream_t s) {
-  const int nb = reduction_blocks(d.n());
-  if (mode == ST_PROD)
-    k_stencil_sym_t<ST_PROD, RED_THREADS><<<nb, RED_THREADS, 0, s>>>(s4, d.N, d.M, d.K, ex, x, b, y, partial);
-  else if (mode == ST_RESID)
-    k_stencil_sym_t<ST_RESID, RED_THREADS><<<nb, RED_THREADS, 0, s>>>(s4, d.N, d.M, d.K, ex, x, b, y, partial);
-  else
-    k_stencil_sym_t<ST_SUBR, RED_THREADS><<<nb, RED_THREADS, 0, s>>>(s4, d.N, d.M, d.K, ex, x, b, y, partial);
+  stencil_sym_any<true>(s4, ex, d, x, b, y, mode, partial, s);
 }
 
 void stencil_prod_sym_t_f32x(const double* s4, const SymExc& ex, Dims d, const float* x, double* y, hipStream_t s) {
