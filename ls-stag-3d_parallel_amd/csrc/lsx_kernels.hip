@@ -10,6 +10,7 @@
 
 #include "lsx_kernels.hpp"
 
+#include <algorithm>
 #include <cmath>
 
 namespace lsx {
@@ -105,45 +106,23 @@ __device__ inline int slot_diag(int npts) { return npts == 7 ? 3 : 13; }
 
 // Row i of the operator applied to x, accumulated in ascending column order (the CSR order
 // of the reference matrices: [b,s,w,p,e,n,t] on the fine level, sorted columns on Galerkin
-// levels).  acc starts at the given value; subtract: terms are subtracted.  Every load is issued
-// unconditionally (absent neighbours read a present cell) and absent terms leave the sum
-// unchanged, so the loads of a row are in flight together.
+// levels).  acc starts at the given value; subtract: terms are subtracted.  Straight-line code: an
+// absent neighbour, whose coefficient is stored as 0, reads the cell itself, so that all loads of
+// a row are in flight together (a branch per term would wait for each).
 template <int NPTS>
 __device__ inline double row_apply(const double* __restrict__ coef, long n, int i, int x, int y, int z, int N, int M,
                                    int K, const double* __restrict__ xv, double acc, bool subtract) {
-  const int NM = N * M;
-  if (NPTS == 7) {
-    const int off[7] = {-NM, -N, -1, 0, 1, N, NM};
-    const bool ok[7] = {z > 0, y > 0, x > 0, true, x < N - 1, y < M - 1, z < K - 1};
-    double a[7], v[7];
+  const int ox[3] = {x > 0 ? -1 : 0, 0, x < N - 1 ? 1 : 0};
+  const int oy[3] = {y > 0 ? -N : 0, 0, y < M - 1 ? N : 0}, oz[3] = {z > 0 ? -N * M : 0, 0, z < K - 1 ? N * M : 0};
+  double a[NPTS], v[NPTS];
 #pragma unroll
-    for (int q = 0; q < 7; ++q) {
-      a[q] = coef[q * n + i];
-      v[q] = xv[ok[q] ? i + off[q] : i];
-    }
-#pragma unroll
-    for (int q = 0; q < 7; ++q) {
-      const double t = a[q] * v[q];
-      const double s = subtract ? acc - t : acc + t;
-      acc = ok[q] ? s : acc;
-    }
-  } else {
-    const bool okx[3] = {x > 0, true, x < N - 1}, oky[3] = {y > 0, true, y < M - 1}, okz[3] = {z > 0, true, z < K - 1};
-    const int ox[3] = {okx[0] ? -1 : 0, 0, okx[2] ? 1 : 0}, oy[3] = {oky[0] ? -N : 0, 0, oky[2] ? N : 0};
-    const int oz[3] = {okz[0] ? -NM : 0, 0, okz[2] ? NM : 0};
-    double a[27], v[27];
-#pragma unroll
-    for (int q = 0; q < 27; ++q) {
-      a[q] = coef[q * n + i];
-      v[q] = xv[i + ox[q % 3] + oy[q / 3 % 3] + oz[q / 9]];
-    }
-#pragma unroll
-    for (int q = 0; q < 27; ++q) {
-      const double t = a[q] * v[q];
-      const double s = subtract ? acc - t : acc + t;
-      acc = okx[q % 3] && oky[q / 3 % 3] && okz[q / 9] ? s : acc;
-    }
+  for (int q = 0; q < NPTS; ++q) {
+    const int p = NPTS == 27 ? q : (const int[7]){4, 10, 12, 13, 14, 16, 22}[q];
+    a[q] = coef[q * n + i];
+    v[q] = xv[i + ox[p % 3] + oy[p / 3 % 3] + oz[p / 9]];
   }
+#pragma unroll
+  for (int q = 0; q < NPTS; ++q) acc = subtract ? acc - a[q] * v[q] : acc + a[q] * v[q];
   return acc;
 }
 
@@ -341,48 +320,121 @@ __global__ void k_galerkin_odd(const double* __restrict__ cf, int Nf, int Mf, in
   }
 }
 
-// r_c = R r_f on odd-odd-odd levels (R = P^T, fine cells in ascending order)
-__global__ void k_restrict_odd(const double* __restrict__ rf, int Nf, int Mf, int Kf, double* __restrict__ rc, int Nc,
-                               int Mc, int Kc) {
+// One coarse cell of r_c = R r_f and one fine cell of P ch_c; `at` reads a fine (coarse) cell (x, y, z).
+// Straight-line code: an absent tap reads a present cell with weight 0, which leaves the sum as it
+// is, so that all reads are in flight together.
+// Odd-odd-odd levels: R = P^T, fine cells in ascending order.
+template <class F>
+__device__ inline double restrict_cell_odd(F at, int X, int Y, int Z, int Nf, int Mf, int Kf) {
+  auto taps = [](int C, int nf, int (&f)[3], double (&w)[3]) {
+    f[0] = C > 0 ? 2 * C - 1 : 2 * C;
+    f[1] = 2 * C;
+    f[2] = 2 * C + 1 < nf ? 2 * C + 1 : 2 * C;
+    w[0] = C > 0 ? 0.5 : 0.0;
+    w[1] = 1.0;
+    w[2] = 2 * C + 1 < nf ? 0.5 : 0.0;
+  };
+  int fx[3], fy[3], fz[3];
+  double wx[3], wy[3], wz[3], v[27];
+  taps(X, Nf, fx, wx);
+  taps(Y, Mf, fy, wy);
+  taps(Z, Kf, fz, wz);
+#pragma unroll
+  for (int q = 0; q < 27; ++q) v[q] = at(fx[q % 3], fy[q / 3 % 3], fz[q / 9]);
+  double acc = 0.0;
+#pragma unroll
+  for (int q = 0; q < 27; ++q) acc = acc + wx[q % 3] * wy[q / 3 % 3] * wz[q / 9] * v[q];
+  return acc;
+}
+
+// sum of the 2 x 2 x 2 taps of a prolongation, z outermost, x innermost
+template <class F>
+__device__ inline double prolong_taps(F at, const int (&cx)[2], const int (&cy)[2], const int (&cz)[2],
+                                      const double (&wx)[2], const double (&wy)[2], const double (&wz)[2]) {
+  double v[8];
+#pragma unroll
+  for (int q = 0; q < 8; ++q) v[q] = at(cx[q & 1], cy[(q >> 1) & 1], cz[q >> 2]);
+  double acc = 0.0;
+#pragma unroll
+  for (int q = 0; q < 8; ++q) acc = acc + wx[q & 1] * wy[(q >> 1) & 1] * wz[q >> 2] * v[q];
+  return acc;
+}
+
+template <class F>
+__device__ inline double prolong_cell_odd(F at, int x, int y, int z) {
+  auto taps = [](int f, int (&c)[2], double (&w)[2]) {  // axis_w_odd
+    c[0] = f >> 1;
+    c[1] = (f + 1) >> 1;
+    w[0] = f & 1 ? 0.5 : 1.0;
+    w[1] = f & 1 ? 0.5 : 0.0;
+  };
+  int cx[2], cy[2], cz[2];
+  double wx[2], wy[2], wz[2];
+  taps(x, cx, wx);
+  taps(y, cy, wy);
+  taps(z, cz, wz);
+  return prolong_taps(at, cx, cy, cz, wx, wy, wz);
+}
+
+// even-even-even levels: 1/8 of each child in R's row order a,b,c,d,aa,bb,cc,dd; trilinear P
+template <class F>
+__device__ inline double restrict_cell(F at, int X, int Y, int Z) {
+  double acc = 0.0;
+#pragma unroll
+  for (int q = 0; q < 8; ++q) acc = acc + 0.125 * at(2 * X + (q & 1), 2 * Y + ((q >> 1) & 1), 2 * Z + (q >> 2));
+  return acc;
+}
+
+template <class F>
+__device__ inline double prolong_cell(F at, int x, int y, int z, int Nf, int Mf, int Kf) {
+  auto taps = [](int f, int nf, int (&c)[2], double (&w)[2]) {  // axis_w
+    const int p = f >> 1;
+    const bool end = f == 0 || f == nf - 1;
+    c[0] = end || (f & 1) ? p : p - 1;
+    c[1] = end ? p : c[0] + 1;
+    w[0] = end ? 1.0 : (f & 1 ? 0.75 : 0.25);
+    w[1] = end ? 0.0 : (f & 1 ? 0.25 : 0.75);
+  };
+  int cx[2], cy[2], cz[2];
+  double wx[2], wy[2], wz[2];
+  taps(x, Nf, cx, wx);
+  taps(y, Mf, cy, wy);
+  taps(z, Kf, cz, wz);
+  return prolong_taps(at, cx, cy, cz, wx, wy, wz);
+}
+
+// r_c = R r_f (ODD: odd-odd-odd level)
+template <bool ODD>
+__global__ void k_restrict(const double* __restrict__ rf, int Nf, int Mf, int Kf, double* __restrict__ rc, int Nc,
+                           int Mc, int Kc) {
   const long nc = (long)Nc * Mc * Kc;
   const int NMf = Nf * Mf;
+  auto at = [&](int x, int y, int z) { return rf[x + Nf * y + NMf * z]; };
   for (long li = blockIdx.x * (long)blockDim.x + threadIdx.x; li < nc; li += (long)gridDim.x * blockDim.x) {
     int X, Y, Z;
     decode((int)li, Nc, Mc, &X, &Y, &Z);
-    int rx[3], ry[3], rz[3];
-    double wx[3], wy[3], wz[3];
-    const int nx = axis_r_odd(X, Nf, rx, wx), ny = axis_r_odd(Y, Mf, ry, wy), nz = axis_r_odd(Z, Kf, rz, wz);
-    double acc = 0.0;
-    for (int c3 = 0; c3 < nz; ++c3)
-      for (int c2 = 0; c2 < ny; ++c2)
-        for (int c1 = 0; c1 < nx; ++c1) {
-          const double w = wx[c1] * wy[c2] * wz[c3];
-          acc = acc + w * rf[rx[c1] + Nf * ry[c2] + NMf * rz[c3]];
-        }
-    rc[li] = acc;
+    if constexpr (ODD)
+      rc[li] = restrict_cell_odd(at, X, Y, Z, Nf, Mf, Kf);
+    else
+      rc[li] = restrict_cell(at, X, Y, Z);
   }
 }
 
-// ch_f = P ch_c, c_f = ch_f on odd-odd-odd levels
-__global__ void k_prolong_odd(const double* __restrict__ chc, int Nc, int Mc, double* __restrict__ chf,
-                              double* __restrict__ cf, int Nf, int Mf, int Kf) {
+// ch_f = P ch_c, c_f = ch_f (ODD: odd-odd-odd level)
+template <bool ODD>
+__global__ void k_prolong(const double* __restrict__ chc, int Nc, int Mc, double* __restrict__ chf,
+                          double* __restrict__ cf, int Nf, int Mf, int Kf) {
   const long nf = (long)Nf * Mf * Kf;
   const int NMc = Nc * Mc;
+  auto at = [&](int x, int y, int z) { return chc[x + Nc * y + NMc * z]; };
   for (long li = blockIdx.x * (long)blockDim.x + threadIdx.x; li < nf; li += (long)gridDim.x * blockDim.x) {
     int x, y, z;
     decode((int)li, Nf, Mf, &x, &y, &z);
-    int cx[2], cy[2], cz[2], nx, ny, nz;
-    double wx[2], wy[2], wz[2];
-    axis_w_odd(x, cx, wx, &nx);
-    axis_w_odd(y, cy, wy, &ny);
-    axis_w_odd(z, cz, wz, &nz);
-    double acc = 0.0;
-    for (int c3 = 0; c3 < nz; ++c3)
-      for (int c2 = 0; c2 < ny; ++c2)
-        for (int c1 = 0; c1 < nx; ++c1) {
-          const double w = wx[c1] * wy[c2] * wz[c3];
-          acc = acc + w * chc[cx[c1] + Nc * cy[c2] + NMc * cz[c3]];
-        }
+    double acc;
+    if constexpr (ODD)
+      acc = prolong_cell_odd(at, x, y, z);
+    else
+      acc = prolong_cell(at, x, y, z, Nf, Mf, Kf);
     chf[li] = acc;
     cf[li] = acc;
   }
@@ -772,53 +824,6 @@ __global__ void k_stencil_resid(const double* __restrict__ coef, int N, int M, i
   if (threadIdx.x == 0) partial[blockIdx.x] = ss;
 }
 
-// r_c = R r_f: each coarse cell sums 1/8 of its 8 children (R row order a,b,c,d,aa,bb,cc,dd)
-__global__ void k_restrict(const double* __restrict__ rf, int Nf, int Mf, double* __restrict__ rc, int Nc, int Mc,
-                           int Kc) {
-  const long nc = (long)Nc * Mc * Kc;
-  const int NMf = Nf * Mf;
-  for (long li = blockIdx.x * (long)blockDim.x + threadIdx.x; li < nc; li += (long)gridDim.x * blockDim.x) {
-    int X, Y, Z;
-    decode((int)li, Nc, Mc, &X, &Y, &Z);
-    const int a = 2 * X + Nf * 2 * Y + NMf * 2 * Z;
-    double acc = 0.0;
-    acc = acc + 0.125 * rf[a];
-    acc = acc + 0.125 * rf[a + 1];
-    acc = acc + 0.125 * rf[a + Nf];
-    acc = acc + 0.125 * rf[a + Nf + 1];
-    acc = acc + 0.125 * rf[a + NMf];
-    acc = acc + 0.125 * rf[a + NMf + 1];
-    acc = acc + 0.125 * rf[a + NMf + Nf];
-    acc = acc + 0.125 * rf[a + NMf + Nf + 1];
-    rc[li] = acc;
-  }
-}
-
-// ch_f = P ch_c (trilinear), c_f = ch_f
-__global__ void k_prolong(const double* __restrict__ chc, int Nc, int Mc, double* __restrict__ chf,
-                          double* __restrict__ cf, int Nf, int Mf, int Kf) {
-  const long nf = (long)Nf * Mf * Kf;
-  const int NMc = Nc * Mc;
-  for (long li = blockIdx.x * (long)blockDim.x + threadIdx.x; li < nf; li += (long)gridDim.x * blockDim.x) {
-    int x, y, z;
-    decode((int)li, Nf, Mf, &x, &y, &z);
-    int cx[2], cy[2], cz[2], nx, ny, nz;
-    double wx[2], wy[2], wz[2];
-    axis_w(x, Nf, cx, wx, &nx);
-    axis_w(y, Mf, cy, wy, &ny);
-    axis_w(z, Kf, cz, wz, &nz);
-    double acc = 0.0;
-    for (int c3 = 0; c3 < nz; ++c3)
-      for (int c2 = 0; c2 < ny; ++c2)
-        for (int c1 = 0; c1 < nx; ++c1) {
-          const double w = wx[c1] * wy[c2] * wz[c3];
-          acc = acc + w * chc[cx[c1] + Nc * cy[c2] + NMc * cz[c3]];
-        }
-    chf[li] = acc;
-    cf[li] = acc;
-  }
-}
-
 // c = omega * T_dir^{-1} r ; ch += c (smoother_adlj_interface.h:73-82 with the TDMA kernels
 // smoother_adlj_x.h:38-48, smoother_adlj_y.h:36-50).  One thread per line, the Thomas steps in the
 // reference's order.  For z lines the reference reads the first right-hand-side element at index
@@ -1006,39 +1011,289 @@ __global__ void __launch_bounds__(64) k_line_tile(const double* __restrict__ sb,
 }
 
 // lu_decomposition_sparse_matrix.h:216-259 + decomposition_sparse_matrix_interface.h:43-71.
-// The factors (n <= 64) and the right-hand side are staged in LDS by the whole workgroup; thread 0
-// then runs the triangular solves on LDS operands (the same operations in the same order).
+// The factors (n <= 64) and the right-hand side are staged in LDS by the whole workgroup; one
+// wavefront then substitutes, a row to a lane.  Every row's operations keep the reference's order:
+// forward the finished unknowns are subtracted as they come, backward a row's products are formed
+// by all lanes at once and subtracted one after the other.
+struct LuLds {
+  double *L, *U, *scale, *rhs;
+  int* perm;
+};
+// doubles of LDS that lu_lds takes
+__host__ __device__ constexpr int lu_lds_size(int n) { return 2 * n * n + 3 * n; }
+__device__ inline LuLds lu_lds(double* p, int n) {
+  return LuLds{p, p + n * n, p + 2 * n * n, p + 2 * n * n + n, reinterpret_cast<int*>(p + 2 * n * n + 2 * n)};
+}
+__device__ inline void lu_stage(const LuLds& q, int n, const double* __restrict__ scale, const int* __restrict__ perm,
+                                const double* __restrict__ L, const double* __restrict__ U) {
+  for (int k = threadIdx.x; k < n * n; k += blockDim.x) {
+    q.L[k] = L[k];
+    q.U[k] = U[k];
+  }
+  for (int k = threadIdx.x; k < n; k += blockDim.x) {
+    q.scale[k] = scale[k];
+    q.perm[k] = perm[k];
+  }
+}
+// the value of lane j (uniform j)
+__device__ inline double lane_value(double v, int j) {
+  const unsigned long long u = __double_as_longlong(v);
+  const unsigned lo = __builtin_amdgcn_readlane((unsigned)u, j), hi = __builtin_amdgcn_readlane((unsigned)(u >> 32), j);
+  return __longlong_as_double((long long)(((unsigned long long)hi << 32) | lo));
+}
+// x into q.rhs (the first wavefront of the workgroup)
+__device__ inline void lu_substitute(const LuLds& q, int n) {
+  const int lane = threadIdx.x, row = lane < n ? lane : n - 1;
+  double y = q.scale[q.perm[row]] * q.rhs[q.perm[row]];
+  for (int t = 0; t < n; ++t) {
+    const double s = y - q.L[row * n + t] * lane_value(y, t);
+    y = lane > t ? s : y;
+  }
+  double b = 0.0;
+  for (int i = n - 1; i >= 0; --i) {
+    const double p = q.U[i * n + row] * b;
+    double aux = lane_value(y, i);
+    for (int j = i + 1; j < n; ++j) aux -= lane_value(p, j);
+    aux = aux / q.U[i * n + i];
+    b = lane == i ? aux : b;
+  }
+  if (lane < n) q.rhs[lane] = q.scale[lane] * b;
+}
+
 constexpr int LU_SOLVE_THREADS = 256;
 __global__ void __launch_bounds__(LU_SOLVE_THREADS) k_lu_solve(const double* scale, const int* perm,
                                                                const double* L, const double* U, int n,
                                                                const double* __restrict__ b, double* __restrict__ x) {
-  __shared__ double sL[64 * 64], sU[64 * 64], ssc[64], sb[64], slu_b[64], slu_y[64];
-  __shared__ int sp[64];
-  for (int k = threadIdx.x; k < n * n; k += blockDim.x) {
-    sL[k] = L[k];
-    sU[k] = U[k];
+  __shared__ double lds[lu_lds_size(64)];
+  const LuLds q = lu_lds(lds, n);
+  lu_stage(q, n, scale, perm, L, U);
+  for (int k = threadIdx.x; k < n; k += blockDim.x) q.rhs[k] = b[k];
+  __syncthreads();
+  if (threadIdx.x < 64) lu_substitute(q, n);
+  __syncthreads();
+  for (int k = threadIdx.x; k < n; k += blockDim.x) x[k] = q.rhs[k];
+}
+
+// ---- the cascade's small levels in one workgroup -----------------------------------------------
+// A level of a few thousand cells is nothing but latency: its 9 products and 9 line solves per
+// application took 18 launches of 3 to 6 us, whatever its size.  One workgroup runs all small levels
+// (the last one the LU level): the right-hand sides of every level and the current correction in
+// LDS, each thread's part of ch and its one row of a 27-point operator in registers for all sweeps of
+// a level, barriers for launches.  Operations and orders are those of the per-level kernels
+// (k_stencil, k_line_tile, k_restrict, k_prolong, k_lu_solve).  A 7-point level may have 4096 cells
+// and a 27-point level 1024; a 16^3 27-point level would stream 0.9 MB of coefficients through one CU
+// for every sweep (5.8 us at 64 bytes a cycle, no less than its two launches) and stays outside.
+// Measured: 8^3, 4^3 and the LU 38 us (45 launches: 190 us); with a 16^3 7-point level 104 us (7.3 us
+// a sweep, of which the coefficients' and factors' way from L2 takes about half).
+constexpr int CS_THREADS = 512, CS_CELLS = 8, CS_LEN = 17;
+constexpr int CS_LDS = 18432;  // doubles: 144 KB of the CU's 160
+
+// rows of a level in LDS: x fastest with an odd pitch (x lines: adjacent lanes hold adjacent rows)
+struct CsGrid {
+  int N, M, K, P;
+  __device__ CsGrid(Dims d) : N(d.N), M(d.M), K(d.K), P(d.N | 1) {}
+  __device__ int at(int x, int y, int z) const { return x + P * (y + M * z); }
+};
+
+// element i of p by a 32-bit byte offset from a uniform base: one address register a load
+__device__ inline double ld32(const double* __restrict__ p, unsigned i) {
+  return *reinterpret_cast<const double*>(reinterpret_cast<const char*>(p) + i * 8u);
+}
+
+// all sweeps of one level of axes of at most ML cells: c holds the prolonged correction (every
+// cell), chv each thread's own
+template <int NP, int CELLS, int ML>
+__device__ inline void cs_sweeps(const CascadeLevel& L, int n_post, double omega, int z_head_fix, double* __restrict__ r,
+                                 double* __restrict__ c, double (&chv)[CS_CELLS]) {
+  const CsGrid g(L.d);
+  const int n = g.N * g.M * g.K, tid = threadIdx.x;
+  // a thread's one 27-point row stays in registers for all sweeps; several rows are read again by
+  // each sweep, HELD at a time: with the lines' factors they would spill
+  constexpr bool KEEP = CELLS == 1;
+  constexpr int HELD = NP == 27 ? 1 : 2;
+  double a[HELD][NP];
+  unsigned shift = 0;
+  auto rows = [&](int j0) {
+#pragma unroll
+    for (int j = 0; j < HELD; ++j)
+      if (tid + CS_THREADS * (j0 + j) < n)
+#pragma unroll
+        for (int q = 0; q < NP; ++q) a[j][q] = ld32(L.coef + q * n, shift + tid + CS_THREADS * (j0 + j));
+  };
+  if (KEEP) rows(0);
+  int own[CELLS];
+  unsigned okm[CELLS];  // axis neighbours present: bit 0/1 x -/+, 2/3 y, 4/5 z
+#pragma unroll
+  for (int j = 0; j < CELLS; ++j) {
+    const int i = tid + CS_THREADS * j;
+    own[j] = 0;
+    okm[j] = 0;
+    if (i >= n) continue;
+    int x, y, z;
+    decode(i, g.N, g.M, &x, &y, &z);
+    own[j] = g.at(x, y, z);
+    okm[j] = (x > 0) | (x < g.N - 1) << 1 | (y > 0) << 2 | (y < g.M - 1) << 3 | (z > 0) << 4 | (z < g.K - 1) << 5;
   }
-  for (int k = threadIdx.x; k < n; k += blockDim.x) {
-    ssc[k] = scale[k];
-    sp[k] = perm[k];
-    sb[k] = b[k];
+  const int sy = g.P, sz = g.P * g.M;
+  for (int s = 0; s < n_post; ++s)
+#pragma unroll 1
+    for (int dir = 2; dir >= 0; --dir) {  // z, y, x
+      // one thread per line; its couplings and pivots are on their way while the product runs
+      const int len = dir == 0 ? g.N : (dir == 1 ? g.M : g.K);
+      const int stg = dir == 0 ? n / len : (dir == 1 ? g.N : g.N * g.M), stl = dir == 0 ? 1 : (dir == 1 ? sy : sz);
+      const bool line = tid < n / len;
+      const int p = dir == 0 ? 0 : tid % g.N, q = dir == 0 ? tid : tid / g.N;
+      const int g0 = dir == 1 ? p + g.N * g.M * q : tid;  // x lines: of the transposed factors
+      const int l0 = dir == 0 ? g.P * q : (dir == 1 ? p + sz * q : p + sy * q);
+      double fs[ML], fd[ML];
+      if (line) {
+        const double* sb = dir == 0 ? L.xt : L.coef + slot_sub(NP, dir) * n;
+        const double* di = dir == 0 ? L.xt + n : L.dinv[dir];
+#pragma unroll
+        for (int u = 0; u < ML; ++u) {
+          const int k = u < len ? u : len - 1;
+          fs[u] = ld32(sb, g0 + stg * k);
+          fd[u] = ld32(di, g0 + stg * k);
+        }
+      }
+      // r -= A c.  The empty asm statements hide that a sweep's addresses are the last one's: kept
+      // over the sweeps instead of computed again, they spill
+      if (!KEEP) asm volatile("" : "+s"(shift));
+#pragma unroll
+      for (int j = 0; j < CELLS; ++j) {
+        if (!KEEP && j % HELD == 0) rows(j);
+        if (tid + CS_THREADS * j >= n) continue;
+        // straight-line as row_apply: an absent neighbour has coefficient 0 and reads the cell itself
+        int o = own[j];
+        unsigned m = okm[j];
+        asm volatile("" : "+v"(o), "+v"(m));
+        const int ox[3] = {m & 1 ? -1 : 0, 0, m & 2 ? 1 : 0}, oy[3] = {m & 4 ? -sy : 0, 0, m & 8 ? sy : 0};
+        const int oz[3] = {m & 16 ? -sz : 0, 0, m & 32 ? sz : 0};
+        double acc = 0.0, v[NP];
+#pragma unroll
+        for (int q = 0; q < NP; ++q) {
+          const int p = NP == 27 ? q : (const int[7]){4, 10, 12, 13, 14, 16, 22}[q];
+          v[q] = c[o + ox[p % 3] + oy[p / 3 % 3] + oz[p / 9]];
+        }
+#pragma unroll
+        for (int q = 0; q < NP; ++q) acc = acc + a[j % HELD][q] * v[q];
+        r[o] = r[o] - acc;
+      }
+      __syncthreads();
+      // c = omega T^-1 r
+      if (line) {
+        const double* eu = dir == 0 ? L.xt + 2 * n : L.eu[dir];
+        double fe[ML], v[ML];
+#pragma unroll
+        for (int u = 0; u < ML; ++u) {
+          const int k = u < len ? u : len - 1;
+          v[u] = r[l0 + stl * k];
+          fe[u] = ld32(eu, g0 + stg * k);
+        }
+        if (dir == 2 && !z_head_fix) {
+          int hx, hy, hz;
+          decode(q * g.N * g.K + p, g.N, g.M, &hx, &hy, &hz);
+          v[0] = r[g.at(hx, hy, hz)];
+        }
+        v[0] = v[0] * fd[0];
+#pragma unroll
+        for (int u = 1; u < ML; ++u)
+          if (u < len) v[u] = (v[u] - fs[u] * v[u - 1]) * fd[u];  // uniform branch
+        double xnext = 0.0;
+#pragma unroll
+        for (int u = ML - 1; u >= 0; --u)
+          if (u < len) {
+            xnext = v[u] - fe[u] * xnext;
+            c[l0 + stl * u] = xnext * omega;
+          }
+      }
+      __syncthreads();
+#pragma unroll
+      for (int j = 0; j < CELLS; ++j)
+        if (tid + CS_THREADS * j < n) chv[j] = chv[j] + c[own[j]];
+    }
+}
+
+// xt: a level's x couplings, dinv and eu with the line index fastest, so that the threads of
+// k_cascade_small, one per x line, load adjacent values (set-up)
+__global__ void k_x_factors_t(const double* __restrict__ sb, const double* __restrict__ dinv,
+                              const double* __restrict__ eu, int N, int nl, double* __restrict__ xt) {
+  const int i = blockIdx.x * blockDim.x + threadIdx.x, n = N * nl;
+  if (i >= n) return;
+  const int j = i / nl + N * (i % nl);
+  xt[i] = sb[j];
+  xt[n + i] = dinv[j];
+  xt[2 * n + i] = eu[j];
+}
+
+__global__ void __launch_bounds__(CS_THREADS) k_cascade_small(CascadeLevels C, int n_post, double omega, int z_head_fix,
+                                                              const double* __restrict__ lu_scale,
+                                                              const int* __restrict__ lu_perm,
+                                                              const double* __restrict__ Lf,
+                                                              const double* __restrict__ Uf,
+                                                              const double* __restrict__ r0, double* __restrict__ ch0) {
+  __shared__ double lds[CS_LDS];
+  const int tid = threadIdx.x, last = C.count - 1;
+  // r of every level, then c (the largest level's size), then ch of the level below, then the LU
+  double* c = lds + C.off[last + 1];
+  double* chl = c + C.c_size;
+  const int n_last = (int)C.L[last].d.n();
+  const LuLds lu = lu_lds(chl + C.ch_size, n_last);
+  lu_stage(lu, n_last, lu_scale, lu_perm, Lf, Uf);
+  {
+    const CsGrid g(C.L[0].d);
+    const int n = g.N * g.M * g.K;
+    for (int i = tid; i < n; i += CS_THREADS) {
+      int x, y, z;
+      decode(i, g.N, g.M, &x, &y, &z);
+      lds[g.at(x, y, z)] = r0[i];
+    }
   }
   __syncthreads();
-  if (blockIdx.x != 0 || threadIdx.x != 0) return;
-  double* bs = slu_b;  // LDS: as local arrays they would live in scratch memory
-  double* yv = slu_y;
-  for (int i = 0; i < n; ++i) bs[i] = ssc[sp[i]] * sb[sp[i]];
-  for (int i = 0; i < n; ++i) {
-    double aux = bs[i];
-    for (int t = 0; t < i; ++t) aux -= sL[i * n + t] * yv[t];
-    yv[i] = aux;
+  for (int q = 0; q < last; ++q) {
+    const CsGrid f(C.L[q].d), g(C.L[q + 1].d);
+    const double* rf = lds + C.off[q];
+    double* rc = q + 1 == last ? lu.rhs : lds + C.off[q + 1];
+    auto at = [&](int x, int y, int z) { return rf[f.at(x, y, z)]; };
+    for (int i = tid; i < g.N * g.M * g.K; i += CS_THREADS) {
+      int X, Y, Z;
+      decode(i, g.N, g.M, &X, &Y, &Z);
+      const double v = f.N & 1 ? restrict_cell_odd(at, X, Y, Z, f.N, f.M, f.K) : restrict_cell(at, X, Y, Z);
+      rc[q + 1 == last ? i : g.at(X, Y, Z)] = v;
+    }
+    __syncthreads();
   }
-  for (int i = n - 1; i >= 0; --i) {
-    double aux = yv[i];
-    for (int j = i + 1; j < n; ++j) aux -= sU[i * n + j] * bs[j];
-    bs[i] = aux / sU[i * n + i];
+  if (tid < 64) lu_substitute(lu, n_last);
+  __syncthreads();
+  for (int q = last - 1; q >= 0; --q) {
+    const CsGrid f(C.L[q].d), g(C.L[q + 1].d);
+    const int n = f.N * f.M * f.K;
+    const double* chc = q + 1 == last ? lu.rhs : chl;
+    auto at = [&](int x, int y, int z) { return chc[x + g.N * (y + g.M * z)]; };
+    double chv[CS_CELLS];
+#pragma unroll
+    for (int j = 0; j < CS_CELLS; ++j) {
+      const int i = tid + CS_THREADS * j;
+      chv[j] = 0.0;
+      if (i >= n) continue;
+      int x, y, z;
+      decode(i, f.N, f.M, &x, &y, &z);
+      chv[j] = f.N & 1 ? prolong_cell_odd(at, x, y, z) : prolong_cell(at, x, y, z, f.N, f.M, f.K);
+      c[f.at(x, y, z)] = chv[j];
+    }
+    __syncthreads();
+    if (C.L[q].npts == 7)
+      cs_sweeps<7, CS_CELLS, CS_LEN>(C.L[q], n_post, omega, z_head_fix, lds + C.off[q], c, chv);
+    else if (n > CS_THREADS || max(f.N, max(f.M, f.K)) > 9)
+      cs_sweeps<27, CS_CELLS / 4, CS_LEN>(C.L[q], n_post, omega, z_head_fix, lds + C.off[q], c, chv);
+    else
+      cs_sweeps<27, 1, 9>(C.L[q], n_post, omega, z_head_fix, lds + C.off[q], c, chv);
+    double* out = q == 0 ? ch0 : chl;
+#pragma unroll
+    for (int j = 0; j < CS_CELLS; ++j)
+      if (tid + CS_THREADS * j < n) out[tid + CS_THREADS * j] = chv[j];
+    __syncthreads();
   }
-  for (int i = 0; i < n; ++i) x[i] = ssc[i] * bs[i];
 }
 
 // ---- kernels: BLAS-1 ---------------------------------------------------------------------------
@@ -1497,19 +1752,17 @@ void stencil_apply_sym(const double* s4, const SymExc& ex, Dims d, const double*
 }
 
 void restrict_full(const double* rf, Dims df, double* rc, Dims dc, hipStream_t s) {
-  if (df.N & 1) {
-    k_restrict_odd<<<grid_1d(dc.n()), 256, 0, s>>>(rf, df.N, df.M, df.K, rc, dc.N, dc.M, dc.K);
-    return;
-  }
-  k_restrict<<<grid_1d(dc.n()), 256, 0, s>>>(rf, df.N, df.M, rc, dc.N, dc.M, dc.K);
+  if (df.N & 1)
+    k_restrict<true><<<grid_1d(dc.n()), 256, 0, s>>>(rf, df.N, df.M, df.K, rc, dc.N, dc.M, dc.K);
+  else
+    k_restrict<false><<<grid_1d(dc.n()), 256, 0, s>>>(rf, df.N, df.M, df.K, rc, dc.N, dc.M, dc.K);
 }
 
 void prolong_copy(const double* chc, Dims dc, double* chf, double* cf, Dims df, hipStream_t s) {
-  if (df.N & 1) {
-    k_prolong_odd<<<grid_1d(df.n()), 256, 0, s>>>(chc, dc.N, dc.M, chf, cf, df.N, df.M, df.K);
-    return;
-  }
-  k_prolong<<<grid_1d(df.n()), 256, 0, s>>>(chc, dc.N, dc.M, chf, cf, df.N, df.M, df.K);
+  if (df.N & 1)
+    k_prolong<true><<<grid_1d(df.n()), 256, 0, s>>>(chc, dc.N, dc.M, chf, cf, df.N, df.M, df.K);
+  else
+    k_prolong<false><<<grid_1d(df.n()), 256, 0, s>>>(chc, dc.N, dc.M, chf, cf, df.N, df.M, df.K);
 }
 
 void line_solve(const double* coef, int npts, Dims d, int dir, const double* dinv, const double* eu, const double* r,
@@ -1538,6 +1791,38 @@ void line_solve(const double* coef, int npts, Dims d, int dir, const double* din
 void lu_solve(const double* scale, const int* perm, const double* L, const double* U, int n, const double* b,
               double* x, hipStream_t s) {
   k_lu_solve<<<1, LU_SOLVE_THREADS, 0, s>>>(scale, perm, L, U, n, b, x);
+}
+
+bool cascade_small_fits(CascadeLevels& C) {
+  if (C.count < 2 || C.count > CascadeLevels::MAX) return false;
+  auto pitched = [](Dims d) { return (d.N | 1) * d.M * d.K; };
+  const long n_last = C.L[C.count - 1].d.n();
+  C.off[0] = 0;
+  C.c_size = 0;
+  C.ch_size = 0;
+  long total = 0;
+  for (int q = 0; q < C.count; ++q) {
+    const long n = C.L[q].d.n();
+    if (n > (C.L[q].npts == 7 ? CS_CELLS : CS_CELLS / 4) * CS_THREADS) return false;
+    if (q + 1 < C.count && std::max(C.L[q].d.N, std::max(C.L[q].d.M, C.L[q].d.K)) > CS_LEN) return false;
+    if (q + 1 < C.count) {
+      total += pitched(C.L[q].d);
+      C.c_size = std::max(C.c_size, pitched(C.L[q].d));
+      if (q > 0) C.ch_size = std::max(C.ch_size, (int)n);
+    }
+    C.off[q + 1] = (int)total;
+  }
+  return n_last <= 64 && total + C.c_size + C.ch_size + lu_lds_size((int)n_last) <= CS_LDS;
+}
+
+void x_factors_t(const double* coef, int npts, Dims d, const double* dinv, const double* eu, double* xt,
+                 hipStream_t s) {
+  k_x_factors_t<<<div_up(d.n(), 256), 256, 0, s>>>(coef + slot_sub(npts, 0) * d.n(), dinv, eu, d.N, d.M * d.K, xt);
+}
+
+void cascade_small(const CascadeLevels& C, int n_post, double omega, int z_head_fix, const double* lu_scale,
+                   const int* lu_perm, const double* L, const double* U, const double* r, double* ch, hipStream_t s) {
+  k_cascade_small<<<1, CS_THREADS, 0, s>>>(C, n_post, omega, z_head_fix, lu_scale, lu_perm, L, U, r, ch);
 }
 
 void copy(const double* a, double* b, long n, hipStream_t s) { k_copy<<<grid_1d(n), 256, 0, s>>>(a, b, n); }

@@ -71,6 +71,29 @@ void line_solve(const double* coef, int npts, Dims d, int dir, const double* din
 void lu_solve(const double* scale, const int* perm, const double* L, const double* U, int n, const double* b,
               double* x, hipStream_t s);
 
+// The small levels of the cascade in one launch: C.L[0] the first of them, the last the LU level.
+// cascade_small_fits sets the LDS offsets and says whether the levels fit one workgroup (a 7-point
+// level of at most 4096 cells, 27-point levels of at most 1024, axes of at most 17); cascade_small takes the
+// right-hand side of level C.L[0] and writes its correction.
+struct CascadeLevel {
+  Dims d;
+  int npts;
+  const double* coef;
+  const double *dinv[3], *eu[3];
+  const double* xt;  // x couplings, dinv[0] and eu[0] with the line index fastest (x_factors_t)
+};
+struct CascadeLevels {
+  static constexpr int MAX = 12;
+  int count = 0, c_size = 0, ch_size = 0;
+  int off[MAX + 1] = {};
+  CascadeLevel L[MAX] = {};
+};
+void x_factors_t(const double* coef, int npts, Dims d, const double* dinv, const double* eu, double* xt,
+                 hipStream_t s);
+bool cascade_small_fits(CascadeLevels& C);
+void cascade_small(const CascadeLevels& C, int n_post, double omega, int z_head_fix, const double* lu_scale,
+                   const int* lu_perm, const double* L, const double* U, const double* r, double* ch, hipStream_t s);
+
 // ---- BLAS-1 (FP64) ------------------------------------------------------------------------
 void copy(const double* a, double* b, long n, hipStream_t s);
 void fill_zero(double* b, long n, hipStream_t s);  // a kernel, not a memset: safe under graph capture

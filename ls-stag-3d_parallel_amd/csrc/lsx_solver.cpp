@@ -409,6 +409,7 @@ void Solver::build_hierarchy() {
     MGLevel& C = levels.back();
     lu_factor(C.coef.p, C.d, lu_scale.p, lu_perm.p, lu_L.p, lu_U.p, lu_col.p, stream);
   }
+  find_small_levels();
   LSX_HIP(hipGetLastError());
   LSX_HIP(hipStreamSynchronize(stream));
 }
@@ -968,11 +969,23 @@ void Solver::fine_apply(const double* x, const double* b, double* y, int mode) {
 // -----------------------------------------------------------------------------------------------
 void Solver::mg_apply(const double* v, double* z) {
   const int L = (int)levels.size() - 1;
-  copy(v, levels[0].r.p, d0.n(), stream);
-  for (int k = 0; k < L; ++k) restrict_full(levels[k].r.p, levels[k].d, levels[k + 1].r.p, levels[k + 1].d, stream);
-  if (L > 0)
-    lu_solve(lu_scale.p, lu_perm.p, lu_L.p, lu_U.p, (int)levels[L].d.n(), levels[L].r.p, levels[L].ch.p, stream);
-  for (int k = L > 0 ? L - 1 : 0; k >= 0; --k) {
+  // levels from `lc` down run in one launch (per-kernel timing wants the launches one by one)
+  const int lc = timing ? L : small_from;
+  const double* r = v;
+  if (lc > 0 || L == 0) {
+    copy(v, levels[0].r.p, d0.n(), stream);
+    r = levels[0].r.p;
+  }
+  for (int k = 0; k < lc; ++k) {
+    restrict_full(levels[k].r.p, levels[k].d, levels[k + 1].r.p, levels[k + 1].d, stream);
+    r = levels[k + 1].r.p;
+  }
+  if (lc < L)
+    cascade_small(small_lv, opt.n_post, opt.omega, opt.z_head_fix, lu_scale.p, lu_perm.p, lu_L.p, lu_U.p, r,
+                  lc == 0 ? z : levels[lc].ch.p, stream);
+  else if (L > 0)
+    lu_solve(lu_scale.p, lu_perm.p, lu_L.p, lu_U.p, (int)levels[L].d.n(), r, levels[L].ch.p, stream);
+  for (int k = L > 0 ? lc - 1 : 0; k >= 0; --k) {
     MGLevel& lv = levels[k];
     double* ch = k == 0 ? z : lv.ch.p;
     if (L > 0) {
@@ -997,6 +1010,38 @@ void Solver::mg_apply(const double* v, double* z) {
                    opt.z_head_fix, stream);
         if (k == 0) tend(LSX_K_LINE_X + dir, e0);
       }
+  }
+}
+
+// the first level from which all levels fit one workgroup, the last level if there is none
+void Solver::find_small_levels() {
+  const int L = (int)levels.size() - 1;
+  for (small_from = 0; small_from < L; ++small_from) {
+    small_lv = CascadeLevels{};
+    if (L - small_from + 1 > CascadeLevels::MAX) continue;
+    for (int k = small_from; k <= L; ++k) {
+      CascadeLevel& q = small_lv.L[small_lv.count++];
+      const MGLevel& lv = levels[k];
+      q.d = lv.d;
+      q.npts = lv.npts;
+      q.coef = lv.coef.p;
+      for (int dir = 0; dir < 3; ++dir) {
+        q.dinv[dir] = lv.dinv[dir].p;
+        q.eu[dir] = lv.eu[dir].p;
+      }
+    }
+    if (!cascade_small_fits(small_lv)) continue;
+    long total = 0;
+    for (int k = small_from; k < L; ++k) total += 3 * levels[k].d.n();
+    small_xt.alloc(total);
+    double* xt = small_xt.p;
+    for (int k = small_from; k < L; ++k) {
+      const MGLevel& lv = levels[k];
+      x_factors_t(lv.coef.p, lv.npts, lv.d, lv.dinv[0].p, lv.eu[0].p, xt, stream);
+      small_lv.L[k - small_from].xt = xt;
+      xt += 3 * lv.d.n();
+    }
+    return;
   }
 }
 

@@ -133,6 +133,12 @@ class Solver {
   int src_pin = -1;
   void alloc_krylov();
   void mg_apply(const double* v_dev, double* z_dev);
+  // cascade levels small_from .. last, which one workgroup runs in one launch (small_from the last
+  // level: none)
+  CascadeLevels small_lv;
+  DevBuf<double> small_xt;
+  int small_from = 0;
+  void find_small_levels();
   int fgmres(const double* b, double* x);
   int bicgstab(const double* b, double* x);
   double reduce_to_host(const double* dev_scalar);

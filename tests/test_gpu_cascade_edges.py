@@ -23,3 +23,23 @@ def test_one_level_application_is_the_oracles(lsx, dims):
     z = S.precondition(v)
     assert np.abs(z).max() > 0
     assert np.array_equal(z, O.Solver(A, eps=1.0, precond="mg1").mg_apply(v))
+
+
+# 7-point levels of up to 4096 cells and 27-point levels of up to 1024 run in one workgroup, with
+# their restrictions, the coarsest LU and the prolongations: whole grids, from level 1, from level 2
+SMALL = [(4, 4, 4), (8, 4, 6), (3, 3, 3), (5, 5, 3), (12, 12, 12), (20, 12, 12), (16, 16, 16), (17, 17, 9), (17, 17, 17),
+         (9, 5, 33), (20, 20, 20), (24, 24, 24), (40, 24, 24), (33, 33, 33)]
+
+
+@pytest.mark.parametrize("dims", SMALL, ids=["x".join(map(str, d)) for d in SMALL])
+@pytest.mark.parametrize("fix", [False, True])
+def test_cascade_application_is_the_oracles(lsx, dims, fix):
+    g, A = P.synthetic_cut(*dims, seed=sum(dims))
+    S = lsx.MGFGMRES(z_head_fix=fix)
+    S.set(A, np.zeros(A.n), np.zeros(A.n), lsx.Task(eps=1.0))
+    v = np.random.default_rng(3).standard_normal(A.n)
+    z = S.precondition(v)
+    S.kernel_timing(True)  # per-level launches
+    assert np.array_equal(z, S.precondition(v))
+    if not fix:
+        assert np.array_equal(z, O.Solver(A, eps=1.0).mg_apply(v))
