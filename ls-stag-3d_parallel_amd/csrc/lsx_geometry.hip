@@ -310,22 +310,29 @@ __device__ inline double edge_fraction(double f, double fo) {
   return (f * fo < 0) ? ((f > 0) ? (fo / (fo - f)) : (f / (f - fo))) : ((f > -fo) ? 0.0 : 1.0);
 }
 
+// edge fractions of the edges below node (x, y, z) along x, y and z; phi(dx, dy, dz) reads a node near it
+template <class P>
+__device__ inline void alpha_of(P phi, int x, int y, int z, int K, const Box& box, double (&a)[3]) {
+  a[0] = a[1] = a[2] = 1.0;
+  if (in_box(x, y, box)) {
+    const double f = phi(0, 0, 0);
+    a[0] = edge_fraction(f, phi(-1, 0, 0));
+    a[1] = edge_fraction(f, phi(0, -1, 0));
+    a[2] = (z == 0 || z == K - 1) ? ((f > 0.0) ? 0.0 : 1.0) : edge_fraction(f, phi(0, 0, -1));
+  }
+}
+
 __global__ void k_alpha(const double* __restrict__ phi, int N, int M, int K, Box box, double* __restrict__ ax,
                         double* __restrict__ ay, double* __restrict__ az) {
   const long n = (long)N * M * K, NM = (long)N * M;
   for (long i = blockIdx.x * (long)blockDim.x + threadIdx.x; i < n; i += (long)gridDim.x * blockDim.x) {
     int x, y, z;
     decode(i, N, M, &x, &y, &z);
-    double a0 = 1.0, a1 = 1.0, a2 = 1.0;
-    if (in_box(x, y, box)) {
-      const double f = phi[i];
-      a0 = edge_fraction(f, phi[i - 1]);
-      a1 = edge_fraction(f, phi[i - N]);
-      a2 = (z == 0 || z == K - 1) ? ((f > 0.0) ? 0.0 : 1.0) : edge_fraction(f, phi[i - NM]);
-    }
-    ax[i] = a0;
-    ay[i] = a1;
-    az[i] = a2;
+    double a[3];
+    alpha_of([&](int dx, int dy, int dz) { return phi[i + dx + (long)N * dy + NM * dz]; }, x, y, z, K, box, a);
+    ax[i] = a[0];
+    ay[i] = a[1];
+    az[i] = a[2];
   }
 }
 
@@ -357,34 +364,41 @@ __device__ inline int border_type(int x, int y, int z, int N, int M, int K) {
   return FluidCell;
 }
 
+// type code of cell (x, y, z) and of its east, north and top faces; p as in alpha_of
+template <class P>
+__device__ inline int type_of(P p, int x, int y, int z, int N, int M, int K, const Box& box, int (&side)[3]) {
+  int t = border_type(x, y, z, N, M, K);
+  side[0] = side[1] = side[2] = FLUID_SIDE;
+  if (in_box(x, y, box)) {
+    const double phi = p(0, 0, 0), phiW = p(-1, 0, 0), phiS = p(0, -1, 0);
+    const int tT = type_of_side(phi, phiW, p(-1, -1, 0), phiS);
+    if (z == 0 || z == K - 1) {
+      side[0] = type_of_side(phi, phiS, phiS, phi);
+      side[1] = type_of_side(phi, phiW, phiW, phi);
+      side[2] = tT;
+      t = (tT == 0) ? SolidCell : (z == 0 ? B_Border : T_Border);
+    } else {
+      const double phiSB = p(0, -1, -1), phiB = p(0, 0, -1), phiBW = p(-1, 0, -1);
+      side[0] = type_of_side(phi, phiS, phiSB, phiB);
+      side[1] = type_of_side(phi, phiW, phiBW, phiB);
+      side[2] = tT;
+      t = tT * 10000 + type_of_side(phiB, phiBW, p(-1, -1, -1), phiSB);
+    }
+  }
+  return t;
+}
+
 __global__ void k_types(const double* __restrict__ p, int N, int M, int K, Box box, int* __restrict__ type,
                         int* __restrict__ sx, int* __restrict__ sy, int* __restrict__ sz) {
   const long n = (long)N * M * K, NM = (long)N * M;
   for (long i = blockIdx.x * (long)blockDim.x + threadIdx.x; i < n; i += (long)gridDim.x * blockDim.x) {
-    int x, y, z;
+    int x, y, z, side[3];
     decode(i, N, M, &x, &y, &z);
-    int t = border_type(x, y, z, N, M, K);
-    int s0 = FLUID_SIDE, s1 = FLUID_SIDE, s2 = FLUID_SIDE;
-    if (in_box(x, y, box)) {
-      const double phi = p[i], phiW = p[i - 1], phiS = p[i - N];
-      const int tT = type_of_side(phi, phiW, p[i - N - 1], phiS);
-      if (z == 0 || z == K - 1) {
-        s0 = type_of_side(phi, phiS, phiS, phi);
-        s1 = type_of_side(phi, phiW, phiW, phi);
-        s2 = tT;
-        t = (tT == 0) ? SolidCell : (z == 0 ? B_Border : T_Border);
-      } else {
-        const double phiSB = p[i - N - NM], phiB = p[i - NM], phiBW = p[i - NM - 1];
-        s0 = type_of_side(phi, phiS, phiSB, phiB);
-        s1 = type_of_side(phi, phiW, phiBW, phiB);
-        s2 = tT;
-        t = tT * 10000 + type_of_side(phiB, phiBW, p[i - N - 1 - NM], phiSB);
-      }
-    }
-    type[i] = t;
-    sx[i] = s0;
-    sy[i] = s1;
-    sz[i] = s2;
+    type[i] = type_of([&](int dx, int dy, int dz) { return p[i + dx + (long)N * dy + NM * dz]; }, x, y, z, N, M, K, box,
+                      side);
+    sx[i] = side[0];
+    sy[i] = side[1];
+    sz[i] = side[2];
   }
 }
 
@@ -409,6 +423,24 @@ __device__ inline double face_theta(int side, double P0, double P1, double Q0, d
   return t < THETA_EQ_ZERO ? 0.0 : t;
 }
 
+// open fractions of the east, north and top faces of cell (x, y, z); a(c, dx, dy, dz) reads edge
+// fraction c near it
+template <class A>
+__device__ inline void theta_of(A a, const int (&side)[3], int x, int y, int z, int K, const Box& box, double (&t)[3]) {
+  t[0] = t[1] = t[2] = 1.0;
+  if (in_box(x, y, box)) {
+    t[2] = face_theta(side[2], a(1, 0, 0, 0), a(1, -1, 0, 0), a(0, 0, 0, 0), a(0, 0, -1, 0));
+    if (z == 0 || z == K - 1) {
+      const double ay = a(1, 0, 0, 0), ax = a(0, 0, 0, 0);
+      t[0] = ay < THETA_EQ_ZERO ? 0.0 : ay;
+      t[1] = ax < THETA_EQ_ZERO ? 0.0 : ax;
+    } else {
+      t[0] = face_theta(side[0], a(2, 0, 0, 0), a(2, 0, -1, 0), a(1, 0, 0, 0), a(1, 0, 0, -1));
+      t[1] = face_theta(side[1], a(2, 0, 0, 0), a(2, -1, 0, 0), a(0, 0, 0, 0), a(0, 0, 0, -1));
+    }
+  }
+}
+
 __global__ void k_theta(const double* __restrict__ ax, const double* __restrict__ ay, const double* __restrict__ az,
                         const int* __restrict__ sx, const int* __restrict__ sy, const int* __restrict__ sz, int N, int M,
                         int K, Box box, double* __restrict__ tx, double* __restrict__ ty, double* __restrict__ tz) {
@@ -416,21 +448,17 @@ __global__ void k_theta(const double* __restrict__ ax, const double* __restrict_
   for (long i = blockIdx.x * (long)blockDim.x + threadIdx.x; i < n; i += (long)gridDim.x * blockDim.x) {
     int x, y, z;
     decode(i, N, M, &x, &y, &z);
-    double t0 = 1.0, t1 = 1.0, t2 = 1.0;
-    if (in_box(x, y, box)) {
-      t2 = face_theta(sz[i], ay[i], ay[i - 1], ax[i], ax[i - N]);
-      if (z == 0 || z == K - 1) {
-        const double a = ay[i], b = ax[i];
-        t0 = a < THETA_EQ_ZERO ? 0.0 : a;
-        t1 = b < THETA_EQ_ZERO ? 0.0 : b;
-      } else {
-        t0 = face_theta(sx[i], az[i], az[i - N], ay[i], ay[i - NM]);
-        t1 = face_theta(sy[i], az[i], az[i - 1], ax[i], ax[i - NM]);
-      }
-    }
-    tx[i] = t0;
-    ty[i] = t1;
-    tz[i] = t2;
+    const int side[3] = {sx[i], sy[i], sz[i]};
+    double t[3];
+    theta_of(
+        [&](int c, int dx, int dy, int dz) {
+          const long j = i + dx + (long)N * dy + NM * dz;
+          return c == 0 ? ax[j] : (c == 1 ? ay[j] : az[j]);
+        },
+        side, x, y, z, K, box, t);
+    tx[i] = t[0];
+    ty[i] = t[1];
+    tz[i] = t[2];
   }
 }
 
@@ -570,15 +598,83 @@ __device__ inline int find_rule(int code) {
   return -1;
 }
 
+// cut volume of a cell of type ty and full volume fullV; a(c, dx, dy, dz) and t(c, ...) read edge and
+// face fraction c near it
+template <class A, class T>
+__device__ inline double vof_of(int ty, double fullV, A a, T t) {
+  auto at = [](auto f, Ref r) { return f((int)r.comp, (int)r.dx, (int)r.dy, (int)r.dz); };
+  double vol = fullV;
+  if (ty == B_Border || ty == T_Border) {
+    vol *= t(2, 0, 0, 0);
+  } else if (ty == SolidCell) {
+    vol = 0.0;
+  } else if (ty > 0 && ty != FluidCell) {
+    const int k = find_rule(ty);
+    if (k >= 0) {
+      const Rule r = c_rules[k];
+      const double tUp = t(r.axis, 0, 0, 0), tLo = t(r.axis, -(r.axis == 0), -(r.axis == 1), -(r.axis == 2));
+      switch (r.fam) {
+        case F_TET:
+          vol = at(a, r.a) * at(t, r.b) * fullV * ONE_THIRD;
+          break;
+        case F_HEP3:
+          vol = (3.0 - (1.0 - at(a, r.a)) * (1.0 - at(t, r.b))) * fullV * ONE_THIRD;
+          break;
+        case F_PRISM:
+          vol = (tUp + tLo) * fullV * 0.5;
+          break;
+        case F_HEP5: {
+          const double tsel = r.sel ? tUp : tLo;
+          double ap = at(a, r.a);
+          const double denom = 1.0 - ap;
+          double term = 0.0;
+          if (denom > EQ_DOUBLE) {
+            ap /= denom;
+            term = (1.0 - tsel) * (3.0 - 2.0 * at(a, r.b)) * ap * ap * ONE_THIRD;
+          }
+          vol = (tLo + tUp + term) * fullV * 0.5;
+          break;
+        }
+        case F_HEX5: {
+          const double denom = at(a, r.a);
+          double term2 = r.sel ? tUp : tLo;
+          const double other = r.sel ? tLo : tUp;
+          if (denom > EQ_DOUBLE) {
+            const double coef = (1.0 - denom) / denom;
+            term2 *= (1.0 - (1.0 + 2.0 * at(a, r.b)) * coef * coef * ONE_THIRD);
+          }
+          vol = (other + term2) * fullV * 0.5;
+          break;
+        }
+        default: {  // F_HEP6
+          const double tsel = r.sel ? tUp : tLo;
+          const double other = r.sel ? tLo : tUp;
+          double term = 0.0;
+          double al = at(a, r.a);
+          double denom = 1.0 - al;
+          if (denom > EQ_DOUBLE) {
+            al /= denom;
+            term = (3.0 - 2.0 * at(a, r.b)) * al * al;
+          }
+          al = at(a, r.a2);
+          denom = 1.0 - al;
+          if (denom > EQ_DOUBLE) {
+            al /= denom;
+            term += (3.0 - 2.0 * at(a, r.b2)) * al * al;
+          }
+          vol = (other + tsel + (1.0 - tsel) * term * ONE_THIRD) * fullV * 0.5;
+        }
+      }
+    }
+  }
+  return vol + PLUS_TINY;
+}
+
 struct Fields {
   const double* a[3];
   const double* t[3];
   int N, NM;
 };
-
-__device__ inline double at(const double* const* arr, const Fields& F, long i, Ref r) {
-  return arr[(int)r.comp][i + r.dx + (long)F.N * r.dy + (long)F.NM * r.dz];
-}
 
 __global__ void k_vof(const int* __restrict__ type, Fields F, const double* __restrict__ dx,
                       const double* __restrict__ dy, const double* __restrict__ dz, int N, int M, int K,
@@ -587,74 +683,10 @@ __global__ void k_vof(const int* __restrict__ type, Fields F, const double* __re
   for (long i = blockIdx.x * (long)blockDim.x + threadIdx.x; i < n; i += (long)gridDim.x * blockDim.x) {
     int x, y, z;
     decode(i, N, M, &x, &y, &z);
-    const double fullV = dx[x] * dy[y] * dz[z];
-    double vol = fullV;
-    const int t = type[i];
-    if (t == B_Border || t == T_Border) {
-      vol *= F.t[2][i];
-    } else if (t == SolidCell) {
-      vol = 0.0;
-    } else if (t > 0 && t != FluidCell) {
-      const int k = find_rule(t);
-      if (k >= 0) {
-        const Rule r = c_rules[k];
-        const long lowOff = r.axis == 0 ? 1 : (r.axis == 1 ? F.N : F.NM);
-        const double tUp = F.t[r.axis][i], tLo = F.t[r.axis][i - lowOff];
-        switch (r.fam) {
-          case F_TET:
-            vol = at(F.a, F, i, r.a) * at(F.t, F, i, r.b) * fullV * ONE_THIRD;
-            break;
-          case F_HEP3:
-            vol = (3.0 - (1.0 - at(F.a, F, i, r.a)) * (1.0 - at(F.t, F, i, r.b))) * fullV * ONE_THIRD;
-            break;
-          case F_PRISM:
-            vol = (tUp + tLo) * fullV * 0.5;
-            break;
-          case F_HEP5: {
-            const double tsel = r.sel ? tUp : tLo;
-            double ap = at(F.a, F, i, r.a);
-            const double denom = 1.0 - ap;
-            double term = 0.0;
-            if (denom > EQ_DOUBLE) {
-              ap /= denom;
-              term = (1.0 - tsel) * (3.0 - 2.0 * at(F.a, F, i, r.b)) * ap * ap * ONE_THIRD;
-            }
-            vol = (tLo + tUp + term) * fullV * 0.5;
-            break;
-          }
-          case F_HEX5: {
-            const double denom = at(F.a, F, i, r.a);
-            double term2 = r.sel ? tUp : tLo;
-            const double other = r.sel ? tLo : tUp;
-            if (denom > EQ_DOUBLE) {
-              const double coef = (1.0 - denom) / denom;
-              term2 *= (1.0 - (1.0 + 2.0 * at(F.a, F, i, r.b)) * coef * coef * ONE_THIRD);
-            }
-            vol = (other + term2) * fullV * 0.5;
-            break;
-          }
-          default: {  // F_HEP6
-            const double tsel = r.sel ? tUp : tLo;
-            const double other = r.sel ? tLo : tUp;
-            double term = 0.0;
-            double al = at(F.a, F, i, r.a);
-            double denom = 1.0 - al;
-            if (denom > EQ_DOUBLE) {
-              al /= denom;
-              term = (3.0 - 2.0 * at(F.a, F, i, r.b)) * al * al;
-            }
-            al = at(F.a, F, i, r.a2);
-            denom = 1.0 - al;
-            if (denom > EQ_DOUBLE) {
-              al /= denom;
-              term += (3.0 - 2.0 * at(F.a, F, i, r.b2)) * al * al;
-            }
-            vol = (other + tsel + (1.0 - tsel) * term * ONE_THIRD) * fullV * 0.5;
-          }
-        }
-      }
-    }
-    vof[i] = vol + PLUS_TINY;
+    auto rd = [&](const double* const* f) {
+      return [&, f](int c, int ex, int ey, int ez) { return f[c][i + ex + (long)F.N * ey + (long)F.NM * ez]; };
+    };
+    vof[i] = vof_of(type[i], dx[x] * dy[y] * dz[z], rd(F.a), rd(F.t));
   }
 }
 
@@ -668,30 +700,43 @@ __device__ inline bool no_n(int t) { return t == N_Border || t == TN_Edge || t =
 __device__ inline bool no_w(int t) { return t == W_Border || t == TW_Edge || t == BW_Edge || t == NW_Edge || t == SW_Edge || t == TNW_Corner || t == TSW_Corner || t == BNW_Corner || t == BSW_Corner; }
 __device__ inline bool no_e(int t) { return t == E_Border || t == TE_Edge || t == BE_Edge || t == NE_Edge || t == SE_Edge || t == TNE_Corner || t == TSE_Corner || t == BNE_Corner || t == BSE_Corner; }
 
+// the fields near cell i of a whole grid
+struct GridCell {
+  const int* __restrict__ ty;
+  const double* __restrict__ th[3];
+  const double* __restrict__ vo;
+  long i;
+  int N;
+  long NM;
+  __device__ int type() const { return ty[i]; }
+  __device__ double theta(int c, int dx, int dy, int dz) const { return th[c][i + dx + (long)N * dy + NM * dz]; }
+  __device__ double vof(int dx, int dy, int dz) const { return vo[i + dx + (long)N * dy + NM * dz]; }
+};
+
 // Pressure operator row of cell i as 7 coefficients c = [b,s,w,p,e,n,t] (absent = 0): the
 // values of LaplaceDiscreteOperator::calcLap (laplace_discrete_operator.h:107-686) with the
-// staggered masses M = (V_i + V_nb)/2 inlined, and identity rows at the two pinned cells.
-__device__ inline void laplace_row(long i, int x, int y, int z, const int* __restrict__ type,
-                                   const double* __restrict__ tx, const double* __restrict__ ty,
-                                   const double* __restrict__ tz, const double* __restrict__ vof,
-                                   const double* __restrict__ dxs, const double* __restrict__ dys,
-                                   const double* __restrict__ dzs, int N, int M, int pin, double* c) {
+// staggered masses M = (V_i + V_nb)/2 inlined, and identity rows at the two pinned cells.  g reads
+// the cell's type and the face fractions and volumes near it.
+template <class G>
+__device__ inline void laplace_row(const G& g, long i, int x, int y, int z, const double* __restrict__ dxs,
+                                   const double* __restrict__ dys, const double* __restrict__ dzs, int N, int M, int pin,
+                                   double* c) {
   const long NM = (long)N * M;
-  const int t = type[i];
+  const int t = g.type();
   double a_b = 0, a_s = 0, a_w = 0, a_p = 0, a_e = 0, a_n = 0, a_t = 0;
   if (t == SolidCell) {
     a_p = PLUS_TINY;
   } else {
-    const double v = vof[i];
+    const double v = g.vof(0, 0, 0);
     const double ddx = dxs[x], ddy = dys[y], ddz = dzs[z];
     const bool hb = !no_b(t), hs = !no_s(t), hw = !no_w(t), he = !no_e(t), hn = !no_n(t), ht = !no_t(t);
     // masses of the six faces (only the present ones are read)
-    const double imw = hw ? inv_mass(0.5 * (vof[i - 1] + v)) : 0.0;
-    const double ime = he ? inv_mass(0.5 * (v + vof[i + 1])) : 0.0;
-    const double ims = hs ? inv_mass(0.5 * (vof[i - N] + v)) : 0.0;
-    const double imn = hn ? inv_mass(0.5 * (v + vof[i + N])) : 0.0;
-    const double imb = hb ? inv_mass(0.5 * (vof[i - NM] + v)) : 0.0;
-    const double imt = ht ? inv_mass(0.5 * (v + vof[i + NM])) : 0.0;
+    const double imw = hw ? inv_mass(0.5 * (g.vof(-1, 0, 0) + v)) : 0.0;
+    const double ime = he ? inv_mass(0.5 * (v + g.vof(1, 0, 0))) : 0.0;
+    const double ims = hs ? inv_mass(0.5 * (g.vof(0, -1, 0) + v)) : 0.0;
+    const double imn = hn ? inv_mass(0.5 * (v + g.vof(0, 1, 0))) : 0.0;
+    const double imb = hb ? inv_mass(0.5 * (g.vof(0, 0, -1) + v)) : 0.0;
+    const double imt = ht ? inv_mass(0.5 * (v + g.vof(0, 0, 1))) : 0.0;
     if (t == FluidCell) {
       const double dyz = ddy * ddz, dxz = ddx * ddz, dxy = ddy * ddx;
       double aux = dyz * dyz;
@@ -707,12 +752,12 @@ __device__ inline void laplace_row(long i, int x, int y, int z, const int* __res
     } else {
       const double dyz = ddy * ddz, dxz = ddx * ddz, dxy = ddx * ddy;
       double aux;
-      if (hw) { aux = tx[i - 1] * dyz; a_w = aux * aux * imw; }
-      if (he) { aux = tx[i] * dyz; a_e = aux * aux * ime; }
-      if (hs) { aux = ty[i - N] * dxz; a_s = aux * aux * ims; }
-      if (hn) { aux = ty[i] * dxz; a_n = aux * aux * imn; }
-      if (hb) { aux = tz[i - NM] * dxy; a_b = aux * aux * imb; }
-      if (ht) { aux = tz[i] * dxy; a_t = aux * aux * imt; }
+      if (hw) { aux = g.theta(0, -1, 0, 0) * dyz; a_w = aux * aux * imw; }
+      if (he) { aux = g.theta(0, 0, 0, 0) * dyz; a_e = aux * aux * ime; }
+      if (hs) { aux = g.theta(1, 0, -1, 0) * dxz; a_s = aux * aux * ims; }
+      if (hn) { aux = g.theta(1, 0, 0, 0) * dxz; a_n = aux * aux * imn; }
+      if (hb) { aux = g.theta(2, 0, 0, -1) * dxy; a_b = aux * aux * imb; }
+      if (ht) { aux = g.theta(2, 0, 0, 0) * dxy; a_t = aux * aux * imt; }
       bool first = true;
       if (hb) { a_p = -a_b; first = false; }
       if (hs) { a_p = first ? -a_s : a_p - a_s; first = false; }
@@ -744,7 +789,7 @@ __global__ void k_laplace7(const int* __restrict__ type, const double* __restric
     int x, y, z;
     decode(i, N, M, &x, &y, &z);
     double c[7];
-    laplace_row(i, x, y, z, type, tx, ty, tz, vof, dxs, dys, dzs, N, M, pin, c);
+    laplace_row(GridCell{type, {tx, ty, tz}, vof, i, N, (long)N * M}, i, x, y, z, dxs, dys, dzs, N, M, pin, c);
     for (int q = 0; q < 7; ++q) coef[q * n + i] = c[q];
   }
 }
@@ -1072,9 +1117,8 @@ struct RhsIn {
   FlowBc bc;
 };
 
-__device__ inline double rhs_cell(long i, int x, int y, int z, const int* __restrict__ type,
-                                  const double* __restrict__ tx, const double* __restrict__ ty,
-                                  const double* __restrict__ tz, const double* __restrict__ dxa,
+template <class G>
+__device__ inline double rhs_cell(const G& g, long i, int x, int y, int z, const double* __restrict__ dxa,
                                   const double* __restrict__ dya, const double* __restrict__ dza, int N, int M, int K,
                                   const RhsIn& in) {
   const long NM = (long)N * M;
@@ -1082,7 +1126,7 @@ __device__ inline double rhs_cell(long i, int x, int y, int z, const int* __rest
   const double* __restrict__ v = in.v;
   const double* __restrict__ w = in.w;
   const FlowBc& bc = in.bc;
-  const int t = type[i];
+  const int t = g.type();
   const double dx = dxa[x], dy = dya[y], dz = dza[z];
   const long row = y + (long)z * M;
   // flux: initFlux, addFluxNSp, addFluxTBp, setBaseFlux (static body: ibFlux = 0)
@@ -1091,20 +1135,20 @@ __device__ inline double rhs_cell(long i, int x, int y, int z, const int* __rest
   if (x == N - 1) flux = bc.U_E * (dy * dz);
   if (y == 0) flux -= (dx * dz) * bc.V_S;
   if (y == M - 1) flux += (dx * dz) * bc.V_N;
-  if (z == 0) flux -= (dy * dx) * tz[i] * bc.W_B;
-  if (z == K - 1) flux += (dy * dx) * tz[i] * bc.W_T;
+  if (z == 0) flux -= (dy * dx) * g.theta(2, 0, 0, 0) * bc.W_B;
+  if (z == K - 1) flux += (dy * dx) * g.theta(2, 0, 0, 0) * bc.W_T;
   if (in.u_out && x == N - 1) flux = in.u_out[row * (N - 1) + N - 2] * dy * dz;
   // Dx u
   double aux = 0.0;
   {
     const long p = row * (N - 1) + x;
     if (t == SolidCell) aux += 0.0 * u[x == 0 ? p : p - 1];
-    else if (x_east(t)) aux += (-tx[i - 1] * dy * dz) * u[p - 1];
-    else if (x_west(t)) aux += (tx[i] * dy * dz) * u[p];
+    else if (x_east(t)) aux += (-g.theta(0, -1, 0, 0) * dy * dz) * u[p - 1];
+    else if (x_west(t)) aux += (g.theta(0, 0, 0, 0) * dy * dz) * u[p];
     else {
       const double dyz = dy * dz;
-      aux += (-tx[i - 1] * dyz) * u[p - 1];
-      aux += (tx[i] * dyz) * u[p];
+      aux += (-g.theta(0, -1, 0, 0) * dyz) * u[p - 1];
+      aux += (g.theta(0, 0, 0, 0) * dyz) * u[p];
     }
   }
   // (aux + flux) + Dy v
@@ -1112,24 +1156,24 @@ __device__ inline double rhs_cell(long i, int x, int y, int z, const int* __rest
   {
     const long p = (long)z * N * (M - 1) + (long)y * N + x;
     if (t == SolidCell) r += 0.0 * v[y == 0 ? p : p - N];
-    else if (y_north(t)) r += (-ty[i - N] * dx * dz) * v[p - N];
-    else if (y_south(t)) r += (ty[i] * dx * dz) * v[p];
+    else if (y_north(t)) r += (-g.theta(1, 0, -1, 0) * dx * dz) * v[p - N];
+    else if (y_south(t)) r += (g.theta(1, 0, 0, 0) * dx * dz) * v[p];
     else {
       const double dxz = dx * dz;
-      r += (-ty[i - N] * dxz) * v[p - N];
-      r += (ty[i] * dxz) * v[p];
+      r += (-g.theta(1, 0, -1, 0) * dxz) * v[p - N];
+      r += (g.theta(1, 0, 0, 0) * dxz) * v[p];
     }
   }
   // + Dz w
   double auxz = 0.0;
   {
     if (t == SolidCell) auxz += 0.0 * w[z == 0 ? i : i - NM];
-    else if (z_bottom(t)) auxz += (tz[i] * dx * dy) * w[i];
-    else if (z_top(t)) auxz += (-tz[i - NM] * dx * dy) * w[i - NM];
+    else if (z_bottom(t)) auxz += (g.theta(2, 0, 0, 0) * dx * dy) * w[i];
+    else if (z_top(t)) auxz += (-g.theta(2, 0, 0, -1) * dx * dy) * w[i - NM];
     else {
       const double dxy = dx * dy;
-      auxz += (-tz[i - NM] * dxy) * w[i - NM];
-      auxz += (tz[i] * dxy) * w[i];
+      auxz += (-g.theta(2, 0, 0, -1) * dxy) * w[i - NM];
+      auxz += (g.theta(2, 0, 0, 0) * dxy) * w[i];
     }
   }
   r += auxz;
@@ -1147,7 +1191,7 @@ __global__ void k_pressure_rhs(const int* __restrict__ type, const double* __res
     const int z = (int)(i / NM);
     const long r2 = i - (long)z * NM;
     const int y = (int)(r2 / N), x = (int)(r2 - (long)y * N);
-    b[i] = rhs_cell(i, x, y, z, type, tx, ty, tz, dxa, dya, dza, N, M, K, in);
+    b[i] = rhs_cell(GridCell{type, {tx, ty, tz}, nullptr, i, N, NM}, i, x, y, z, dxa, dya, dza, N, M, K, in);
   }
 }
 
@@ -1255,17 +1299,20 @@ void pressure_rhs(const int* type, const double* tx, const double* ty, const dou
 // change of the geometry is that of the Lagrangian F = J(theta, p) + lambda . (b - A p) with p and
 // lambda held fixed.  F is a sum over cells of terms that read the level set at the corners of
 // the cell and of its six neighbours, after an oscillation fix that reads one node further:
-// corner c reaches the cells c + [-2, 3]^3.  Corners 6 apart in every direction therefore have
-// disjoint reach, so one pair of geometry rebuilds with all corners of one of the 216 classes
-// (x mod 6, y mod 6, z mod 6) moved by +h and -h gives the central difference dF/dphi_c of
-// every corner of the class at once, summed over its reach.  Differences are taken per
-// coefficient (c+ - c-) before they meet p, so the large cancelling products of A p never enter
-// them.  A Bezier body then chains dF/dphi to its control values through the closest point:
-// phi = sgn |X - S(u*, v*)| gives dphi/dP_ij = -sgn (X - S)/|X - S| B_i(u*) B_j(v*) (the
-// minimiser's own change does not enter at a minimum).
+// corner c reaches the cells c + [-2, 3]^3, and dF/dphi_c is the central difference of those cells'
+// terms with the corner moved by +h and -h.  Differences are taken per coefficient (c+ - c-)
+// before they meet p, so the large cancelling products of A p never enter them.  A Bezier body
+// then chains dF/dphi to its control values through the closest point: phi = sgn |X - S(u*, v*)|
+// gives dphi/dP_ij = -sgn (X - S)/|X - S| B_i(u*) B_j(v*) (the minimiser's own change does not
+// enter at a minimum).
+//
+// A corner whose level set and whose neighbours' along the axes, before and after the fix, lie on one
+// side of the surface by more than the step changes no edge fraction and no sign, so its difference
+// is exactly 0: only the corners along the surface are worked on (k_active_*: their list, in index order), one
+// workgroup each (k_corner), which rebuilds the geometry of the 6^3 cells around its corner twice in
+// LDS and reads the unmoved geometry outside them.  72 x 64 x 64 cells, 3210 corners: 224 us (two
+// rebuilds of the whole grid for each of 216 classes of corners 6 apart: 59 ms).
 namespace {
-
-constexpr int SG_SPACING = 6;
 
 __device__ inline bool cut_cell(int t) { return t > 0 && t != FluidCell; }
 
@@ -1294,116 +1341,269 @@ __global__ void k_drag(const int* __restrict__ type, const double* __restrict__ 
   if (threadIdx.x == 0) partial[blockIdx.x] = lds[0];
 }
 
-__device__ inline int corner_class(int x, int y, int z) {
-  return x % SG_SPACING + SG_SPACING * (y % SG_SPACING) + SG_SPACING * SG_SPACING * (z % SG_SPACING);
+template <class G>
+__device__ inline double drag_cell(const G& g, int x, int y, int z, const double* dys, const double* dzs, const Box& box,
+                                   double p) {
+  if (!in_box(x, y, box) || !cut_cell(g.type())) return 0.0;
+  return (g.theta(0, -1, 0, 0) - g.theta(0, 0, 0, 0)) * dys[y] * dzs[z] * p;
 }
 
-__global__ void k_perturb(const double* __restrict__ phi_raw, int N, int M, int K, Box box, int cls, double h,
-                          double* __restrict__ phi_p, double* __restrict__ phi_m) {
+// whether moving corner i by h can change the geometry: its level set and its neighbours', before
+// (raw) and after (phi) the oscillation fix, do not all lie on one side by more than the step
+__device__ inline bool corner_active(const double* __restrict__ raw, const double* __restrict__ phi, long i, int N, int M,
+                                     int K, const Box& box, double h) {
+  int x, y, z;
+  decode(i, N, M, &x, &y, &z);
+  if (!in_box(x, y, box)) return false;
+  const long NM = (long)N * M;
+  const double t = 2.0 * (EQ_DOUBLE + h);
+  const bool inside = raw[i] > 0.0;
+  auto apart = [&](bool there, long j) {
+    const long k = there ? j : i;
+    const double r = raw[k], f = phi[k];
+    return inside ? !(r > t && f > t) : !(r < -t && f < -t);
+  };
+  return apart(true, i) || apart(x - 1 >= box.hs, i - 1) || apart(x + 1 < box.hf, i + 1) ||
+         apart(y - 1 >= box.vs, i - N) || apart(y + 1 < box.vf, i + N) || apart(z > 0, i - NM) ||
+         apart(z + 1 < K, i + NM);
+}
+
+// The list of active corners in index order: blocks of AC_NODES consecutive nodes count theirs
+// (list null), one workgroup turns the counts into offsets and the total (k_active_scan), and the
+// blocks write (ranks within a block by ballots).
+constexpr int AC_NODES = 1024;
+__global__ void __launch_bounds__(256) k_active(const double* __restrict__ raw, const double* __restrict__ phi, int N, int M, int K, Box box, double h,
+                                                int* __restrict__ count, int* __restrict__ list) {
+  __shared__ int waves[4];
   const long n = (long)N * M * K;
-  for (long i = blockIdx.x * (long)blockDim.x + threadIdx.x; i < n; i += (long)gridDim.x * blockDim.x) {
-    int x, y, z;
-    decode(i, N, M, &x, &y, &z);
-    const double v = phi_raw[i];
-    const bool on = in_box(x, y, box) && corner_class(x, y, z) == cls;
-    phi_p[i] = on ? v + h : v;
-    phi_m[i] = on ? v - h : v;
-  }
-}
-
-__device__ inline double drag_cell(const GeoView& g, long i, int x, int y, int z, const double* dys,
-                                   const double* dzs, const Box& box, double p) {
-  if (!in_box(x, y, box) || !cut_cell(g.type[i])) return 0.0;
-  return (g.tx[i - 1] - g.tx[i]) * dys[y] * dzs[z] * p;
-}
-
-__global__ void k_lagr_diff(GeoView gp, GeoView gm, const double* __restrict__ dxs, const double* __restrict__ dys,
-                            const double* __restrict__ dzs, int N, int M, int K, Box box, int pin,
-                            const double* __restrict__ p, const double* __restrict__ lam, int objective, int has_rhs,
-                            RhsIn rin, double inv2h, double* __restrict__ dF) {
-  const long n = (long)N * M * K, NM = (long)N * M;
-  for (long i = blockIdx.x * (long)blockDim.x + threadIdx.x; i < n; i += (long)gridDim.x * blockDim.x) {
-    int x, y, z;
-    decode(i, N, M, &x, &y, &z);
-    double dJ = 0.0;
-    if (objective == OBJ_DRAG_X && in_box(x, y, box)) {
-      const bool cp = cut_cell(gp.type[i]), cm = cut_cell(gm.type[i]);
-      if (cp && cm) {
-        const double dw = gp.tx[i - 1] - gm.tx[i - 1], de = gp.tx[i] - gm.tx[i];
-        dJ = (dw - de) * dys[y] * dzs[z] * p[i];
-      } else {
-        dJ = drag_cell(gp, i, x, y, z, dys, dzs, box, p[i]) - drag_cell(gm, i, x, y, z, dys, dzs, box, p[i]);
-      }
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  int at = list ? count[blockIdx.x] : 0;
+  for (int q = 0; q < AC_NODES / 256; ++q) {
+    const long i = (long)blockIdx.x * AC_NODES + q * 256 + threadIdx.x;
+    const bool on = i < n && corner_active(raw, phi, i, N, M, K, box, h);
+    const unsigned long long m = __ballot(on);
+    if (lane == 0) waves[wave] = __popcll(m);
+    __syncthreads();
+    int before = 0, all = 0;
+    for (int w = 0; w < 4; ++w) {
+      before += w < wave ? waves[w] : 0;
+      all += waves[w];
     }
-    double ca[7], cb[7];
-    laplace_row(i, x, y, z, gp.type, gp.tx, gp.ty, gp.tz, gp.vof, dxs, dys, dzs, N, M, pin, ca);
-    laplace_row(i, x, y, z, gm.type, gm.tx, gm.ty, gm.tz, gm.vof, dxs, dys, dzs, N, M, pin, cb);
-    const long nb[7] = {i - NM, i - N, i - 1, i, i + 1, i + N, i + NM};
-    const bool has[7] = {z > 0, y > 0, x > 0, true, x < N - 1, y < M - 1, z < K - 1};
-    double dAp = 0.0;
-    for (int q = 0; q < 7; ++q)
-      if (has[q]) dAp += (ca[q] - cb[q]) * p[nb[q]];
-    double db = 0.0;
-    if (has_rhs)
-      db = rhs_cell(i, x, y, z, gp.type, gp.tx, gp.ty, gp.tz, dxs, dys, dzs, N, M, K, rin) -
-           rhs_cell(i, x, y, z, gm.type, gm.tx, gm.ty, gm.tz, dxs, dys, dzs, N, M, K, rin);
-    dF[i] = (dJ + lam[i] * (db - dAp)) * inv2h;
+    if (list && on) list[at + before + __popcll(m & ((1ull << lane) - 1))] = (int)i;
+    at += all;
+    __syncthreads();
   }
+  if (!list && threadIdx.x == 0) count[blockIdx.x] = at;
 }
 
-// g[c] = sum of dF over the reach of corner c, for the corners of class `cls`
-__global__ void k_corner_gather(const double* __restrict__ dF, int N, int M, int K, Box box, int cls,
-                                double* __restrict__ g) {
-  const long n = (long)N * M * K, NM = (long)N * M;
-  for (long c = blockIdx.x * (long)blockDim.x + threadIdx.x; c < n; c += (long)gridDim.x * blockDim.x) {
-    int x, y, z;
-    decode(c, N, M, &x, &y, &z);
-    if (!in_box(x, y, box) || corner_class(x, y, z) != cls) continue;
-    double acc = 0.0;
-    for (int zz = z - 2; zz <= z + 3; ++zz) {
-      if (zz < 0 || zz >= K) continue;
-      for (int yy = y - 2; yy <= y + 3; ++yy) {
-        if (yy < 0 || yy >= M) continue;
-        for (int xx = x - 2; xx <= x + 3; ++xx) {
-          if (xx < 0 || xx >= N) continue;
-          acc += dF[xx + (long)N * yy + NM * zz];
+__global__ void __launch_bounds__(1024) k_active_scan(int* __restrict__ count, int nb) {
+  __shared__ int sum[1024];
+  const int per = (nb + 1023) / 1024, lo = threadIdx.x * per, hi = lo + per < nb ? lo + per : nb;
+  int mine = 0;
+  for (int b = lo; b < hi; ++b) mine += count[b];
+  sum[threadIdx.x] = mine;
+  __syncthreads();
+  for (int st = 1; st < 1024; st <<= 1) {
+    const int v = (int)threadIdx.x >= st ? sum[threadIdx.x - st] : 0;
+    __syncthreads();
+    sum[threadIdx.x] += v;
+    __syncthreads();
+  }
+  int at = sum[threadIdx.x] - mine;
+  for (int b = lo; b < hi; ++b) {
+    const int c = count[b];
+    count[b] = at;
+    at += c;
+  }
+  if (threadIdx.x == 1023) count[nb] = sum[1023];
+}
+
+// One moved geometry around a corner: nodes and cells c + [-1, 4]^3.
+constexpr int PA = 6, PCELLS = PA * PA * PA;
+struct Patch {
+  double phi[PCELLS], a[3][PCELLS], t[3][PCELLS], vof[PCELLS];
+  int type[PCELLS];
+};
+// the fields near a cell at (lx, ly, lz) of the patch, grid index i: the patch's inside it, the
+// unmoved geometry's outside
+struct PatchCell {
+  const Patch* s;
+  const GeoBase& g;
+  int lx, ly, lz;
+  long i;
+  int N;
+  long NM;
+  __device__ double get(const double* in, const double* __restrict__ out, int dx, int dy, int dz) const {
+    const int a = lx + dx, b = ly + dy, c = lz + dz;
+    const bool local = (unsigned)a < PA && (unsigned)b < PA && (unsigned)c < PA;
+    return local ? in[a + PA * (b + PA * c)] : out[i + dx + (long)N * dy + NM * dz];
+  }
+  __device__ double phi(int dx, int dy, int dz) const { return get(s->phi, g.phi, dx, dy, dz); }
+  __device__ double alpha(int c, int dx, int dy, int dz) const { return get(s->a[c], g.a[c], dx, dy, dz); }
+  __device__ double theta(int c, int dx, int dy, int dz) const { return get(s->t[c], g.t[c], dx, dy, dz); }
+  __device__ double vof(int dx, int dy, int dz) const { return get(s->vof, g.vof, dx, dy, dz); }
+  __device__ int type() const {
+    const bool local = (unsigned)lx < PA && (unsigned)ly < PA && (unsigned)lz < PA;
+    return local ? s->type[lx + PA * (ly + PA * lz)] : g.type[i];
+  }
+};
+
+// g[c] = dF/dphi_c of the listed corners, a workgroup at a time; total = count[nb] of the list.
+// Every stage is the whole grid's (alpha_of, type_of, theta_of, vof_of, laplace_row, rhs_cell), one
+// thread per cell of the patch and both moves in turn; the terms of the 216 reached cells are added
+// in index order.  Bound by the latency of its dozen stages; 35 KB of LDS let four share a CU.
+__global__ void __launch_bounds__(256) k_corner(GeoBase g, const int* __restrict__ list, const int* __restrict__ total,
+                                                const double* __restrict__ dxs, const double* __restrict__ dys,
+                                                const double* __restrict__ dzs, int N, int M, int K, Box box, int pin,
+                                                const double* __restrict__ p, const double* __restrict__ lam,
+                                                int objective, int has_rhs, RhsIn rin, double h, double inv2h,
+                                                double* __restrict__ out) {
+  __shared__ Patch S[2];
+  __shared__ double dF[PCELLS];
+  const long NM = (long)N * M;
+  const int tid = threadIdx.x, n_active = total[0];
+  const int lx = tid % PA, ly = tid / PA % PA, lz = tid / (PA * PA);
+  for (int w = blockIdx.x; w < n_active; w += gridDim.x) {
+    const long c = list[w];
+    int cx, cy, cz;
+    decode(c, N, M, &cx, &cy, &cz);
+    const int x = cx - 1 + lx, y = cy - 1 + ly, z = cz - 1 + lz;
+    const long i = x + (long)N * y + NM * z;
+    const bool own = tid < PCELLS && x >= 0 && x < N && y >= 0 && y < M && z >= 0 && z < K;
+    auto raw = [&](int m, long j) {  // the moved level set before the oscillation fix
+      const double v = g.raw[j];
+      return j == c ? (m == 0 ? v + h : v - h) : v;
+    };
+    // oscillation fix (k_osc_flags, k_osc_iter): nodes below the patch hold their unmoved final values
+    bool flag[2] = {false, false};
+    if (own)
+      for (int m = 0; m < 2; ++m) {
+        const double f = raw(m, i);
+        S[m].phi[tid] = f;
+        if (in_box(x, y, box) && f > EQ_DOUBLE)
+          flag[m] = raw(m, i + 1) < 0 || raw(m, i + N) < 0 || (z > 0 && z < K - 1 && raw(m, i + NM) < 0);
+      }
+    for (;;) {
+      __syncthreads();
+      double nxt[2];
+      bool changed = false;
+      for (int m = 0; m < 2; ++m)
+        if (flag[m]) {
+          const PatchCell q{&S[m], g, lx, ly, lz, i, N, NM};
+          double f = raw(m, i);
+          check_osc(f, q.phi(-1, 0, 0), raw(m, i + 1));
+          check_osc(f, q.phi(0, -1, 0), raw(m, i + N));
+          if (z > 0 && z < K - 1) check_osc(f, q.phi(0, 0, -1), raw(m, i + NM));
+          changed = changed || f != S[m].phi[tid];
+          nxt[m] = f;
         }
-      }
+      if (!__syncthreads_or(changed)) break;
+      for (int m = 0; m < 2; ++m)
+        if (flag[m]) S[m].phi[tid] = nxt[m];
     }
-    g[c] = acc;
+    int side[2][3];
+    if (own)
+      for (int m = 0; m < 2; ++m) {
+        const PatchCell q{&S[m], g, lx, ly, lz, i, N, NM};
+        auto phi = [&](int dx, int dy, int dz) { return q.phi(dx, dy, dz); };
+        double a[3];
+        alpha_of(phi, x, y, z, K, box, a);
+        for (int k = 0; k < 3; ++k) S[m].a[k][tid] = a[k];
+        S[m].type[tid] = type_of(phi, x, y, z, N, M, K, box, side[m]);
+      }
+    __syncthreads();
+    if (own)
+      for (int m = 0; m < 2; ++m) {
+        const PatchCell q{&S[m], g, lx, ly, lz, i, N, NM};
+        double t[3];
+        theta_of([&](int k, int dx, int dy, int dz) { return q.alpha(k, dx, dy, dz); }, side[m], x, y, z, K, box, t);
+        for (int k = 0; k < 3; ++k) S[m].t[k][tid] = t[k];
+      }
+    __syncthreads();
+    if (own)
+      for (int m = 0; m < 2; ++m) {
+        const PatchCell q{&S[m], g, lx, ly, lz, i, N, NM};
+        S[m].vof[tid] = vof_of(
+            S[m].type[tid], dxs[x] * dys[y] * dzs[z],
+            [&](int k, int dx, int dy, int dz) { return q.alpha(k, dx, dy, dz); },
+            [&](int k, int dx, int dy, int dz) { return q.theta(k, dx, dy, dz); });
+      }
+    __syncthreads();
+    // the reached cells c + [-2, 3]^3: one cell before the patch's in every direction
+    const int rx = x - 1, ry = y - 1, rz = z - 1;
+    if (tid < PCELLS) {
+      double v = 0.0;
+      if (rx >= 0 && rx < N && ry >= 0 && ry < M && rz >= 0 && rz < K) {
+        const long r = rx + (long)N * ry + NM * rz;
+        const PatchCell gp{&S[0], g, lx - 1, ly - 1, lz - 1, r, N, NM}, gm{&S[1], g, lx - 1, ly - 1, lz - 1, r, N, NM};
+        double dJ = 0.0;
+        if (objective == OBJ_DRAG_X && in_box(rx, ry, box)) {
+          if (cut_cell(gp.type()) && cut_cell(gm.type())) {
+            const double dw = gp.theta(0, -1, 0, 0) - gm.theta(0, -1, 0, 0);
+            const double de = gp.theta(0, 0, 0, 0) - gm.theta(0, 0, 0, 0);
+            dJ = (dw - de) * dys[ry] * dzs[rz] * p[r];
+          } else {
+            dJ = drag_cell(gp, rx, ry, rz, dys, dzs, box, p[r]) - drag_cell(gm, rx, ry, rz, dys, dzs, box, p[r]);
+          }
+        }
+        double ca[7], cb[7];
+        laplace_row(gp, r, rx, ry, rz, dxs, dys, dzs, N, M, pin, ca);
+        laplace_row(gm, r, rx, ry, rz, dxs, dys, dzs, N, M, pin, cb);
+        const long nb[7] = {r - NM, r - N, r - 1, r, r + 1, r + N, r + NM};
+        const bool has[7] = {rz > 0, ry > 0, rx > 0, true, rx < N - 1, ry < M - 1, rz < K - 1};
+        double dAp = 0.0;
+        for (int q = 0; q < 7; ++q)
+          if (has[q]) dAp += (ca[q] - cb[q]) * p[nb[q]];
+        double db = 0.0;
+        if (has_rhs)
+          db = rhs_cell(gp, r, rx, ry, rz, dxs, dys, dzs, N, M, K, rin) -
+               rhs_cell(gm, r, rx, ry, rz, dxs, dys, dzs, N, M, K, rin);
+        v = (dJ + lam[r] * (db - dAp)) * inv2h;
+      }
+      dF[tid] = v;
+    }
+    __syncthreads();
+    if (tid == 0) {
+      double acc = 0.0;
+#pragma unroll 8
+      for (int q = 0; q < PCELLS; ++q) acc += dF[q];
+      out[c] = acc;
+    }
+    __syncthreads();
   }
 }
 
-// per corner with g != 0: winning patch, its parameters and w = g dphi/dS (3 values)
-__global__ void k_bz_hits(const double* __restrict__ g, const double* __restrict__ cx, const double* __restrict__ cy,
-                          const double* __restrict__ cz, int N, int M, int K, Box box, Body body,
-                          int* __restrict__ hf, double* __restrict__ huv, double* __restrict__ hw) {
-  const long n = (long)N * M * K;
-  for (long i = blockIdx.x * (long)blockDim.x + threadIdx.x; i < n; i += (long)gridDim.x * blockDim.x) {
-    int x, y, z;
-    decode(i, N, M, &x, &y, &z);
-    int f = -1;
-    if (in_box(x, y, box) && g[i] != 0.0) {
-      BzHit hit;
-      bezier_closest(body.ctrl, body.c, body.a, cx[x], cy[y], cz[z], hit);
-      if (hit.dist > 0.0) {
-        f = hit.f;
-        huv[2 * i] = hit.u;
-        huv[2 * i + 1] = hit.v;
-        for (int c = 0; c < 3; ++c) hw[3 * i + c] = g[i] * (-hit.sgn * hit.r[c] / hit.dist);
-      }
+// per listed corner with g != 0: winning patch, its parameters and w = g dphi/dS (3 values)
+__global__ void k_bz_hits(const double* __restrict__ g, const int* __restrict__ list, int count,
+                          const double* __restrict__ cx, const double* __restrict__ cy, const double* __restrict__ cz,
+                          int N, int M, Body body, int* __restrict__ hf, double* __restrict__ huv,
+                          double* __restrict__ hw) {
+  const int l = blockIdx.x * blockDim.x + threadIdx.x;
+  if (l >= count) return;
+  const long i = list[l];
+  int x, y, z;
+  decode(i, N, M, &x, &y, &z);
+  int f = -1;
+  if (g[i] != 0.0) {
+    BzHit hit;
+    bezier_closest(body.ctrl, body.c, body.a, cx[x], cy[y], cz[z], hit);
+    if (hit.dist > 0.0) {
+      f = hit.f;
+      huv[2 * l] = hit.u;
+      huv[2 * l + 1] = hit.v;
+      for (int c = 0; c < 3; ++c) hw[3 * l + c] = g[i] * (-hit.sgn * hit.r[c] / hit.dist);
     }
-    hf[i] = f;
   }
+  hf[l] = f;
 }
 
-// one workgroup per control point (f, i, j): out[(f*16 + i*4 + j)*3 + c] = sum over its corners
+// one workgroup per control point (f, i, j): out[(f*16 + i*4 + j)*3 + c] = sum over the listed corners
 __global__ void k_bz_reduce(const int* __restrict__ hf, const double* __restrict__ huv, const double* __restrict__ hw,
-                            long n, double* __restrict__ out) {
+                            int count, double* __restrict__ out) {
   __shared__ double lds[3][256];
   const int cp = blockIdx.x, f = cp / 16, bi = (cp / 4) % 4, bj = cp % 4;
   double acc[3] = {0.0, 0.0, 0.0};
-  for (long k = threadIdx.x; k < n; k += blockDim.x) {
+  for (int k = threadIdx.x; k < count; k += blockDim.x) {
     if (hf[k] != f) continue;
     double bu[4], dbu[4], ddbu[4], bv[4], dbv[4], ddbv[4];
     bz_basis(huv[2 * k], bu, dbu, ddbu);
@@ -1480,29 +1680,33 @@ double drag(const int* type, const double* tx, const double* dy, const double* d
   return J;
 }
 
-void perturb_class(const double* phi_raw, int N, int M, int K, Box box, int cls, double h, double* phi_p,
-                   double* phi_m, hipStream_t s) {
-  k_perturb<<<grid_1d((long)N * M * K), 256, 0, s>>>(phi_raw, N, M, K, box, cls, h, phi_p, phi_m);
+int active_blocks(long n) { return (int)((n + AC_NODES - 1) / AC_NODES); }
+
+void active_corners(const double* phi_raw, const double* phi, int N, int M, int K, Box box, double h, int* count, int* list,
+                    hipStream_t s) {
+  const int nb = active_blocks((long)N * M * K);
+  if (!list) {
+    k_active<<<nb, 256, 0, s>>>(phi_raw, phi, N, M, K, box, h, count, nullptr);
+    k_active_scan<<<1, 1024, 0, s>>>(count, nb);
+  } else {
+    k_active<<<nb, 256, 0, s>>>(phi_raw, phi, N, M, K, box, h, count, list);
+  }
 }
 
-void lagrangian_diff(const GeoView& gp, const GeoView& gm, const double* dx, const double* dy, const double* dz, int N,
-                     int M, int K, Box box, int pin, const double* p, const double* lam, int objective,
-                     const RhsArgs* rhs, double h, double* dF, hipStream_t s) {
+void corner_gradient(const GeoBase& g, const int* list, const int* total, int most, const double* dx, const double* dy,
+                     const double* dz, int N, int M, int K, Box box, int pin, const double* p, const double* lam,
+                     int objective, const RhsArgs* rhs, double h, double* out, hipStream_t s) {
   RhsIn in{nullptr, nullptr, nullptr, nullptr, nullptr, FlowBc{0, 0, 0, 0, 0, 0}};
   if (rhs) in = RhsIn{rhs->u, rhs->v, rhs->w, rhs->u_west, rhs->u_out, rhs->bc};
-  k_lagr_diff<<<grid_1d((long)N * M * K), 256, 0, s>>>(gp, gm, dx, dy, dz, N, M, K, box, pin, p, lam, objective,
-                                                       rhs ? 1 : 0, in, 0.5 / h, dF);
+  if (most < 1) return;
+  k_corner<<<most < 4096 ? most : 4096, 256, 0, s>>>(g, list, total, dx, dy, dz, N, M, K, box, pin, p, lam, objective,
+                                                     rhs ? 1 : 0, in, h, 0.5 / h, out);
 }
 
-void corner_gather(const double* dF, int N, int M, int K, Box box, int cls, double* g, hipStream_t s) {
-  k_corner_gather<<<grid_1d((long)N * M * K), 256, 0, s>>>(dF, N, M, K, box, cls, g);
-}
-
-void bezier_chain(const double* g, const double* cx, const double* cy, const double* cz, int N, int M, int K, Box box,
-                  Body body, int* hf, double* huv, double* hw, double* out, hipStream_t s) {
-  const long n = (long)N * M * K;
-  k_bz_hits<<<grid_1d(n), 256, 0, s>>>(g, cx, cy, cz, N, M, K, box, body, hf, huv, hw);
-  k_bz_reduce<<<96, 256, 0, s>>>(hf, huv, hw, n, out);
+void bezier_chain(const double* g, const int* list, int count, const double* cx, const double* cy, const double* cz,
+                  int N, int M, Body body, int* hf, double* huv, double* hw, double* out, hipStream_t s) {
+  if (count > 0) k_bz_hits<<<(count + 63) / 64, 64, 0, s>>>(g, list, count, cx, cy, cz, N, M, body, hf, huv, hw);
+  k_bz_reduce<<<96, 256, 0, s>>>(hf, huv, hw, count, out);
 }
 
 }  // namespace geo
