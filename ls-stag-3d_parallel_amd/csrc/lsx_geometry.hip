@@ -1308,10 +1308,15 @@ void pressure_rhs(const int* type, const double* tx, const double* ty, const dou
 //
 // A corner whose level set and whose neighbours' along the axes, before and after the fix, lie on one
 // side of the surface by more than the step changes no edge fraction and no sign, so its difference
-// is exactly 0: only the corners along the surface are worked on (k_active_*: their list, in index order), one
+// is exactly 0: where the fix moved no node that another fixed node had read (at most two of its
+// passes, every body of a few cells' thickness), only the corners along the surface are worked on (k_active_*: their list, in index order), one
 // workgroup each (k_corner), which rebuilds the geometry of the 6^3 cells around its corner twice in
 // LDS and reads the unmoved geometry outside them.  72 x 64 x 64 cells, 3210 corners: 224 us (two
-// rebuilds of the whole grid for each of 216 classes of corners 6 apart: 59 ms).
+// rebuilds of the whole grid for each of 216 classes of corners 6 apart: 59 ms).  Longer chains of
+// fixed nodes carry a move out of the corner's reach; such bodies keep the classes: corners 6 apart
+// in every direction have disjoint reach, so one pair of rebuilds with all corners of a class
+// (x mod 6, y mod 6, z mod 6) moved gives the differences of all of them, and what a chain carries
+// further is counted with the class's next corner.
 namespace {
 
 __device__ inline bool cut_cell(int t) { return t > 0 && t != FluidCell; }
@@ -1348,6 +1353,99 @@ __device__ inline double drag_cell(const G& g, int x, int y, int z, const double
   return (g.theta(0, -1, 0, 0) - g.theta(0, 0, 0, 0)) * dys[y] * dzs[z] * p;
 }
 
+// ---- all corners of a class at once
+constexpr int SG_SPACING = 6;
+
+__device__ inline int corner_class(int x, int y, int z) {
+  return x % SG_SPACING + SG_SPACING * (y % SG_SPACING) + SG_SPACING * SG_SPACING * (z % SG_SPACING);
+}
+
+__global__ void k_perturb(const double* __restrict__ phi_raw, int N, int M, int K, Box box, int cls, double h,
+                          double* __restrict__ phi_p, double* __restrict__ phi_m) {
+  const long n = (long)N * M * K;
+  for (long i = blockIdx.x * (long)blockDim.x + threadIdx.x; i < n; i += (long)gridDim.x * blockDim.x) {
+    int x, y, z;
+    decode(i, N, M, &x, &y, &z);
+    const double v = phi_raw[i];
+    const bool on = in_box(x, y, box) && corner_class(x, y, z) == cls;
+    phi_p[i] = on ? v + h : v;
+    phi_m[i] = on ? v - h : v;
+  }
+}
+
+// (F_i(+) - F_i(-)) / 2h of cell i from its fields in the two moved geometries
+struct LagrArgs {
+  const double *dxs, *dys, *dzs, *p, *lam;
+  int N, M, K, pin, objective, has_rhs;
+  Box box;
+  RhsIn rin;
+  double inv2h;
+};
+template <class G>
+__device__ inline double lagr_diff(const G& gp, const G& gm, long i, int x, int y, int z, const LagrArgs& a) {
+  const int N = a.N, M = a.M, K = a.K;
+  const long NM = (long)N * M;
+  const double* __restrict__ p = a.p;
+  double dJ = 0.0;
+  if (a.objective == OBJ_DRAG_X && in_box(x, y, a.box)) {
+    if (cut_cell(gp.type()) && cut_cell(gm.type())) {
+      const double dw = gp.theta(0, -1, 0, 0) - gm.theta(0, -1, 0, 0);
+      const double de = gp.theta(0, 0, 0, 0) - gm.theta(0, 0, 0, 0);
+      dJ = (dw - de) * a.dys[y] * a.dzs[z] * p[i];
+    } else {
+      dJ = drag_cell(gp, x, y, z, a.dys, a.dzs, a.box, p[i]) - drag_cell(gm, x, y, z, a.dys, a.dzs, a.box, p[i]);
+    }
+  }
+  double ca[7], cb[7];
+  laplace_row(gp, i, x, y, z, a.dxs, a.dys, a.dzs, N, M, a.pin, ca);
+  laplace_row(gm, i, x, y, z, a.dxs, a.dys, a.dzs, N, M, a.pin, cb);
+  const long nb[7] = {i - NM, i - N, i - 1, i, i + 1, i + N, i + NM};
+  const bool has[7] = {z > 0, y > 0, x > 0, true, x < N - 1, y < M - 1, z < K - 1};
+  double dAp = 0.0;
+  for (int q = 0; q < 7; ++q)
+    if (has[q]) dAp += (ca[q] - cb[q]) * p[nb[q]];
+  double db = 0.0;
+  if (a.has_rhs)
+    db = rhs_cell(gp, i, x, y, z, a.dxs, a.dys, a.dzs, N, M, K, a.rin) -
+         rhs_cell(gm, i, x, y, z, a.dxs, a.dys, a.dzs, N, M, K, a.rin);
+  return (dJ + a.lam[i] * (db - dAp)) * a.inv2h;
+}
+
+__global__ void k_lagr_diff(GeoView gp, GeoView gm, LagrArgs a, double* __restrict__ dF) {
+  const long n = (long)a.N * a.M * a.K, NM = (long)a.N * a.M;
+  for (long i = blockIdx.x * (long)blockDim.x + threadIdx.x; i < n; i += (long)gridDim.x * blockDim.x) {
+    int x, y, z;
+    decode(i, a.N, a.M, &x, &y, &z);
+    const GridCell cp{gp.type, {gp.tx, gp.ty, gp.tz}, gp.vof, i, a.N, NM};
+    const GridCell cm{gm.type, {gm.tx, gm.ty, gm.tz}, gm.vof, i, a.N, NM};
+    dF[i] = lagr_diff(cp, cm, i, x, y, z, a);
+  }
+}
+
+// g[c] = sum of dF over the reach of corner c, for the corners of class `cls`
+__global__ void k_corner_gather(const double* __restrict__ dF, int N, int M, int K, Box box, int cls,
+                                double* __restrict__ g) {
+  const long n = (long)N * M * K, NM = (long)N * M;
+  for (long c = blockIdx.x * (long)blockDim.x + threadIdx.x; c < n; c += (long)gridDim.x * blockDim.x) {
+    int x, y, z;
+    decode(c, N, M, &x, &y, &z);
+    if (!in_box(x, y, box) || corner_class(x, y, z) != cls) continue;
+    double acc = 0.0;
+    for (int zz = z - 2; zz <= z + 3; ++zz) {
+      if (zz < 0 || zz >= K) continue;
+      for (int yy = y - 2; yy <= y + 3; ++yy) {
+        if (yy < 0 || yy >= M) continue;
+        for (int xx = x - 2; xx <= x + 3; ++xx) {
+          if (xx < 0 || xx >= N) continue;
+          acc += dF[xx + (long)N * yy + NM * zz];
+        }
+      }
+    }
+    g[c] = acc;
+  }
+}
+
+// ---- the corners along the surface, one workgroup each
 // whether moving corner i by h can change the geometry: its level set and its neighbours', before
 // (raw) and after (phi) the oscillation fix, do not all lie on one side by more than the step
 __device__ inline bool corner_active(const double* __restrict__ raw, const double* __restrict__ phi, long i, int N, int M,
@@ -1368,11 +1466,12 @@ __device__ inline bool corner_active(const double* __restrict__ raw, const doubl
          apart(z + 1 < K, i + NM);
 }
 
-// The list of active corners in index order: blocks of AC_NODES consecutive nodes count theirs
+// The list of active corners (g given: of those with g != 0) in index order: blocks of AC_NODES consecutive nodes count theirs
 // (list null), one workgroup turns the counts into offsets and the total (k_active_scan), and the
 // blocks write (ranks within a block by ballots).
 constexpr int AC_NODES = 1024;
-__global__ void __launch_bounds__(256) k_active(const double* __restrict__ raw, const double* __restrict__ phi, int N, int M, int K, Box box, double h,
+__global__ void __launch_bounds__(256) k_active(const double* __restrict__ raw, const double* __restrict__ phi, const double* __restrict__ g,
+                                                int N, int M, int K, Box box, double h,
                                                 int* __restrict__ count, int* __restrict__ list) {
   __shared__ int waves[4];
   const long n = (long)N * M * K;
@@ -1380,7 +1479,7 @@ __global__ void __launch_bounds__(256) k_active(const double* __restrict__ raw, 
   int at = list ? count[blockIdx.x] : 0;
   for (int q = 0; q < AC_NODES / 256; ++q) {
     const long i = (long)blockIdx.x * AC_NODES + q * 256 + threadIdx.x;
-    const bool on = i < n && corner_active(raw, phi, i, N, M, K, box, h);
+    const bool on = i < n && (g ? g[i] != 0.0 : corner_active(raw, phi, i, N, M, K, box, h));
     const unsigned long long m = __ballot(on);
     if (lane == 0) waves[wave] = __popcll(m);
     __syncthreads();
@@ -1453,11 +1552,10 @@ struct PatchCell {
 // thread per cell of the patch and both moves in turn; the terms of the 216 reached cells are added
 // in index order.  Bound by the latency of its dozen stages; 35 KB of LDS let four share a CU.
 __global__ void __launch_bounds__(256) k_corner(GeoBase g, const int* __restrict__ list, const int* __restrict__ total,
-                                                const double* __restrict__ dxs, const double* __restrict__ dys,
-                                                const double* __restrict__ dzs, int N, int M, int K, Box box, int pin,
-                                                const double* __restrict__ p, const double* __restrict__ lam,
-                                                int objective, int has_rhs, RhsIn rin, double h, double inv2h,
-                                                double* __restrict__ out) {
+                                                LagrArgs la, double h, double* __restrict__ out) {
+  const int N = la.N, M = la.M, K = la.K;
+  const Box& box = la.box;
+  const double *__restrict__ dxs = la.dxs, *__restrict__ dys = la.dys, *__restrict__ dzs = la.dzs;
   __shared__ Patch S[2];
   __shared__ double dF[PCELLS];
   const long NM = (long)N * M;
@@ -1536,29 +1634,7 @@ __global__ void __launch_bounds__(256) k_corner(GeoBase g, const int* __restrict
       if (rx >= 0 && rx < N && ry >= 0 && ry < M && rz >= 0 && rz < K) {
         const long r = rx + (long)N * ry + NM * rz;
         const PatchCell gp{&S[0], g, lx - 1, ly - 1, lz - 1, r, N, NM}, gm{&S[1], g, lx - 1, ly - 1, lz - 1, r, N, NM};
-        double dJ = 0.0;
-        if (objective == OBJ_DRAG_X && in_box(rx, ry, box)) {
-          if (cut_cell(gp.type()) && cut_cell(gm.type())) {
-            const double dw = gp.theta(0, -1, 0, 0) - gm.theta(0, -1, 0, 0);
-            const double de = gp.theta(0, 0, 0, 0) - gm.theta(0, 0, 0, 0);
-            dJ = (dw - de) * dys[ry] * dzs[rz] * p[r];
-          } else {
-            dJ = drag_cell(gp, rx, ry, rz, dys, dzs, box, p[r]) - drag_cell(gm, rx, ry, rz, dys, dzs, box, p[r]);
-          }
-        }
-        double ca[7], cb[7];
-        laplace_row(gp, r, rx, ry, rz, dxs, dys, dzs, N, M, pin, ca);
-        laplace_row(gm, r, rx, ry, rz, dxs, dys, dzs, N, M, pin, cb);
-        const long nb[7] = {r - NM, r - N, r - 1, r, r + 1, r + N, r + NM};
-        const bool has[7] = {rz > 0, ry > 0, rx > 0, true, rx < N - 1, ry < M - 1, rz < K - 1};
-        double dAp = 0.0;
-        for (int q = 0; q < 7; ++q)
-          if (has[q]) dAp += (ca[q] - cb[q]) * p[nb[q]];
-        double db = 0.0;
-        if (has_rhs)
-          db = rhs_cell(gp, r, rx, ry, rz, dxs, dys, dzs, N, M, K, rin) -
-               rhs_cell(gm, r, rx, ry, rz, dxs, dys, dzs, N, M, K, rin);
-        v = (dJ + lam[r] * (db - dAp)) * inv2h;
+        v = lagr_diff(gp, gm, r, rx, ry, rz, la);
       }
       dF[tid] = v;
     }
@@ -1682,25 +1758,46 @@ double drag(const int* type, const double* tx, const double* dy, const double* d
 
 int active_blocks(long n) { return (int)((n + AC_NODES - 1) / AC_NODES); }
 
-void active_corners(const double* phi_raw, const double* phi, int N, int M, int K, Box box, double h, int* count, int* list,
-                    hipStream_t s) {
+void active_corners(const double* phi_raw, const double* phi, const double* g, int N, int M, int K, Box box, double h,
+                    int* count, int* list, hipStream_t s) {
   const int nb = active_blocks((long)N * M * K);
   if (!list) {
-    k_active<<<nb, 256, 0, s>>>(phi_raw, phi, N, M, K, box, h, count, nullptr);
+    k_active<<<nb, 256, 0, s>>>(phi_raw, phi, g, N, M, K, box, h, count, nullptr);
     k_active_scan<<<1, 1024, 0, s>>>(count, nb);
   } else {
-    k_active<<<nb, 256, 0, s>>>(phi_raw, phi, N, M, K, box, h, count, list);
+    k_active<<<nb, 256, 0, s>>>(phi_raw, phi, g, N, M, K, box, h, count, list);
   }
+}
+
+static LagrArgs lagr_args(const double* dx, const double* dy, const double* dz, int N, int M, int K, Box box, int pin,
+                          const double* p, const double* lam, int objective, const RhsArgs* rhs, double h) {
+  RhsIn in{nullptr, nullptr, nullptr, nullptr, nullptr, FlowBc{0, 0, 0, 0, 0, 0}};
+  if (rhs) in = RhsIn{rhs->u, rhs->v, rhs->w, rhs->u_west, rhs->u_out, rhs->bc};
+  return LagrArgs{dx, dy, dz, p, lam, N, M, K, pin, objective, rhs ? 1 : 0, box, in, 0.5 / h};
 }
 
 void corner_gradient(const GeoBase& g, const int* list, const int* total, int most, const double* dx, const double* dy,
                      const double* dz, int N, int M, int K, Box box, int pin, const double* p, const double* lam,
                      int objective, const RhsArgs* rhs, double h, double* out, hipStream_t s) {
-  RhsIn in{nullptr, nullptr, nullptr, nullptr, nullptr, FlowBc{0, 0, 0, 0, 0, 0}};
-  if (rhs) in = RhsIn{rhs->u, rhs->v, rhs->w, rhs->u_west, rhs->u_out, rhs->bc};
   if (most < 1) return;
-  k_corner<<<most < 4096 ? most : 4096, 256, 0, s>>>(g, list, total, dx, dy, dz, N, M, K, box, pin, p, lam, objective,
-                                                     rhs ? 1 : 0, in, h, 0.5 / h, out);
+  k_corner<<<most < 4096 ? most : 4096, 256, 0, s>>>(
+      g, list, total, lagr_args(dx, dy, dz, N, M, K, box, pin, p, lam, objective, rhs, h), h, out);
+}
+
+void perturb_class(const double* phi_raw, int N, int M, int K, Box box, int cls, double h, double* phi_p,
+                   double* phi_m, hipStream_t s) {
+  k_perturb<<<grid_1d((long)N * M * K), 256, 0, s>>>(phi_raw, N, M, K, box, cls, h, phi_p, phi_m);
+}
+
+void lagrangian_diff(const GeoView& gp, const GeoView& gm, const double* dx, const double* dy, const double* dz, int N,
+                     int M, int K, Box box, int pin, const double* p, const double* lam, int objective,
+                     const RhsArgs* rhs, double h, double* dF, hipStream_t s) {
+  k_lagr_diff<<<grid_1d((long)N * M * K), 256, 0, s>>>(
+      gp, gm, lagr_args(dx, dy, dz, N, M, K, box, pin, p, lam, objective, rhs, h), dF);
+}
+
+void corner_gather(const double* dF, int N, int M, int K, Box box, int cls, double* g, hipStream_t s) {
+  k_corner_gather<<<grid_1d((long)N * M * K), 256, 0, s>>>(dF, N, M, K, box, cls, g);
 }
 
 void bezier_chain(const double* g, const int* list, int count, const double* cx, const double* cy, const double* cz,

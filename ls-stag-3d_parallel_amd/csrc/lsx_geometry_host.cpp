@@ -162,6 +162,33 @@ void Geometry::stage_flow(const double* u, const double* v, const double* w, con
   }
 }
 
+void Geometry::Work::alloc(long n) {
+  raw.alloc(n);
+  phi.alloc(n);
+  tmp.alloc(n);
+  ax.alloc(n);
+  ay.alloc(n);
+  az.alloc(n);
+  tx.alloc(n);
+  ty.alloc(n);
+  tz.alloc(n);
+  vof.alloc(n);
+  type.alloc(n);
+  sx.alloc(n);
+  sy.alloc(n);
+  sz.alloc(n);
+  flag.alloc(n);
+}
+
+void Geometry::rebuild_from(Work& w) {
+  if (geo::oscillation_fix(w.raw.p, w.phi.p, w.tmp.p, w.flag.p, dchanged.p, N, M, K, box_, stream) < 0)
+    throw Error(LSX_ERR_HIP, "level-set oscillation fix failed");
+  geo::alpha(w.phi.p, N, M, K, box_, w.ax.p, w.ay.p, w.az.p, stream);
+  geo::types(w.phi.p, N, M, K, box_, w.type.p, w.sx.p, w.sy.p, w.sz.p, stream);
+  geo::theta(w.ax.p, w.ay.p, w.az.p, w.sx.p, w.sy.p, w.sz.p, N, M, K, box_, w.tx.p, w.ty.p, w.tz.p, stream);
+  geo::vof(w.type.p, w.ax.p, w.ay.p, w.az.p, w.tx.p, w.ty.p, w.tz.p, dx.p, dy.p, dz.p, N, M, K, w.vof.p, stream);
+}
+
 double Geometry::drag(const double* p, double* dJdp, int mem) {
   if (!built) throw Error(LSX_ERR_STATE, "geometry not built");
   if (!p) throw Error(LSX_ERR_ARG, "null pressure");
@@ -261,21 +288,41 @@ void Geometry::shape_gradient(const double* p, const double* lam, int objective,
   LSX_HIP(hipMemsetAsync(sg_g.p, 0, nn * sizeof(double), stream));
   const int nb = geo::active_blocks(nn);
   sg_count.alloc(nb + 1);
-  geo::active_corners(phi_raw.p, phi.p, N, M, K, box_, h, sg_count.p, nullptr, stream);
+  auto list_corners = [&](const double* g) {
+    geo::active_corners(phi_raw.p, phi.p, g, N, M, K, box_, h, sg_count.p, nullptr, stream);
+    int count = 0;
+    LSX_HIP(hipMemcpyAsync(&count, sg_count.p + nb, sizeof(int), hipMemcpyDeviceToHost, stream));
+    LSX_HIP(hipStreamSynchronize(stream));
+    if ((size_t)count > sg_list.n) {  // with room for the next body's
+      const size_t cap = (size_t)count + count / 4;
+      sg_list.alloc(cap);
+      sg_f.alloc(cap);
+      sg_uv.alloc(2 * cap);
+      sg_w.alloc(3 * cap);
+    }
+    if (count > 0) geo::active_corners(phi_raw.p, phi.p, g, N, M, K, box_, h, sg_count.p, sg_list.p, stream);
+    return count;
+  };
   int active = 0;
-  LSX_HIP(hipMemcpyAsync(&active, sg_count.p + nb, sizeof(int), hipMemcpyDeviceToHost, stream));
-  LSX_HIP(hipStreamSynchronize(stream));
-  if ((size_t)active > sg_list.n) {  // with room for the next body's
-    const size_t cap = (size_t)active + active / 4;
-    sg_list.alloc(cap);
-    sg_f.alloc(cap);
-    sg_uv.alloc(2 * cap);
-    sg_w.alloc(3 * cap);
+  if (osc_passes <= 2) {
+    active = list_corners(nullptr);
+    const geo::GeoBase base{phi_raw.p, phi.p, {ax.p, ay.p, az.p}, {tx.p, ty.p, tz.p}, vof.p, type.p};
+    geo::corner_gradient(base, sg_list.p, sg_count.p + nb, active, dx.p, dy.p, dz.p, N, M, K, box_, pin, dp, dl,
+                         objective, rhs, h, sg_g.p, stream);
+  } else {  // fixed nodes that read fixed nodes: a move may leave its corner's reach
+    wp.alloc(nn);
+    wm.alloc(nn);
+    sg_dF.alloc(nn);
+    for (int cls = 0; cls < 216; ++cls) {
+      geo::perturb_class(phi_raw.p, N, M, K, box_, cls, h, wp.raw.p, wm.raw.p, stream);
+      rebuild_from(wp);
+      rebuild_from(wm);
+      geo::lagrangian_diff(wp.view(), wm.view(), dx.p, dy.p, dz.p, N, M, K, box_, pin, dp, dl, objective, rhs, h,
+                           sg_dF.p, stream);
+      geo::corner_gather(sg_dF.p, N, M, K, box_, cls, sg_g.p, stream);
+    }
+    if (dJdctrl) active = list_corners(sg_g.p);
   }
-  if (active > 0) geo::active_corners(phi_raw.p, phi.p, N, M, K, box_, h, sg_count.p, sg_list.p, stream);
-  const geo::GeoBase base{phi_raw.p, phi.p, {ax.p, ay.p, az.p}, {tx.p, ty.p, tz.p}, vof.p, type.p};
-  geo::corner_gradient(base, sg_list.p, sg_count.p + nb, active, dx.p, dy.p, dz.p, N, M, K, box_, pin, dp, dl, objective,
-                       rhs, h, sg_g.p, stream);
   LSX_HIP(hipGetLastError());
   if (dJdphi)
     LSX_HIP(hipMemcpyAsync(dJdphi, sg_g.p, nn * sizeof(double),
