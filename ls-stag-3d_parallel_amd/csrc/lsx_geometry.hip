@@ -1308,15 +1308,16 @@ void pressure_rhs(const int* type, const double* tx, const double* ty, const dou
 //
 // A corner whose level set and whose neighbours' along the axes, before and after the fix, lie on one
 // side of the surface by more than the step changes no edge fraction and no sign, so its difference
-// is exactly 0: where the fix moved no node that another fixed node had read (at most two of its
-// passes, every body of a few cells' thickness), only the corners along the surface are worked on (k_active_*: their list, in index order), one
-// workgroup each (k_corner), which rebuilds the geometry of the 6^3 cells around its corner twice in
-// LDS and reads the unmoved geometry outside them.  72 x 64 x 64 cells, 3210 corners: 224 us (two
-// rebuilds of the whole grid for each of 216 classes of corners 6 apart: 59 ms).  Longer chains of
-// fixed nodes carry a move out of the corner's reach; such bodies keep the classes: corners 6 apart
-// in every direction have disjoint reach, so one pair of rebuilds with all corners of a class
-// (x mod 6, y mod 6, z mod 6) moved gives the differences of all of them, and what a chain carries
-// further is counted with the class's next corner.
+// is exactly 0: only the corners along the surface are worked on (k_active: their list, in index
+// order), one workgroup each (k_corner), which rebuilds the geometry around its corner twice in LDS
+// and reads the unmoved geometry outside it.  72 x 64 x 64 cells, 3210 corners: 224 us (two rebuilds
+// of the whole grid for each of 216 classes of corners: 59 ms).
+//
+// A fixed node may have read another fixed node; such chains carry a move beyond its corner's
+// reach.  There (more than two passes of the fix) the corners of a class, 6 apart in every
+// direction with disjoint reach, move together, and what a chain carries further counts with the
+// class's corner that reaches it: the fixed nodes' values under each class's two moves come from a
+// table (k_chain_table), and the corners whose cells read a chained node are listed too.
 namespace {
 
 __device__ inline bool cut_cell(int t) { return t > 0 && t != FluidCell; }
@@ -1353,24 +1354,11 @@ __device__ inline double drag_cell(const G& g, int x, int y, int z, const double
   return (g.theta(0, -1, 0, 0) - g.theta(0, 0, 0, 0)) * dys[y] * dzs[z] * p;
 }
 
-// ---- all corners of a class at once
-constexpr int SG_SPACING = 6;
+// Corners 6 apart in every direction move together: their classes (x mod 6, y mod 6, z mod 6).
+constexpr int SG_SPACING = 6, SG_CLASSES = SG_SPACING * SG_SPACING * SG_SPACING;
 
 __device__ inline int corner_class(int x, int y, int z) {
   return x % SG_SPACING + SG_SPACING * (y % SG_SPACING) + SG_SPACING * SG_SPACING * (z % SG_SPACING);
-}
-
-__global__ void k_perturb(const double* __restrict__ phi_raw, int N, int M, int K, Box box, int cls, double h,
-                          double* __restrict__ phi_p, double* __restrict__ phi_m) {
-  const long n = (long)N * M * K;
-  for (long i = blockIdx.x * (long)blockDim.x + threadIdx.x; i < n; i += (long)gridDim.x * blockDim.x) {
-    int x, y, z;
-    decode(i, N, M, &x, &y, &z);
-    const double v = phi_raw[i];
-    const bool on = in_box(x, y, box) && corner_class(x, y, z) == cls;
-    phi_p[i] = on ? v + h : v;
-    phi_m[i] = on ? v - h : v;
-  }
 }
 
 // (F_i(+) - F_i(-)) / 2h of cell i from its fields in the two moved geometries
@@ -1411,41 +1399,6 @@ __device__ inline double lagr_diff(const G& gp, const G& gm, long i, int x, int 
   return (dJ + a.lam[i] * (db - dAp)) * a.inv2h;
 }
 
-__global__ void k_lagr_diff(GeoView gp, GeoView gm, LagrArgs a, double* __restrict__ dF) {
-  const long n = (long)a.N * a.M * a.K, NM = (long)a.N * a.M;
-  for (long i = blockIdx.x * (long)blockDim.x + threadIdx.x; i < n; i += (long)gridDim.x * blockDim.x) {
-    int x, y, z;
-    decode(i, a.N, a.M, &x, &y, &z);
-    const GridCell cp{gp.type, {gp.tx, gp.ty, gp.tz}, gp.vof, i, a.N, NM};
-    const GridCell cm{gm.type, {gm.tx, gm.ty, gm.tz}, gm.vof, i, a.N, NM};
-    dF[i] = lagr_diff(cp, cm, i, x, y, z, a);
-  }
-}
-
-// g[c] = sum of dF over the reach of corner c, for the corners of class `cls`
-__global__ void k_corner_gather(const double* __restrict__ dF, int N, int M, int K, Box box, int cls,
-                                double* __restrict__ g) {
-  const long n = (long)N * M * K, NM = (long)N * M;
-  for (long c = blockIdx.x * (long)blockDim.x + threadIdx.x; c < n; c += (long)gridDim.x * blockDim.x) {
-    int x, y, z;
-    decode(c, N, M, &x, &y, &z);
-    if (!in_box(x, y, box) || corner_class(x, y, z) != cls) continue;
-    double acc = 0.0;
-    for (int zz = z - 2; zz <= z + 3; ++zz) {
-      if (zz < 0 || zz >= K) continue;
-      for (int yy = y - 2; yy <= y + 3; ++yy) {
-        if (yy < 0 || yy >= M) continue;
-        for (int xx = x - 2; xx <= x + 3; ++xx) {
-          if (xx < 0 || xx >= N) continue;
-          acc += dF[xx + (long)N * yy + NM * zz];
-        }
-      }
-    }
-    g[c] = acc;
-  }
-}
-
-// ---- the corners along the surface, one workgroup each
 // whether moving corner i by h can change the geometry: its level set and its neighbours', before
 // (raw) and after (phi) the oscillation fix, do not all lie on one side by more than the step
 __device__ inline bool corner_active(const double* __restrict__ raw, const double* __restrict__ phi, long i, int N, int M,
@@ -1466,12 +1419,14 @@ __device__ inline bool corner_active(const double* __restrict__ raw, const doubl
          apart(z + 1 < K, i + NM);
 }
 
-// The list of active corners (g given: of those with g != 0) in index order: blocks of AC_NODES consecutive nodes count theirs
+// Lists of nodes in index order: AC_FIXED those that the oscillation fix changed, AC_CORNERS the active
+// corners and those marked.  Blocks of AC_NODES consecutive nodes count theirs
 // (list null), one workgroup turns the counts into offsets and the total (k_active_scan), and the
 // blocks write (ranks within a block by ballots).
 constexpr int AC_NODES = 1024;
-__global__ void __launch_bounds__(256) k_active(const double* __restrict__ raw, const double* __restrict__ phi, const double* __restrict__ g,
-                                                int N, int M, int K, Box box, double h,
+__global__ void __launch_bounds__(256) k_active(const double* __restrict__ raw, const double* __restrict__ phi,
+                                                const unsigned char* __restrict__ mark, int mode, int N, int M, int K,
+                                                Box box, double h,
                                                 int* __restrict__ count, int* __restrict__ list) {
   __shared__ int waves[4];
   const long n = (long)N * M * K;
@@ -1479,7 +1434,8 @@ __global__ void __launch_bounds__(256) k_active(const double* __restrict__ raw, 
   int at = list ? count[blockIdx.x] : 0;
   for (int q = 0; q < AC_NODES / 256; ++q) {
     const long i = (long)blockIdx.x * AC_NODES + q * 256 + threadIdx.x;
-    const bool on = i < n && (g ? g[i] != 0.0 : corner_active(raw, phi, i, N, M, K, box, h));
+    const bool on = i < n && (mode == AC_FIXED ? raw[i] != phi[i]
+                                               : (mark && mark[i]) || corner_active(raw, phi, i, N, M, K, box, h));
     const unsigned long long m = __ballot(on);
     if (lane == 0) waves[wave] = __popcll(m);
     __syncthreads();
@@ -1517,16 +1473,105 @@ __global__ void __launch_bounds__(1024) k_active_scan(int* __restrict__ count, i
   if (threadIdx.x == 1023) count[nb] = sum[1023];
 }
 
-// One moved geometry around a corner: nodes and cells c + [-1, 4]^3.
-constexpr int PA = 6, PCELLS = PA * PA * PA;
+// Index of node j in the sorted list of fixed nodes.
+__device__ inline int find_node(const int* __restrict__ list, int count, int j) {
+  int lo = 0, hi = count - 1;
+  while (lo < hi) {
+    const int mid = (lo + hi) >> 1;
+    if (list[mid] < j)
+      lo = mid + 1;
+    else
+      hi = mid;
+  }
+  return lo;
+}
+
+// The level set with the corners of a class moved by +h (move 0) or -h (move 1), before the fix and,
+// from the values `val` of the fixed nodes, after it.
+struct MovedLevelSet {
+  const double* __restrict__ raw0;
+  const double* __restrict__ phi0;
+  const int* __restrict__ list;  // fixed nodes
+  const double* val;
+  int count, cls, move, N, M;
+  double h;
+  Box box;
+  __device__ double raw(long j) const {
+    int x, y, z;
+    decode(j, N, M, &x, &y, &z);
+    const double v = raw0[j];
+    const bool on = in_box(x, y, box) && corner_class(x, y, z) == cls;
+    return on ? (move == 0 ? v + h : v - h) : v;
+  }
+  __device__ double fixed(long j) const {
+    return raw0[j] != phi0[j] ? val[find_node(list, count, (int)j)] : raw(j);
+  }
+};
+
+// table[(cls * 2 + move) * count + l] = level set of fixed node l after the fix with the corners of class cls
+// moved: one workgroup per class and move repeats k_osc_iter's pass over the list until nothing
+// changes (a node depends on lower ones only, so that is the ordered sweep's result whatever the
+// order of the updates within a pass)
+__global__ void __launch_bounds__(256) k_chain_table(const double* __restrict__ raw0, const double* __restrict__ phi0,
+                                                     const int* __restrict__ list, int count, int N, int M, int K,
+                                                     Box box, double h, double* table) {
+  const long NM = (long)N * M;
+  volatile double* val = table + (long)blockIdx.x * count;
+  const MovedLevelSet f{raw0, phi0, list, table + (long)blockIdx.x * count, count, (int)blockIdx.x / 2,
+                        (int)blockIdx.x % 2, N, M, h, box};
+  for (int l = threadIdx.x; l < count; l += blockDim.x) val[l] = phi0[list[l]];
+  for (;;) {
+    __threadfence_block();
+    __syncthreads();
+    bool changed = false;
+    for (int l = threadIdx.x; l < count; l += blockDim.x) {
+      const long j = list[l];
+      const int z = (int)(j / NM);
+      auto lower = [&](long k) {
+        return raw0[k] != phi0[k] ? (double)val[find_node(list, count, (int)k)] : f.raw(k);
+      };
+      double v = f.raw(j);
+      check_osc(v, lower(j - 1), f.raw(j + 1));
+      check_osc(v, lower(j - N), f.raw(j + N));
+      if (z > 0 && z < K - 1) check_osc(v, lower(j - NM), f.raw(j + NM));
+      if (v != val[l]) {
+        val[l] = v;
+        changed = true;
+      }
+    }
+    if (!__syncthreads_or(changed)) break;
+  }
+}
+
+// mark the corners whose cells read a fixed node next to a lower fixed one: its cells' rows reach the
+// corners within 4 of it
+__global__ void __launch_bounds__(256) k_chain_mark(const double* __restrict__ raw0, const double* __restrict__ phi0,
+                                                    const int* __restrict__ list, int N, int M, int K, Box box,
+                                                    unsigned char* __restrict__ mark) {
+  const long NM = (long)N * M, j = list[blockIdx.x];
+  int x, y, z;
+  decode(j, N, M, &x, &y, &z);
+  auto fixed = [&](long k) { return raw0[k] != phi0[k]; };
+  if (!fixed(j - 1) && !fixed(j - N) && !(z > 0 && fixed(j - NM))) return;
+  for (int q = threadIdx.x; q < 729; q += blockDim.x) {
+    const int cx = x + q % 9 - 4, cy = y + q / 9 % 9 - 4, cz = z + q / 81 - 4;
+    if (cx >= 0 && cx < N && cy >= 0 && cy < M && cz >= 0 && cz < K && in_box(cx, cy, box))
+      mark[cx + (long)N * cy + NM * cz] = 1;
+  }
+}
+
+// One moved geometry around a corner: cells c + [LO, LO + PA - 1]^3.
+template <int PA>
 struct Patch {
-  double phi[PCELLS], a[3][PCELLS], t[3][PCELLS], vof[PCELLS];
-  int type[PCELLS];
+  static constexpr int CELLS = PA * PA * PA;
+  double phi[CELLS], a[3][CELLS], t[3][CELLS], vof[CELLS];
+  int type[CELLS];
 };
 // the fields near a cell at (lx, ly, lz) of the patch, grid index i: the patch's inside it, the
 // unmoved geometry's outside
+template <int PA>
 struct PatchCell {
-  const Patch* s;
+  const Patch<PA>* s;
   const GeoBase& g;
   int lx, ly, lz;
   long i;
@@ -1547,93 +1592,117 @@ struct PatchCell {
   }
 };
 
-// g[c] = dF/dphi_c of the listed corners, a workgroup at a time; total = count[nb] of the list.
-// Every stage is the whole grid's (alpha_of, type_of, theta_of, vof_of, laplace_row, rhs_cell), one
-// thread per cell of the patch and both moves in turn; the terms of the 216 reached cells are added
-// in index order.  Bound by the latency of its dozen stages; 35 KB of LDS let four share a CU.
-__global__ void __launch_bounds__(256) k_corner(GeoBase g, const int* __restrict__ list, const int* __restrict__ total,
-                                                LagrArgs la, double h, double* __restrict__ out) {
+// out[c] = dF/dphi_c of the listed corners, a workgroup at a time.  Every stage is the whole grid's
+// (alpha_of, type_of, theta_of, vof_of, laplace_row, rhs_cell), one thread per cell of the patch and
+// both moves in turn; the terms of the 216 reached cells are added in index order.  Bound by the
+// latency of its dozen stages.  Without chains the corner's move changes nodes and cells c + [-1, 4]^3 at
+// most and the fix is repeated in LDS (31 KB: four workgroups share a CU); CHAIN: every cell and edge
+// that the rows of the reach read, c + [-4, 4]^3, with the fixed nodes' values from the table.
+template <bool CHAIN>
+__global__ void __launch_bounds__(CHAIN ? 768 : 256) k_corner(GeoBase g, const int* __restrict__ list, int n_active,
+                                                              LagrArgs la, double h, const int* __restrict__ fixed,
+                                                              int n_fixed, const double* __restrict__ table,
+                                                              double* __restrict__ out) {
+  constexpr int PA = CHAIN ? 9 : 6, LO = CHAIN ? -4 : -1, CELLS = PA * PA * PA, RA = 6, REACH = RA * RA * RA;
+  __shared__ Patch<PA> S[2];
+  __shared__ double dF[REACH];
   const int N = la.N, M = la.M, K = la.K;
   const Box& box = la.box;
   const double *__restrict__ dxs = la.dxs, *__restrict__ dys = la.dys, *__restrict__ dzs = la.dzs;
-  __shared__ Patch S[2];
-  __shared__ double dF[PCELLS];
   const long NM = (long)N * M;
-  const int tid = threadIdx.x, n_active = total[0];
+  const int tid = threadIdx.x;
   const int lx = tid % PA, ly = tid / PA % PA, lz = tid / (PA * PA);
   for (int w = blockIdx.x; w < n_active; w += gridDim.x) {
     const long c = list[w];
     int cx, cy, cz;
     decode(c, N, M, &cx, &cy, &cz);
-    const int x = cx - 1 + lx, y = cy - 1 + ly, z = cz - 1 + lz;
+    const int x = cx + LO + lx, y = cy + LO + ly, z = cz + LO + lz;
     const long i = x + (long)N * y + NM * z;
-    const bool own = tid < PCELLS && x >= 0 && x < N && y >= 0 && y < M && z >= 0 && z < K;
-    auto raw = [&](int m, long j) {  // the moved level set before the oscillation fix
-      const double v = g.raw[j];
-      return j == c ? (m == 0 ? v + h : v - h) : v;
-    };
-    // oscillation fix (k_osc_flags, k_osc_iter): nodes below the patch hold their unmoved final values
-    bool flag[2] = {false, false};
-    if (own)
-      for (int m = 0; m < 2; ++m) {
-        const double f = raw(m, i);
-        S[m].phi[tid] = f;
-        if (in_box(x, y, box) && f > EQ_DOUBLE)
-          flag[m] = raw(m, i + 1) < 0 || raw(m, i + N) < 0 || (z > 0 && z < K - 1 && raw(m, i + NM) < 0);
-      }
-    for (;;) {
-      __syncthreads();
-      double nxt[2];
-      bool changed = false;
-      for (int m = 0; m < 2; ++m)
-        if (flag[m]) {
-          const PatchCell q{&S[m], g, lx, ly, lz, i, N, NM};
-          double f = raw(m, i);
-          check_osc(f, q.phi(-1, 0, 0), raw(m, i + 1));
-          check_osc(f, q.phi(0, -1, 0), raw(m, i + N));
-          if (z > 0 && z < K - 1) check_osc(f, q.phi(0, 0, -1), raw(m, i + NM));
-          changed = changed || f != S[m].phi[tid];
-          nxt[m] = f;
+    const bool own = tid < CELLS && x >= 0 && x < N && y >= 0 && y < M && z >= 0 && z < K;
+    if constexpr (!CHAIN) {
+      auto raw = [&](int m, long j) {  // the moved level set before the oscillation fix
+        const double v = g.raw[j];
+        return j == c ? (m == 0 ? v + h : v - h) : v;
+      };
+      // oscillation fix (k_osc_flags, k_osc_iter): nodes below the patch hold their unmoved final values
+      bool flag[2] = {false, false};
+      if (own)
+#pragma unroll
+        for (int m = 0; m < 2; ++m) {
+          const double f = raw(m, i);
+          S[m].phi[tid] = f;
+          if (in_box(x, y, box) && f > EQ_DOUBLE)
+            flag[m] = raw(m, i + 1) < 0 || raw(m, i + N) < 0 || (z > 0 && z < K - 1 && raw(m, i + NM) < 0);
         }
-      if (!__syncthreads_or(changed)) break;
-      for (int m = 0; m < 2; ++m)
-        if (flag[m]) S[m].phi[tid] = nxt[m];
+      for (;;) {
+        __syncthreads();
+        double nxt[2];
+        bool changed = false;
+#pragma unroll
+        for (int m = 0; m < 2; ++m)
+          if (flag[m]) {
+            const PatchCell<PA> q{&S[m], g, lx, ly, lz, i, N, NM};
+            double f = raw(m, i);
+            check_osc(f, q.phi(-1, 0, 0), raw(m, i + 1));
+            check_osc(f, q.phi(0, -1, 0), raw(m, i + N));
+            if (z > 0 && z < K - 1) check_osc(f, q.phi(0, 0, -1), raw(m, i + NM));
+            changed = changed || f != S[m].phi[tid];
+            nxt[m] = f;
+          }
+        if (!__syncthreads_or(changed)) break;
+#pragma unroll
+        for (int m = 0; m < 2; ++m)
+          if (flag[m]) S[m].phi[tid] = nxt[m];
+      }
     }
     int side[2][3];
     if (own)
+#pragma unroll
       for (int m = 0; m < 2; ++m) {
-        const PatchCell q{&S[m], g, lx, ly, lz, i, N, NM};
-        auto phi = [&](int dx, int dy, int dz) { return q.phi(dx, dy, dz); };
+        const PatchCell<PA> q{&S[m], g, lx, ly, lz, i, N, NM};
+        const int cls = corner_class(cx, cy, cz);
+        const MovedLevelSet f{g.raw, g.phi, fixed, table + (long)(cls * 2 + m) * n_fixed, n_fixed, cls, m, N, M, h, box};
+        auto phi = [&](int dx, int dy, int dz) {
+          if constexpr (CHAIN)
+            return f.fixed(i + dx + (long)N * dy + NM * dz);
+          else
+            return q.phi(dx, dy, dz);
+        };
         double a[3];
         alpha_of(phi, x, y, z, K, box, a);
         for (int k = 0; k < 3; ++k) S[m].a[k][tid] = a[k];
         S[m].type[tid] = type_of(phi, x, y, z, N, M, K, box, side[m]);
       }
     __syncthreads();
+    // (CHAIN: what the patch's first layer of faces and volumes lacks below it, no row of the reach reads)
     if (own)
+#pragma unroll
       for (int m = 0; m < 2; ++m) {
-        const PatchCell q{&S[m], g, lx, ly, lz, i, N, NM};
+        const PatchCell<PA> q{&S[m], g, lx, ly, lz, i, N, NM};
         double t[3];
         theta_of([&](int k, int dx, int dy, int dz) { return q.alpha(k, dx, dy, dz); }, side[m], x, y, z, K, box, t);
         for (int k = 0; k < 3; ++k) S[m].t[k][tid] = t[k];
       }
     __syncthreads();
     if (own)
+#pragma unroll
       for (int m = 0; m < 2; ++m) {
-        const PatchCell q{&S[m], g, lx, ly, lz, i, N, NM};
+        const PatchCell<PA> q{&S[m], g, lx, ly, lz, i, N, NM};
         S[m].vof[tid] = vof_of(
             S[m].type[tid], dxs[x] * dys[y] * dzs[z],
             [&](int k, int dx, int dy, int dz) { return q.alpha(k, dx, dy, dz); },
             [&](int k, int dx, int dy, int dz) { return q.theta(k, dx, dy, dz); });
       }
     __syncthreads();
-    // the reached cells c + [-2, 3]^3: one cell before the patch's in every direction
-    const int rx = x - 1, ry = y - 1, rz = z - 1;
-    if (tid < PCELLS) {
+    // the reached cells c + [-2, 3]^3
+    if (tid < REACH) {
+      const int ex = tid % RA - 2, ey = tid / RA % RA - 2, ez = tid / (RA * RA) - 2;
+      const int rx = cx + ex, ry = cy + ey, rz = cz + ez;
       double v = 0.0;
       if (rx >= 0 && rx < N && ry >= 0 && ry < M && rz >= 0 && rz < K) {
         const long r = rx + (long)N * ry + NM * rz;
-        const PatchCell gp{&S[0], g, lx - 1, ly - 1, lz - 1, r, N, NM}, gm{&S[1], g, lx - 1, ly - 1, lz - 1, r, N, NM};
+        const PatchCell<PA> gp{&S[0], g, ex - LO, ey - LO, ez - LO, r, N, NM};
+        const PatchCell<PA> gm{&S[1], g, ex - LO, ey - LO, ez - LO, r, N, NM};
         v = lagr_diff(gp, gm, r, rx, ry, rz, la);
       }
       dF[tid] = v;
@@ -1642,7 +1711,7 @@ __global__ void __launch_bounds__(256) k_corner(GeoBase g, const int* __restrict
     if (tid == 0) {
       double acc = 0.0;
 #pragma unroll 8
-      for (int q = 0; q < PCELLS; ++q) acc += dF[q];
+      for (int q = 0; q < REACH; ++q) acc += dF[q];
       out[c] = acc;
     }
     __syncthreads();
@@ -1758,15 +1827,18 @@ double drag(const int* type, const double* tx, const double* dy, const double* d
 
 int active_blocks(long n) { return (int)((n + AC_NODES - 1) / AC_NODES); }
 
-void active_corners(const double* phi_raw, const double* phi, const double* g, int N, int M, int K, Box box, double h,
-                    int* count, int* list, hipStream_t s) {
+void list_nodes(const double* phi_raw, const double* phi, const unsigned char* mark, int mode, int N, int M, int K,
+                Box box, double h, int* count, int* list, hipStream_t s) {
   const int nb = active_blocks((long)N * M * K);
-  if (!list) {
-    k_active<<<nb, 256, 0, s>>>(phi_raw, phi, g, N, M, K, box, h, count, nullptr);
-    k_active_scan<<<1, 1024, 0, s>>>(count, nb);
-  } else {
-    k_active<<<nb, 256, 0, s>>>(phi_raw, phi, g, N, M, K, box, h, count, list);
-  }
+  k_active<<<nb, 256, 0, s>>>(phi_raw, phi, mark, mode, N, M, K, box, h, count, list);
+  if (!list) k_active_scan<<<1, 1024, 0, s>>>(count, nb);
+}
+
+void chain_tables(const double* phi_raw, const double* phi, const int* fixed, int n_fixed, int N, int M, int K, Box box,
+                  double h, double* table, unsigned char* mark, hipStream_t s) {
+  (void)hipMemsetAsync(mark, 0, (size_t)N * M * K, s);
+  k_chain_mark<<<n_fixed, 256, 0, s>>>(phi_raw, phi, fixed, N, M, K, box, mark);
+  k_chain_table<<<2 * SG_CLASSES, 256, 0, s>>>(phi_raw, phi, fixed, n_fixed, N, M, K, box, h, table);
 }
 
 static LagrArgs lagr_args(const double* dx, const double* dy, const double* dz, int N, int M, int K, Box box, int pin,
@@ -1776,28 +1848,17 @@ static LagrArgs lagr_args(const double* dx, const double* dy, const double* dz, 
   return LagrArgs{dx, dy, dz, p, lam, N, M, K, pin, objective, rhs ? 1 : 0, box, in, 0.5 / h};
 }
 
-void corner_gradient(const GeoBase& g, const int* list, const int* total, int most, const double* dx, const double* dy,
-                     const double* dz, int N, int M, int K, Box box, int pin, const double* p, const double* lam,
-                     int objective, const RhsArgs* rhs, double h, double* out, hipStream_t s) {
-  if (most < 1) return;
-  k_corner<<<most < 4096 ? most : 4096, 256, 0, s>>>(
-      g, list, total, lagr_args(dx, dy, dz, N, M, K, box, pin, p, lam, objective, rhs, h), h, out);
-}
-
-void perturb_class(const double* phi_raw, int N, int M, int K, Box box, int cls, double h, double* phi_p,
-                   double* phi_m, hipStream_t s) {
-  k_perturb<<<grid_1d((long)N * M * K), 256, 0, s>>>(phi_raw, N, M, K, box, cls, h, phi_p, phi_m);
-}
-
-void lagrangian_diff(const GeoView& gp, const GeoView& gm, const double* dx, const double* dy, const double* dz, int N,
-                     int M, int K, Box box, int pin, const double* p, const double* lam, int objective,
-                     const RhsArgs* rhs, double h, double* dF, hipStream_t s) {
-  k_lagr_diff<<<grid_1d((long)N * M * K), 256, 0, s>>>(
-      gp, gm, lagr_args(dx, dy, dz, N, M, K, box, pin, p, lam, objective, rhs, h), dF);
-}
-
-void corner_gather(const double* dF, int N, int M, int K, Box box, int cls, double* g, hipStream_t s) {
-  k_corner_gather<<<grid_1d((long)N * M * K), 256, 0, s>>>(dF, N, M, K, box, cls, g);
+void corner_gradient(const GeoBase& g, const int* list, int count, const int* fixed, int n_fixed, const double* table,
+                     const double* dx, const double* dy, const double* dz, int N, int M, int K, Box box, int pin,
+                     const double* p, const double* lam, int objective, const RhsArgs* rhs, double h, double* out,
+                     hipStream_t s) {
+  if (count < 1) return;
+  const LagrArgs la = lagr_args(dx, dy, dz, N, M, K, box, pin, p, lam, objective, rhs, h);
+  const int blocks = count < 4096 ? count : 4096;
+  if (table)
+    k_corner<true><<<blocks, 768, 0, s>>>(g, list, count, la, h, fixed, n_fixed, table, out);
+  else
+    k_corner<false><<<blocks, 256, 0, s>>>(g, list, count, la, h, nullptr, 0, nullptr, out);
 }
 
 void bezier_chain(const double* g, const int* list, int count, const double* cx, const double* cy, const double* cz,

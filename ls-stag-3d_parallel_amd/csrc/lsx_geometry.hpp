@@ -82,11 +82,6 @@ struct GeoBase {
   const double *raw, *phi, *a[3], *t[3], *vof;
   const int* type;
 };
-// its fields that operator rows, right-hand side and drag read
-struct GeoView {
-  const int* type;
-  const double *tx, *ty, *tz, *vof;
-};
 // the flow fields the pressure right-hand side is assembled from (device pointers)
 struct RhsArgs {
   const double *u, *v, *w, *u_west, *u_out;
@@ -105,28 +100,26 @@ void drag_noalloc(const int* type, const double* tx, const double* dy, const dou
 // Address of the library's drag scratch array on the current device (looked up once per device
 // with hipGetSymbolAddress); 0, or a negative value when the lookup fails.
 int drag_scratch(double** out);
-// phi_p = phi_raw + h, phi_m = phi_raw - h at the in-box corners of class cls (x%6 + 6 (y%6) + 36 (z%6))
-void perturb_class(const double* phi_raw, int N, int M, int K, Box box, int cls, double h, double* phi_p,
-                   double* phi_m, hipStream_t s);
-// dF[i] = (F_i(+) - F_i(-)) / 2h with F_i = J_i + lambda_i (b_i - (A p)_i); rhs null: b fixed
-void lagrangian_diff(const GeoView& gp, const GeoView& gm, const double* dx, const double* dy, const double* dz, int N,
-                     int M, int K, Box box, int pin, const double* p, const double* lam, int objective,
-                     const RhsArgs* rhs, double h, double* dF, hipStream_t s);
-// g[c] = sum of dF over cells c + [-2, 3]^3 for the corners c of class cls
-void corner_gather(const double* dF, int N, int M, int K, Box box, int cls, double* g, hipStream_t s);
-// The corners that a move by h can change the geometry at (g given: those with g != 0), in index order.
-// list null: fills
+// Lists of nodes in index order: AC_FIXED those that the oscillation fix changed, AC_CORNERS the corners
+// that a move by h can change the geometry at and (mark given) the marked ones.  list null: fills
 // count[0 .. nb) with the offsets of nb = active_blocks(n) blocks of nodes and count[nb] with the
-// number of corners; list given (after that): writes them.
+// number of listed ones; list given (after that): writes them.
+enum { AC_FIXED = 0, AC_CORNERS = 1 };
 int active_blocks(long n);
-void active_corners(const double* phi_raw, const double* phi, const double* g, int N, int M, int K, Box box, double h,
-                    int* count, int* list, hipStream_t s);
-// out[c] = sum over the cells c + [-2, 3]^3 of (F_i(+) - F_i(-)) / 2h with corner c moved by +h and -h and
-// F_i = J_i + lambda_i (b_i - (A p)_i), for the listed corners (total: their number in device
-// memory, most: on the host); rhs null: b fixed
-void corner_gradient(const GeoBase& g, const int* list, const int* total, int most, const double* dx, const double* dy,
-                     const double* dz, int N, int M, int K, Box box, int pin, const double* p, const double* lam,
-                     int objective, const RhsArgs* rhs, double h, double* out, hipStream_t s);
+void list_nodes(const double* phi_raw, const double* phi, const unsigned char* mark, int mode, int N, int M, int K,
+                Box box, double h, int* count, int* list, hipStream_t s);
+// Where fixed nodes have read fixed nodes: table gets their values with the corners of each class moved
+// by +h and -h (432 n_fixed doubles), mark (n bytes) the corners whose cells read such a node.
+constexpr int CHAIN_MOVES = 432;
+void chain_tables(const double* phi_raw, const double* phi, const int* fixed, int n_fixed, int N, int M, int K, Box box,
+                  double h, double* table, unsigned char* mark, hipStream_t s);
+// out[c] = sum over the cells c + [-2, 3]^3 of (F_i(+) - F_i(-)) / 2h with F_i = J_i + lambda_i (b_i - (A p)_i), for
+// the count listed corners, moved by +h and -h one by one, or (table given) together with the others of
+// their class; rhs null: b fixed
+void corner_gradient(const GeoBase& g, const int* list, int count, const int* fixed, int n_fixed, const double* table,
+                     const double* dx, const double* dy, const double* dz, int N, int M, int K, Box box, int pin,
+                     const double* p, const double* lam, int objective, const RhsArgs* rhs, double h, double* out,
+                     hipStream_t s);
 // out[288] = sum over the count listed corners of g dphi/dctrl through the closest point (hf, huv, hw: count,
 // 2 count, 3 count scratch)
 void bezier_chain(const double* g, const int* list, int count, const double* cx, const double* cy, const double* cz,

@@ -162,31 +162,18 @@ void Geometry::stage_flow(const double* u, const double* v, const double* w, con
   }
 }
 
-void Geometry::Work::alloc(long n) {
-  raw.alloc(n);
-  phi.alloc(n);
-  tmp.alloc(n);
-  ax.alloc(n);
-  ay.alloc(n);
-  az.alloc(n);
-  tx.alloc(n);
-  ty.alloc(n);
-  tz.alloc(n);
-  vof.alloc(n);
-  type.alloc(n);
-  sx.alloc(n);
-  sy.alloc(n);
-  sz.alloc(n);
-  flag.alloc(n);
-}
-
-void Geometry::rebuild_from(Work& w) {
-  if (geo::oscillation_fix(w.raw.p, w.phi.p, w.tmp.p, w.flag.p, dchanged.p, N, M, K, box_, stream) < 0)
-    throw Error(LSX_ERR_HIP, "level-set oscillation fix failed");
-  geo::alpha(w.phi.p, N, M, K, box_, w.ax.p, w.ay.p, w.az.p, stream);
-  geo::types(w.phi.p, N, M, K, box_, w.type.p, w.sx.p, w.sy.p, w.sz.p, stream);
-  geo::theta(w.ax.p, w.ay.p, w.az.p, w.sx.p, w.sy.p, w.sz.p, N, M, K, box_, w.tx.p, w.ty.p, w.tz.p, stream);
-  geo::vof(w.type.p, w.ax.p, w.ay.p, w.az.p, w.tx.p, w.ty.p, w.tz.p, dx.p, dy.p, dz.p, N, M, K, w.vof.p, stream);
+// nodes of a list (geo::AC_*) into `list`, which grows with some room for the next body's; their number
+int Geometry::list_nodes(int mode, const unsigned char* mark, double h, DevBuf<int>& list) {
+  const int nb = geo::active_blocks(n());
+  sg_count.alloc(nb + 1);
+  geo::list_nodes(phi_raw.p, phi.p, mark, mode, N, M, K, box_, h, sg_count.p, nullptr, stream);
+  int count = 0;
+  LSX_HIP(hipMemcpyAsync(&count, sg_count.p + nb, sizeof(int), hipMemcpyDeviceToHost, stream));
+  LSX_HIP(hipStreamSynchronize(stream));
+  if ((size_t)count > list.n) list.alloc((size_t)count + count / 4);
+  if (count > 0)
+    geo::list_nodes(phi_raw.p, phi.p, mark, mode, N, M, K, box_, h, sg_count.p, list.p, stream);
+  return count;
 }
 
 double Geometry::drag(const double* p, double* dJdp, int mem) {
@@ -286,49 +273,30 @@ void Geometry::shape_gradient(const double* p, const double* lam, int objective,
   }
   sg_g.alloc(nn);
   LSX_HIP(hipMemsetAsync(sg_g.p, 0, nn * sizeof(double), stream));
-  const int nb = geo::active_blocks(nn);
-  sg_count.alloc(nb + 1);
-  auto list_corners = [&](const double* g) {
-    geo::active_corners(phi_raw.p, phi.p, g, N, M, K, box_, h, sg_count.p, nullptr, stream);
-    int count = 0;
-    LSX_HIP(hipMemcpyAsync(&count, sg_count.p + nb, sizeof(int), hipMemcpyDeviceToHost, stream));
-    LSX_HIP(hipStreamSynchronize(stream));
-    if ((size_t)count > sg_list.n) {  // with room for the next body's
-      const size_t cap = (size_t)count + count / 4;
-      sg_list.alloc(cap);
-      sg_f.alloc(cap);
-      sg_uv.alloc(2 * cap);
-      sg_w.alloc(3 * cap);
-    }
-    if (count > 0) geo::active_corners(phi_raw.p, phi.p, g, N, M, K, box_, h, sg_count.p, sg_list.p, stream);
-    return count;
-  };
-  int active = 0;
-  if (osc_passes <= 2) {
-    active = list_corners(nullptr);
-    const geo::GeoBase base{phi_raw.p, phi.p, {ax.p, ay.p, az.p}, {tx.p, ty.p, tz.p}, vof.p, type.p};
-    geo::corner_gradient(base, sg_list.p, sg_count.p + nb, active, dx.p, dy.p, dz.p, N, M, K, box_, pin, dp, dl,
-                         objective, rhs, h, sg_g.p, stream);
-  } else {  // fixed nodes that read fixed nodes: a move may leave its corner's reach
-    wp.alloc(nn);
-    wm.alloc(nn);
-    sg_dF.alloc(nn);
-    for (int cls = 0; cls < 216; ++cls) {
-      geo::perturb_class(phi_raw.p, N, M, K, box_, cls, h, wp.raw.p, wm.raw.p, stream);
-      rebuild_from(wp);
-      rebuild_from(wm);
-      geo::lagrangian_diff(wp.view(), wm.view(), dx.p, dy.p, dz.p, N, M, K, box_, pin, dp, dl, objective, rhs, h,
-                           sg_dF.p, stream);
-      geo::corner_gather(sg_dF.p, N, M, K, box_, cls, sg_g.p, stream);
-    }
-    if (dJdctrl) active = list_corners(sg_g.p);
+  // fixed nodes that have read fixed nodes (a third pass of the fix): corners move by classes
+  int n_fixed = 0;
+  if (osc_passes > 2) {
+    n_fixed = list_nodes(geo::AC_FIXED, nullptr, h, sg_fixed);
+    if ((size_t)n_fixed * geo::CHAIN_MOVES > sg_table.n) sg_table.alloc((size_t)(n_fixed + n_fixed / 4) * geo::CHAIN_MOVES);
+    if (n_fixed > 0)
+      geo::chain_tables(phi_raw.p, phi.p, sg_fixed.p, n_fixed, N, M, K, box_, h, sg_table.p, flag.p, stream);
   }
+  const bool chain = n_fixed > 0;
+  const int active = list_nodes(geo::AC_CORNERS, chain ? flag.p : nullptr, h, sg_list);
+  const geo::GeoBase base{phi_raw.p, phi.p, {ax.p, ay.p, az.p}, {tx.p, ty.p, tz.p}, vof.p, type.p};
+  geo::corner_gradient(base, sg_list.p, active, sg_fixed.p, n_fixed, chain ? sg_table.p : nullptr, dx.p, dy.p, dz.p, N, M,
+                       K, box_, pin, dp, dl, objective, rhs, h, sg_g.p, stream);
   LSX_HIP(hipGetLastError());
   if (dJdphi)
     LSX_HIP(hipMemcpyAsync(dJdphi, sg_g.p, nn * sizeof(double),
                            mem == LSX_MEM_HOST ? hipMemcpyDeviceToHost : hipMemcpyDeviceToDevice, stream));
   if (dJdctrl) {
     sg_out.alloc(288);
+    if ((size_t)active > sg_f.n) {
+      sg_f.alloc(sg_list.n);
+      sg_uv.alloc(2 * sg_list.n);
+      sg_w.alloc(3 * sg_list.n);
+    }
     geo::bezier_chain(sg_g.p, sg_list.p, active, cx.p, cy.p, cz.p, N, M, body_, sg_f.p, sg_uv.p, sg_w.p, sg_out.p,
                       stream);
     LSX_HIP(hipGetLastError());

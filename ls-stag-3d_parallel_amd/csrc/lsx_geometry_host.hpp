@@ -97,21 +97,11 @@ class Geometry {
   DevBuf<double> bez;  // Bezier control values (device)
   geo::Body body_{};
   geo::Box box_{};
-  // shape-gradient work, by classes: two moved geometries and dF per cell
-  struct Work {
-    DevBuf<double> raw, phi, tmp, ax, ay, az, tx, ty, tz, vof;
-    DevBuf<int> type, sx, sy, sz;
-    DevBuf<unsigned char> flag;
-    void alloc(long n);
-    geo::GeoView view() const { return geo::GeoView{type.p, tx.p, ty.p, tz.p, vof.p}; }
-  };
-  Work wp, wm;
-  DevBuf<double> sg_dF;
-  void rebuild_from(Work& w);  // fields of w from w.raw (oscillation fix onwards)
-  // by corners: the list of active corners and its offsets, g per corner, closest points of
-  // the listed ones
-  DevBuf<double> sg_g, sg_uv, sg_w, sg_partial, sg_out;
-  DevBuf<int> sg_count, sg_list, sg_f;
+  // shape-gradient work: node lists and their offsets, the fixed nodes' values per class and move, g
+  // per corner, closest points of the listed corners
+  DevBuf<double> sg_g, sg_uv, sg_w, sg_partial, sg_out, sg_table;
+  DevBuf<int> sg_count, sg_list, sg_fixed, sg_f;
+  int list_nodes(int mode, const unsigned char* mark, double h, DevBuf<int>& list);
 };
 
 }  // namespace lsx
