@@ -696,16 +696,8 @@ void Solver::vcycle_run(const double* v, T* z, const float* b32) {
   } else {
     b0 = v;
   }
-  // levels from `lc` down are small enough for one workgroup: a single launch does their cycle
-  int lc = L + 1;
-  const bool fuse_ok = opt.coarse_fuse && (!dense_c.p || vlev[L].L.d.n() <= vc::COARSE_DENSE);
-  for (int l = 1; l <= L && fuse_ok; ++l)
-    if (rb_level(l) && vlev[l].L.d.n() <= vc::COARSE_CELLS && L - l + 1 <= vc::COARSE_MAX) {
-      lc = l;
-      break;
-    }
-  if (lc == L) lc = L + 1;  // the LU level alone gains nothing
-  const int top = lc <= L ? lc : L;
+  vc::CoarseLevels<T> C;
+  const int top = coarse_levels<T>(C);
   for (int l = 0; l < top; ++l) {
     VStore& S = vlev[l];
     T* x = l == 0 ? z : vx<T>(S);
@@ -713,18 +705,10 @@ void Solver::vcycle_run(const double* v, T* z, const float* b32) {
     smooth<T>(l, x, b, opt.n_pre, true);
     vc::resid_restrict<T>(S.L, x, b, vb<T>(vlev[l + 1]), stream);
   }
-  if (lc <= L) {
-    vc::CoarseLevels<T> C;
-    C.count = L - lc + 1;
-    for (int q = 0; q < C.count; ++q) {
-      C.L[q] = vlev[lc + q].L;
-      C.x[q] = vx<T>(vlev[lc + q]);
-      C.b[q] = vb<T>(vlev[lc + q]);
-    }
-    vc::coarse_cycle<T>(C, opt.n_pre, opt.n_post, lu_scale.p, lu_perm.p, lu_L.p, lu_U.p, dense_c.p, stream);
-  } else {
+  if (C.count)
+    vc::coarse_cycle<T>(C, 0, opt.n_pre, opt.n_post, lu_scale.p, lu_perm.p, lu_L.p, lu_U.p, dense_c.p, stream);
+  else
     coarse_solve<T>(false);
-  }
   for (int l = top - 1; l >= 0; --l) {
     VStore& S = vlev[l];
     T* x = l == 0 ? z : vx<T>(S);
@@ -732,6 +716,24 @@ void Solver::vcycle_run(const double* v, T* z, const float* b32) {
     vc::prolong_add<T>(vx<T>(vlev[l + 1]), vlev[l + 1].L.d, x, S.L.d, stream);
     smooth<T>(l, x, b, opt.n_post, false, true);  // lines z, y, x: the cycle is symmetric in its line order
   }
+}
+
+// The levels from the returned one down are small enough for one workgroup, which runs their cycle in
+// a single launch (C, empty if there are none: the last level is then returned)
+template <class T>
+int Solver::coarse_levels(vc::CoarseLevels<T>& C) {
+  const int L = (int)vlev.size() - 1;
+  if (!opt.coarse_fuse || (dense_c.p && vlev[L].L.d.n() > vc::COARSE_DENSE)) return L;
+  for (int l = 1; l < L; ++l) {  // the LU level alone gains nothing
+    if (!rb_level(l) || L - l + 1 > vc::COARSE_MAX) continue;
+    C.count = L - l + 1;
+    for (int q = 0; q < C.count; ++q) C.L[q] = vlev[l + q].L;
+    C.x = vx<T>(vlev[l]);
+    C.b = vb<T>(vlev[l]);
+    if (vc::coarse_fits<T>(C)) return l;
+  }
+  C.count = 0;
+  return L;
 }
 
 // `sweeps` smoothing sweeps of level l on x (zero_guess: x is taken as 0 and not read).
@@ -823,7 +825,7 @@ void Solver::smooth(int l, T* x, const T* b, int sweeps, bool zero_guess, bool r
 
 // The transpose of vcycle_apply: its steps in reverse order, each transposed (half-sweeps in the
 // opposite colour order on A^T, restriction by P^T, prolongation by the transposed sum
-// restriction, the symmetric coarsest LU unchanged).  Levels are launched one by one.
+// restriction, the symmetric coarsest LU unchanged).
 template <class T>
 void Solver::vcycle_apply_tr(const double* v, T* z) {
   const int L = (int)vlev.size() - 1;
@@ -843,7 +845,9 @@ void Solver::vcycle_apply_tr(const double* v, T* z) {
         S.dr.alloc(S.L.d.n());
     }
   }
-  for (int l = 0; l < L; ++l) {
+  vc::CoarseLevels<T> C;
+  const int top = coarse_levels<T>(C);
+  for (int l = 0; l < top; ++l) {
     VStore& S = vlev[l];
     T* x = l == 0 ? z : vx<T>(S);
     const T* b = l == 0 ? b0 : vb<T>(S);
@@ -851,8 +855,11 @@ void Solver::vcycle_apply_tr(const double* v, T* z) {
     vc::resid_tr<T>(S.L, x, b, vr<T>(S), stream);
     vc::restrict_pt<T>(vr<T>(S), S.L.d, vb<T>(vlev[l + 1]), stream);
   }
-  coarse_solve<T>(true);
-  for (int l = L - 1; l >= 0; --l) {
+  if (C.count)
+    vc::coarse_cycle<T>(C, 1, opt.n_post, opt.n_pre, lu_scale.p, lu_perm.p, lu_L.p, lu_U.p, dense_r.p, stream);
+  else
+    coarse_solve<T>(true);
+  for (int l = top - 1; l >= 0; --l) {
     VStore& S = vlev[l];
     T* x = l == 0 ? z : vx<T>(S);
     const T* b = l == 0 ? b0 : vb<T>(S);

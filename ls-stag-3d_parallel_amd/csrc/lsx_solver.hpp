@@ -158,6 +158,8 @@ class Solver {
   DevBuf<double> dense_c, dense_r, dense_part;
   template <class T>
   void coarse_solve(bool transposed);
+  template <class T>
+  int coarse_levels(vc::CoarseLevels<T>& C);
   DevBuf<double> cwork;   // correction increment c (fine size, reused on every level)
   DevBuf<double> partial, scalars;
   DevBuf<double> mpartial, cgs_h;  // block Gram-Schmidt partial sums and coefficients

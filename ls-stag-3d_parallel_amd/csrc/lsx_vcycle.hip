@@ -13,6 +13,7 @@
 #include <algorithm>
 #include <type_traits>
 
+#include "lsx_lu.hpp"
 #include "lsx_vcycle.hpp"
 
 namespace lsx {
@@ -371,20 +372,20 @@ __device__ inline T offdiag_fsum(const T* __restrict__ x, const FT* __restrict__
   return fw * xw + fe * xe + fs_ * xs + fn * xn + fb * xb + ft * xt;
 }
 
-// one colour of a red-black sweep; work item t (from start, by stride) owns the t-th cell of it.
+// one colour of a red-black sweep; thread t owns the t-th cell of it.
 // zero_guess: 0 normal; 1 x is zero before this half-sweep; 2 first update of this colour after
 // a zero start (its values are not read).  An empty row (1/a_p stored as 0) keeps its value, so
 // that every step has the form x + W (b - A x) and the cycle's transpose is the transposed cycle.
 template <class T, class FT>
-__device__ inline void rbgs_body(T* __restrict__ x, const T* __restrict__ b, const FT* __restrict__ ae,
-                                 const FT* __restrict__ an, const FT* __restrict__ at, const T* __restrict__ s, T fs,
-                                 int N, int M, int K, int color, int pin0, int pin1, int zero_guess, long start,
-                                 long stride) {
+__global__ void k_rbgs(T* __restrict__ x, const T* __restrict__ b, const FT* __restrict__ ae, const FT* __restrict__ an,
+                       const FT* __restrict__ at, const T* __restrict__ s, T fs, int N, int M, int K, int color,
+                       int pin0, int pin1, int zero_guess) {
   // 32-bit index arithmetic (a level has fewer than 2^31 cells); the neighbours' loads are issued
   // unconditionally (offdiag_u: the same sum in the same order)
   const unsigned half_row = (unsigned)(N + 1) / 2;
   const unsigned total = half_row * (unsigned)M * (unsigned)K;
-  for (long t = start; t < (long)total; t += stride) {
+  const long stride = (long)gridDim.x * blockDim.x;
+  for (long t = blockIdx.x * (long)blockDim.x + threadIdx.x; t < (long)total; t += stride) {
     const unsigned tt = (unsigned)t, row = tt / half_row;
     const int yy = (int)(row % (unsigned)M), zz = (int)(row / (unsigned)M);
     const int xx = 2 * (int)(tt - row * half_row) + ((yy + zz + color) & 1);
@@ -403,14 +404,6 @@ __device__ inline void rbgs_body(T* __restrict__ x, const T* __restrict__ b, con
     }
     x[i] = v;
   }
-}
-
-template <class T, class FT>
-__global__ void k_rbgs(T* __restrict__ x, const T* __restrict__ b, const FT* __restrict__ ae, const FT* __restrict__ an,
-                       const FT* __restrict__ at, const T* __restrict__ s, T fs, int N, int M, int K, int color,
-                       int pin0, int pin1, int zero_guess) {
-  rbgs_body<T, FT>(x, b, ae, an, at, s, fs, N, M, K, color, pin0, pin1, zero_guess,
-                   blockIdx.x * (long)blockDim.x + threadIdx.x, (long)gridDim.x * blockDim.x);
 }
 
 // bc = sum over the children of (b - A x): one thread per fine cell (64 adjacent x by 2 y by 2 z
@@ -546,32 +539,45 @@ __device__ inline float axis_wt(int f, int nf, int C) {
   return v;
 }
 
-template <class T>
-__global__ void k_restrict_pt(const T* __restrict__ r, int Nf, int Mf, int Kf, T* __restrict__ bc) {
-  const int Nc = (Nf + 1) / 2, Mc = (Mf + 1) / 2, Kc = (Kf + 1) / 2;
-  const long nc = (long)Nc * Mc * Kc, NMf = (long)Nf * Mf;
-  for (long I = blockIdx.x * (long)blockDim.x + threadIdx.x; I < nc; I += (long)gridDim.x * blockDim.x) {
-    int X, Y, Z;
-    decode(I, Nc, Mc, &X, &Y, &Z);
-    T acc = 0;
-    for (int fz = 2 * Z - 1; fz <= 2 * Z + 2; ++fz) {
-      if (fz < 0 || fz >= Kf) continue;
-      const float wz = axis_wt(fz, Kf, Z);
-      if (wz == 0.0f) continue;
-      for (int fy = 2 * Y - 1; fy <= 2 * Y + 2; ++fy) {
-        if (fy < 0 || fy >= Mf) continue;
-        const float wy = axis_wt(fy, Mf, Y);
-        if (wy == 0.0f) continue;
-        for (int fx = 2 * X - 1; fx <= 2 * X + 2; ++fx) {
-          if (fx < 0 || fx >= Nf) continue;
-          const float wx = axis_wt(fx, Nf, X);
-          if (wx == 0.0f) continue;
-          acc += (T)(wx * wy * wz) * r[fx + (long)Nf * fy + NMf * fz];
-        }
-      }
+// One coarse cell of P^T r: the 4 x 4 x 4 fine cells around it, z outermost; `at` reads a fine cell.
+// Straight-line code: a tap without weight (or past the level) reads the cell's first child.
+template <class T, class F>
+__device__ inline T restrict_pt_cell(F at, int X, int Y, int Z, int Nf, int Mf, int Kf) {
+  auto taps = [](int C, int nf, int (&f)[4], float (&w)[4]) {
+#pragma unroll
+    for (int k = 0; k < 4; ++k) {
+      const int q = 2 * C - 1 + k;
+      const bool in = q >= 0 && q < nf;
+      w[k] = in ? axis_wt(q, nf, C) : 0.0f;
+      f[k] = in ? q : 2 * C;
     }
-    bc[I] = acc;
+  };
+  int fx[4], fy[4], fz[4];
+  float wx[4], wy[4], wz[4];
+  taps(X, Nf, fx, wx);
+  taps(Y, Mf, fy, wy);
+  taps(Z, Kf, fz, wz);
+  T acc = 0;
+#pragma unroll
+  for (int c3 = 0; c3 < 4; ++c3) {
+    T v[16];
+#pragma unroll
+    for (int q = 0; q < 16; ++q) v[q] = at(fx[q & 3], fy[q >> 2], fz[c3]);
+#pragma unroll
+    for (int q = 0; q < 16; ++q) acc += (T)(wx[q & 3] * wy[q >> 2] * wz[c3]) * v[q];
   }
+  return acc;
+}
+
+template <class T>
+__global__ void __launch_bounds__(256) k_restrict_pt(const T* __restrict__ r, int Nf, int Mf, int Kf,
+                                                     T* __restrict__ bc) {
+  const int Nc = (Nf + 1) / 2, Mc = (Mf + 1) / 2, Kc = (Kf + 1) / 2;
+  const long I = blockIdx.x * (long)blockDim.x + threadIdx.x, NMf = (long)Nf * Mf;
+  if (I >= (long)Nc * Mc * Kc) return;
+  int X, Y, Z;
+  decode(I, Nc, Mc, &X, &Y, &Z);
+  bc[I] = restrict_pt_cell<T>([&](int x, int y, int z) { return r[x + (long)Nf * y + NMf * z]; }, X, Y, Z, Nf, Mf, Kf);
 }
 
 template <class T>
@@ -585,40 +591,32 @@ __global__ void k_prolong_inject_add(const T* __restrict__ xc, int Nc, int Mc, T
   }
 }
 
+// the trilinear prolongation at fine cell (x, y, z); `at` reads a coarse cell.  Always two taps per axis
+// (an absent second tap reads the first with weight 0), so that the eight loads are straight-line code
+template <class T, class F>
+__device__ inline T prolong_value(F at, int Nf, int Mf, int Kf, int x, int y, int z) {
+  int cx[2], cy[2], cz[2], nx, ny, nz;
+  float wx[2], wy[2], wz[2];
+  axis_w(x, Nf, cx, wx, &nx);
+  axis_w(y, Mf, cy, wy, &ny);
+  axis_w(z, Kf, cz, wz, &nz);
+  if (nx < 2) { cx[1] = cx[0]; wx[1] = 0.f; }
+  if (ny < 2) { cy[1] = cy[0]; wy[1] = 0.f; }
+  if (nz < 2) { cz[1] = cz[0]; wz[1] = 0.f; }
+  T v[8];
+#pragma unroll
+  for (int c = 0; c < 8; ++c) v[c] = at(cx[c & 1], cy[(c >> 1) & 1], cz[c >> 2]);
+  T acc = 0;
+#pragma unroll
+  for (int c = 0; c < 8; ++c) acc += (T)(wx[c & 1] * wy[(c >> 1) & 1] * wz[c >> 2]) * v[c];
+  return acc;
+}
+
 template <class T>
 __device__ inline void prolong_cell(const T* __restrict__ xc, int Nc, int Mc, T* __restrict__ xf, int Nf, int Mf,
                                     int Kf, long i, int x, int y, int z) {
   const long NMc = (long)Nc * Mc;
-  {
-    int cx[2], cy[2], cz[2], nx, ny, nz;
-    float wx[2], wy[2], wz[2];
-    axis_w(x, Nf, cx, wx, &nx);
-    axis_w(y, Mf, cy, wy, &ny);
-    axis_w(z, Kf, cz, wz, &nz);
-    // always two taps per axis (an absent second tap reads the first with weight 0), so that the
-    // eight loads are straight-line code
-    if (nx < 2) { cx[1] = cx[0]; wx[1] = 0.f; }
-    if (ny < 2) { cy[1] = cy[0]; wy[1] = 0.f; }
-    if (nz < 2) { cz[1] = cz[0]; wz[1] = 0.f; }
-    T v[8];
-#pragma unroll
-    for (int c = 0; c < 8; ++c) v[c] = xc[cx[c & 1] + Nc * cy[(c >> 1) & 1] + NMc * cz[c >> 2]];
-    T acc = 0;
-#pragma unroll
-    for (int c = 0; c < 8; ++c) acc += (T)(wx[c & 1] * wy[(c >> 1) & 1] * wz[c >> 2]) * v[c];
-    xf[i] += acc;
-  }
-}
-
-template <class T>
-__device__ inline void prolong_add_body(const T* __restrict__ xc, int Nc, int Mc, T* __restrict__ xf, int Nf, int Mf,
-                                        int Kf, long start, long stride) {
-  const long nf = (long)Nf * Mf * Kf;
-  for (long i = start; i < nf; i += stride) {
-    int x, y, z;
-    decode(i, Nf, Mf, &x, &y, &z);
-    prolong_cell<T>(xc, Nc, Mc, xf, Nf, Mf, Kf, i, x, y, z);
-  }
+  xf[i] += prolong_value<T>([&](int X, int Y, int Z) { return xc[X + (long)Nc * Y + NMc * Z]; }, Nf, Mf, Kf, x, y, z);
 }
 
 // One thread per coarse cell (64 x by 4 y coarse cells per block, blocks x fastest, then y, then
@@ -689,144 +687,221 @@ __global__ void __launch_bounds__(256) k_prolong_add(const T* __restrict__ xc, i
   if (x < Nf && y < Mf) prolong_cell<T>(xc, Nc, Mc, xf, Nf, Mf, Kf, x + (long)Nf * (y + (long)Mf * z), x, y, z);
 }
 
+// a / b for 0 <= a < 2^13, b > 0 (inv = 1 / b in FP32): the quotient's distance from the next integer,
+// at least 1 / 2b, exceeds the product's rounding, a / b 2^-22.  An integer division is some 40
+// instructions, and a phase of the small levels is hardly more
+__device__ inline int small_div(int a, float inv) { return (int)(((float)a + 0.5f) * inv); }
+
+// ---- red-black sweeps with the cells' data in registers -----------------------------------------
+// The cells of one level in a workgroup of COARSE_THREADS threads: each thread keeps the right-hand
+// side, 1/a_p and the six faces of NI cells of either colour in registers for all sweeps, x lives in
+// LDS.  The updates are those of k_rbgs / k_rbgs_tr (the same operands in the same order; an absent
+// neighbour has face 0 and reads the cell itself).
+template <class T, int NI>
+struct RbCells {
+  T f[2][NI][6], s[2][NI], b[2][NI];  // faces w, e, s, n, b, t (absent ones 0)
+  int at[2][NI];                      // cell in LDS, -1: none
+  unsigned near[2][NI];               // neighbours present, bit per face
+
+  // cells of a level (N x M x K, x in LDS in the level's order), right-hand side rhs(i)
+  template <class FT, class B>
+  __device__ void load(const Level& L, B rhs) {
+    const int N = L.d.N, M = L.d.M, K = L.d.K, NM = N * M;
+    const FT *fe = (const FT*)L.f_e, *fn = (const FT*)L.f_n, *ft = (const FT*)L.f_t;
+    const T* sv = (const T*)L.s;
+    const int half_row = (N + 1) / 2, total = half_row * M * K;
+    const float ih = 1.0f / (float)half_row, im = 1.0f / (float)M;
+#pragma unroll
+    for (int c = 0; c < 2; ++c)
+#pragma unroll
+      for (int j = 0; j < NI; ++j) {
+        const int t = (int)threadIdx.x + COARSE_THREADS * j, row = small_div(t, ih);
+        const int z = small_div(row, im), y = row - z * M, x = 2 * (t - row * half_row) + ((y + z + c) & 1);
+        at[c][j] = -1;
+        if (t >= total || x >= N) continue;
+        const int i = x + N * row;
+        const bool hw = x > 0, he = x < N - 1, hs = y > 0, hn = y < M - 1, hb = z > 0, ht = z < K - 1;
+        at[c][j] = i;
+        near[c][j] = hw | he << 1 | hs << 2 | hn << 3 | hb << 4 | ht << 5;
+        s[c][j] = sv[i];
+        b[c][j] = rhs(i);
+        const T w0 = (T)fe[hw ? i - 1 : i], e0 = (T)fe[i], s0 = (T)fn[hs ? i - N : i], n0 = (T)fn[i];
+        const T b0 = (T)ft[hb ? i - NM : i], t0 = (T)ft[i];
+        f[c][j][0] = hw ? w0 : (T)0;
+        f[c][j][1] = he ? e0 : (T)0;
+        f[c][j][2] = hs ? s0 : (T)0;
+        f[c][j][3] = hn ? n0 : (T)0;
+        f[c][j][4] = hb ? b0 : (T)0;
+        f[c][j][5] = ht ? t0 : (T)0;
+      }
+  }
+  __device__ T offdiag(const T* x, int c, int j, int sy, int sz) const {
+    const int i = at[c][j];
+    const unsigned m = near[c][j];
+    const T xw = x[m & 1 ? i - 1 : i], xe = x[m & 2 ? i + 1 : i], xs = x[m & 4 ? i - sy : i], xn = x[m & 8 ? i + sy : i];
+    const T xb = x[m & 16 ? i - sz : i], xt = x[m & 32 ? i + sz : i];
+    const T* q = f[c][j];
+    return q[0] * xw + q[1] * xe + q[2] * xs + q[3] * xn + q[4] * xb + q[5] * xt;
+  }
+  // one colour (c a constant after unrolling); zero: as k_rbgs's zero_guess
+  template <int C>
+  __device__ void half(T* x, T fs, int sy, int sz, int zero) const {
+#pragma unroll
+    for (int j = 0; j < NI; ++j) {
+      // from a zero start the other colour is cleared: its update reads the cell itself for absent
+      // neighbours
+      if (zero == 1 && at[1 - C][j] >= 0) x[at[1 - C][j]] = (T)0;
+      if (at[C][j] < 0) continue;
+      const T si = s[C][j], bi = b[C][j];
+      if (zero == 1) {
+        x[at[C][j]] = bi * si;  // 0 on an empty row
+      } else {
+        const T v = (bi - fs * offdiag(x, C, j, sy, sz)) * si;
+        if (si != (T)0) x[at[C][j]] = v;  // an empty row keeps its value
+      }
+    }
+  }
+  // residual b - A x of every cell into r
+  __device__ void residual(const T* x, T fs, int sy, int sz, T* r) const {
+#pragma unroll
+    for (int c = 0; c < 2; ++c)
+#pragma unroll
+      for (int j = 0; j < NI; ++j) {
+        if (at[c][j] < 0) continue;
+        const T si = s[c][j], ap = si != (T)0 ? (T)1 / si : (T)0;
+        const T r0 = b[c][j] - ap * x[at[c][j]];
+        r[at[c][j]] = r0 - fs * offdiag(x, c, j, sy, sz);
+      }
+  }
+};
+
 // The small levels of the cycle in one workgroup: pre-smoothing and restriction down to the
-// coarsest level, its dense LU solve (FP64, thread 0, the factors of lu_factor), then
+// coarsest level, its dense LU solve (FP64, the factors of lu_factor) or dense inverse, then
 // prolongation and post-smoothing back up; barriers separate the phases (one launch instead of
-// ~10 per level).  Level q of C is levels[first + q]; the last one is the LU level.
-template <class T, class FT>
+// ~10 per level).  Level q of C is levels[first + q]; the last one is the LU level.  x, b and the
+// residual live in LDS, the cells' coefficients in registers (RbCells): a phase is one round of LDS
+// reads, where reading x and the faces from L2 took 2 us a phase.  TR: the transposed cycle (colours
+// black then red, restriction by P^T, prolongation by R^T, pre- and post-sweeps exchanged by the
+// caller); the coarse levels are symmetric and hold no pinned rows.
+// Measured with 16^3, 8^3, 4^3 and 2^3 levels: see the figures at vc::coarse_cycle.
+template <class T, class FT, bool TR>
 __global__ void __launch_bounds__(COARSE_THREADS) k_coarse_cycle(CoarseLevels<T> C, int n_pre, int n_post,
                                                                 const double* __restrict__ lu_scale,
                                                                 const int* __restrict__ lu_perm,
                                                                 const double* __restrict__ Lf,
                                                                 const double* __restrict__ Uf,
                                                                 const double* __restrict__ dinv) {
-  const long tid = threadIdx.x, nth = blockDim.x;
-  const int last = C.count - 1;
-  int n_last = 0;
-  T* x_last = nullptr;
-  const T* b_last = nullptr;
+  constexpr int NI = COARSE_ITEMS, FIRST = TR ? 1 : 0;
+  // x of every level, b of every level, the residual of one level; then the LU's operands
+  constexpr int TAIL = COARSE_CELLS + lu_lds_size(COARSE_LU) > lu_lds_size(64) ? COARSE_CELLS + lu_lds_size(COARSE_LU)
+                                                                              : lu_lds_size(64);
+  __shared__ double lds[2 * COARSE_SUM + TAIL];
+  T* xs = reinterpret_cast<T*>(lds);
+  T* bs = xs + COARSE_SUM;
+  T* res = bs + COARSE_SUM;
+  const int tid = threadIdx.x, last = C.count - 1;
+  const int n_last = (int)C.L[last].d.n();
+  // factors of up to COARSE_LU unknowns have room of their own and are staged at once, larger ones
+  // take the residual's place when it is done with
+  const bool early = n_last <= COARSE_LU;
+  const LuLds lu = lu_lds(early ? lds + 2 * COARSE_SUM + COARSE_CELLS : lds + 2 * COARSE_SUM, n_last);
+  {
+    const int n = (int)C.L[0].d.n();
+    T v[COARSE_CELLS / COARSE_THREADS];
 #pragma unroll
-  for (int q = 0; q < COARSE_MAX; ++q)
-    if (q == last) {
-      n_last = (int)C.L[q].d.n();
-      x_last = C.x[q];
-      b_last = C.b[q];
-    }
-  // the LU factors of the last level (at most 64 unknowns) are staged in LDS by the whole
-  // workgroup at the start: thread 0's triangular solves then wait on LDS, not on one
-  // (by then evicted) global load after another
-  __shared__ double sL[64 * 64], sU[64 * 64], ssc[64], slu_b[64], slu_y[64];
-  __shared__ int sperm[64];
-  __shared__ T sres[COARSE_CELLS];  // residuals of the level being restricted
-  if (!dinv) {
-    const int n = n_last;
-    for (int k = (int)tid; k < n * n; k += (int)nth) {
-      sL[k] = Lf[k];
-      sU[k] = Uf[k];
-    }
-    for (int k = (int)tid; k < n; k += (int)nth) {
-      ssc[k] = lu_scale[k];
-      sperm[k] = lu_perm[k];
-    }
+    for (int j = 0; j < COARSE_CELLS / COARSE_THREADS; ++j)
+      if (tid + j * COARSE_THREADS < n) v[j] = C.b[tid + j * COARSE_THREADS];
+    if (!dinv && early) lu_stage(lu, n_last, lu_scale, lu_perm, Lf, Uf);
+#pragma unroll
+    for (int j = 0; j < COARSE_CELLS / COARSE_THREADS; ++j)
+      if (tid + j * COARSE_THREADS < n) bs[tid + j * COARSE_THREADS] = v[j];
   }
   __syncthreads();
-  for (int q = 0; q < COARSE_MAX - 1; ++q) {
-    if (q < last) {
-      const Level& L = C.L[q];
-      const FT* e = (const FT*)L.f_e;
-      const FT* nn = (const FT*)L.f_n;
-      const FT* t = (const FT*)L.f_t;
-      const T* s = (const T*)L.s;
-      for (int sw = 0; sw < n_pre; ++sw) {
-        rbgs_body<T, FT>(C.x[q], C.b[q], e, nn, t, s, (T)L.fscale, L.d.N, L.d.M, L.d.K, 0, L.pin0, L.pin1,
-                         sw == 0 ? 1 : 0, tid, nth);
-        __syncthreads();
-        rbgs_body<T, FT>(C.x[q], C.b[q], e, nn, t, s, (T)L.fscale, L.d.N, L.d.M, L.d.K, 1, L.pin0, L.pin1,
-                         sw == 0 ? 2 : 0, tid, nth);
-        __syncthreads();
-      }
-      // residual restriction: every cell's residual into LDS (one thread per cell), then each coarse
-      // cell sums its children in the order of k_resid_restrict_cells (the same values; one cell's
-      // loads per thread instead of eight keeps the kernel clear of register spills)
-      {
-        const T* x = C.x[q];
-        const T* b = C.b[q];
-        const T fs = (T)L.fscale;
-        const int N = L.d.N, M = L.d.M, K = L.d.K, n = N * M * K;
-        for (int i = (int)tid; i < n; i += (int)nth) {
-          int xx, yy, zz;
-          decode(i, N, M, &xx, &yy, &zz);
-          const T si = s[i];
-          const T ap = si != (T)0 ? (T)1 / si : (T)0;
-          T r = b[i] - ap * x[i];
-          const T od = offdiag_u<T, FT>(x, e, nn, t, i, xx, yy, zz, N, M, K);
-          if (i != L.pin0 && i != L.pin1) r -= fs * od;
-          sres[i] = r;
-        }
-        __syncthreads();
-        const int Nc = (N + 1) / 2, Mc = (M + 1) / 2, nc = Nc * Mc * ((K + 1) / 2);
-        T* bc = C.b[q + 1];
-        for (int I = (int)tid; I < nc; I += (int)nth) {
-          int X, Y, Z;
-          decode(I, Nc, Mc, &X, &Y, &Z);
-          T acc = 0;
-#pragma unroll
-          for (int c = 0; c < 8; ++c) {
-            const int cx = 2 * X + (c & 1), cy = 2 * Y + ((c >> 1) & 1), cz = 2 * Z + (c >> 2);
-            acc += cx < N && cy < M && cz < K ? sres[cx + N * (cy + M * cz)] : (T)0;  // odd axes: one child
-          }
-          bc[I] = acc;
-        }
-        __syncthreads();
-      }
-    }
-  }
-  if (dinv) {  // dense inverse of the last level, column-major: x_i = sum_j inv[j n + i] b_j
-    const int n = n_last;
-    const T* bb = b_last;
-    for (int i = (int)tid; i < n; i += (int)nth) {
-      double acc = 0.0;
-      for (int j = 0; j < n; ++j) acc += dinv[(long)j * n + i] * (double)bb[j];
-      x_last[i] = (T)acc;
-    }
-  } else if (tid == 0) {
-    const int n = n_last;
-    const T* bb = b_last;
-    double* bs = slu_b;  // LDS: as local arrays they would live in scratch memory
-    double* yv = slu_y;
-    for (int i = 0; i < n; ++i) bs[i] = ssc[sperm[i]] * (double)bb[sperm[i]];
-    for (int i = 0; i < n; ++i) {
-      double aux = bs[i];
-      for (int k = 0; k < i; ++k) aux -= sL[i * n + k] * yv[k];
-      yv[i] = aux;
-    }
-    for (int i = n - 1; i >= 0; --i) {
-      double aux = yv[i];
-      for (int j = i + 1; j < n; ++j) aux -= sU[i * n + j] * bs[j];
-      bs[i] = aux / sU[i * n + i];
-    }
-    for (int i = 0; i < n; ++i) x_last[i] = (T)(ssc[i] * bs[i]);
-  }
-  __syncthreads();
-  for (int q = COARSE_MAX - 2; q >= 0; --q) {
-    if (q < last) {
-      const Level& L = C.L[q];
-      const FT* e = (const FT*)L.f_e;
-      const FT* nn = (const FT*)L.f_n;
-      const FT* t = (const FT*)L.f_t;
-      const T* s = (const T*)L.s;
-      prolong_add_body<T>(C.x[q + 1], C.L[q + 1].d.N, C.L[q + 1].d.M, C.x[q], L.d.N, L.d.M, L.d.K, tid, nth);
+  int off = 0;
+  for (int q = 0; q < last; ++q) {
+    const Level& L = C.L[q];
+    const int N = L.d.N, M = L.d.M, K = L.d.K, n = N * M * K;
+    T* x = xs + off;
+    const T fs = (T)L.fscale;
+    RbCells<T, NI> cells;
+    cells.template load<FT>(L, [&](int i) { return bs[off + i]; });
+    for (int sw = 0; sw < n_pre; ++sw) {
+      cells.template half<FIRST>(x, fs, N, N * M, sw == 0 ? 1 : 0);
       __syncthreads();
-      for (int sw = 0; sw < n_post; ++sw) {
-        rbgs_body<T, FT>(C.x[q], C.b[q], e, nn, t, s, (T)L.fscale, L.d.N, L.d.M, L.d.K, 0, L.pin0, L.pin1, 0, tid,
-                         nth);
-        __syncthreads();
-        rbgs_body<T, FT>(C.x[q], C.b[q], e, nn, t, s, (T)L.fscale, L.d.N, L.d.M, L.d.K, 1, L.pin0, L.pin1, 0, tid,
-                         nth);
-        __syncthreads();
+      cells.template half<1 - FIRST>(x, fs, N, N * M, sw == 0 ? 2 : 0);
+      __syncthreads();
+    }
+    cells.residual(x, fs, N, N * M, res);
+    __syncthreads();
+    const int Nc = (N + 1) / 2, Mc = (M + 1) / 2, nc = Nc * Mc * ((K + 1) / 2);
+    const float inc = 1.0f / (float)Nc, imc = 1.0f / (float)Mc;
+    for (int I = tid; I < nc; I += COARSE_THREADS) {
+      const int R = small_div(I, inc), X = I - R * Nc, Z = small_div(R, imc), Y = R - Z * Mc;
+      T acc = 0;
+      if constexpr (TR) {
+        acc = restrict_pt_cell<T>([&](int a, int b, int c) { return res[a + N * (b + M * c)]; }, X, Y, Z, N, M, K);
+      } else {
+#pragma unroll
+        for (int c = 0; c < 8; ++c) {
+          const int cx = 2 * X + (c & 1), cy = 2 * Y + ((c >> 1) & 1), cz = 2 * Z + (c >> 2);
+          const bool in = cx < N && cy < M && cz < K;  // odd axes: one child
+          const T v = res[in ? cx + N * (cy + M * cz) : 0];
+          acc += in ? v : (T)0;
+        }
       }
+      bs[off + n + I] = acc;
+    }
+    off += n;
+    __syncthreads();
+  }
+  T* xl = xs + off;
+  const T* bl = bs + off;
+  if (dinv) {  // dense inverse of the last level, column-major: x_i = sum_j inv[j n + i] b_j
+    for (int i = tid; i < n_last; i += COARSE_THREADS) {
+      double acc = 0.0;
+      for (int j = 0; j < n_last; ++j) acc += dinv[(long)j * n_last + i] * (double)bl[j];
+      xl[i] = (T)acc;
+    }
+  } else {
+    if (!early) {
+      lu_stage(lu, n_last, lu_scale, lu_perm, Lf, Uf);
+      __syncthreads();
+    }
+    if (tid < 64) {
+      if (tid < n_last) lu.rhs[tid] = (double)bl[tid];
+      lu_substitute(lu, n_last);
+      if (tid < n_last) xl[tid] = (T)lu.rhs[tid];
     }
   }
+  __syncthreads();
+  for (int q = last - 1; q >= 0; --q) {
+    const Level& L = C.L[q];
+    const int N = L.d.N, M = L.d.M, K = L.d.K, n = N * M * K;
+    const int Nc = C.L[q + 1].d.N, Mc = C.L[q + 1].d.M;
+    const T* xc = xs + off;
+    off -= n;
+    T* x = xs + off;
+    const T fs = (T)L.fscale;
+    RbCells<T, NI> cells;
+    cells.template load<FT>(L, [&](int i) { return bs[off + i]; });
+    const float in = 1.0f / (float)N, im = 1.0f / (float)M;
+    for (int i = tid; i < n; i += COARSE_THREADS) {
+      const int r = small_div(i, in), a = i - r * N, c = small_div(r, im), b = r - c * M;
+      if constexpr (TR)
+        x[i] += xc[(a >> 1) + Nc * ((b >> 1) + Mc * (c >> 1))];
+      else
+        x[i] += prolong_value<T>([&](int X, int Y, int Z) { return xc[X + Nc * (Y + Mc * Z)]; }, N, M, K, a, b, c);
+    }
+    __syncthreads();
+    for (int sw = 0; sw < n_post; ++sw) {
+      cells.template half<FIRST>(x, fs, N, N * M, 0);
+      __syncthreads();
+      cells.template half<1 - FIRST>(x, fs, N, N * M, 0);
+      __syncthreads();
+    }
+  }
+  const int n = (int)C.L[0].d.n();
+  for (int i = tid; i < n; i += COARSE_THREADS) C.x[i] = xs[i];
 }
 
 // ---- coarsest level as a dense inverse ---------------------------------------------------------
@@ -2023,7 +2098,7 @@ void resid_tr<float>(const Level& L, const float* x, const float* b, float* r, h
 template <class T>
 void restrict_pt(const T* r, Dims df, T* bc, hipStream_t s) {
   const long nc = (long)((df.N + 1) / 2) * ((df.M + 1) / 2) * ((df.K + 1) / 2);
-  k_restrict_pt<T><<<grid_1d(nc), 256, 0, s>>>(r, df.N, df.M, df.K, bc);
+  k_restrict_pt<T><<<(unsigned)((nc + 255) / 256), 256, 0, s>>>(r, df.N, df.M, df.K, bc);
 }
 template <class T>
 void prolong_inject_add(const T* xc, Dims dc, T* xf, Dims df, hipStream_t s) {
@@ -2158,15 +2233,38 @@ template void copy_vec<float>(const float*, float*, long, hipStream_t);
 template void copy_vec<double>(const double*, double*, long, hipStream_t);
 
 template <class T>
-void coarse_cycle(const CoarseLevels<T>& C, int n_pre, int n_post, const double* lu_scale, const int* lu_perm,
+bool coarse_fits(const CoarseLevels<T>& C) {
+  if (C.count < 2 || C.count > COARSE_MAX) return false;
+  long sum = 0;
+  for (int q = 0; q < C.count; ++q) {
+    const Dims& d = C.L[q].d;
+    sum += d.n();
+    if (q + 1 < C.count && (d.n() > COARSE_CELLS || (long)((d.N + 1) / 2) * d.M * d.K > COARSE_ITEMS * COARSE_THREADS))
+      return false;
+    if (C.L[q].pin0 >= 0 || C.L[q].pin1 >= 0) return false;
+  }
+  return sum <= COARSE_SUM;
+}
+template bool coarse_fits<float>(const CoarseLevels<float>&);
+template bool coarse_fits<double>(const CoarseLevels<double>&);
+
+template <class T>
+void coarse_cycle(const CoarseLevels<T>& C, int trans, int n_pre, int n_post, const double* lu_scale, const int* lu_perm,
                   const double* L, const double* U, const double* dinv, hipStream_t s) {
-  if (C.count < 2 || C.count > COARSE_MAX) return;
-  if (C.L[0].ftype == FACE_F16)
-    k_coarse_cycle<T, _Float16><<<1, COARSE_THREADS, 0, s>>>(C, n_pre, n_post, lu_scale, lu_perm, L, U, dinv);
-  else if (C.L[0].ftype == FACE_F32)
-    k_coarse_cycle<T, float><<<1, COARSE_THREADS, 0, s>>>(C, n_pre, n_post, lu_scale, lu_perm, L, U, dinv);
+#define LSX_COARSE(FT)                                                                                             \
+  do {                                                                                                             \
+    if (trans)                                                                                                     \
+      k_coarse_cycle<T, FT, true><<<1, COARSE_THREADS, 0, s>>>(C, n_pre, n_post, lu_scale, lu_perm, L, U, dinv);   \
+    else                                                                                                           \
+      k_coarse_cycle<T, FT, false><<<1, COARSE_THREADS, 0, s>>>(C, n_pre, n_post, lu_scale, lu_perm, L, U, dinv);  \
+  } while (0)
+  if constexpr (std::is_same<T, double>::value)
+    LSX_COARSE(double);
+  else if (C.L[0].ftype == FACE_F16)
+    LSX_COARSE(_Float16);
   else
-    k_coarse_cycle<T, double><<<1, COARSE_THREADS, 0, s>>>(C, n_pre, n_post, lu_scale, lu_perm, L, U, dinv);
+    LSX_COARSE(float);
+#undef LSX_COARSE
 }
 
 void dense_inverse(const double* fe, const double* fn, const double* ft, const double* dg, Dims d, double* inv_c,
@@ -2208,10 +2306,10 @@ void prolong_add(const T* xc, Dims dc, T* xf, Dims df, hipStream_t s) {
 }
 template void prolong_add<float>(const float*, Dims, float*, Dims, hipStream_t);
 template void prolong_add<double>(const double*, Dims, double*, Dims, hipStream_t);
-template void coarse_cycle<float>(const CoarseLevels<float>&, int, int, const double*, const int*, const double*,
+template void coarse_cycle<float>(const CoarseLevels<float>&, int, int, int, const double*, const int*, const double*,
                                   const double*, const double*, hipStream_t);
-template void coarse_cycle<double>(const CoarseLevels<double>&, int, int, const double*, const int*, const double*,
-                                   const double*, const double*, hipStream_t);
+template void coarse_cycle<double>(const CoarseLevels<double>&, int, int, int, const double*, const int*,
+                                   const double*, const double*, const double*, hipStream_t);
 
 template <class A, class B>
 void convert(const A* a, B* b, long n, hipStream_t s) {

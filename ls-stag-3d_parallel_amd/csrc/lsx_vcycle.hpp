@@ -51,18 +51,22 @@ void diag_rule(double* fe, const double* fn, const double* ft, const double* dg,
                double* partial, double* out, hipStream_t s);
 
 // The small levels handled by one workgroup in a single launch (k_coarse_cycle): levels with at
-// most COARSE_CELLS cells (16^3; a 32^3 level already runs faster on the whole device), down to
-// and including the LU level.
+// most COARSE_CELLS cells (16^3) and COARSE_ITEMS cells of a colour per thread, COARSE_SUM cells in
+// all, down to and including the LU level.  x, b: the first level's, in memory.
 constexpr int COARSE_MAX = 8;
 constexpr int COARSE_THREADS = 1024;
 constexpr long COARSE_CELLS = 4096;
+constexpr int COARSE_ITEMS = 2, COARSE_SUM = 5120;
+constexpr int COARSE_LU = 40;  // unknowns whose LU factors have LDS of their own
 template <class T>
 struct CoarseLevels {
   int count = 0;
   Level L[COARSE_MAX];
-  T* x[COARSE_MAX] = {};
-  T* b[COARSE_MAX] = {};
+  T* x = nullptr;
+  const T* b = nullptr;
 };
+template <class T>
+bool coarse_fits(const CoarseLevels<T>& C);
 
 // ---- setup (FP64 temporaries) --------------------------------------------------------------
 // faces and diagonal of the finest level from the FP64 7-plane operator [b,s,w,p,e,n,t]; a face
@@ -108,10 +112,11 @@ template <class T>
 void prolong_add(const T* xc, Dims dc, T* xf, Dims df, hipStream_t s);
 template <class A, class B>
 void convert(const A* a, B* b, long n, hipStream_t s);
-// the small levels of the cycle in one launch: C.b[0] holds the right-hand side of the first of
-// them, C.x[0] receives its correction (lu_*: the dense LU factors of the last level)
+// the small levels of the cycle (trans: the transposed one) in one launch: C.b holds the right-hand side
+// of the first of them, C.x receives its correction (lu_*: the dense LU factors of the last level,
+// or dinv its dense inverse, column-major)
 template <class T>
-void coarse_cycle(const CoarseLevels<T>& C, int n_pre, int n_post, const double* lu_scale, const int* lu_perm,
+void coarse_cycle(const CoarseLevels<T>& C, int trans, int n_pre, int n_post, const double* lu_scale, const int* lu_perm,
                   const double* L, const double* U, const double* dinv, hipStream_t s);
 
 // Coarsest level of a capped hierarchy (DENSE_MAX unknowns at most) as a dense FP64 inverse,
