@@ -69,7 +69,9 @@ typedef struct lsx_options {
   int graphs;        /* V-cycle: 1 = replay each cycle from a captured HIP graph (one per basis slot) */
   int smoother;      /* V-cycle: LSX_SMOOTH_RBGS (default) or LSX_SMOOTH_LINE                  */
   int fused_sweep;   /* V-cycle red-black: 1 = both colours in one pass on a finest level of
-                        >= 2^23 cells (default), 2 = on every level, 0 = never (half-sweeps)    */
+                        >= 2^23 cells, all sweeps of a side in one launch on levels of <= 2^18
+                        (default); 2 = one pass per sweep on every level; 0 = half-sweeps.
+                        All give the same bits                                                  */
   int line_levels;   /* V-cycle with LSX_SMOOTH_LINE: the finest line_levels levels are smoothed
                         with lines, coarser ones with red-black sweeps; 0 = every level (default) */
   int diag_faces;    /* V-cycle: 1 = on levels whose rows sum to zero (checked at set-up: every

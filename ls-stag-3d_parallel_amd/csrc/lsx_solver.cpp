@@ -564,7 +564,7 @@ void Solver::build_vcycle() {
         S.fxt.alloc(nl);
       else
         S.dxt.alloc(nl);
-    } else if (fused_level(l)) {  // second iterate buffer of the one-pass sweeps
+    } else if (fused_level(l) || tile_size(l)) {  // second iterate buffer of the one-pass sweeps
       if (m32)
         S.fxt.alloc(nl);
       else
@@ -702,6 +702,10 @@ void Solver::vcycle_run(const double* v, T* z, const float* b32) {
     VStore& S = vlev[l];
     T* x = l == 0 ? z : vx<T>(S);
     const T* b = l == 0 ? b0 : vb<T>(S);
+    if (tile_level(l)) {
+      vc::rb_pre<T>(S.L, vxt<T>(S), b, vlev[l + 1].L.d, vb<T>(vlev[l + 1]), opt.n_pre, stream);
+      continue;
+    }
     smooth<T>(l, x, b, opt.n_pre, true);
     vc::resid_restrict<T>(S.L, x, b, vb<T>(vlev[l + 1]), stream);
   }
@@ -713,6 +717,10 @@ void Solver::vcycle_run(const double* v, T* z, const float* b32) {
     VStore& S = vlev[l];
     T* x = l == 0 ? z : vx<T>(S);
     const T* b = l == 0 ? b0 : vb<T>(S);
+    if (tile_level(l)) {
+      vc::rb_post<T>(S.L, 0, vxt<T>(S), x, b, vx<T>(vlev[l + 1]), vlev[l + 1].L.d, opt.n_post, stream);
+      continue;
+    }
     vc::prolong_add<T>(vx<T>(vlev[l + 1]), vlev[l + 1].L.d, x, S.L.d, stream);
     smooth<T>(l, x, b, opt.n_post, false, true);  // lines z, y, x: the cycle is symmetric in its line order
   }
@@ -851,8 +859,12 @@ void Solver::vcycle_apply_tr(const double* v, T* z) {
     VStore& S = vlev[l];
     T* x = l == 0 ? z : vx<T>(S);
     const T* b = l == 0 ? b0 : vb<T>(S);
-    smooth<T>(l, x, b, opt.n_post, true, false);  // transposed post-smoothing (lines x, y, z)
-    vc::resid_tr<T>(S.L, x, b, vr<T>(S), stream);
+    if (tile_level(l)) {
+      vc::rb_pre_tr<T>(S.L, vxt<T>(S), b, vr<T>(S), opt.n_post, stream);
+    } else {
+      smooth<T>(l, x, b, opt.n_post, true, false);  // transposed post-smoothing (lines x, y, z)
+      vc::resid_tr<T>(S.L, x, b, vr<T>(S), stream);
+    }
     vc::restrict_pt<T>(vr<T>(S), S.L.d, vb<T>(vlev[l + 1]), stream);
   }
   if (C.count)
@@ -863,6 +875,10 @@ void Solver::vcycle_apply_tr(const double* v, T* z) {
     VStore& S = vlev[l];
     T* x = l == 0 ? z : vx<T>(S);
     const T* b = l == 0 ? b0 : vb<T>(S);
+    if (tile_level(l)) {
+      vc::rb_post<T>(S.L, 1, vxt<T>(S), x, b, vx<T>(vlev[l + 1]), vlev[l + 1].L.d, opt.n_pre, stream);
+      continue;
+    }
     vc::prolong_inject_add<T>(vx<T>(vlev[l + 1]), vlev[l + 1].L.d, x, S.L.d, stream);
     smooth<T>(l, x, b, opt.n_pre, false, true);  // transposed pre-smoothing (lines z, y, x)
   }

@@ -207,6 +207,18 @@ class Solver {
   bool fused_level(int l) const {
     return opt.fused_sweep == 2 || (opt.fused_sweep == 1 && l == 0 && levels[l].d.n() >= (1L << 23));
   }
+  // red-black levels that take each side of their cycle in one launch of overlapping tiles (per-kernel
+  // timing wants level 0's sweeps one by one).  Up to 64^3 cells: a tile of 8^3 cells computes a
+  // region of 16^3, which is free while the tiles fill the 256 CUs once or twice.  One side of
+  // V(2,2), tiles against half-sweeps, us: 48^3 FP32 10 / 18, FP64 13 / 18; 56^3 FP64 transposed 17
+  // / 29; 64^3 FP32 16 / 19, FP64 23 / 22 (and four launches fewer); 80^3 FP32 24 / 29, FP64 45 / 39;
+  // 96^3 FP64 75 / 65
+  static constexpr long RB_TILE_CELLS = 1L << 18;
+  bool tile_size(int l) const {
+    return opt.fused_sweep == 1 && rb_level(l) && !fused_level(l) && levels[l].d.N > 1 && levels[l].d.n() <= RB_TILE_CELLS &&
+           opt.n_pre <= vc::RB_TILE_SWEEPS && opt.n_post <= vc::RB_TILE_SWEEPS;
+  }
+  bool tile_level(int l) const { return tile_size(l) && !(timing && l == 0); }
   // levels smoothed by line relaxation: every level, or the finest opt.line_levels of them
   bool line_level(int l) const {
     return opt.smoother == LSX_SMOOTH_LINE && (opt.line_levels <= 0 || l < opt.line_levels);

@@ -783,7 +783,8 @@ struct RbCells {
 // reads, where reading x and the faces from L2 took 2 us a phase.  TR: the transposed cycle (colours
 // black then red, restriction by P^T, prolongation by R^T, pre- and post-sweeps exchanged by the
 // caller); the coarse levels are symmetric and hold no pinned rows.
-// Measured with 16^3, 8^3, 4^3 and 2^3 levels: see the figures at vc::coarse_cycle.
+// Measured with levels of 16^3, 8^3, 4^3 and 2^3 cells: FP64 71 -> 38 us, FP32 28 -> 19 us; most of it is
+// loads of coefficients, which nothing overlaps, and the LU's chain (3 us).
 template <class T, class FT, bool TR>
 __global__ void __launch_bounds__(COARSE_THREADS) k_coarse_cycle(CoarseLevels<T> C, int n_pre, int n_post,
                                                                 const double* __restrict__ lu_scale,
@@ -902,6 +903,254 @@ __global__ void __launch_bounds__(COARSE_THREADS) k_coarse_cycle(CoarseLevels<T>
   }
   const int n = (int)C.L[0].d.n();
   for (int i = tid; i < n; i += COARSE_THREADS) C.x[i] = xs[i];
+}
+
+// ---- all sweeps of a level in one launch -------------------------------------------------------
+// On a level of some 10^4 to 10^5 cells a half-sweep is a launch and one trip to memory (4.4 us at
+// 24 x 16 x 16 cells as at 48 x 32 x 32), and the four of a V(2,2) side and the residual's restriction or
+// the prolongation make five.  k_rb_tile takes them in one: a workgroup owns a tile of
+// (16 - 2 H)^3 cells and works on the 16^3 region around it, H = 2 sweeps: a half-sweep's values
+// are right one cell less deep into the region than the one before, the tile's are after all of them.
+// The halo is computed by its neighbours' workgroups too, from the same values by the same operations
+// (those of k_rbgs / k_rbgs_tr, k_resid_restrict_cells, k_prolong_add8), so the result is the same bit
+// for bit.  A thread holds the coefficients of two x pairs, one of either colour in each; x lies in LDS
+// by colour (a wavefront reads 64 consecutive words for each neighbour), what a cell reads past
+// the region is padding whose value never reaches the tile.  The iterate between the two sides
+// needs a buffer of its own, since neighbours read what a tile replaces.
+// MODE: RB_PRE from a zero start, residual restricted to bc; RB_PRE_TR the transposed cycle's (black
+// first, residual of A^T written to bc as a fine vector); RB_POST prolongation of xc added to x_in,
+// then the sweeps; RB_POST_TR its R^T.  Needs N >= 2 and byte offsets below 2^31.
+// Bound by latency up to one workgroup per CU (launch, one trip to memory, 4 half-sweeps: 9-10 us), by
+// the instructions of the halo beyond it.  One side of a 48^3 level, FP32: 18 -> 10 us (before), 14 + 4
+// -> 9 us (after); a fourth of the first version's time went into one load per coefficient with its
+// address, hence the pairs.  FP32 before-sides take two workgroups per CU (64 registers); the
+// after-sides would spill (64^3: 26 us against 18).
+enum RbTile { RB_PRE, RB_PRE_TR, RB_POST, RB_POST_TR };
+constexpr int RB_R = 16;
+
+template <class T>
+struct __attribute__((packed, aligned(alignof(T)))) Two {
+  T a, b;
+};
+template <class T>
+__device__ inline T ld1(const T* p, int i) {
+  return *(const T*)((const char*)p + (unsigned)(i * (int)sizeof(T)));
+}
+// values at i and i + 1 of a row; `shift`: i is the row's last cell, the second value is not used
+template <class V, class T>
+__device__ inline void ld2(const T* p, int i, int shift, V (&v)[2]) {
+  const Two<T> q = *(const Two<T>*)((const char*)p + (unsigned)((i - shift) * (int)sizeof(T)));
+  v[0] = (V)(shift ? q.b : q.a);
+  v[1] = (V)q.b;
+}
+
+template <class T, class FT, int MODE, bool DFF>
+__global__ void __launch_bounds__(COARSE_THREADS, sizeof(T) == 4 && (MODE == RB_PRE || MODE == RB_PRE_TR) ? 8 : 4)
+    k_rb_tile(Level L, const T* __restrict__ x_in, T* __restrict__ x_out, const T* __restrict__ b,
+              const T* __restrict__ xc, int Nc, int Mc, int Kc, T* __restrict__ bc, int sweeps, DiagRule<T> dr) {
+  constexpr bool TR = MODE == RB_PRE_TR || MODE == RB_POST_TR, PRE = MODE == RB_PRE || MODE == RB_PRE_TR;
+  constexpr int NI = 2, FIRST = TR ? 1 : 0, R = RB_R, HALF = R * R * R / 2, SY = R / 2, SZ = R * R / 2;
+  constexpr int CR = R / 2 + 2;  // coarse cells per axis that the region's prolongation reads
+  __shared__ T lds[2 * HALF + 3 * SZ];
+  __shared__ T aux[MODE == RB_PRE ? 2 * HALF : PRE ? 1 : CR * CR * CR];  // residuals / coarse values
+  const int N = L.d.N, M = L.d.M, K = L.d.K, H = 2 * sweeps, W = R - 2 * H;
+  const int gx = (N + W - 1) / W, gy = (M + W - 1) / W;
+  const int lb = xcd_order(blockIdx.x, gridDim.x);
+  const int tx = lb % gx * W, ty = lb / gx % gy * W, tz = lb / (gx * gy) * W;  // the tile's first cell
+  const int x0 = tx - H, y0 = ty - H, z0 = tz - H;                            // the region's (even)
+  const int NM = N * M, t = threadIdx.x;
+  const T fs = (T)L.fscale;
+  const FT *fe = (const FT*)L.f_e, *fn = (const FT*)L.f_n, *ft = (const FT*)L.f_t;
+  const T* sv = (const T*)L.s;
+  T* const mine = lds + SZ + t;  // colour c, pair j of this thread: mine[c (HALF + SZ) + COARSE_THREADS j]
+  constexpr int CS = HALF + SZ;
+  if constexpr (!PRE) {
+    if (t < CR * CR * CR) {
+      const int q = t / CR, cx = t - q * CR, cz = q / CR, cy = q - cz * CR;
+      const int X = min(max((x0 >> 1) - 1 + cx, 0), Nc - 1), Y = min(max((y0 >> 1) - 1 + cy, 0), Mc - 1);
+      const int Z = min(max((z0 >> 1) - 1 + cz, 0), Kc - 1);
+      aux[t] = ld1(xc, X + Nc * (Y + Mc * Z));
+    }
+  }
+  const int px = 2 * (t & 7), ly = (t >> 3) & 15, lz = t >> 7;
+  const int sw = (ly + lz) & 1;  // the pair's first cell has colour sw
+  const int X = x0 + px, Y = y0 + ly;
+  const bool in_xy = X >= 0 && X < N && Y >= 0 && Y < M, two = X + 1 < N;
+  T f[2][NI][6], s[2][NI], r[2][NI], xp[NI][2];  // by colour (xp: by position in the pair)
+  unsigned flags = 0;                            // bit 4 j + c: pinned; bit 4 j + 2 + c: marked east face
+#pragma unroll
+  for (int j = 0; j < NI; ++j) {
+    const int Z = z0 + lz + SY * j;
+    const bool in = in_xy && Z >= 0 && Z < K;
+    const int i = in ? X + N * Y + NM * Z : 0, shift = in && !two ? 1 : 0;
+    T e[2], n[2], so[2], to[2], bo[2], sp[2], bp[2];
+    const T w0 = (T)ld1(fe, i - (in && X > 0 ? 1 : 0));
+    ld2(fe, i, shift, e);
+    ld2(fn, i, shift, n);
+    ld2(fn, i - (in && Y > 0 ? N : 0), shift, so);
+    ld2(ft, i, shift, to);
+    ld2(ft, i - (in && Z > 0 ? NM : 0), shift, bo);
+    ld2(sv, i, shift, sp);
+    ld2(b, i, shift, bp);
+    if constexpr (!PRE) ld2(x_in, i, shift, xp[j]);
+    T g[2][6];
+    unsigned fl[2];
+#pragma unroll
+    for (int k = 0; k < 2; ++k) {
+      const int q = i + k;
+      const bool is = in && (k == 0 || two), pin = is && (q == L.pin0 || q == L.pin1);
+      // A: a pinned row is an identity row; A^T: a row that is not pinned drops its couplings to
+      // pinned cells
+      auto keep = [&](bool there, int nb) {
+        return is && there && (TR ? pin || (nb != L.pin0 && nb != L.pin1) : !pin);
+      };
+      const T west = k == 0 ? w0 : e[0];
+      g[k][0] = keep(X + k > 0, q - 1) ? west : (T)0;
+      g[k][1] = keep(X + k < N - 1, q + 1) ? e[k] : (T)0;
+      g[k][2] = keep(Y > 0, q - N) ? so[k] : (T)0;
+      g[k][3] = keep(Y < M - 1, q + N) ? n[k] : (T)0;
+      g[k][4] = keep(Z > 0, q - NM) ? bo[k] : (T)0;
+      g[k][5] = keep(Z < K - 1, q + NM) ? to[k] : (T)0;
+      sp[k] = is ? sp[k] : (T)0;
+      bp[k] = is ? bp[k] : (T)0;
+      fl[k] = (pin ? 1u : 0u) | (__builtin_signbit(e[k]) ? 4u : 0u);
+    }
+#pragma unroll
+    for (int c = 0; c < 2; ++c) {
+#pragma unroll
+      for (int d = 0; d < 6; ++d) f[c][j][d] = sw ? g[1 - c][d] : g[c][d];
+      s[c][j] = sw ? sp[1 - c] : sp[c];
+      r[c][j] = sw ? bp[1 - c] : bp[c];
+      flags |= (sw ? fl[1 - c] : fl[c]) << (4 * j + c);
+    }
+  }
+  auto col = [&](int c) { return sw ^ c; };  // position of colour c's cell in the pair
+  auto offdiag = [&](int c, int j) {
+    const T* o = mine + (1 - c) * CS + COARSE_THREADS * j;
+    const T* h = o + col(c);
+    const T xw = h[-1], xe = h[0], xs = o[-SY], xn = o[SY], xb = o[-SZ], xt = o[SZ];
+    const T* q = f[c][j];
+    return q[0] * xw + q[1] * xe + q[2] * xs + q[3] * xn + q[4] * xb + q[5] * xt;
+  };
+  auto half = [&](auto colour) {
+    constexpr int C = decltype(colour)::value;
+#pragma unroll
+    for (int j = 0; j < NI; ++j) {
+      const T v = (r[C][j] - fs * offdiag(C, j)) * s[C][j];
+      if (s[C][j] != (T)0) mine[C * CS + COARSE_THREADS * j] = v;  // an empty row keeps its value
+    }
+    __syncthreads();
+  };
+  if constexpr (PRE) {  // from zero: the first colour's update reads nothing
+#pragma unroll
+    for (int j = 0; j < NI; ++j) {
+      mine[FIRST * CS + COARSE_THREADS * j] = r[FIRST][j] * s[FIRST][j];
+      mine[(1 - FIRST) * CS + COARSE_THREADS * j] = (T)0;
+    }
+    __syncthreads();
+  } else {
+    __syncthreads();
+    // as prolong_value: taps (p - 1, p) of an even cell, (p, p + 1) of an odd one, weights 1/4 and
+    // 3/4 (1 for the cell's own parent at the level's ends, where the other tap's 0 changes no bit)
+    const T* v0 = aux + (t & 7) + CR * (((ly >> 1) + (ly & 1)) + CR * ((lz >> 1) + (lz & 1)));
+    auto weights = [](int x, int n, float (&w)[2]) {
+      const bool odd = x & 1, end = x == n - 1 || x == 0;
+      w[0] = odd ? (end ? 1.f : 0.75f) : (end ? 0.f : 0.25f);
+      w[1] = odd ? (end ? 0.f : 0.25f) : (end ? 1.f : 0.75f);
+    };
+    float wx[2][2], wy[2];
+    weights(X, N, wx[0]);
+    weights(X + 1, N, wx[1]);
+    weights(Y, M, wy);
+#pragma unroll
+    for (int j = 0; j < NI; ++j) {
+      const int Z = z0 + lz + SY * j;
+      const T* vj = v0 + CR * CR * (SY / 2) * j;
+      T add[2] = {0, 0};
+      if constexpr (TR) {
+        add[0] = add[1] = vj[1 + CR * (1 - (ly & 1)) + CR * CR * (1 - (lz & 1))];
+      } else {
+        float wz[2];
+        weights(Z, K, wz);
+#pragma unroll
+        for (int zc = 0; zc < 2; ++zc)
+#pragma unroll
+          for (int yc = 0; yc < 2; ++yc) {
+            const T* q = vj + CR * yc + CR * CR * zc;
+            const T v[3] = {q[0], q[1], q[2]};
+#pragma unroll
+            for (int k = 0; k < 2; ++k)
+#pragma unroll
+              for (int c = 0; c < 2; ++c) add[k] += (T)(wx[k][c] * wy[yc] * wz[zc]) * v[k + c];
+          }
+      }
+#pragma unroll
+      for (int k = 0; k < 2; ++k) {
+        const bool is = in_xy && X + k < N && Z >= 0 && Z < K;
+        mine[(sw ^ k) * CS + COARSE_THREADS * j] = is ? xp[j][k] + add[k] : (T)0;
+      }
+    }
+    __syncthreads();
+    half(std::integral_constant<int, FIRST>{});
+  }
+  half(std::integral_constant<int, 1 - FIRST>{});
+#pragma unroll 1
+  for (int k = 1; k < sweeps; ++k) {
+    half(std::integral_constant<int, FIRST>{});
+    half(std::integral_constant<int, 1 - FIRST>{});
+  }
+#pragma unroll
+  for (int j = 0; j < NI; ++j) {
+    const int Z = z0 + lz + SY * j, i = X + N * Y + NM * Z;
+    const bool own = in_xy && px >= H && px < H + W && ly >= H && ly < H + W && Z >= tz && Z < tz + W && Z < K;
+    T xv[2], rv[2];
+#pragma unroll
+    for (int c = 0; c < 2; ++c) {
+      xv[c] = mine[c * CS + COARSE_THREADS * j];
+      rv[c] = 0;
+      if constexpr (PRE) {
+        const T* q = f[c][j];
+        const T si = s[c][j];
+        if constexpr (DFF) {
+          const bool pin = flags >> (4 * j + c) & 1, mark = flags >> (4 * j + 2 + c) & 1;
+          const T fsum = q[0] + q[1] + q[2] + q[3] + q[4] + q[5];
+          const T ap = pin ? (T)1 : dr.of_marked(fs * fsum, (long)(i + col(c)), mark);
+          const T r0 = r[c][j] - ap * xv[c];
+          rv[c] = r0 - fs * offdiag(c, j);
+        } else {
+          const T ap = si != (T)0 ? (T)1 / si : (T)0;
+          const T r0 = r[c][j] - ap * xv[c];
+          rv[c] = r0 - fs * offdiag(c, j);
+        }
+        if constexpr (MODE == RB_PRE) aux[c * HALF + COARSE_THREADS * j + t] = rv[c];
+      }
+    }
+    if (own) {
+      auto put = [&](T* p, const T (&v)[2]) {
+        const T a = sw ? v[1] : v[0], c = sw ? v[0] : v[1];
+        if (two)
+          *(Two<T>*)(p + i) = Two<T>{a, c};
+        else
+          p[i] = a;
+      };
+      put(x_out, xv);
+      if constexpr (MODE == RB_PRE_TR) put(bc, rv);
+    }
+  }
+  if constexpr (MODE == RB_PRE) {
+    __syncthreads();
+    const int V = W / 2, q = t / V, cx = t - q * V, cz = q / V, cy = q - cz * V;
+    const int Cx = tx / 2 + cx, Cy = ty / 2 + cy, Cz = tz / 2 + cz;
+    if (cz < V && Cx < Nc && Cy < Mc && Cz < Kc) {
+      T acc = 0;
+#pragma unroll
+      for (int k = 0; k < 8; ++k) {  // absent children (odd axes) have residual 0
+        const int yy = H + 2 * cy + ((k >> 1) & 1), zz = H + 2 * cz + (k >> 2), c = (k ^ yy ^ zz) & 1;
+        acc += aux[c * HALF + H / 2 + cx + SY * yy + SZ * zz];
+      }
+      bc[Cx + Nc * (Cy + Mc * Cz)] = acc;
+    }
+  }
 }
 
 // ---- coarsest level as a dense inverse ---------------------------------------------------------
@@ -2231,6 +2480,58 @@ void copy_vec(const T* a, T* b, long n, hipStream_t s) {
 }
 template void copy_vec<float>(const float*, float*, long, hipStream_t);
 template void copy_vec<double>(const double*, double*, long, hipStream_t);
+
+template <class T, class FT>
+static void rb_tile_t(const Level& L, int mode, const T* x_in, T* x_out, const T* b, const T* xc, Dims dc, T* bc,
+                      int sweeps, hipStream_t s) {
+  const int W = RB_R - 4 * sweeps;
+  const unsigned blocks = (unsigned)((long)((L.d.N + W - 1) / W) * ((L.d.M + W - 1) / W) * ((L.d.K + W - 1) / W));
+  const DiagRule<T> dr = diag_rule<T>(L);
+#define LSX_TILE(MODE, DFF) \
+  k_rb_tile<T, FT, MODE, DFF><<<blocks, COARSE_THREADS, 0, s>>>(L, x_in, x_out, b, xc, dc.N, dc.M, dc.K, bc, sweeps, dr)
+  if (mode == RB_PRE && L.dff)
+    LSX_TILE(RB_PRE, true);
+  else if (mode == RB_PRE)
+    LSX_TILE(RB_PRE, false);
+  else if (mode == RB_PRE_TR)
+    LSX_TILE(RB_PRE_TR, false);
+  else if (mode == RB_POST)
+    LSX_TILE(RB_POST, false);
+  else
+    LSX_TILE(RB_POST_TR, false);
+#undef LSX_TILE
+}
+template <class T>
+static void rb_tile(const Level& L, int mode, const T* x_in, T* x_out, const T* b, const T* xc, Dims dc, T* bc,
+                    int sweeps, hipStream_t s) {
+  if constexpr (std::is_same<T, double>::value)
+    rb_tile_t<T, double>(L, mode, x_in, x_out, b, xc, dc, bc, sweeps, s);
+  else if (L.ftype == FACE_F16)
+    rb_tile_t<T, _Float16>(L, mode, x_in, x_out, b, xc, dc, bc, sweeps, s);
+  else
+    rb_tile_t<T, float>(L, mode, x_in, x_out, b, xc, dc, bc, sweeps, s);
+}
+
+template <class T>
+void rb_pre(const Level& L, T* x, const T* b, Dims dc, T* bc, int sweeps, hipStream_t s) {
+  rb_tile<T>(L, RB_PRE, nullptr, x, b, nullptr, dc, bc, sweeps, s);
+}
+template <class T>
+void rb_pre_tr(const Level& L, T* x, const T* b, T* r, int sweeps, hipStream_t s) {
+  rb_tile<T>(L, RB_PRE_TR, nullptr, x, b, nullptr, Dims{0, 0, 0}, r, sweeps, s);
+}
+template <class T>
+void rb_post(const Level& L, int trans, const T* x_in, T* x_out, const T* b, const T* xc, Dims dc, int sweeps,
+             hipStream_t s) {
+  rb_tile<T>(L, trans ? RB_POST_TR : RB_POST, x_in, x_out, b, xc, dc, nullptr, sweeps, s);
+}
+template void rb_pre<float>(const Level&, float*, const float*, Dims, float*, int, hipStream_t);
+template void rb_pre<double>(const Level&, double*, const double*, Dims, double*, int, hipStream_t);
+template void rb_pre_tr<float>(const Level&, float*, const float*, float*, int, hipStream_t);
+template void rb_pre_tr<double>(const Level&, double*, const double*, double*, int, hipStream_t);
+template void rb_post<float>(const Level&, int, const float*, float*, const float*, const float*, Dims, int, hipStream_t);
+template void rb_post<double>(const Level&, int, const double*, double*, const double*, const double*, Dims, int,
+                              hipStream_t);
 
 template <class T>
 bool coarse_fits(const CoarseLevels<T>& C) {

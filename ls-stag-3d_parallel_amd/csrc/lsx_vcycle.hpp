@@ -119,6 +119,18 @@ template <class T>
 void coarse_cycle(const CoarseLevels<T>& C, int trans, int n_pre, int n_post, const double* lu_scale, const int* lu_perm,
                   const double* L, const double* U, const double* dinv, hipStream_t s);
 
+// one side of a red-black level's cycle in one launch (k_rb_tile), sweeps 1 or 2, bit-identical to the
+// launches one by one.  rb_pre: x = sweeps from 0, bc = sum restriction of the residual; rb_pre_tr: the
+// transposed cycle's sweeps, r = b - A^T x; rb_post: x_out = sweeps from x_in + P xc (trans: R^T xc)
+constexpr int RB_TILE_SWEEPS = 2;
+template <class T>
+void rb_pre(const Level& L, T* x, const T* b, Dims dc, T* bc, int sweeps, hipStream_t s);
+template <class T>
+void rb_pre_tr(const Level& L, T* x, const T* b, T* r, int sweeps, hipStream_t s);
+template <class T>
+void rb_post(const Level& L, int trans, const T* x_in, T* x_out, const T* b, const T* xc, Dims dc, int sweeps,
+             hipStream_t s);
+
 // Coarsest level of a capped hierarchy (DENSE_MAX unknowns at most) as a dense FP64 inverse,
 // formed at setup by Gauss-Jordan elimination with partial pivoting on the scaled operator:
 // inv_c column-major (inv_c[j n + i] = inv(i, j)), inv_r row-major; work holds 2 n^2 + 2 n + 1
