@@ -326,6 +326,7 @@ int lsx_geometry_shape_gradient(lsx_geometry* g, const double* p, const double* 
   if (mem != LSX_MEM_HOST && mem != LSX_MEM_DEVICE) return LSX_ERR_ARG;
   if (u && !bc) return LSX_ERR_ARG;
   return guarded([&] {
+    lsx::BlockPool::Scope blocks(g->impl.spare);
     lsx::FlowStage st;
     if (u) g->impl.stage_flow(u, v, w, u_west, u_out, *bc, mem, st);
     g->impl.shape_gradient(p, lambda, objective, u ? &st.args : nullptr, pin, h_rel, dJdphi, dJdctrl, mem);
@@ -374,6 +375,7 @@ int lsx_adjoint_backward(lsx_tape* t, const double* dJdp, int objective, const d
       LSX_HIP(hipMemset(dJdb, 0, n * sizeof(double)));
     S.solve_adjoint(dJdp, dJdb, mem, it, norm_r);
     if (dJdctrl) {
+      lsx::BlockPool::Scope blocks(G.spare);
       lsx::FlowStage st;
       if (u) G.stage_flow(u, v, w, u_west, u_out, *bc, mem, st);
       lsx::DevBuf<double> lam;

@@ -60,6 +60,7 @@ Geometry::~Geometry() {
 }
 
 void Geometry::build(const geo::Body& body_in, geo::Box box, const double* host_ctrl) {
+  BlockPool::Scope blocks(spare);
   if (box.hs < 1 || box.vs < 1 || box.hf > N - 1 || box.vf > M - 1 || box.hs >= box.hf || box.vs >= box.vf)
     throw Error(LSX_ERR_ARG, "geometry box must lie inside the domain's interior");
   if (body_in.kind != geo::BODY_SPHERE && body_in.kind != geo::BODY_ELLIPSOID && body_in.kind != geo::BODY_BEZIER6)
@@ -177,6 +178,7 @@ int Geometry::list_nodes(int mode, const unsigned char* mark, double h, DevBuf<i
 }
 
 double Geometry::drag(const double* p, double* dJdp, int mem) {
+  BlockPool::Scope blocks(spare);
   if (!built) throw Error(LSX_ERR_STATE, "geometry not built");
   if (!p) throw Error(LSX_ERR_ARG, "null pressure");
   const long nn = n();
@@ -248,6 +250,7 @@ void Geometry::drag_noalloc(const double* p, double* J, double* dJdp) {
 
 void Geometry::shape_gradient(const double* p, const double* lam, int objective, const geo::RhsArgs* rhs, int pin,
                               double h_rel, double* dJdphi, double* dJdctrl, int mem) {
+  BlockPool::Scope blocks(spare);
   if (!built) throw Error(LSX_ERR_STATE, "geometry not built");
   if (!p || !lam) throw Error(LSX_ERR_ARG, "null pressure or adjoint");
   if (objective != geo::OBJ_NONE && objective != geo::OBJ_DRAG_X) throw Error(LSX_ERR_ARG, "unknown objective");
@@ -341,6 +344,7 @@ void Geometry::laplace7(int pin, double* coef_dev, hipStream_t s) const {
 
 void Geometry::pressure_rhs(const double* u, const double* v, const double* w, const double* u_west,
                             const double* u_out, const lsx_flow_bc& bc, double* b, int mem) {
+  BlockPool::Scope blocks(spare);
   if (!built) throw Error(LSX_ERR_STATE, "geometry not built");
   const long nn = n(), nu = (long)(N - 1) * M * K, nv = (long)N * (M - 1) * K, nw = (long)N * M * (K - 1);
   const long nrow = (long)M * K;
@@ -381,6 +385,7 @@ void Geometry::pressure_rhs(const double* u, const double* v, const double* w, c
 
 void Geometry::correct(const double* dp, const double* us, const double* vs, const double* ws, double* u, double* v,
                        double* w, double* p, double coef, int mem) {
+  BlockPool::Scope blocks(spare);
   if (!built) throw Error(LSX_ERR_STATE, "geometry not built");
   const long nn = n(), nu = (long)(N - 1) * M * K, nv = (long)N * (M - 1) * K, nw = (long)N * M * (K - 1);
   if (mem == LSX_MEM_DEVICE) {

@@ -81,6 +81,7 @@ class Geometry {
   long n() const { return (long)N * M * K; }
   bool built = false;
   long build_count = 0;
+  BlockPool spare;  // the host-array calls' device copies
 
  private:
   hipStream_t stream = nullptr;

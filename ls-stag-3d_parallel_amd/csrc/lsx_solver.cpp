@@ -74,7 +74,8 @@ hipEvent_t Solver::ev_take() {
 }
 
 void Solver::clear_graphs() {
-  for (CycleGraph& g : cgraphs) (void)hipGraphExecDestroy(g.exec);
+  for (CycleGraph& g : cgraphs)
+    if (g.exec) (void)hipGraphExecDestroy(g.exec);
   cgraphs.clear();
 }
 
@@ -244,6 +245,7 @@ void Solver::setup_levels(int N, int M, int K) {
 }
 
 void Solver::set_geometry(const Geometry& g, int pin) {
+  BlockPool::Scope blocks(spare);
   check_dims(g.N, g.M, g.K);
   ready = false;
   values_dirty = false;
@@ -260,6 +262,7 @@ void Solver::set_geometry(const Geometry& g, int pin) {
 }
 
 void Solver::set_helmholtz(const Geometry& g, int dir, double nu, double coef_time, int flow) {
+  BlockPool::Scope blocks(spare);
   if (dir < 0 || dir > 2) throw Error(LSX_ERR_ARG, "velocity component must be 0 (u), 1 (v) or 2 (w)");
   const int N = g.N - (dir == 0), M = g.M - (dir == 1), K = g.K - (dir == 2);
   check_dims(N, M, K);
@@ -277,6 +280,7 @@ void Solver::set_helmholtz(const Geometry& g, int dir, double nu, double coef_ti
 
 void Solver::set_fields(int N, int M, int K, const double* dx, const double* dy, const double* dz, const int* type,
                         const double* thx, const double* thy, const double* thz, const double* vof, int pin, int mem) {
+  BlockPool::Scope blocks(spare);
   check_dims(N, M, K);
   if (!dx || !dy || !dz || !type || !thx || !thy || !thz || !vof) throw Error(LSX_ERR_ARG, "null mesh field");
   if (mem != LSX_MEM_HOST && mem != LSX_MEM_DEVICE) throw Error(LSX_ERR_ARG, "mem must be LSX_MEM_HOST or LSX_MEM_DEVICE");
@@ -311,6 +315,7 @@ void Solver::set_fields(int N, int M, int K, const double* dx, const double* dy,
 }
 
 void Solver::set_csr(int N, int M, int K, const int* rp, const int* cl, const double* vl, long nnz, int mem) {
+  BlockPool::Scope blocks(spare);
   check_dims(N, M, K);
   src_geo = nullptr;
   if (!rp || !cl || !vl || nnz <= 0) throw Error(LSX_ERR_ARG, "null CSR array or empty matrix");
@@ -364,6 +369,7 @@ void Solver::update_values(const double* vl, int mem) {
 }
 
 void Solver::rebuild() {
+  BlockPool::Scope blocks(spare);
   if (!ready) throw Error(LSX_ERR_STATE, "rebuild before set_csr");
   build_hierarchy();
   values_dirty = false;
@@ -654,11 +660,20 @@ void Solver::vcycle_apply(const double* v, T* z, const float* b32) {
   }
   // one captured graph per (v, z) pair: the Krylov loops apply the cycle to a fixed set of
   // basis slots, so a graph replays every launch of a cycle with one submission
-  for (const CycleGraph& g : cgraphs)
-    if (g.v == v && g.z == (const void*)z && g.b32 == b32) {
-      LSX_HIP(hipGraphLaunch(g.exec, stream));
-      return;
-    }
+  CycleGraph* mine = nullptr;
+  for (CycleGraph& g : cgraphs)
+    if (g.v == v && g.z == (const void*)z && g.b32 == b32) mine = &g;
+  if (mine && mine->exec) {
+    LSX_HIP(hipGraphLaunch(mine->exec, stream));
+    return;
+  }
+  // a pair's first cycle since the set-up runs eagerly: capture and instantiation (46 us) pay from
+  // the second replay on, and a set-up per solve uses each pair once
+  if (!mine) {
+    cgraphs.push_back({v, (const void*)z, b32, nullptr});
+    vcycle_run<T>(v, z, b32);
+    return;
+  }
   hipGraph_t graph = nullptr;
   LSX_HIP(hipStreamBeginCapture(stream, hipStreamCaptureModeThreadLocal));
   capturing = true;
@@ -676,7 +691,7 @@ void Solver::vcycle_apply(const double* v, T* z, const float* b32) {
   const hipError_t ie = hipGraphInstantiate(&exec, graph, nullptr, nullptr, 0);
   (void)hipGraphDestroy(graph);
   LSX_HIP(ie);
-  cgraphs.push_back({v, (const void*)z, b32, exec});
+  mine->exec = exec;
   LSX_HIP(hipGraphLaunch(exec, stream));
 }
 
