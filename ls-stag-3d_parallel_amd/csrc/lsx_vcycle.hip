@@ -1608,10 +1608,11 @@ __device__ inline T wave_get(T v, int src, bool ok) {
   return r;
 }
 
-// CPL consecutive elements of p from index i (i a multiple of CPL) as one wide load
+// CPL consecutive elements of p from index i as one wide load, aligned to the element (rows of a
+// length that is no multiple of CPL start anywhere)
 template <class E, int C>
 __device__ inline void ld_pack(const E* __restrict__ p, long i, E (&out)[C]) {
-  struct alignas(sizeof(E) * C) Pack {
+  struct __attribute__((packed, aligned(alignof(E)))) Pack {
     E v[C];
   };
   const Pack pk = *reinterpret_cast<const Pack*>(p + i);
@@ -1619,9 +1620,10 @@ __device__ inline void ld_pack(const E* __restrict__ p, long i, E (&out)[C]) {
   for (int j = 0; j < C; ++j) out[j] = pk.v[j];
 }
 
-// The rows of cells i0 .. i0 + CPL - 1 of one x line (i0 = row start + CPL * lane, N a multiple
-// of CPL): the same rows as line_row, each array read with one wide load per lane.  The lines'
-// neighbours in y and z exist or not for the whole row; pinned cells are checked per cell.
+// The rows of cells i0 .. i0 + CPL - 1 of one x line (i0 = row start + CPL * lane): the same rows
+// as line_row, each array read with one wide load per lane.  The lines' neighbours in y and z
+// exist or not for the whole row; pinned cells are checked per cell.  Cells past the row's end are
+// decoupled identity rows (their loads read the next row).
 template <class T, class FT, int CPL, bool ZERO, bool DFF>
 __device__ inline void line_rows_x(const T* __restrict__ x, const T* __restrict__ b, const FT* __restrict__ ae,
                                    const FT* __restrict__ an, const FT* __restrict__ at, const T* __restrict__ s,
@@ -1681,10 +1683,11 @@ __device__ inline void line_rows_x(const T* __restrict__ x, const T* __restrict_
       empty = sv[j] == (T)0;
     }
     const bool ident = own && !trans, cut = ident || empty;
-    lo[j] = cut ? (T)0 : cw;
-    up[j] = cut ? (T)0 : ce;
-    dg[j] = cut ? (T)1 : ap;
-    rh[j] = ident ? bi : (empty ? xi : bi - off);
+    const bool past = CPL > 1 && k >= N;
+    lo[j] = cut || past ? (T)0 : cw;
+    up[j] = cut || past ? (T)0 : ce;
+    dg[j] = cut || past ? (T)1 : ap;
+    rh[j] = past ? (T)0 : (ident ? bi : (empty ? xi : bi - off));
   }
 }
 
@@ -1706,7 +1709,9 @@ __global__ void __launch_bounds__(256) k_line_x(const T* __restrict__ x_in, T* _
   const long row = live ? row_t : (long)M * K - 1;
   const int yy = (int)(row % M), zz = (int)(row / M);
   T lo[CPL], dg[CPL], up[CPL], rh[CPL];
-  if (N % CPL == 0 && lane * CPL < N) {
+  // a lane across the row's end reads on into the next row, of its neighbours' rows too, where
+  // that row is there.  129 x 111 x 95 FP32: one cell a load 22.6 us, so 13.6
+  if (lane * CPL < N && (lane * CPL + CPL <= N || row < (long)M * K - M - 1)) {
     line_rows_x<T, FT, CPL, ZERO, DFF>(x_in, b, ae, an, at, s, fs, row * N + lane * CPL, lane * CPL, yy, zz, N, M,
                                        K, pin0, pin1, TRANS, lo, dg, up, rh, dr);
   } else {
@@ -1788,11 +1793,18 @@ __global__ void __launch_bounds__(256) k_line_x(const T* __restrict__ x_in, T* _
   const T xe = r * recip0(d);
   const T xl0 = wave_get<LANES>(xe, lane - 1, lane > 0);
   const T xl = lane > 0 ? xl0 : (T)0;
+  struct __attribute__((packed, aligned(alignof(T)))) Pack {
+    T v[CPL];
+  } out;
 #pragma unroll
-  for (int j = 0; j < CPL; ++j) {
-    const int k = lane * CPL + j;
-    const T v = j == CPL - 1 ? xe : G[j] + H[j] * xl + Q[j] * xe;
-    if (live && k < N) x_out[row * N + k] = v;
+  for (int j = 0; j < CPL; ++j) out.v[j] = j == CPL - 1 ? xe : G[j] + H[j] * xl + Q[j] * xe;
+  T* const to = x_out + row * N + lane * CPL;
+  if (live && lane * CPL + CPL <= N) {
+    *reinterpret_cast<Pack*>(to) = out;
+  } else if (live) {
+#pragma unroll
+    for (int j = 0; j < CPL; ++j)
+      if (lane * CPL + j < N) to[j] = out.v[j];
   }
 }
 
@@ -1919,9 +1931,10 @@ __global__ void __launch_bounds__(1024) k_line_seg(const T* __restrict__ x_in, T
   // Line groups in XCD-contiguous order, columns fastest: the halo columns and neighbouring
   // planes a workgroup reads are read by workgroups of the same XCD at about the same time
   // (measured fetch 26 instead of 35 B/cell, 24 B/cell compulsory reads; 9 % less time).  y lines:
-  // LPW adjacent x of one (y = 0, z) row; z lines: LPW consecutive cells p = x + N y of the (x, y)
-  // plane, so that every row load is one aligned 128-byte line whatever N is (the same groups as
-  // x runs of one row when LPW divides N)
+  // LPW adjacent x of one (y = 0, z) row (groups of consecutive (x, z) across the rows' ends leave no
+  // lane idle but read two runs per row: 129 x 111 x 95 FP32 21 us against 17); z lines: LPW
+  // consecutive cells p = x + N y of the (x, y) plane, so that every row load is one aligned
+  // 128-byte line whatever N is (the same groups as x runs of one row when LPW divides N)
   const int gxb = (N + LPW - 1) / LPW;
   const int lb = xcd_order(blockIdx.x, gridDim.x);
   bool live;
@@ -1935,11 +1948,10 @@ __global__ void __launch_bounds__(1024) k_line_seg(const T* __restrict__ x_in, T
   } else {
     p0 = (long)lb * LPW;
     pl = p0 + LPW - 1 < NM - 1 ? p0 + LPW - 1 : NM - 1;
-    const long pr = p0 + lane;
-    live = pr < NM;
-    const long pc = live ? pr : NM - 1;
-    xx = (int)(pc % N);
-    other = (int)(pc / N);
+    live = p0 + lane < NM;
+    const unsigned pc = (unsigned)(live ? p0 + lane : NM - 1);
+    other = (int)(pc / (unsigned)N);
+    xx = (int)(pc - (unsigned)other * (unsigned)N);
   }
   const int len = DIR == 1 ? M : K;
   const long stride = DIR == 1 ? (long)N : NM;
@@ -1952,8 +1964,8 @@ __global__ void __launch_bounds__(1024) k_line_seg(const T* __restrict__ x_in, T
   T le = (T)0, de = (T)1, ue = (T)0, re = (T)0;  // row of the last cell
   T Gb = (T)0, Hb = (T)1, Qb = (T)0;              // the cell before the last, in (x_L, x_E)
   T Gf = (T)0, Hf = (T)0, Qf = (T)1;              // the first cell, in (x_L, x_E)
-  // the elimination of the segment; FULL: a segment of SEG rows (every segment of a line whose
-  // length is a multiple of SEG), whose masks are then known at compile time
+  // the elimination of the segment; FULL: segments of SEG rows (a line whose length is a multiple of
+  // SEG), whose masks are then known at compile time
   auto eliminate = [&](auto full_tag) {
     constexpr bool FULL = decltype(full_tag)::value;
     const int nrow = FULL ? SEG : cnt;
@@ -2055,10 +2067,13 @@ __global__ void __launch_bounds__(1024) k_line_seg(const T* __restrict__ x_in, T
       }
     }
   };
-  if (cnt == SEG)
+  // one of the two for the whole workgroup: a wavefront with a full and a partial segment would go
+  // through both, and the others wait for it (17 x 14 x 12: 7.7 us a z pass, so 5.8)
+  if (len % SEG == 0)
     eliminate(std::true_type{});
   else
     eliminate(std::false_type{});
+  int xe_plane = 7;
   if ((S & (S - 1)) == 0) {
     // S a power of two (<= 32): the reduced systems are solved inside wavefronts.  Each thread
     // posts its partial last-cell row and its first cell; after one barrier thread t takes
@@ -2100,7 +2115,8 @@ __global__ void __launch_bounds__(1024) k_line_seg(const T* __restrict__ x_in, T
     IF(7, ts, tl) = r * recip0(d);
     __syncthreads();
   } else {
-    // general S: cyclic reduction across the wavefronts through LDS, one barrier pair per step
+    // general S: cyclic reduction across the wavefronts through LDS, one barrier per step: the steps
+    // post their rows to planes 0-3 and 4-7 in turn
     IF(4, seg, lane) = Gf;
     IF(5, seg, lane) = Hf;
     IF(6, seg, lane) = Qf;
@@ -2114,29 +2130,31 @@ __global__ void __launch_bounds__(1024) k_line_seg(const T* __restrict__ x_in, T
     T d = de + le * Qb + ue * H1;
     T c = ue * Q1;
     T r = re - le * Gb - ue * G1;
+    int to = 0;
     for (int st = 1; st < S; st <<= 1) {  // S is uniform over the workgroup
-      IF(0, seg, lane) = a;
-      IF(1, seg, lane) = d;
-      IF(2, seg, lane) = c;
-      IF(3, seg, lane) = r;
+      IF(to, seg, lane) = a;
+      IF(to + 1, seg, lane) = d;
+      IF(to + 2, seg, lane) = c;
+      IF(to + 3, seg, lane) = r;
       __syncthreads();
       const bool okm = seg - st >= 0, okp = seg + st < S;
-      const T am = okm ? IF(0, seg - st, lane) : (T)0, dm = okm ? IF(1, seg - st, lane) : (T)1;
-      const T cm = okm ? IF(2, seg - st, lane) : (T)0, rm = okm ? IF(3, seg - st, lane) : (T)0;
-      const T ap = okp ? IF(0, seg + st, lane) : (T)0, dp = okp ? IF(1, seg + st, lane) : (T)1;
-      const T cq = okp ? IF(2, seg + st, lane) : (T)0, rp = okp ? IF(3, seg + st, lane) : (T)0;
+      const T am = okm ? IF(to, seg - st, lane) : (T)0, dm = okm ? IF(to + 1, seg - st, lane) : (T)1;
+      const T cm = okm ? IF(to + 2, seg - st, lane) : (T)0, rm = okm ? IF(to + 3, seg - st, lane) : (T)0;
+      const T ap = okp ? IF(to, seg + st, lane) : (T)0, dp = okp ? IF(to + 1, seg + st, lane) : (T)1;
+      const T cq = okp ? IF(to + 2, seg + st, lane) : (T)0, rp = okp ? IF(to + 3, seg + st, lane) : (T)0;
       const T al = -a * recip0(dm), ga = -c * recip0(dp);
       a = al * am;
       c = ga * cq;
       d = d + al * cm + ga * ap;
       r = r + al * rm + ga * rp;
-      __syncthreads();
+      to ^= 4;
     }
-    IF(7, seg, lane) = r * recip0(d);
+    xe_plane = to + 3;
+    IF(xe_plane, seg, lane) = r * recip0(d);
     __syncthreads();
   }
-  const T xe = IF(7, seg, lane);
-  const T xl = seg > 0 ? IF(7, seg - 1, lane) : (T)0;
+  const T xe = IF(xe_plane, seg, lane);
+  const T xl = seg > 0 ? IF(xe_plane, seg - 1, lane) : (T)0;
   if (live) {
 #pragma unroll
     for (int k = 0; k < SEG; ++k)
