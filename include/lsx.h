@@ -65,7 +65,8 @@ typedef struct lsx_options {
                         a grid with a short axis) is solved by its dense FP64 inverse */
   int z_head_fix;    /* 0 = reproduce the reference z-line head read (default) */
   int ortho;         /* LSX_ORTHO_*: FGMRES orthogonalisation                    */
-  int coarse_fuse;   /* V-cycle: 1 = levels of <= 4096 cells in one launch (default), 0 = per level */
+  int coarse_fuse;   /* V-cycle: 1 = levels of <= 4096 cells (with lines: <= 1024) in one launch (default),
+                        0 = per level                                                           */
   int graphs;        /* V-cycle: 1 = replay each cycle from a captured HIP graph (one per basis slot) */
   int smoother;      /* V-cycle: LSX_SMOOTH_RBGS (default) or LSX_SMOOTH_LINE                  */
   int fused_sweep;   /* V-cycle red-black: 1 = both colours in one pass on a finest level of

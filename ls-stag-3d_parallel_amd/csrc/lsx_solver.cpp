@@ -725,7 +725,8 @@ void Solver::vcycle_run(const double* v, T* z, const float* b32) {
     vc::resid_restrict<T>(S.L, x, b, vb<T>(vlev[l + 1]), stream);
   }
   if (C.count)
-    vc::coarse_cycle<T>(C, 0, opt.n_pre, opt.n_post, lu_scale.p, lu_perm.p, lu_L.p, lu_U.p, dense_c.p, stream);
+    (line_level(top) ? vc::line_cycle<T> : vc::coarse_cycle<T>)(C, 0, opt.n_pre, opt.n_post, lu_scale.p, lu_perm.p, lu_L.p,
+                                                               lu_U.p, dense_c.p, stream);
   else
     coarse_solve<T>(false);
   for (int l = top - 1; l >= 0; --l) {
@@ -748,12 +749,12 @@ int Solver::coarse_levels(vc::CoarseLevels<T>& C) {
   const int L = (int)vlev.size() - 1;
   if (!opt.coarse_fuse || (dense_c.p && vlev[L].L.d.n() > vc::COARSE_DENSE)) return L;
   for (int l = 1; l < L; ++l) {  // the LU level alone gains nothing
-    if (!rb_level(l) || L - l + 1 > vc::COARSE_MAX) continue;
+    if ((!rb_level(l) && !line_level(l)) || L - l + 1 > vc::COARSE_MAX) continue;
     C.count = L - l + 1;
     for (int q = 0; q < C.count; ++q) C.L[q] = vlev[l + q].L;
     C.x = vx<T>(vlev[l]);
     C.b = vb<T>(vlev[l]);
-    if (vc::coarse_fits<T>(C)) return l;
+    if (rb_level(l) ? vc::coarse_fits<T>(C) : line_level(L - 1) && vc::coarse_line_fits<T>(C)) return l;
   }
   C.count = 0;
   return L;
@@ -883,7 +884,8 @@ void Solver::vcycle_apply_tr(const double* v, T* z) {
     vc::restrict_pt<T>(vr<T>(S), S.L.d, vb<T>(vlev[l + 1]), stream);
   }
   if (C.count)
-    vc::coarse_cycle<T>(C, 1, opt.n_post, opt.n_pre, lu_scale.p, lu_perm.p, lu_L.p, lu_U.p, dense_r.p, stream);
+    (line_level(top) ? vc::line_cycle<T> : vc::coarse_cycle<T>)(C, 1, opt.n_post, opt.n_pre, lu_scale.p, lu_perm.p, lu_L.p,
+                                                               lu_U.p, dense_r.p, stream);
   else
     coarse_solve<T>(true);
   for (int l = top - 1; l >= 0; --l) {

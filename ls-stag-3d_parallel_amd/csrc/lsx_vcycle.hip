@@ -775,6 +775,69 @@ struct RbCells {
   }
 };
 
+// Restriction of a level's residual in LDS to its coarse level's right-hand side (sum over the
+// children, TR: P^T)
+template <class T, bool TR>
+__device__ inline void coarse_restrict(const T* res, int N, int M, int K, T* bc) {
+  const int Nc = (N + 1) / 2, Mc = (M + 1) / 2, nc = Nc * Mc * ((K + 1) / 2);
+  const float inc = 1.0f / (float)Nc, imc = 1.0f / (float)Mc;
+  for (int I = threadIdx.x; I < nc; I += COARSE_THREADS) {
+    const int R = small_div(I, inc), X = I - R * Nc, Z = small_div(R, imc), Y = R - Z * Mc;
+    T acc = 0;
+    if constexpr (TR) {
+      acc = restrict_pt_cell<T>([&](int a, int b, int c) { return res[a + N * (b + M * c)]; }, X, Y, Z, N, M, K);
+    } else {
+#pragma unroll
+      for (int c = 0; c < 8; ++c) {
+        const int cx = 2 * X + (c & 1), cy = 2 * Y + ((c >> 1) & 1), cz = 2 * Z + (c >> 2);
+        const bool in = cx < N && cy < M && cz < K;  // odd axes: one child
+        const T v = res[in ? cx + N * (cy + M * cz) : 0];
+        acc += in ? v : (T)0;
+      }
+    }
+    bc[I] = acc;
+  }
+}
+// x += P xc (TR: R^T xc), both in LDS
+template <class T, bool TR>
+__device__ inline void coarse_prolong(const T* xc, int N, int M, int K, T* x) {
+  const int Nc = (N + 1) / 2, Mc = (M + 1) / 2, n = N * M * K;
+  const float in = 1.0f / (float)N, im = 1.0f / (float)M;
+  for (int i = threadIdx.x; i < n; i += COARSE_THREADS) {
+    const int r = small_div(i, in), a = i - r * N, c = small_div(r, im), b = r - c * M;
+    if constexpr (TR)
+      x[i] += xc[(a >> 1) + Nc * ((b >> 1) + Mc * (c >> 1))];
+    else
+      x[i] += prolong_value<T>([&](int X, int Y, int Z) { return xc[X + Nc * (Y + Mc * Z)]; }, N, M, K, a, b, c);
+  }
+}
+// The coarsest level (n unknowns, b and x in LDS): its dense inverse, column-major, x_i = sum_j inv[j n
+// + i] b_j, or its LU, staged by the caller if `staged`
+template <class T>
+__device__ inline void coarse_bottom(const LuLds& lu, int n, bool staged, const double* __restrict__ lu_scale,
+                                     const int* __restrict__ lu_perm, const double* __restrict__ Lf,
+                                     const double* __restrict__ Uf, const double* __restrict__ dinv, const T* b, T* x) {
+  const int tid = threadIdx.x;
+  if (dinv) {
+    for (int i = tid; i < n; i += COARSE_THREADS) {
+      double acc = 0.0;
+      for (int j = 0; j < n; ++j) acc += dinv[(long)j * n + i] * (double)b[j];
+      x[i] = (T)acc;
+    }
+  } else {
+    if (!staged) {
+      lu_stage(lu, n, lu_scale, lu_perm, Lf, Uf);
+      __syncthreads();
+    }
+    if (tid < 64) {
+      if (tid < n) lu.rhs[tid] = (double)b[tid];
+      lu_substitute(lu, n);
+      if (tid < n) x[tid] = (T)lu.rhs[tid];
+    }
+  }
+  __syncthreads();
+}
+
 // The small levels of the cycle in one workgroup: pre-smoothing and restriction down to the
 // coarsest level, its dense LU solve (FP64, the factors of lu_factor) or dense inverse, then
 // prolongation and post-smoothing back up; barriers separate the phases (one launch instead of
@@ -834,65 +897,21 @@ __global__ void __launch_bounds__(COARSE_THREADS) k_coarse_cycle(CoarseLevels<T>
     }
     cells.residual(x, fs, N, N * M, res);
     __syncthreads();
-    const int Nc = (N + 1) / 2, Mc = (M + 1) / 2, nc = Nc * Mc * ((K + 1) / 2);
-    const float inc = 1.0f / (float)Nc, imc = 1.0f / (float)Mc;
-    for (int I = tid; I < nc; I += COARSE_THREADS) {
-      const int R = small_div(I, inc), X = I - R * Nc, Z = small_div(R, imc), Y = R - Z * Mc;
-      T acc = 0;
-      if constexpr (TR) {
-        acc = restrict_pt_cell<T>([&](int a, int b, int c) { return res[a + N * (b + M * c)]; }, X, Y, Z, N, M, K);
-      } else {
-#pragma unroll
-        for (int c = 0; c < 8; ++c) {
-          const int cx = 2 * X + (c & 1), cy = 2 * Y + ((c >> 1) & 1), cz = 2 * Z + (c >> 2);
-          const bool in = cx < N && cy < M && cz < K;  // odd axes: one child
-          const T v = res[in ? cx + N * (cy + M * cz) : 0];
-          acc += in ? v : (T)0;
-        }
-      }
-      bs[off + n + I] = acc;
-    }
+    coarse_restrict<T, TR>(res, N, M, K, bs + off + n);
     off += n;
     __syncthreads();
   }
-  T* xl = xs + off;
-  const T* bl = bs + off;
-  if (dinv) {  // dense inverse of the last level, column-major: x_i = sum_j inv[j n + i] b_j
-    for (int i = tid; i < n_last; i += COARSE_THREADS) {
-      double acc = 0.0;
-      for (int j = 0; j < n_last; ++j) acc += dinv[(long)j * n_last + i] * (double)bl[j];
-      xl[i] = (T)acc;
-    }
-  } else {
-    if (!early) {
-      lu_stage(lu, n_last, lu_scale, lu_perm, Lf, Uf);
-      __syncthreads();
-    }
-    if (tid < 64) {
-      if (tid < n_last) lu.rhs[tid] = (double)bl[tid];
-      lu_substitute(lu, n_last);
-      if (tid < n_last) xl[tid] = (T)lu.rhs[tid];
-    }
-  }
-  __syncthreads();
+  coarse_bottom<T>(lu, n_last, early, lu_scale, lu_perm, Lf, Uf, dinv, bs + off, xs + off);
   for (int q = last - 1; q >= 0; --q) {
     const Level& L = C.L[q];
     const int N = L.d.N, M = L.d.M, K = L.d.K, n = N * M * K;
-    const int Nc = C.L[q + 1].d.N, Mc = C.L[q + 1].d.M;
     const T* xc = xs + off;
     off -= n;
     T* x = xs + off;
     const T fs = (T)L.fscale;
     RbCells<T, NI> cells;
     cells.template load<FT>(L, [&](int i) { return bs[off + i]; });
-    const float in = 1.0f / (float)N, im = 1.0f / (float)M;
-    for (int i = tid; i < n; i += COARSE_THREADS) {
-      const int r = small_div(i, in), a = i - r * N, c = small_div(r, im), b = r - c * M;
-      if constexpr (TR)
-        x[i] += xc[(a >> 1) + Nc * ((b >> 1) + Mc * (c >> 1))];
-      else
-        x[i] += prolong_value<T>([&](int X, int Y, int Z) { return xc[X + Nc * (Y + Mc * Z)]; }, N, M, K, a, b, c);
-    }
+    coarse_prolong<T, TR>(xc, N, M, K, x);
     __syncthreads();
     for (int sw = 0; sw < n_post; ++sw) {
       cells.template half<FIRST>(x, fs, N, N * M, 0);
@@ -2166,6 +2185,254 @@ __global__ void __launch_bounds__(1024) k_line_seg(const T* __restrict__ x_in, T
   }
 }
 
+// ---- small line-relaxed levels in one workgroup --------------------------------------------------
+// One line pass over a level in LDS (x_in, x_out, b, faces in operator units, reciprocals of s), bit
+// for bit as k_line_x<CPL 1> and k_line_seg: the directions differ in strides only.  A: the first
+// direction across the line, B: the second.
+__device__ inline float fma_of(float a, float b, float c) { return __builtin_fmaf(a, b, c); }
+__device__ inline double fma_of(double a, double b, double c) { return __builtin_fma(a, b, c); }
+template <class T>
+struct LineCells {
+  const T *e, *n, *t, *ap, *b;
+};
+template <class T, bool TR>
+struct SmallLines {
+  const T *fL, *fA, *fB, *ap, *b;
+  int sL, sA, sB;   // strides along the line and across
+  int len, nA, nB;  // cells along the line and across
+
+  __device__ SmallLines(const Dims& d, int dir, const LineCells<T>& c) {
+    fL = dir == 0 ? c.e : dir == 1 ? c.n : c.t;
+    fA = dir == 0 ? c.n : c.e;
+    fB = dir == 2 ? c.n : c.t;
+    sL = dir == 0 ? 1 : dir == 1 ? d.N : d.N * d.M;
+    sA = dir == 0 ? d.N : 1;
+    sB = dir == 2 ? d.N : d.N * d.M;
+    len = dir == 0 ? d.N : dir == 1 ? d.M : d.K;
+    nA = dir == 0 ? d.M : d.N;
+    nB = dir == 2 ? d.M : d.K;
+    ap = c.ap;
+    b = c.b;
+  }
+  // row of cell k of line (p, q)
+  template <bool FIRST>
+  __device__ inline void row(const T* x, int k, int p, int q, T& lo, T& dg, T& up, T& rh) const {
+  #pragma clang fp contract(fast)  // as line_row
+    const int i = k * sL + p * sA + q * sB;
+    const bool l0 = k > 0, l1 = k < len - 1, a0 = p > 0, a1 = p < nA - 1, b0 = q > 0, b1 = q < nB - 1;
+    const int ia0 = a0 ? i - sA : i, ia1 = a1 ? i + sA : i, ib0 = b0 ? i - sB : i, ib1 = b1 ? i + sB : i;
+    const T d = ap[i], xi = x[i];
+    const T fl = fL[l0 ? i - sL : i], fu = fL[i];
+    const T fa = fA[ia0], fc = fA[i], fb = fB[ib0], fd = fB[i];
+    const T ca0 = a0 ? fa : (T)0, ca1 = a1 ? fc : (T)0, cb0 = b0 ? fb : (T)0, cb1 = b1 ? fd : (T)0;
+    // the sum as the compiler contracts it in the passes launched one by one: line_row and line_rows_x
+    // round the second product, SegLine::row (FIRST) the first
+    const T first = FIRST ? fma_of(ca1, x[ia1], ca0 * x[ia0]) : fma_of(ca0, x[ia0], ca1 * x[ia1]);
+    const T off = fma_of(cb1, x[ib1], fma_of(cb0, x[ib0], first));
+    const bool empty = d == (T)0;
+    lo = empty || !l0 ? (T)0 : fl;
+    up = empty || !l1 ? (T)0 : fu;
+    dg = empty ? (T)1 : d;
+    rh = empty ? xi : b[i] - off;
+  }
+  // x lines: W lanes a line (W >= len, a power of two), cyclic reduction as k_line_x<CPL 1>
+  __device__ inline void lanes(const T* x, T* y) const {
+  #pragma clang fp contract(fast)  // as k_line_x
+    const int W = len <= 8 ? 8 : len <= 16 ? 16 : len <= 32 ? 32 : 64, lines = nA * nB;
+    const int k = threadIdx.x & (W - 1), step = COARSE_THREADS / W;
+    const float ia = 1.0f / (float)nA;
+    for (int l0 = 0; l0 < lines; l0 += step) {  // the same trips for every thread: shuffles
+      const int l = l0 + (int)threadIdx.x / W;
+      const bool live = l < lines && k < len;
+      const int lc = l < lines ? l : lines - 1, q = small_div(lc, ia), p = lc - q * nA;
+      T a = (T)0, d = (T)1, c = (T)0, r = (T)0;
+      if (live) row<false>(x, k, p, q, a, d, c, r);
+      for (int st = 1; st < len; st <<= 1) {
+        const bool okm = k - st >= 0, okp = k + st < W;
+        const int sm = okm ? k - st : k, sp = okp ? k + st : k;
+        const T am0 = __shfl(a, sm, W), dm0 = __shfl(d, sm, W), cm0 = __shfl(c, sm, W), rm0 = __shfl(r, sm, W);
+        const T ap0 = __shfl(a, sp, W), dp0 = __shfl(d, sp, W), cp0 = __shfl(c, sp, W), rp0 = __shfl(r, sp, W);
+        const T am = okm ? am0 : (T)0, dm = okm ? dm0 : (T)1, cm = okm ? cm0 : (T)0, rm = okm ? rm0 : (T)0;
+        const T ap = okp ? ap0 : (T)0, dp = okp ? dp0 : (T)1, cq = okp ? cp0 : (T)0, rp = okp ? rp0 : (T)0;
+        const T al = -a * recip0(dm), ga = -c * recip0(dp);
+        a = al * am;
+        c = ga * cq;
+        d = d + al * cm + ga * ap;
+        r = r + al * rm + ga * rp;
+      }
+      if (live) y[k * sL + p * sA + q * sB] = r * recip0(d);
+    }
+  }
+  // y and z lines of at most 2 SEG cells: a thread a segment, as k_line_seg with S = 1 or 2; the second
+  // segment of a line sits 32 lanes further
+  __device__ inline void segments(const T* x, T* y) const {
+  #pragma clang fp contract(fast)  // as k_line_seg
+    const bool twin = len > SEG;
+    const int lines = nA * nB, t = threadIdx.x, seg = twin ? (t >> 5) & 1 : 0;
+    const int l = twin ? (t >> 6) * 32 + (t & 31) : t;
+    const bool live = l < lines;
+    const int lc = live ? l : lines - 1, q = small_div(lc, 1.0f / (float)nA), p = lc - q * nA;
+    const int k0 = seg * SEG, cnt = len - k0 < SEG ? len - k0 : SEG;
+    if (!__any(live)) return;
+    T G[SEG], H[SEG], Q[SEG];
+    T le = (T)0, de = (T)1, ue = (T)0, re = (T)0, cp = (T)0, gp = (T)0, hp = (T)1;
+#pragma unroll
+    for (int k = 0; k < SEG; ++k) {
+      T lo, dg, up, rh;
+      row<!TR>(x, k0 + (k < cnt ? k : cnt - 1), p, q, lo, dg, up, rh);
+      const bool el = k < cnt - 1, last = k == cnt - 1;
+      const T winv = recip0(dg - lo * cp);
+      const T gn = (rh - lo * gp) * winv, hn = -lo * hp * winv, cn = up * winv;
+      gp = el ? gn : gp;
+      hp = el ? hn : hp;
+      cp = el ? cn : cp;
+      G[k] = gp;
+      H[k] = hp;
+      Q[k] = cp;
+      le = last ? lo : le;
+      de = last ? dg : de;
+      ue = last ? up : ue;
+      re = last ? rh : re;
+    }
+    T Gb = (T)0, Hb = (T)1, Qb = (T)0, Gn = (T)0, Hn = (T)0, Qn = (T)1;
+#pragma unroll
+    for (int k = SEG - 2; k >= 0; --k) {
+      const bool act = k < cnt - 1, bl = k == cnt - 2;
+      const T c = Q[k];
+      const T gn = G[k] - c * Gn, hn = H[k] - c * Hn, qn = -c * Qn;
+      Gn = act ? gn : Gn;
+      Hn = act ? hn : Hn;
+      Qn = act ? qn : Qn;
+      G[k] = Gn;
+      H[k] = Hn;
+      Q[k] = Qn;
+      Gb = bl ? Gn : Gb;
+      Hb = bl ? Hn : Hb;
+      Qb = bl ? Qn : Qb;
+    }
+    const T Gf = cnt > 1 ? Gn : (T)0, Hf = cnt > 1 ? Hn : (T)0, Qf = cnt > 1 ? Qn : (T)1;
+    const int w = t & 63;
+    const bool nx = twin && seg == 0;
+    const T g1 = __shfl(Gf, w ^ 32, 64), h1 = __shfl(Hf, w ^ 32, 64), q1 = __shfl(Qf, w ^ 32, 64);
+    const T G1 = nx ? g1 : (T)0, H1 = nx ? h1 : (T)0, Q1 = nx ? q1 : (T)0;
+    T a = le * Hb;
+    const T d0 = de + le * Qb, r0 = re - le * Gb;
+    T d = d0 + ue * H1, c = ue * Q1, r = r0 - ue * G1;
+    if (twin) {
+      const T ao = __shfl(a, w ^ 32, 64), dd = __shfl(d, w ^ 32, 64), co = __shfl(c, w ^ 32, 64), ro = __shfl(r, w ^ 32, 64);
+      const bool m = seg == 1;
+      const T am = m ? ao : (T)0, dm = m ? dd : (T)1, cm = m ? co : (T)0, rm = m ? ro : (T)0;
+      const T ap = m ? (T)0 : ao, dp = m ? (T)1 : dd, cq = m ? (T)0 : co, rp = m ? (T)0 : ro;
+      const T al = -a * recip0(dm), ga = -c * recip0(dp);
+      a = al * am;
+      c = ga * cq;
+      d = d + al * cm + ga * ap;
+      r = r + al * rm + ga * rp;
+    }
+    const T xe = r * recip0(d), xo = __shfl(xe, w ^ 32, 64), xl = seg > 0 ? xo : (T)0;
+    if (live) {
+#pragma unroll
+      for (int k = 0; k < SEG; ++k)
+        if (k < cnt) y[(k0 + k) * sL + p * sA + q * sB] = k == cnt - 1 ? xe : G[k] + H[k] * xl + Q[k] * xe;
+    }
+  }
+};
+
+// The small levels of a line-relaxed cycle in one workgroup, as k_coarse_cycle: x, its second
+// buffer, b and the coefficients in LDS.  Launched one by one, 12 line passes of a level of 9 x 7 x 6 or 5 x 4 x 3 cells
+// cost 3.6 to 4.8 us each, a launch's time; so both levels with transfers and LU take 68 us where
+// their launches took 117 (4.4 us x 24 passes, transfers, LU).  TR: the transposed cycle's transfers (the coarse
+// levels are symmetric and hold no pinned rows).
+template <class T, class FT, bool TR>
+__global__ void __launch_bounds__(COARSE_THREADS) k_line_cycle(CoarseLevels<T> C, int n_pre, int n_post,
+                                                              const double* __restrict__ lu_scale,
+                                                              const int* __restrict__ lu_perm,
+                                                              const double* __restrict__ Lf,
+                                                              const double* __restrict__ Uf,
+                                                              const double* __restrict__ dinv) {
+  constexpr int SUM = COARSE_LINE_SUM;
+  __shared__ T lds[7 * SUM];
+  __shared__ double lu_space[lu_lds_size(64)];
+  T *xs = lds, *ys = lds + SUM, *bs = lds + 2 * SUM;
+  const int tid = threadIdx.x, last = C.count - 1;
+  const int n_last = (int)C.L[last].d.n();
+  const LuLds lu = lu_lds(lu_space, n_last > 64 ? 0 : n_last);
+  if (!dinv) lu_stage(lu, n_last, lu_scale, lu_perm, Lf, Uf);
+  for (int i = tid; i < (int)C.L[0].d.n(); i += COARSE_THREADS) bs[i] = C.b[i];
+  T *ce = lds + 3 * SUM, *cn = lds + 4 * SUM, *ct = lds + 5 * SUM, *ca = lds + 6 * SUM;
+  for (int q = 0, o = 0; q < last; ++q) {
+    const Level& L = C.L[q];
+    const int n = (int)L.d.n();
+    const T fs = (T)L.fscale;
+    for (int i = tid; i < n; i += COARSE_THREADS) {
+      ce[o + i] = fs * (T)((const FT*)L.f_e)[i];
+      cn[o + i] = fs * (T)((const FT*)L.f_n)[i];
+      ct[o + i] = fs * (T)((const FT*)L.f_t)[i];
+      ca[o + i] = recip0(((const T*)L.s)[i]);
+      xs[o + i] = (T)0;
+    }
+    o += n;
+  }
+  unsigned in_y = 0;  // bit q: level q's iterate is in ys
+  int off = 0;
+  // passes over level q, its iterate in x to begin with; forward: lines x, y, z, else z, y, x
+  auto smooth = [&](int q, int sweeps, bool rev) {
+    for (int p = 0; p < 3 * sweeps; ++p) {
+      const int dir = rev ? 2 - p % 3 : p % 3;
+      const bool fromy = in_y >> q & 1;
+      const T* x = (fromy ? ys : xs) + off;
+      T* y = (fromy ? xs : ys) + off;
+      const SmallLines<T, TR> lines(C.L[q].d, dir, LineCells<T>{ce + off, cn + off, ct + off, ca + off, bs + off});
+      if (dir == 0)
+        lines.lanes(x, y);
+      else
+        lines.segments(x, y);
+      in_y ^= 1u << q;
+      __syncthreads();
+    }
+  };
+  for (int q = 0; q < last; ++q) {
+    const Level& L = C.L[q];
+    const int N = L.d.N, M = L.d.M, K = L.d.K, n = N * M * K;
+    __syncthreads();
+    smooth(q, n_pre, false);
+    const bool fromy = in_y >> q & 1;
+    const T* x = (fromy ? ys : xs) + off;
+    T* res = (fromy ? xs : ys) + off;
+    const FT *fe = (const FT*)L.f_e, *fn = (const FT*)L.f_n, *ft = (const FT*)L.f_t;
+    const T *sv = (const T*)L.s, fs = (T)L.fscale;
+    const float in = 1.0f / (float)N, im = 1.0f / (float)M;
+    const int NM = N * M;
+    for (int i = tid; i < n; i += COARSE_THREADS) {
+      const int rw = small_div(i, in), X = i - rw * N, Z = small_div(rw, im), Y = rw - Z * M;
+      const bool hw = X > 0, he = X < N - 1, hs = Y > 0, hn = Y < M - 1, hb = Z > 0, ht = Z < K - 1;
+      const T w = (T)fe[hw ? i - 1 : i], e = (T)fe[i], so = (T)fn[hs ? i - N : i], no = (T)fn[i];
+      const T bo = (T)ft[hb ? i - NM : i], to = (T)ft[i], si = sv[i], ap = si != (T)0 ? (T)1 / si : (T)0;
+      const T od = (hw ? w : (T)0) * x[hw ? i - 1 : i] + (he ? e : (T)0) * x[he ? i + 1 : i] +
+                   (hs ? so : (T)0) * x[hs ? i - N : i] + (hn ? no : (T)0) * x[hn ? i + N : i] +
+                   (hb ? bo : (T)0) * x[hb ? i - NM : i] + (ht ? to : (T)0) * x[ht ? i + NM : i];
+      const T r0 = bs[off + i] - ap * x[i];
+      res[i] = r0 - fs * od;
+    }
+    __syncthreads();
+    coarse_restrict<T, TR>(res, N, M, K, bs + off + n);
+    off += n;
+    __syncthreads();
+  }
+  coarse_bottom<T>(lu, n_last, true, lu_scale, lu_perm, Lf, Uf, dinv, bs + off, xs + off);
+  for (int q = last - 1; q >= 0; --q) {
+    const Level& L = C.L[q];
+    const T* xc = (in_y >> (q + 1) & 1 ? ys : xs) + off;
+    off -= L.d.N * L.d.M * L.d.K;
+    coarse_prolong<T, TR>(xc, L.d.N, L.d.M, L.d.K, (in_y >> q & 1 ? ys : xs) + off);
+    __syncthreads();
+    smooth(q, n_post, true);
+  }
+  const int n = (int)C.L[0].d.n();
+  const T* x = in_y & 1 ? ys : xs;
+  for (int i = tid; i < n; i += COARSE_THREADS) C.x[i] = x[i];
+}
+
 }  // namespace
 
 // ================================================================================================
@@ -2566,6 +2833,40 @@ bool coarse_fits(const CoarseLevels<T>& C) {
 }
 template bool coarse_fits<float>(const CoarseLevels<float>&);
 template bool coarse_fits<double>(const CoarseLevels<double>&);
+
+template <class T>
+bool coarse_line_fits(const CoarseLevels<T>& C) {
+  if (C.count < 2 || C.count > COARSE_MAX) return false;
+  long sum = 0;
+  for (int q = 0; q < C.count; ++q) {
+    const Dims& d = C.L[q].d;
+    sum += d.n();
+    // a y or z line takes one thread, or two of a wavefront
+    auto too_many = [](long lines, int len) { return lines > (len > SEG ? COARSE_THREADS / 2 : COARSE_THREADS); };
+    if (q + 1 < C.count && (d.n() > COARSE_LINE_CELLS || d.N > 64 || d.M > 2 * SEG || d.K > 2 * SEG || C.L[q].dff ||
+                            too_many((long)d.N * d.K, d.M) || too_many((long)d.N * d.M, d.K)))
+      return false;
+    if (sizeof(T) == 4 && q + 1 < C.count && C.L[q].ftype != FACE_F16) return false;
+    if (C.L[q].pin0 >= 0 || C.L[q].pin1 >= 0) return false;
+  }
+  return sum <= COARSE_LINE_SUM;
+}
+template bool coarse_line_fits<float>(const CoarseLevels<float>&);
+template bool coarse_line_fits<double>(const CoarseLevels<double>&);
+
+template <class T>
+void line_cycle(const CoarseLevels<T>& C, int trans, int n_pre, int n_post, const double* lu_scale, const int* lu_perm,
+                const double* L, const double* U, const double* dinv, hipStream_t s) {
+  using FT = std::conditional_t<std::is_same<T, double>::value, double, _Float16>;
+  if (trans)
+    k_line_cycle<T, FT, true><<<1, COARSE_THREADS, 0, s>>>(C, n_pre, n_post, lu_scale, lu_perm, L, U, dinv);
+  else
+    k_line_cycle<T, FT, false><<<1, COARSE_THREADS, 0, s>>>(C, n_pre, n_post, lu_scale, lu_perm, L, U, dinv);
+}
+template void line_cycle<float>(const CoarseLevels<float>&, int, int, int, const double*, const int*, const double*,
+                                const double*, const double*, hipStream_t);
+template void line_cycle<double>(const CoarseLevels<double>&, int, int, int, const double*, const int*, const double*,
+                                 const double*, const double*, hipStream_t);
 
 template <class T>
 void coarse_cycle(const CoarseLevels<T>& C, int trans, int n_pre, int n_post, const double* lu_scale, const int* lu_perm,

@@ -67,6 +67,13 @@ struct CoarseLevels {
 };
 template <class T>
 bool coarse_fits(const CoarseLevels<T>& C);
+// The same for line-relaxed levels (k_line_cycle): x lines of at most 64 cells, y and z lines of
+// at most 16, COARSE_LINE_CELLS cells a level (at 17 x 14 x 12 a pass in one workgroup takes as
+// long as its launch, 4 to 5 us, at 9 x 7 x 6 and 5 x 4 x 3 2.2 against 4.4), COARSE_LINE_SUM in all.
+constexpr long COARSE_LINE_CELLS = 1024;
+constexpr int COARSE_LINE_SUM = 1536;
+template <class T>
+bool coarse_line_fits(const CoarseLevels<T>& C);
 
 // ---- setup (FP64 temporaries) --------------------------------------------------------------
 // faces and diagonal of the finest level from the FP64 7-plane operator [b,s,w,p,e,n,t]; a face
@@ -115,6 +122,9 @@ void convert(const A* a, B* b, long n, hipStream_t s);
 // the small levels of the cycle (trans: the transposed one) in one launch: C.b holds the right-hand side
 // of the first of them, C.x receives its correction (lu_*: the dense LU factors of the last level,
 // or dinv its dense inverse, column-major)
+template <class T>
+void line_cycle(const CoarseLevels<T>& C, int trans, int n_pre, int n_post, const double* lu_scale, const int* lu_perm,
+                const double* L, const double* U, const double* dinv, hipStream_t s);
 template <class T>
 void coarse_cycle(const CoarseLevels<T>& C, int trans, int n_pre, int n_post, const double* lu_scale, const int* lu_perm,
                   const double* L, const double* U, const double* dinv, hipStream_t s);

@@ -35,3 +35,23 @@ def test_line_sweep_of_any_row(lsx, dims, precision, tol):
     t = abs(Bx @ y - b @ BTy) / (np.linalg.norm(Bx) * np.linalg.norm(y))
     print(f"dims={dims} precision={precision} rel err {e[0]:.3e} from zero {e[1]:.3e} transpose {t:.3e}", flush=True)
     assert max(e) <= tol and t <= tol
+
+
+@pytest.mark.parametrize("precision", ["fp64-vcycle", "mixed"])
+@pytest.mark.parametrize("dims", [(33, 28, 24), (32, 32, 32), (18, 13, 11), (100, 30, 10), (17, 5, 32), (40, 24, 33)])
+def test_small_line_levels_in_one_launch_are_bitwise(lsx, dims, precision):
+    """The one-workgroup cycle over small line-relaxed levels gives the bits of the launches one by
+    one, forward and transposed: y and z lines of one and two segments, x lines of up to 50 cells."""
+    g, A = P.synthetic_cut(*dims, seed=11)
+    act = A.to_scipy().diagonal() < 0
+    rng = np.random.default_rng(3)
+    v, w = (rng.standard_normal(A.n) * act for _ in range(2))
+    for n_pre, n_post in ((2, 2), (1, 2), (2, 1), (3, 1)):
+        z = []
+        for fuse in (True, False):
+            S = lsx.solver("fgmres", precision, smoother="line", coarse_fuse=fuse)
+            S.set(A, np.zeros(A.n), np.zeros(A.n), lsx.mixed_task(1.0, n_pre=n_pre, n_post=n_post))
+            z.append((S.precondition(v), S.precondition_transpose(w), S.precondition(w)))
+        for a, c in zip(*z):
+            assert np.linalg.norm(a) > 0 and np.array_equal(a, c), (n_pre, n_post, np.abs(a - c).max())
+    print(f"dims={dims} precision={precision} levels={S.num_levels()}", flush=True)
