@@ -40,6 +40,7 @@ void stencil_apply_sym_t(const double* s4, const SymExc& ex, Dims d, const doubl
 // a fixed order into out[out_index] (device memory).
 constexpr int RED_THREADS = 256;
 constexpr int CGS_MAX = 32;
+constexpr int RED_BLOCKS_MAX = 1024;
 int reduction_blocks(long n);
 
 // ---- setup --------------------------------------------------------------------------------
@@ -102,8 +103,9 @@ void scale_copy(const double* w, const double* normw, double* v, long n, hipStre
 void scale_copy_f32(const double* w, const double* normw, double* v, float* vf, long n, hipStream_t s);
 void dot_partial(const double* a, const double* b, long n, double* partial, hipStream_t s);
 void finalize(const double* partial, int nb, double* out, int sqrt_flag, hipStream_t s);
-// w -= h*v ; then partial dot(w, vnext) (vnext may be null => partial sum of w^2)
-void axpy_dot(double* w, const double* v, const double* h, const double* vnext, long n, double* partial,
+// h = sum of the reduction_blocks(n) partials `pin`; w -= h*v ; then partial dot(w, vnext) into `pout`
+// (vnext may be null => partial sum of w^2; pout must not be pin)
+void axpy_dot(double* w, const double* v, const double* pin, double* h, const double* vnext, long n, double* pout,
               hipStream_t s);
 // x += sum_k y_k z_k in the order k = last..0 (coefficients from host array, up to 64)
 void sol_update(double* x, const double* Z, long ldz, const double* yk, int count, long n, hipStream_t s);

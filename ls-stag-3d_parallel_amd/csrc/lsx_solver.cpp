@@ -50,7 +50,7 @@ Solver::Solver(const lsx_options& o, hipStream_t s) : opt(o) {
   }
   err.alloc(1);
   scalars.alloc(SC_H + 256 * 257 / 2 + 8);
-  partial.alloc(2048);
+  partial.alloc(2 * RED_BLOCKS_MAX);
   mpartial.alloc((size_t)CGS_MAX * CGS_BLOCKS_MAX);
   cgs_h.alloc(2 * CGS_MAX);
 }
@@ -1231,20 +1231,18 @@ int Solver::fgmres(const double* b, double* x) {
         }
       } else {
         // modified Gram-Schmidt: h_i = w . v_i ; w -= h_i v_i  (the dot of the next basis vector
-        // is fused into the update pass; the last pass yields ||w||^2)
-        dot_partial(w.p, V.p, n, partial.p, stream);
-        finalize(partial.p, nb, dH + hColStart, 0, stream);
+        // is fused into the update pass, which sums its partials in the next one; the last pass yields
+        // ||w||^2); the partials alternate between two halves
+        double* half[2] = {partial.p, partial.p + RED_BLOCKS_MAX};
+        dot_partial(w.p, V.p, n, half[0], stream);
         for (int i = 0; i <= j; ++i) {
           const double* vi = V.p + (size_t)i * n;
           const double* vnext = i < j ? V.p + (size_t)(i + 1) * n : nullptr;
           if (vnext) tbeg(LSX_K_ORTHO, &e0);
-          axpy_dot(w.p, vi, dH + hColStart + i, vnext, n, partial.p, stream);
+          axpy_dot(w.p, vi, half[i & 1], dH + hColStart + i, vnext, n, half[(i + 1) & 1], stream);
           if (vnext) tend(LSX_K_ORTHO, e0);
-          if (vnext)
-            finalize(partial.p, nb, dH + hColStart + i + 1, 0, stream);
-          else
-            finalize(partial.p, nb, dnorm, 1, stream);
         }
+        finalize(half[(j + 1) & 1], nb, dnorm, 1, stream);
         hNum = hColStart + j + 1;
         LSX_HIP(hipMemcpyAsync(hcol.data(), dH + hColStart, (j + 1) * sizeof(double), hipMemcpyDeviceToHost, stream));
         LSX_HIP(hipMemcpyAsync(&normW, dnorm, sizeof(double), hipMemcpyDeviceToHost, stream));
