@@ -46,10 +46,12 @@ __device__ inline bool in_box(int x, int y, const Box& b) { return x >= b.hs && 
 // Newton steps from the cube-sphere inverse of the point (a coordinate at its bound with the
 // gradient pointing out holds there while the other takes a 1D step; Gauss-Newton where the
 // Hessian is not positive definite), smallest distance wins, side from (x - S) . (S_u x S_v).
-__constant__ int BZ_A[6] = {0, 0, 1, 1, 2, 2};
-__constant__ double BZ_S[6] = {1.0, -1.0, 1.0, -1.0, 1.0, -1.0};
-__constant__ int BZ_U[6] = {1, 2, 2, 0, 0, 1};
-__constant__ int BZ_V[6] = {2, 1, 0, 2, 1, 0};
+// BZ_A = {0, 0, 1, 1, 2, 2}, BZ_S = {1, -1, 1, -1, 1, -1}, BZ_U = {1, 2, 2, 0, 0, 1}, BZ_V = {2, 1, 0, 2, 1, 0}
+__device__ inline int bz_next_axis(int a, int k) { return a + k < 3 ? a + k : a + k - 3; }
+__device__ inline int bz_a(int f) { return f >> 1; }
+__device__ inline int bz_u(int f) { return bz_next_axis(f >> 1, 1 + (f & 1)); }
+__device__ inline int bz_v(int f) { return bz_next_axis(f >> 1, 2 - (f & 1)); }
+__device__ inline double bz_pick(const double* d, int k) { return k == 0 ? d[0] : (k == 1 ? d[1] : d[2]); }
 
 __device__ inline void bz_basis(double t, double* b, double* db, double* ddb) {
   const double s = 1.0 - t;
@@ -128,12 +130,12 @@ struct BzHit {
 // after it would repeat it exactly.
 __device__ inline double bz_patch(const double* __restrict__ P, int f, const double* X, const double* d, double& u,
                                   double& v, double* r, double& side) {
-  const double da = fabs(d[BZ_A[f]]);
+  const double da = fabs(bz_pick(d, bz_a(f)));
   u = 0.5;
   v = 0.5;
   if (da > 0.0) {
-    u = bz_clamp(0.5 * (d[BZ_U[f]] / da + 1.0));
-    v = bz_clamp(0.5 * (d[BZ_V[f]] / da + 1.0));
+    u = bz_clamp(0.5 * (bz_pick(d, bz_u(f)) / da + 1.0));
+    v = bz_clamp(0.5 * (bz_pick(d, bz_v(f)) / da + 1.0));
   }
   double S[3], Su[3], Sv[3];
   for (int it = 0; it < 12; ++it) {
@@ -177,16 +179,34 @@ __device__ inline double bz_patch(const double* __restrict__ P, int f, const dou
   return bz_dot(r, r);
 }
 
-// squared distance from X to the bounding box of patch P's control points (the patch lies in
-// their convex hull)
-__device__ inline double bz_box_dist2(const double* __restrict__ P, const double* X) {
+// A workgroup's copy of the control values, a patch BZ_STRIDE apart (lanes on different patches read
+// different banks), and the bounding box of each patch's control points (the patch lies in their
+// convex hull)
+constexpr int BZ_STRIDE = 53;
+struct BzBody {
+  double P[6 * BZ_STRIDE], lo[18], hi[18];
+};
+// every thread of the workgroup takes part
+__device__ inline void bz_load(const double* __restrict__ ctrl, BzBody& B) {
+  for (int k = threadIdx.x; k < 288; k += blockDim.x) B.P[k / 48 * BZ_STRIDE + k % 48] = ctrl[k];
+  __syncthreads();
+  if (threadIdx.x < 18) {
+    const double* P = B.P + threadIdx.x / 3 * BZ_STRIDE + threadIdx.x % 3;
+    double lo = P[0], hi = P[0];
+    for (int k = 1; k < 16; ++k) {
+      lo = fmin(lo, P[3 * k]);
+      hi = fmax(hi, P[3 * k]);
+    }
+    B.lo[threadIdx.x] = lo;
+    B.hi[threadIdx.x] = hi;
+  }
+  __syncthreads();
+}
+// squared distance from X to the bounding box of patch f
+__device__ inline double bz_box_dist2(const BzBody& B, int f, const double* X) {
   double acc = 0.0;
   for (int c = 0; c < 3; ++c) {
-    double lo = P[c], hi = P[c];
-    for (int k = 1; k < 16; ++k) {
-      lo = fmin(lo, P[3 * k + c]);
-      hi = fmax(hi, P[3 * k + c]);
-    }
+    const double lo = B.lo[3 * f + c], hi = B.hi[3 * f + c];
     const double e = X[c] < lo ? lo - X[c] : (X[c] > hi ? X[c] - hi : 0.0);
     acc += e * e;
   }
@@ -194,34 +214,32 @@ __device__ inline double bz_box_dist2(const double* __restrict__ P, const double
 }
 
 // The patch with the smallest distance wins, the lowest index among equal distances.  Each point
-// first searches its home patch (the cube face its normalised direction points to); another
-// patch is searched only if its control-point box comes within the best distance so far plus a
-// margin of 1e-12, far above rounding (a patch further away cannot win or tie).  The loops run
-// over the patches in order so that the control values stay uniform over the wavefront.
-__device__ double bezier_closest(const double* __restrict__ ctrl, const double* c0, const double* a0, double x,
-                                 double y, double z, BzHit& hit) {
+// first searches its home patch (the cube face its normalised direction points to), then, in
+// order, every other patch whose control-point box comes within the best distance so far plus a
+// margin of 1e-12, far above rounding (a patch further away cannot win or tie).  A search is up to
+// 13 evaluations in FP64, so what counts is how many a wavefront makes: the lanes search their
+// own patches at the same time, control values from LDS, where going through the patches in turn
+// with uniform control values took every patch that any lane of the wavefront needed.
+__device__ void bezier_closest(const BzBody& B, const double* c0, const double* a0, double x, double y, double z,
+                               BzHit& hit) {
   const double X[3] = {x, y, z};
   double d[3];
   for (int c = 0; c < 3; ++c) d[c] = (X[c] - c0[c]) / a0[c];
   int ax = 0;
+  double da = d[0];
   for (int c = 1; c < 3; ++c)
-    if (fabs(d[c]) > fabs(d[ax])) ax = c;
-  const int home = 2 * ax + (d[ax] < 0.0 ? 1 : 0);  // faces 2a, 2a + 1: normal axis a, sign + / -
-  double best = 0.0, side = 0.0;
-  // pass 0 searches the home patch, pass 1 the others (one call site: one copy of the search)
-  for (int k = 0; k < 12; ++k) {
-    const int f = k < 6 ? k : k - 6;
-    const double* P = ctrl + f * 48;
-    if (k < 6) {
-      if (f != home) continue;
-    } else {
-      if (f == home) continue;
-      const double m = sqrt(bz_box_dist2(P, X)) - 1e-12;
-      if (m > 0.0 && m * m > best) continue;
+    if (fabs(d[c]) > fabs(da)) {
+      ax = c;
+      da = d[c];
     }
+  const int home = 2 * ax + (da < 0.0 ? 1 : 0);  // faces 2a, 2a + 1: normal axis a, sign + / -
+  double best = 0.0, side = 0.0;
+  int f = home, next = 0;
+  bool first = true;
+  for (;;) {
     double u, v, r[3], sd;
-    const double dist2 = bz_patch(P, f, X, d, u, v, r, sd);
-    if (k < 6 || dist2 < best || (dist2 == best && f < hit.f)) {
+    const double dist2 = bz_patch(B.P + f * BZ_STRIDE, f, X, d, u, v, r, sd);
+    if (first || dist2 < best || (dist2 == best && f < hit.f)) {
       best = dist2;
       side = sd;
       hit.f = f;
@@ -229,17 +247,18 @@ __device__ double bezier_closest(const double* __restrict__ ctrl, const double* 
       hit.v = v;
       for (int c = 0; c < 3; ++c) hit.r[c] = r[c];
     }
+    first = false;
+    for (; next < 6; ++next) {
+      if (next == home) continue;
+      const double m = sqrt(bz_box_dist2(B, next, X)) - 1e-12;
+      if (!(m > 0.0 && m * m > best)) break;
+    }
+    if (next >= 6) break;
+    f = next++;
   }
   const double dist = sqrt(best);
   hit.dist = dist;
   hit.sgn = side > 0.0 ? -1.0 : 1.0;
-  return side > 0.0 ? -dist : dist;
-}
-
-__device__ inline double bezier_phi(const double* __restrict__ ctrl, const double* c0, const double* a0, double x,
-                                    double y, double z) {
-  BzHit hit;
-  return bezier_closest(ctrl, c0, a0, x, y, z, hit);
 }
 
 // ---- level set -------------------------------------------------------------------------------
@@ -254,8 +273,6 @@ __global__ void k_level_set(const double* __restrict__ cx, const double* __restr
       if (body.kind == BODY_SPHERE) {
         const double qx = cx[x] - body.c[0], qy = cy[y] - body.c[1], qz = cz[z] - body.c[2];
         v = body.a[0] - sqrt(qx * qx + qy * qy + qz * qz);
-      } else if (body.kind == BODY_BEZIER6) {
-        v = bezier_phi(body.ctrl, body.c, body.a, cx[x], cy[y], cz[z]);
       } else {
         const double s = fmin(body.a[0], fmin(body.a[1], body.a[2]));
         const double qx = (cx[x] - body.c[0]) / body.a[0], qy = (cy[y] - body.c[1]) / body.a[1],
@@ -265,6 +282,28 @@ __global__ void k_level_set(const double* __restrict__ cx, const double* __restr
     }
     phi[i] = v;
   }
+}
+
+// the level set of a Bezier body, a wavefront to 4 x 4 x 4 nodes (neighbours search the same patches),
+// a workgroup to 8 x 8 x 4.  64^3: 480 us with 64 nodes of a row a wavefront and the patches in
+// turn, 232 so (the shape gradient's closest points at 72 x 64 x 64: 238 -> 75)
+__global__ void __launch_bounds__(256) k_level_set_bezier(const double* __restrict__ cx, const double* __restrict__ cy,
+                                                          const double* __restrict__ cz, int N, int M, int K, Box box,
+                                                          Body body, double* __restrict__ phi) {
+  __shared__ BzBody B;
+  bz_load(body.ctrl, B);
+  const int gx = (N + 7) / 8, gy = (M + 7) / 8, t = threadIdx.x, w = t >> 6;
+  const int x = (int)(blockIdx.x % gx) * 8 + (w & 1) * 4 + (t & 3);
+  const int y = (int)(blockIdx.x / gx % gy) * 8 + (w >> 1) * 4 + ((t >> 2) & 3);
+  const int z = (int)(blockIdx.x / gx / gy) * 4 + ((t >> 4) & 3);
+  if (x >= N || y >= M || z >= K) return;
+  double v = 0.0;
+  if (in_box(x, y, box)) {
+    BzHit hit;
+    bezier_closest(B, body.c, body.a, cx[x], cy[y], cz[z], hit);
+    v = hit.sgn < 0.0 ? -hit.dist : hit.dist;
+  }
+  phi[x + (long)N * (y + (long)M * z)] = v;
 }
 
 __global__ void k_osc_flags(const double* __restrict__ phi, int N, int M, int K, Box box, unsigned char* __restrict__ flag) {
@@ -1015,7 +1054,11 @@ int rule_count() { return N_RULES; }
 
 void level_set(const double* cx, const double* cy, const double* cz, int N, int M, int K, Box box, Body body,
                double* phi, hipStream_t s) {
-  k_level_set<<<grid_1d((long)N * M * K), 256, 0, s>>>(cx, cy, cz, N, M, K, box, body, phi);
+  if (body.kind == BODY_BEZIER6)
+    k_level_set_bezier<<<(unsigned)((long)((N + 7) / 8) * ((M + 7) / 8) * ((K + 3) / 4)), 256, 0, s>>>(cx, cy, cz, N, M, K,
+                                                                                              box, body, phi);
+  else
+    k_level_set<<<grid_1d((long)N * M * K), 256, 0, s>>>(cx, cy, cz, N, M, K, box, body, phi);
 }
 
 int oscillation_fix(const double* phi0, double* phi, double* tmp, unsigned char* flag, int* changed, int N, int M,
@@ -1719,10 +1762,12 @@ __global__ void __launch_bounds__(CHAIN ? 768 : 256) k_corner(GeoBase g, const i
 }
 
 // per listed corner with g != 0: winning patch, its parameters and w = g dphi/dS (3 values)
-__global__ void k_bz_hits(const double* __restrict__ g, const int* __restrict__ list, int count,
+__global__ void __launch_bounds__(64) k_bz_hits(const double* __restrict__ g, const int* __restrict__ list, int count,
                           const double* __restrict__ cx, const double* __restrict__ cy, const double* __restrict__ cz,
                           int N, int M, Body body, int* __restrict__ hf, double* __restrict__ huv,
                           double* __restrict__ hw) {
+  __shared__ BzBody B;
+  bz_load(body.ctrl, B);
   const int l = blockIdx.x * blockDim.x + threadIdx.x;
   if (l >= count) return;
   const long i = list[l];
@@ -1731,7 +1776,7 @@ __global__ void k_bz_hits(const double* __restrict__ g, const int* __restrict__ 
   int f = -1;
   if (g[i] != 0.0) {
     BzHit hit;
-    bezier_closest(body.ctrl, body.c, body.a, cx[x], cy[y], cz[z], hit);
+    bezier_closest(B, body.c, body.a, cx[x], cy[y], cz[z], hit);
     if (hit.dist > 0.0) {
       f = hit.f;
       huv[2 * l] = hit.u;
