@@ -102,6 +102,9 @@ void scale_copy(const double* w, const double* normw, double* v, long n, hipStre
 // v = (1/normw) w and vf = (float)v in one pass
 void scale_copy_f32(const double* w, const double* normw, double* v, float* vf, long n, hipStream_t s);
 void dot_partial(const double* a, const double* b, long n, double* partial, hipStream_t s);
+// out[0] = a . b, out[1] = c . d, each to the bits of dot_partial + finalize
+void dot2(const double* a, const double* b, const double* c, const double* d, long n, double* partial, double* out,
+          hipStream_t s);
 void finalize(const double* partial, int nb, double* out, int sqrt_flag, hipStream_t s);
 // h = sum of the reduction_blocks(n) partials `pin`; w -= h*v ; then partial dot(w, vnext) into `pout`
 // (vnext may be null => partial sum of w^2; pout must not be pin)
@@ -140,8 +143,7 @@ void sol_update_f32(double* x, const float* Z, long ldz, const double* yk, int c
 void bicg_s_update(double* nu, const double* r, double* sv, double alpha, long n, hipStream_t s);
 void bicg_sol_update(const double* sv, double* y, double* z, double* x, double* t, double* r, double alpha, double w,
                      long n, hipStream_t s);
-void bicg_p_update(double* p, const double* nu, const double* r, double coef, double beta, long n, double* partial,
-                   hipStream_t s);
+void bicg_p_update(double* p, const double* nu, const double* r, double coef, double beta, long n, hipStream_t s);
 void sub_vec(const double* b, const double* z, double* r, long n, hipStream_t s);  // r = b - z
 
 }  // namespace lsx

@@ -18,6 +18,7 @@ constexpr int SC_NORM = 0;    // residual / ||w|| results
 constexpr int SC_TINY = 1;    // max |diag| of a level during setup
 constexpr int SC_TMP = 2;     // scratch dot results
 constexpr int SC_SIGMA = 4;   // the two pinned cells' face sums (V-cycle setup)
+constexpr int SC_PAIR = 6;    // two dots at once
 constexpr int SC_H = 8;       // Hessenberg column entries H[hNum]
 }  // namespace
 
@@ -1092,6 +1093,12 @@ double Solver::reduce_to_host(const double* dev_scalar) {
   return h;
 }
 
+void Solver::dot2(const double* a, const double* b, const double* c, const double* d, long n, double (&out)[2]) {
+  lsx::dot2(a, b, c, d, n, partial.p, scalars.p + SC_PAIR, stream);
+  LSX_HIP(hipMemcpyAsync(out, scalars.p + SC_PAIR, 2 * sizeof(double), hipMemcpyDeviceToHost, stream));
+  LSX_HIP(hipStreamSynchronize(stream));
+}
+
 double Solver::dot(const double* a, const double* b, long n, double* out_dev) {
   dot_partial(a, b, n, partial.p, stream);
   finalize(partial.p, reduction_blocks(n), out_dev, 0, stream);
@@ -1306,36 +1313,33 @@ int Solver::fgmres(const double* b, double* x) {
 // -----------------------------------------------------------------------------------------------
 int Solver::bicgstab(const double* b, double* x) {
   const long n = d0.n();
-  const int nb = reduction_blocks(n);
   double* tmp = scalars.p + SC_TMP;
-  double* dnorm = scalars.p + SC_NORM;
   int iters = 1;
   fine_apply(x, nullptr, bz.p, ST_PROD);
   sub_vec(b, bz.p, br.p, n, stream);
-  norm_r = std::sqrt(dot(br.p, br.p, n, tmp));
+  const double norm2 = dot(br.p, br.p, n, tmp);
+  norm_r = std::sqrt(norm2);
   if (norm_r > opt.eps) {
     copy(br.p, brr.p, n, stream);
     copy(br.p, bp.p, n, stream);
+    double rho = norm2;  // brr . br, of the residual that the iteration starts from
     do {
       precond(bp.p, by.p);
       fine_apply(by.p, nullptr, bnu.p, ST_PROD);
-      double vs = dot(brr.p, br.p, n, tmp);
-      double coef = dot(brr.p, bnu.p, n, tmp);
+      double vs = rho, coef = dot(brr.p, bnu.p, n, tmp), q[2];
       const double alpha = vs / coef;
       bicg_s_update(bnu.p, br.p, bs.p, alpha, n, stream);
       precond(bs.p, bz.p);
       fine_apply(bz.p, nullptr, bt.p, ST_PROD);
-      double wv = dot(bt.p, bs.p, n, tmp);
-      coef = dot(bt.p, bt.p, n, tmp);
-      wv /= coef;
+      dot2(bt.p, bs.p, bt.p, bt.p, n, q);
+      double wv = q[0] / q[1];
       bicg_sol_update(bs.p, by.p, bz.p, x, bt.p, br.p, alpha, wv, n, stream);
       coef = wv / alpha;
       vs *= coef;
-      double beta = dot(brr.p, br.p, n, tmp);
-      beta /= vs;
-      bicg_p_update(bp.p, bnu.p, br.p, coef, beta, n, partial.p, stream);
-      finalize(partial.p, nb, dnorm, 1, stream);
-      norm_r = reduce_to_host(dnorm);
+      dot2(brr.p, br.p, br.p, br.p, n, q);
+      rho = q[0];
+      bicg_p_update(bp.p, bnu.p, br.p, coef, rho / vs, n, stream);
+      norm_r = std::sqrt(q[1]);
       ++iters;
     } while ((norm_r > opt.eps) && (iters < opt.max_it));
   }

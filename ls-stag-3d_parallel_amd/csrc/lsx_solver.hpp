@@ -224,6 +224,7 @@ class Solver {
   int bicgstab(const double* b, double* x);
   double reduce_to_host(const double* dev_scalar);
   double dot(const double* a, const double* b, long n, double* out_dev);
+  void dot2(const double* a, const double* b, const double* c, const double* d, long n, double (&out)[2]);
 
   hipStream_t stream = nullptr;
   bool own_stream = false;
