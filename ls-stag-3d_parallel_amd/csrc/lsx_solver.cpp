@@ -14,7 +14,6 @@ namespace lsx {
 
 namespace {
 // scalar slots in `scalars`
-constexpr int SC_NORM = 0;    // residual / ||w|| results
 constexpr int SC_TINY = 1;    // max |diag| of a level during setup
 constexpr int SC_TMP = 2;     // scratch dot results
 constexpr int SC_SIGMA = 4;   // the two pinned cells' face sums (V-cycle setup)
@@ -53,7 +52,7 @@ Solver::Solver(const lsx_options& o, hipStream_t s) : opt(o) {
   scalars.alloc(SC_H + 256 * 257 / 2 + 8);
   partial.alloc(2 * RED_BLOCKS_MAX);
   mpartial.alloc((size_t)CGS_MAX * CGS_BLOCKS_MAX);
-  cgs_h.alloc(2 * CGS_MAX);
+  cgs_h.alloc(2 * CGS_MAX + 1);
 }
 
 Solver::~Solver() {
@@ -1113,7 +1112,10 @@ int Solver::fgmres(const double* b, double* x) {
   const int m = opt.restart;
   const int m_size = m * (m + 1) / 2;
   const int nb = reduction_blocks(n);
-  double* dnorm = scalars.p + SC_NORM;
+  // norms follow the Gram-Schmidt coefficients in memory, so that a step copies once to the host: behind
+  // both passes' here, behind the column with modified Gram-Schmidt
+  double* const dnorm = cgs_h.p + 2 * CGS_MAX;
+  const double* dscale = dnorm;  // ||w|| of the vector to normalise
   double* dH = scalars.p + SC_H;
   const double eps = opt.eps;
   const MGLevel& F = levels[0];
@@ -1162,11 +1164,12 @@ int Solver::fgmres(const double* b, double* x) {
   int iters = 1;
   double normW = norm_r;
   double curH = norm_r;
-  std::vector<double> hcol(m + 2), hcgs(2 * CGS_MAX);
+  std::vector<double> hcol(m + 2), hcgs(2 * CGS_MAX + 1);
   bool resume = false;  // a V-cycle loop whose estimate converged but whose true residual did not
   for (;;) {
     // normW lives on the device for the scaling kernel
     LSX_HIP(hipMemcpyAsync(dnorm, &normW, sizeof(double), hipMemcpyHostToDevice, stream));
+    dscale = dnorm;
     for (int j = 0, hColStart = 0, hNum = 0; j < m; ++j, hColStart = hNum, ++iters) {
       double* vj = V.p + (size_t)j * n;
       double* zj = m32 ? nullptr : Z.p + (size_t)j * n;
@@ -1175,10 +1178,10 @@ int Solver::fgmres(const double* b, double* x) {
       if (scaled) sc[j] = 1.0;
       if (m32) {
         // v_j = w / ||w|| and its FP32 copy (the cycle's finest right-hand side) in one pass
-        if (scaled) scale_copy_f32(w.p, dnorm, vj, slot32(j), n, stream);
+        if (scaled) scale_copy_f32(w.p, dscale, vj, slot32(j), n, stream);
         vcycle_apply<float>(vj, zj32, slot32(j));
       } else {
-        if (scaled) scale_copy(w.p, dnorm, vj, n, stream);
+        if (scaled) scale_copy(w.p, dscale, vj, n, stream);
         if (vcyc())
           vcycle_apply<double>(vj, zj);
         else
@@ -1228,9 +1231,10 @@ int Solver::fgmres(const double* b, double* x) {
           }
         }
         hNum = hColStart + j + 1;
-        LSX_HIP(hipMemcpyAsync(hcgs.data(), cgs_h.p, 2 * CGS_MAX * sizeof(double), hipMemcpyDeviceToHost, stream));
-        LSX_HIP(hipMemcpyAsync(&normW, dnorm, sizeof(double), hipMemcpyDeviceToHost, stream));
+        LSX_HIP(hipMemcpyAsync(hcgs.data(), cgs_h.p, hcgs.size() * sizeof(double), hipMemcpyDeviceToHost, stream));
         LSX_HIP(hipStreamSynchronize(stream));
+        normW = hcgs[2 * CGS_MAX];
+        dscale = dnorm;
         for (int i = 0; i <= j; ++i) hcol[i] = cgs_passes == 2 ? hcgs[i] + hcgs[CGS_MAX + i] : hcgs[i];
         if (unnorm) {  // back to the orthonormal basis: h_i / (s_i s_j); u_{j+1} = ||w|| v_{j+1}
           for (int i = 0; i <= j; ++i) hcol[i] /= sc[i] * sc[j];
@@ -1249,11 +1253,13 @@ int Solver::fgmres(const double* b, double* x) {
           axpy_dot(w.p, vi, half[i & 1], dH + hColStart + i, vnext, n, half[(i + 1) & 1], stream);
           if (vnext) tend(LSX_K_ORTHO, e0);
         }
-        finalize(half[(j + 1) & 1], nb, dnorm, 1, stream);
+        double* const norm = dH + hColStart + j + 1;
+        finalize(half[(j + 1) & 1], nb, norm, 1, stream);
+        dscale = norm;
         hNum = hColStart + j + 1;
-        LSX_HIP(hipMemcpyAsync(hcol.data(), dH + hColStart, (j + 1) * sizeof(double), hipMemcpyDeviceToHost, stream));
-        LSX_HIP(hipMemcpyAsync(&normW, dnorm, sizeof(double), hipMemcpyDeviceToHost, stream));
+        LSX_HIP(hipMemcpyAsync(hcol.data(), dH + hColStart, (j + 2) * sizeof(double), hipMemcpyDeviceToHost, stream));
         LSX_HIP(hipStreamSynchronize(stream));
+        normW = hcol[j + 1];
       }
       for (int i = 0; i <= j; ++i) H[hColStart + i] = hcol[i];
       curH = H[hColStart];
