@@ -1667,11 +1667,10 @@ __device__ inline T wave_get(T v, int src, bool ok) {
   return r;
 }
 
-// CPL consecutive elements of p from index i as one wide load, aligned to the element (rows of a
-// length that is no multiple of CPL start anywhere)
-template <class E, int C>
+// CPL consecutive elements of p from index i (ODD: any i, else a multiple of CPL) as one wide load
+template <bool ODD, class E, int C>
 __device__ inline void ld_pack(const E* __restrict__ p, long i, E (&out)[C]) {
-  struct __attribute__((packed, aligned(alignof(E)))) Pack {
+  struct __attribute__((packed, aligned(ODD ? alignof(E) : sizeof(E) * C))) Pack {
     E v[C];
   };
   const Pack pk = *reinterpret_cast<const Pack*>(p + i);
@@ -1681,9 +1680,9 @@ __device__ inline void ld_pack(const E* __restrict__ p, long i, E (&out)[C]) {
 
 // The rows of cells i0 .. i0 + CPL - 1 of one x line (i0 = row start + CPL * lane): the same rows
 // as line_row, each array read with one wide load per lane.  The lines' neighbours in y and z
-// exist or not for the whole row; pinned cells are checked per cell.  Cells past the row's end are
-// decoupled identity rows (their loads read the next row).
-template <class T, class FT, int CPL, bool ZERO, bool DFF>
+// exist or not for the whole row; pinned cells are checked per cell.  ODD (N no multiple of CPL):
+// cells past the row's end are decoupled identity rows (their loads read the next row).
+template <class T, class FT, int CPL, bool ZERO, bool DFF, bool ODD>
 __device__ inline void line_rows_x(const T* __restrict__ x, const T* __restrict__ b, const FT* __restrict__ ae,
                                    const FT* __restrict__ an, const FT* __restrict__ at, const T* __restrict__ s,
                                    T fs, long i0, int k0, int yy, int zz, int N, int M, int K, int pin0, int pin1,
@@ -1695,21 +1694,21 @@ __device__ inline void line_rows_x(const T* __restrict__ x, const T* __restrict_
   const long is0 = ys ? i0 - N : i0, in0 = yn ? i0 + N : i0, ib0 = zb ? i0 - NM : i0, it0 = zt ? i0 + NM : i0;
   T sv[CPL], bv[CPL];
   FT fev[CPL], fnv[CPL], fsv[CPL], ftv[CPL], fbv[CPL];
-  if constexpr (!DFF) ld_pack<T, CPL>(s, i0, sv);
-  ld_pack<T, CPL>(b, i0, bv);
-  ld_pack<FT, CPL>(ae, i0, fev);
-  ld_pack<FT, CPL>(an, i0, fnv);
-  ld_pack<FT, CPL>(an, is0, fsv);
-  ld_pack<FT, CPL>(at, i0, ftv);
-  ld_pack<FT, CPL>(at, ib0, fbv);
+  if constexpr (!DFF) ld_pack<ODD, T, CPL>(s, i0, sv);
+  ld_pack<ODD, T, CPL>(b, i0, bv);
+  ld_pack<ODD, FT, CPL>(ae, i0, fev);
+  ld_pack<ODD, FT, CPL>(an, i0, fnv);
+  ld_pack<ODD, FT, CPL>(an, is0, fsv);
+  ld_pack<ODD, FT, CPL>(at, i0, ftv);
+  ld_pack<ODD, FT, CPL>(at, ib0, fbv);
   const FT fw0 = ae[k0 > 0 ? i0 - 1 : i0];
   T xv[CPL], xs[CPL], xn[CPL], xb[CPL], xt[CPL];
   if constexpr (!ZERO) {
-    ld_pack<T, CPL>(x, i0, xv);
-    ld_pack<T, CPL>(x, is0, xs);
-    ld_pack<T, CPL>(x, in0, xn);
-    ld_pack<T, CPL>(x, ib0, xb);
-    ld_pack<T, CPL>(x, it0, xt);
+    ld_pack<ODD, T, CPL>(x, i0, xv);
+    ld_pack<ODD, T, CPL>(x, is0, xs);
+    ld_pack<ODD, T, CPL>(x, in0, xn);
+    ld_pack<ODD, T, CPL>(x, ib0, xb);
+    ld_pack<ODD, T, CPL>(x, it0, xt);
   }
   auto pinned = [&](long j) { return j == pin0 || j == pin1; };
 #pragma unroll
@@ -1742,7 +1741,7 @@ __device__ inline void line_rows_x(const T* __restrict__ x, const T* __restrict_
       empty = sv[j] == (T)0;
     }
     const bool ident = own && !trans, cut = ident || empty;
-    const bool past = CPL > 1 && k >= N;
+    const bool past = ODD && k >= N;
     lo[j] = cut || past ? (T)0 : cw;
     up[j] = cut || past ? (T)0 : ce;
     dg[j] = cut || past ? (T)1 : ap;
@@ -1752,7 +1751,7 @@ __device__ inline void line_rows_x(const T* __restrict__ x, const T* __restrict_
 
 // LANES = 64: one wavefront per line; LANES = 32: two lines per wavefront (lines of at most
 // 32 CPL cells: shorter cyclic reduction, wider loads per lane)
-template <class T, class FT, int CPL, bool ZERO, bool TRANS, bool DFF, int LANES = 64>
+template <class T, class FT, int CPL, bool ZERO, bool TRANS, bool DFF, int LANES, bool ODD>
 __global__ void __launch_bounds__(256) k_line_x(const T* __restrict__ x_in, T* __restrict__ x_out,
                                                 const T* __restrict__ b, const FT* __restrict__ ae,
                                                 const FT* __restrict__ an, const FT* __restrict__ at,
@@ -1768,10 +1767,11 @@ __global__ void __launch_bounds__(256) k_line_x(const T* __restrict__ x_in, T* _
   const long row = live ? row_t : (long)M * K - 1;
   const int yy = (int)(row % M), zz = (int)(row / M);
   T lo[CPL], dg[CPL], up[CPL], rh[CPL];
-  // a lane across the row's end reads on into the next row, of its neighbours' rows too, where
-  // that row is there.  129 x 111 x 95 FP32: one cell a load 22.6 us, so 13.6
-  if (lane * CPL < N && (lane * CPL + CPL <= N || row < (long)M * K - M - 1)) {
-    line_rows_x<T, FT, CPL, ZERO, DFF>(x_in, b, ae, an, at, s, fs, row * N + lane * CPL, lane * CPL, yy, zz, N, M,
+  // ODD: a lane across the row's end reads on into the next row, of its neighbours' rows too, where
+  // that row is there.  129 x 111 x 95 FP32: one cell a load 22.6 us, so 13.6.  Rows of whole lanes
+  // have a variant of their own: 256^3 FP64 215 us, through this one 240
+  if (lane * CPL < N && (!ODD || lane * CPL + CPL <= N || row < (long)M * K - M - 1)) {
+    line_rows_x<T, FT, CPL, ZERO, DFF, ODD>(x_in, b, ae, an, at, s, fs, row * N + lane * CPL, lane * CPL, yy, zz, N, M,
                                        K, pin0, pin1, TRANS, lo, dg, up, rh, dr);
   } else {
 #pragma unroll
@@ -1852,18 +1852,11 @@ __global__ void __launch_bounds__(256) k_line_x(const T* __restrict__ x_in, T* _
   const T xe = r * recip0(d);
   const T xl0 = wave_get<LANES>(xe, lane - 1, lane > 0);
   const T xl = lane > 0 ? xl0 : (T)0;
-  struct __attribute__((packed, aligned(alignof(T)))) Pack {
-    T v[CPL];
-  } out;
 #pragma unroll
-  for (int j = 0; j < CPL; ++j) out.v[j] = j == CPL - 1 ? xe : G[j] + H[j] * xl + Q[j] * xe;
-  T* const to = x_out + row * N + lane * CPL;
-  if (live && lane * CPL + CPL <= N) {
-    *reinterpret_cast<Pack*>(to) = out;
-  } else if (live) {
-#pragma unroll
-    for (int j = 0; j < CPL; ++j)
-      if (lane * CPL + j < N) to[j] = out.v[j];
+  for (int j = 0; j < CPL; ++j) {
+    const int k = lane * CPL + j;
+    const T v = j == CPL - 1 ? xe : G[j] + H[j] * xl + Q[j] * xe;
+    if (live && k < N) x_out[row * N + k] = v;
   }
 }
 
@@ -1970,7 +1963,14 @@ struct SegLine {
   }
 };
 
-template <class T, class FT, int DIR, bool ZERO, bool TRANS, bool DFF>
+// Lines of whole segments (len a multiple of SEG) have a variant of the elimination whose masks are known
+// at compile time; a workgroup takes one variant (a wavefront with a full and a partial segment went
+// through both while the others waited: 17 x 14 x 12 7.7 us a z pass, so 5.8).  WHOLE: a kernel of that
+// variant alone, for large FP64 levels (WHOLE_CELLS).  256^3 FP64 y / z 207 / 236 us, 213 / 239 with
+// the choice at run time; but the code of a kernel of its own is cold on a small level: 65 x 56 x 48
+// FP32 8.7 / 9.5 us against 6.6 / 7.1
+constexpr long WHOLE_CELLS = 1L << 20;
+template <class T, class FT, int DIR, bool ZERO, bool TRANS, bool DFF, bool WHOLE>
 __global__ void __launch_bounds__(1024) k_line_seg(const T* __restrict__ x_in, T* __restrict__ x_out,
                                                    const T* __restrict__ b, const FT* __restrict__ ae,
                                                    const FT* __restrict__ an, const FT* __restrict__ at,
@@ -2016,15 +2016,14 @@ __global__ void __launch_bounds__(1024) k_line_seg(const T* __restrict__ x_in, T
   const long stride = DIR == 1 ? (long)N : NM;
   const long base = DIR == 1 ? xx + NM * other : xx + (long)N * other;
   const int k0 = seg * SEG;
-  const int cnt = len - k0 < SEG ? len - k0 : SEG;  // >= 1
+  const int cnt = WHOLE || len - k0 >= SEG ? SEG : len - k0;  // >= 1
   // Straight-line code over the SEG rows (rows past the segment's end re-read its last row and
   // are masked), so that the loads of all of them are in flight together.
   T G[SEG], H[SEG], Q[SEG];
   T le = (T)0, de = (T)1, ue = (T)0, re = (T)0;  // row of the last cell
   T Gb = (T)0, Hb = (T)1, Qb = (T)0;              // the cell before the last, in (x_L, x_E)
   T Gf = (T)0, Hf = (T)0, Qf = (T)1;              // the first cell, in (x_L, x_E)
-  // the elimination of the segment; FULL: segments of SEG rows (a line whose length is a multiple of
-  // SEG), whose masks are then known at compile time
+  // the elimination of the segment; FULL: every segment has SEG rows
   auto eliminate = [&](auto full_tag) {
     constexpr bool FULL = decltype(full_tag)::value;
     const int nrow = FULL ? SEG : cnt;
@@ -2126,13 +2125,14 @@ __global__ void __launch_bounds__(1024) k_line_seg(const T* __restrict__ x_in, T
       }
     }
   };
-  // one of the two for the whole workgroup: a wavefront with a full and a partial segment would go
-  // through both, and the others wait for it (17 x 14 x 12: 7.7 us a z pass, so 5.8)
-  if (len % SEG == 0)
+  if constexpr (WHOLE) {
     eliminate(std::true_type{});
-  else
-    eliminate(std::false_type{});
-  int xe_plane = 7;
+  } else {
+    if (len % SEG == 0)
+      eliminate(std::true_type{});
+    else
+      eliminate(std::false_type{});
+  }
   if ((S & (S - 1)) == 0) {
     // S a power of two (<= 32): the reduced systems are solved inside wavefronts.  Each thread
     // posts its partial last-cell row and its first cell; after one barrier thread t takes
@@ -2174,8 +2174,7 @@ __global__ void __launch_bounds__(1024) k_line_seg(const T* __restrict__ x_in, T
     IF(7, ts, tl) = r * recip0(d);
     __syncthreads();
   } else {
-    // general S: cyclic reduction across the wavefronts through LDS, one barrier per step: the steps
-    // post their rows to planes 0-3 and 4-7 in turn
+    // general S: cyclic reduction across the wavefronts through LDS, one barrier pair per step
     IF(4, seg, lane) = Gf;
     IF(5, seg, lane) = Hf;
     IF(6, seg, lane) = Qf;
@@ -2189,31 +2188,29 @@ __global__ void __launch_bounds__(1024) k_line_seg(const T* __restrict__ x_in, T
     T d = de + le * Qb + ue * H1;
     T c = ue * Q1;
     T r = re - le * Gb - ue * G1;
-    int to = 0;
     for (int st = 1; st < S; st <<= 1) {  // S is uniform over the workgroup
-      IF(to, seg, lane) = a;
-      IF(to + 1, seg, lane) = d;
-      IF(to + 2, seg, lane) = c;
-      IF(to + 3, seg, lane) = r;
+      IF(0, seg, lane) = a;
+      IF(1, seg, lane) = d;
+      IF(2, seg, lane) = c;
+      IF(3, seg, lane) = r;
       __syncthreads();
       const bool okm = seg - st >= 0, okp = seg + st < S;
-      const T am = okm ? IF(to, seg - st, lane) : (T)0, dm = okm ? IF(to + 1, seg - st, lane) : (T)1;
-      const T cm = okm ? IF(to + 2, seg - st, lane) : (T)0, rm = okm ? IF(to + 3, seg - st, lane) : (T)0;
-      const T ap = okp ? IF(to, seg + st, lane) : (T)0, dp = okp ? IF(to + 1, seg + st, lane) : (T)1;
-      const T cq = okp ? IF(to + 2, seg + st, lane) : (T)0, rp = okp ? IF(to + 3, seg + st, lane) : (T)0;
+      const T am = okm ? IF(0, seg - st, lane) : (T)0, dm = okm ? IF(1, seg - st, lane) : (T)1;
+      const T cm = okm ? IF(2, seg - st, lane) : (T)0, rm = okm ? IF(3, seg - st, lane) : (T)0;
+      const T ap = okp ? IF(0, seg + st, lane) : (T)0, dp = okp ? IF(1, seg + st, lane) : (T)1;
+      const T cq = okp ? IF(2, seg + st, lane) : (T)0, rp = okp ? IF(3, seg + st, lane) : (T)0;
       const T al = -a * recip0(dm), ga = -c * recip0(dp);
       a = al * am;
       c = ga * cq;
       d = d + al * cm + ga * ap;
       r = r + al * rm + ga * rp;
-      to ^= 4;
+      __syncthreads();
     }
-    xe_plane = to + 3;
-    IF(xe_plane, seg, lane) = r * recip0(d);
+    IF(7, seg, lane) = r * recip0(d);
     __syncthreads();
   }
-  const T xe = IF(xe_plane, seg, lane);
-  const T xl = seg > 0 ? IF(xe_plane, seg - 1, lane) : (T)0;
+  const T xe = IF(7, seg, lane);
+  const T xl = seg > 0 ? IF(7, seg - 1, lane) : (T)0;
   if (live) {
 #pragma unroll
     for (int k = 0; k < SEG; ++k)
@@ -2698,23 +2695,29 @@ static void line_pass_z(const Level& L, int dir, const T* x_in, T* x_out, const 
   if (dir == 0) {
     // the FP64 x-line pass reads 1/a_p even on a Level::dff level: rebuilding a_p there measured
     // slower at 256^3 (226 against 195 us), the FP32 one faster (80 against 99 us)
-#define LSX_LINE_X(CPL, LANES)                                                                                 \
-  do {                                                                                                         \
-    const int blocks = (int)(((long)d.M * d.K + 256 / LANES - 1) / (256 / LANES));                             \
-    if (trans)                                                                                                 \
-      k_line_x<T, FT, CPL, ZERO, true, false, LANES><<<blocks, 256, 0, s>>>(x_in, x_out, b, ae, an, at, sv, fs, \
-                                                                            d.N, d.M, d.K, L.pin0, L.pin1, dr); \
-    else if (L.dff && sizeof(T) == 4)                                                                          \
-      k_line_x<T, FT, CPL, ZERO, false, true, LANES><<<blocks, 256, 0, s>>>(x_in, x_out, b, ae, an, at, sv, fs, \
-                                                                            d.N, d.M, d.K, L.pin0, L.pin1, dr); \
-    else                                                                                                       \
-      k_line_x<T, FT, CPL, ZERO, false, false, LANES><<<blocks, 256, 0, s>>>(x_in, x_out, b, ae, an, at, sv,    \
-                                                                             fs, d.N, d.M, d.K, L.pin0, L.pin1, \
-                                                                             dr);                               \
+#define LSX_LINE_X_ODD(CPL, LANES, ODD)                                                                         \
+  do {                                                                                                          \
+    const int blocks = (int)(((long)d.M * d.K + 256 / LANES - 1) / (256 / LANES));                              \
+    if (trans)                                                                                                  \
+      k_line_x<T, FT, CPL, ZERO, true, false, LANES, ODD>                                                       \
+          <<<blocks, 256, 0, s>>>(x_in, x_out, b, ae, an, at, sv, fs, d.N, d.M, d.K, L.pin0, L.pin1, dr);       \
+    else if (L.dff && sizeof(T) == 4)                                                                           \
+      k_line_x<T, FT, CPL, ZERO, false, true, LANES, ODD>                                                       \
+          <<<blocks, 256, 0, s>>>(x_in, x_out, b, ae, an, at, sv, fs, d.N, d.M, d.K, L.pin0, L.pin1, dr);       \
+    else                                                                                                        \
+      k_line_x<T, FT, CPL, ZERO, false, false, LANES, ODD>                                                      \
+          <<<blocks, 256, 0, s>>>(x_in, x_out, b, ae, an, at, sv, fs, d.N, d.M, d.K, L.pin0, L.pin1, dr);       \
+  } while (0)
+#define LSX_LINE_X(CPL, LANES)                                                                                  \
+  do {                                                                                                          \
+    if (d.N % CPL == 0)                                                                                         \
+      LSX_LINE_X_ODD(CPL, LANES, false);                                                                        \
+    else                                                                                                        \
+      LSX_LINE_X_ODD(CPL, LANES, true);                                                                         \
   } while (0)
     // lines of up to 128 cells: two per wavefront, four cells per lane
     if (d.N <= 64)
-      LSX_LINE_X(1, 64);
+      LSX_LINE_X_ODD(1, 64, false);
     else if (d.N <= 128)
       LSX_LINE_X(4, 32);
     else if (d.N <= 256)
@@ -2722,15 +2725,24 @@ static void line_pass_z(const Level& L, int dir, const T* x_in, T* x_out, const 
     else
       LSX_LINE_X(8, 64);
 #undef LSX_LINE_X
+#undef LSX_LINE_X_ODD
   } else {
     const int len = dir == 1 ? d.M : d.K;
     const int S = (len + SEG - 1) / SEG;
     constexpr int LPW = lpw<T>();
     const dim3 grid(dir == 1 ? ((d.N + LPW - 1) / LPW) * d.K : (unsigned)((d.N * (long)d.M + LPW - 1) / LPW));
     const size_t lds = 8 * (size_t)S * (LPW + 1) * sizeof(T);
-#define LSX_LINE_SEG(DIR, TR, DFF)                                                                             \
-  k_line_seg<T, FT, DIR, ZERO, TR, DFF><<<grid, LPW * S, lds, s>>>(x_in, x_out, b, ae, an, at, sv, fs, d.N, d.M,  \
-                                                                   d.K, L.pin0, L.pin1, S, dr)
+#define LSX_LINE_SEG(DIR, TR, DFF)                                                                              \
+  do {                                                                                                          \
+    if (sizeof(T) == 8 && len % SEG == 0 && d.n() >= WHOLE_CELLS)                                                \
+      k_line_seg<T, FT, DIR, ZERO, TR, DFF, sizeof(T) == 8><<<grid, LPW * S, lds, s>>>(x_in, x_out, b, ae, an, at, sv, fs, \
+                                                                             d.N, d.M, d.K, L.pin0, L.pin1, S,  \
+                                                                             dr);                               \
+    else                                                                                                        \
+      k_line_seg<T, FT, DIR, ZERO, TR, DFF, false><<<grid, LPW * S, lds, s>>>(x_in, x_out, b, ae, an, at, sv,   \
+                                                                              fs, d.N, d.M, d.K, L.pin0,        \
+                                                                              L.pin1, S, dr);                   \
+  } while (0)
     if (dir == 1) {
       if (trans)
         LSX_LINE_SEG(1, true, false);
