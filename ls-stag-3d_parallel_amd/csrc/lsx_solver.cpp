@@ -74,8 +74,11 @@ hipEvent_t Solver::ev_take() {
 }
 
 void Solver::clear_graphs() {
-  for (CycleGraph& g : cgraphs)
+  if (!cgraphs.empty()) capture_first = false;
+  for (CycleGraph& g : cgraphs) {
+    if (g.uses > 1) capture_first = true;
     if (g.exec) (void)hipGraphExecDestroy(g.exec);
+  }
   cgraphs.clear();
 }
 
@@ -663,16 +666,20 @@ void Solver::vcycle_apply(const double* v, T* z, const float* b32) {
   CycleGraph* mine = nullptr;
   for (CycleGraph& g : cgraphs)
     if (g.v == v && g.z == (const void*)z && g.b32 == b32) mine = &g;
+  if (mine) ++mine->uses;
   if (mine && mine->exec) {
     LSX_HIP(hipGraphLaunch(mine->exec, stream));
     return;
   }
-  // a pair's first cycle since the set-up runs eagerly: capture and instantiation (46 us) pay from
-  // the second replay on, and a set-up per solve uses each pair once
   if (!mine) {
-    cgraphs.push_back({v, (const void*)z, b32, nullptr});
-    vcycle_run<T>(v, z, b32);
-    return;
+    cgraphs.push_back({v, (const void*)z, b32, nullptr, 1});
+    mine = &cgraphs.back();
+    // capture and instantiation (46 us at 64^3) pay from the second use on: where the last set-up was
+    // replaced before a pair came twice (a set-up per solve), a pair's first cycle runs eagerly
+    if (!capture_first) {
+      vcycle_run<T>(v, z, b32);
+      return;
+    }
   }
   hipGraph_t graph = nullptr;
   LSX_HIP(hipStreamBeginCapture(stream, hipStreamCaptureModeThreadLocal));

@@ -326,8 +326,10 @@ class Solver {
     const double* v;
     const void* z;
     const float* b32;
-    hipGraphExec_t exec;  // null after the first, eager cycle
+    hipGraphExec_t exec;  // null after a first, eager cycle
+    long uses;
   };
+  bool capture_first = true;  // false: the set-up before this one used no pair twice
   std::vector<CycleGraph> cgraphs;
   bool capturing = false;
   void clear_graphs();
