@@ -1964,12 +1964,14 @@ struct SegLine {
 };
 
 // Lines of whole segments (len a multiple of SEG) have a variant of the elimination whose masks are known
-// at compile time; a workgroup takes one variant (a wavefront with a full and a partial segment went
-// through both while the others waited: 17 x 14 x 12 7.7 us a z pass, so 5.8).  WHOLE: a kernel of that
-// variant alone, for large FP64 levels (WHOLE_CELLS).  256^3 FP64 y / z 207 / 236 us, 213 / 239 with
-// the choice at run time; but the code of a kernel of its own is cold on a small level: 65 x 56 x 48
-// FP32 8.7 / 9.5 us against 6.6 / 7.1
+// at compile time.  A workgroup takes one variant (a wavefront with a full and a partial segment went
+// through both while the others waited: 17 x 14 x 12 7.7 us a z pass, so 5.8), but on lines of more
+// than SPLIT_S segments, where one wavefront of many has both (mixed momentum solve of a 256 x 256 x
+// 255 mesh 17.2 ms, so 16.3).  WHOLE: a kernel of that variant alone, for large levels: 256^3 FP64
+// y / z 207 / 236 us, 213 / 239 with the choice at run time, and 1.5 % of the mixed 256^3 solve; on
+// a small level the code of a kernel of its own is cold: 65 x 56 x 48 FP32 8.7 / 9.5 us against 6.6 / 7.1
 constexpr long WHOLE_CELLS = 1L << 20;
+constexpr int SPLIT_S = 16;
 template <class T, class FT, int DIR, bool ZERO, bool TRANS, bool DFF, bool WHOLE>
 __global__ void __launch_bounds__(1024) k_line_seg(const T* __restrict__ x_in, T* __restrict__ x_out,
                                                    const T* __restrict__ b, const FT* __restrict__ ae,
@@ -2128,7 +2130,7 @@ __global__ void __launch_bounds__(1024) k_line_seg(const T* __restrict__ x_in, T
   if constexpr (WHOLE) {
     eliminate(std::true_type{});
   } else {
-    if (len % SEG == 0)
+    if (len % SEG == 0 || (S > SPLIT_S && cnt == SEG))
       eliminate(std::true_type{});
     else
       eliminate(std::false_type{});
@@ -2376,10 +2378,10 @@ struct SmallLines {
 };
 
 // The small levels of a line-relaxed cycle in one workgroup, as k_coarse_cycle: x, its second
-// buffer, b and the coefficients in LDS.  Launched one by one, 12 line passes of a level of 9 x 7 x 6 or 5 x 4 x 3 cells
-// cost 3.6 to 4.8 us each, a launch's time; so both levels with transfers and LU take 68 us where
-// their launches took 117 (4.4 us x 24 passes, transfers, LU).  TR: the transposed cycle's transfers (the coarse
-// levels are symmetric and hold no pinned rows).
+// buffer, b and the coefficients in LDS.  Launched one by one, 12 line passes of a level of 9 x 7 x 6
+// or 5 x 4 x 3 cells cost 3.6 to 4.8 us each, a launch's time; so both levels with transfers and LU
+// take 68 us where their launches took 117 (4.4 us x 24 passes, transfers, LU).  TR: the transposed
+// cycle's transfers (the coarse levels are symmetric and hold no pinned rows).
 template <class T, class FT, bool TR>
 __global__ void __launch_bounds__(COARSE_THREADS) k_line_cycle(CoarseLevels<T> C, int n_pre, int n_post,
                                                               const double* __restrict__ lu_scale,
@@ -2734,8 +2736,8 @@ static void line_pass_z(const Level& L, int dir, const T* x_in, T* x_out, const 
     const size_t lds = 8 * (size_t)S * (LPW + 1) * sizeof(T);
 #define LSX_LINE_SEG(DIR, TR, DFF)                                                                              \
   do {                                                                                                          \
-    if (sizeof(T) == 8 && len % SEG == 0 && d.n() >= WHOLE_CELLS)                                                \
-      k_line_seg<T, FT, DIR, ZERO, TR, DFF, sizeof(T) == 8><<<grid, LPW * S, lds, s>>>(x_in, x_out, b, ae, an, at, sv, fs, \
+    if (len % SEG == 0 && d.n() >= WHOLE_CELLS)                                                                 \
+      k_line_seg<T, FT, DIR, ZERO, TR, DFF, true><<<grid, LPW * S, lds, s>>>(x_in, x_out, b, ae, an, at, sv, fs, \
                                                                              d.N, d.M, d.K, L.pin0, L.pin1, S,  \
                                                                              dr);                               \
     else                                                                                                        \
