@@ -1964,15 +1964,17 @@ struct SegLine {
 };
 
 // Lines of whole segments (len a multiple of SEG) have a variant of the elimination whose masks are known
-// at compile time.  A workgroup takes one variant (a wavefront with a full and a partial segment went
-// through both while the others waited: 17 x 14 x 12 7.7 us a z pass, so 5.8), but on lines of more
-// than SPLIT_S segments, where one wavefront of many has both (mixed momentum solve of a 256 x 256 x
-// 255 mesh 17.2 ms, so 16.3).  WHOLE: a kernel of that variant alone, for large levels: 256^3 FP64
-// y / z 207 / 236 us, 213 / 239 with the choice at run time, and 1.5 % of the mixed 256^3 solve; on
-// a small level the code of a kernel of its own is cold: 65 x 56 x 48 FP32 8.7 / 9.5 us against 6.6 / 7.1
+// at compile time.  SEG_ANY: a workgroup takes one variant (a wavefront with a full and a partial segment
+// went through both while the others waited: 17 x 14 x 12 7.7 us a z pass, so 5.8).  SEG_SPLIT: lines of
+// more than SPLIT_S segments with a partial one, where one wavefront of many has both (mixed momentum
+// solve of a 256 x 256 x 255 mesh 17.2 ms, so 16.3).  SEG_WHOLE: the variant alone, for large
+// levels: 256^3 FP64 y / z 207 / 236 us, 213 / 239 with the choice at run time; FP32 with a_p from the
+// faces keeps the choice (90 / 101 us against 94 / 107), and on a small level the code of
+// a kernel of its own is cold (65 x 56 x 48 FP32 8.7 / 9.5 us against 6.6 / 7.1)
+enum SegMode { SEG_ANY, SEG_SPLIT, SEG_WHOLE };
 constexpr long WHOLE_CELLS = 1L << 20;
 constexpr int SPLIT_S = 16;
-template <class T, class FT, int DIR, bool ZERO, bool TRANS, bool DFF, bool WHOLE>
+template <class T, class FT, int DIR, bool ZERO, bool TRANS, bool DFF, int MODE>
 __global__ void __launch_bounds__(1024) k_line_seg(const T* __restrict__ x_in, T* __restrict__ x_out,
                                                    const T* __restrict__ b, const FT* __restrict__ ae,
                                                    const FT* __restrict__ an, const FT* __restrict__ at,
@@ -2018,7 +2020,7 @@ __global__ void __launch_bounds__(1024) k_line_seg(const T* __restrict__ x_in, T
   const long stride = DIR == 1 ? (long)N : NM;
   const long base = DIR == 1 ? xx + NM * other : xx + (long)N * other;
   const int k0 = seg * SEG;
-  const int cnt = WHOLE || len - k0 >= SEG ? SEG : len - k0;  // >= 1
+  const int cnt = MODE == SEG_WHOLE || len - k0 >= SEG ? SEG : len - k0;  // >= 1
   // Straight-line code over the SEG rows (rows past the segment's end re-read its last row and
   // are masked), so that the loads of all of them are in flight together.
   T G[SEG], H[SEG], Q[SEG];
@@ -2127,10 +2129,10 @@ __global__ void __launch_bounds__(1024) k_line_seg(const T* __restrict__ x_in, T
       }
     }
   };
-  if constexpr (WHOLE) {
+  if constexpr (MODE == SEG_WHOLE) {
     eliminate(std::true_type{});
   } else {
-    if (len % SEG == 0 || (S > SPLIT_S && cnt == SEG))
+    if (MODE == SEG_SPLIT ? cnt == SEG : len % SEG == 0)
       eliminate(std::true_type{});
     else
       eliminate(std::false_type{});
@@ -2734,16 +2736,17 @@ static void line_pass_z(const Level& L, int dir, const T* x_in, T* x_out, const 
     constexpr int LPW = lpw<T>();
     const dim3 grid(dir == 1 ? ((d.N + LPW - 1) / LPW) * d.K : (unsigned)((d.N * (long)d.M + LPW - 1) / LPW));
     const size_t lds = 8 * (size_t)S * (LPW + 1) * sizeof(T);
-#define LSX_LINE_SEG(DIR, TR, DFF)                                                                              \
-  do {                                                                                                          \
-    if (len % SEG == 0 && d.n() >= WHOLE_CELLS)                                                                 \
-      k_line_seg<T, FT, DIR, ZERO, TR, DFF, true><<<grid, LPW * S, lds, s>>>(x_in, x_out, b, ae, an, at, sv, fs, \
-                                                                             d.N, d.M, d.K, L.pin0, L.pin1, S,  \
-                                                                             dr);                               \
-    else                                                                                                        \
-      k_line_seg<T, FT, DIR, ZERO, TR, DFF, false><<<grid, LPW * S, lds, s>>>(x_in, x_out, b, ae, an, at, sv,   \
-                                                                              fs, d.N, d.M, d.K, L.pin0,        \
-                                                                              L.pin1, S, dr);                   \
+#define LSX_LINE_SEG_MODE(DIR, TR, DFF, MODE)                                                                \
+  k_line_seg<T, FT, DIR, ZERO, TR, DFF, MODE><<<grid, LPW * S, lds, s>>>(x_in, x_out, b, ae, an, at, sv, fs, d.N, \
+                                                                         d.M, d.K, L.pin0, L.pin1, S, dr)
+#define LSX_LINE_SEG(DIR, TR, DFF)                                                                           \
+  do {                                                                                                       \
+    if ((sizeof(T) == 8 || !DFF) && len % SEG == 0 && d.n() >= WHOLE_CELLS)                                  \
+      LSX_LINE_SEG_MODE(DIR, TR, DFF, (sizeof(T) == 8 || !DFF ? SEG_WHOLE : SEG_ANY));                       \
+    else if (len % SEG != 0 && S > SPLIT_S)                                                                  \
+      LSX_LINE_SEG_MODE(DIR, TR, DFF, SEG_SPLIT);                                                            \
+    else                                                                                                     \
+      LSX_LINE_SEG_MODE(DIR, TR, DFF, SEG_ANY);                                                              \
   } while (0)
     if (dir == 1) {
       if (trans)
@@ -2761,6 +2764,7 @@ static void line_pass_z(const Level& L, int dir, const T* x_in, T* x_out, const 
         LSX_LINE_SEG(2, false, false);
     }
 #undef LSX_LINE_SEG
+#undef LSX_LINE_SEG_MODE
   }
 }
 
