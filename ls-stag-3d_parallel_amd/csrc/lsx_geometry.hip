@@ -1462,6 +1462,9 @@ __device__ inline bool corner_active(const double* __restrict__ raw, const doubl
          apart(z + 1 < K, i + NM);
 }
 
+// whether the oscillation fix changed a node (a NaN, which it leaves alone, differs from itself)
+__device__ inline bool node_fixed(double raw, double phi) { return raw < phi || raw > phi; }
+
 // Lists of nodes in index order: AC_FIXED those that the oscillation fix changed, AC_CORNERS the active
 // corners and those marked.  Blocks of AC_NODES consecutive nodes count theirs
 // (list null), one workgroup turns the counts into offsets and the total (k_active_scan), and the
@@ -1477,7 +1480,7 @@ __global__ void __launch_bounds__(256) k_active(const double* __restrict__ raw, 
   int at = list ? count[blockIdx.x] : 0;
   for (int q = 0; q < AC_NODES / 256; ++q) {
     const long i = (long)blockIdx.x * AC_NODES + q * 256 + threadIdx.x;
-    const bool on = i < n && (mode == AC_FIXED ? raw[i] != phi[i]
+    const bool on = i < n && (mode == AC_FIXED ? node_fixed(raw[i], phi[i])
                                                : (mark && mark[i]) || corner_active(raw, phi, i, N, M, K, box, h));
     const unsigned long long m = __ballot(on);
     if (lane == 0) waves[wave] = __popcll(m);
@@ -1547,7 +1550,7 @@ struct MovedLevelSet {
     return on ? (move == 0 ? v + h : v - h) : v;
   }
   __device__ double fixed(long j) const {
-    return raw0[j] != phi0[j] ? val[find_node(list, count, (int)j)] : raw(j);
+    return node_fixed(raw0[j], phi0[j]) ? val[find_node(list, count, (int)j)] : raw(j);
   }
 };
 
@@ -1571,7 +1574,7 @@ __global__ void __launch_bounds__(256) k_chain_table(const double* __restrict__ 
       const long j = list[l];
       const int z = (int)(j / NM);
       auto lower = [&](long k) {
-        return raw0[k] != phi0[k] ? (double)val[find_node(list, count, (int)k)] : f.raw(k);
+        return node_fixed(raw0[k], phi0[k]) ? (double)val[find_node(list, count, (int)k)] : f.raw(k);
       };
       double v = f.raw(j);
       check_osc(v, lower(j - 1), f.raw(j + 1));
@@ -1594,7 +1597,7 @@ __global__ void __launch_bounds__(256) k_chain_mark(const double* __restrict__ r
   const long NM = (long)N * M, j = list[blockIdx.x];
   int x, y, z;
   decode(j, N, M, &x, &y, &z);
-  auto fixed = [&](long k) { return raw0[k] != phi0[k]; };
+  auto fixed = [&](long k) { return node_fixed(raw0[k], phi0[k]); };
   if (!fixed(j - 1) && !fixed(j - N) && !(z > 0 && fixed(j - NM))) return;
   for (int q = threadIdx.x; q < 729; q += blockDim.x) {
     const int cx = x + q % 9 - 4, cy = y + q / 9 % 9 - 4, cz = z + q / 81 - 4;

@@ -153,8 +153,17 @@ double bezier_level_set(const double* ctrl, const double* center, const double* 
   const double X[3] = {x, y, z};
   double d[3];
   for (int c = 0; c < 3; ++c) d[c] = (X[c] - center[c]) / axes[c];
-  double best = -1.0, side = 0.0;
-  for (int f = 0; f < 6; ++f) {
+  // the patch that the point's direction meets first, then the others in order: the same winner
+  // whatever the order, but that a NaN distance to the first patch stays
+  int axis = 0;
+  for (int c = 1; c < 3; ++c)
+    if (std::fabs(d[c]) > std::fabs(d[axis])) axis = c;
+  const int home = 2 * axis + (d[axis] < 0.0 ? 1 : 0);
+  double best = 0.0, side = 0.0;
+  int won = -1;
+  for (int k = 0; k < 7; ++k) {
+    const int f = k == 0 ? home : k - 1;
+    if (k > 0 && f == home) continue;
     const double* P = ctrl + f * 48;
     const int a = FACE_A[f], bu = FACE_U[f], bv = FACE_V[f];
     const double da = std::fabs(d[a]);
@@ -202,8 +211,9 @@ double bezier_level_set(const double* ctrl, const double* center, const double* 
     double r[3];
     for (int c = 0; c < 3; ++c) r[c] = X[c] - S[c];
     const double dist2 = dot3(r, r);
-    if (best < 0.0 || dist2 < best) {
+    if (won < 0 || dist2 < best || (dist2 == best && f < won)) {
       best = dist2;
+      won = f;
       const double n[3] = {Su[1] * Sv[2] - Su[2] * Sv[1], Su[2] * Sv[0] - Su[0] * Sv[2],
                            Su[0] * Sv[1] - Su[1] * Sv[0]};
       side = dot3(r, n);

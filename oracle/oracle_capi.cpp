@@ -145,6 +145,18 @@ int lsxo_geom_build_bezier(void* p, const double* ctrl, const double* center, co
   return 0;
 }
 
+// Cut-cell geometry of given corner values (before the oscillation fix).
+int lsxo_geom_build_level_set(void* p, const double* phi, int hs, int hf, int vs, int vf) {
+  auto* h = static_cast<GeomH*>(p);
+  try {
+    build_cut_geometry_from(h->g, Box{hs, hf, vs, vf}, phi);
+  } catch (std::exception& e) {
+    g_err = e.what();
+    return -1;
+  }
+  return 0;
+}
+
 int lsxo_geom_get_level_set(void* p, double* phi, double* ax, double* ay, double* az, int* sx, int* sy, int* sz) {
   auto* h = static_cast<GeomH*>(p);
   const long n = h->g.ncells();

@@ -409,15 +409,29 @@ void build_vof(Geometry& g) {
       }
 }
 
-void build_cut_geometry(Geometry& g, const Box& box, const std::function<double(double, double, double)>& phi_fn) {
+static void check_box(const Geometry& g, const Box& box) {
   if (box.hs < 1 || box.vs < 1 || box.hf > g.N - 1 || box.vf > g.M - 1 || box.hs >= box.hf || box.vs >= box.vf)
     throw std::runtime_error("geometry box must lie inside the domain's interior");
-  corner_level_set(g, box, phi_fn);
+}
+
+static void build_from_level_set(Geometry& g, const Box& box) {
   build_alpha(g, box);
   build_types(g, box);
   build_theta(g, box);
   build_vof(g);
   g.build_masses();
+}
+
+void build_cut_geometry(Geometry& g, const Box& box, const std::function<double(double, double, double)>& phi_fn) {
+  check_box(g, box);
+  corner_level_set(g, box, phi_fn);
+  build_from_level_set(g, box);
+}
+
+void build_cut_geometry_from(Geometry& g, const Box& box, const double* phi) {
+  check_box(g, box);
+  g.phi.assign(phi, phi + g.ncells());
+  build_from_level_set(g, box);
 }
 
 }  // namespace lsxo

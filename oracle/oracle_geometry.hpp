@@ -52,6 +52,8 @@ void build_types(Geometry& g, const Box& box);
 void build_theta(Geometry& g, const Box& box);
 void build_vof(Geometry& g);
 void build_cut_geometry(Geometry& g, const Box& box, const std::function<double(double, double, double)>& phi_fn);
+// the same from given corner values, one per cell
+void build_cut_geometry_from(Geometry& g, const Box& box, const double* phi);
 int vof_table_size();
 std::vector<double> cell_centres(const std::vector<double>& widths, double origin);
 Csr build_laplace(const Geometry& g, bool pin_outlet);
