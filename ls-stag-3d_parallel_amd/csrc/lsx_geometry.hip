@@ -1462,11 +1462,56 @@ __device__ inline bool corner_active(const double* __restrict__ raw, const doubl
          apart(z + 1 < K, i + NM);
 }
 
-// whether the oscillation fix changed a node (a NaN, which it leaves alone, differs from itself)
-__device__ inline bool node_fixed(double raw, double phi) { return raw < phi || raw > phi; }
+// Bits of a node's mark: a corner whose cells read a chained node; a node that the oscillation fix can
+// change in some moved geometry.
+constexpr unsigned char MARK_CORNER = 1, MARK_FIXABLE = 2;
 
-// Lists of nodes in index order: AC_FIXED those that the oscillation fix changed, AC_CORNERS the active
-// corners and those marked.  Blocks of AC_NODES consecutive nodes count theirs
+// The fix can change node i in direction `st` only if a move by h (of one node of the three at most: those
+// that move together are 6 apart) can leave it above the threshold between two nodes below 0.  The
+// upper neighbour is read unfixed, the lower one fixed: below 0 by itself or because the fix
+// brought it there.  NaN compares false: such a node is never fixed.
+__device__ inline bool between(const double* __restrict__ raw, long i, long st, double h) {
+  return raw[i] + h > EQ_DOUBLE && raw[i + st] - h < 0;
+}
+
+// marks of the nodes whose neighbours are low enough by themselves, 0 on all others
+__global__ void __launch_bounds__(256) k_fixable_first(const double* __restrict__ raw, int N, int M, int K, Box box,
+                                                       double h, unsigned char* __restrict__ mark) {
+  const long n = (long)N * M * K, NM = (long)N * M;
+  for (long i = blockIdx.x * (long)blockDim.x + threadIdx.x; i < n; i += (long)gridDim.x * blockDim.x) {
+    int x, y, z;
+    decode(i, N, M, &x, &y, &z);
+    bool on = false;
+    if (in_box(x, y, box)) {
+      auto dir = [&](long st) { return between(raw, i, st, h) && raw[i - st] - h < 0; };
+      on = dir(1) || dir(N) || (z > 0 && z < K - 1 && dir(NM));
+    }
+    mark[i] = on ? MARK_FIXABLE : 0;
+  }
+}
+
+// marks of the nodes above a marked one; state[0]: there is such a node (the fix chains in some moved
+// geometry), state[1]: one was not marked yet.  Repeated until none is added.
+__global__ void __launch_bounds__(256) k_fixable_next(const double* __restrict__ raw, int N, int M, int K, Box box,
+                                                      double h, const unsigned char* __restrict__ cur,
+                                                      unsigned char* __restrict__ nxt, int* __restrict__ state) {
+  const long n = (long)N * M * K, NM = (long)N * M;
+  for (long i = blockIdx.x * (long)blockDim.x + threadIdx.x; i < n; i += (long)gridDim.x * blockDim.x) {
+    int x, y, z;
+    decode(i, N, M, &x, &y, &z);
+    bool above = false;
+    if (in_box(x, y, box)) {
+      auto dir = [&](long st) { return cur[i - st] != 0 && between(raw, i, st, h); };
+      above = dir(1) || dir(N) || (z > 0 && z < K - 1 && dir(NM));
+    }
+    if (above) state[0] = 1;
+    if (above && !cur[i]) state[1] = 1;
+    nxt[i] = above ? MARK_FIXABLE : cur[i];
+  }
+}
+
+// Lists of nodes in index order: AC_FIXABLE the nodes marked so, AC_CORNERS the active corners and those
+// marked.  Blocks of AC_NODES consecutive nodes count theirs
 // (list null), one workgroup turns the counts into offsets and the total (k_active_scan), and the
 // blocks write (ranks within a block by ballots).
 constexpr int AC_NODES = 1024;
@@ -1480,8 +1525,9 @@ __global__ void __launch_bounds__(256) k_active(const double* __restrict__ raw, 
   int at = list ? count[blockIdx.x] : 0;
   for (int q = 0; q < AC_NODES / 256; ++q) {
     const long i = (long)blockIdx.x * AC_NODES + q * 256 + threadIdx.x;
-    const bool on = i < n && (mode == AC_FIXED ? node_fixed(raw[i], phi[i])
-                                               : (mark && mark[i]) || corner_active(raw, phi, i, N, M, K, box, h));
+    const bool on = i < n && (mode == AC_FIXABLE ? (mark[i] & MARK_FIXABLE) != 0
+                                                 : (mark && (mark[i] & MARK_CORNER)) ||
+                                                       corner_active(raw, phi, i, N, M, K, box, h));
     const unsigned long long m = __ballot(on);
     if (lane == 0) waves[wave] = __popcll(m);
     __syncthreads();
@@ -1519,7 +1565,7 @@ __global__ void __launch_bounds__(1024) k_active_scan(int* __restrict__ count, i
   if (threadIdx.x == 1023) count[nb] = sum[1023];
 }
 
-// Index of node j in the sorted list of fixed nodes.
+// Index of node j in the sorted list of fixable nodes.
 __device__ inline int find_node(const int* __restrict__ list, int count, int j) {
   int lo = 0, hi = count - 1;
   while (lo < hi) {
@@ -1533,11 +1579,11 @@ __device__ inline int find_node(const int* __restrict__ list, int count, int j) 
 }
 
 // The level set with the corners of a class moved by +h (move 0) or -h (move 1), before the fix and,
-// from the values `val` of the fixed nodes, after it.
+// from the values `val` of the fixable nodes, after it.
 struct MovedLevelSet {
   const double* __restrict__ raw0;
-  const double* __restrict__ phi0;
-  const int* __restrict__ list;  // fixed nodes
+  const unsigned char* __restrict__ mark;
+  const int* __restrict__ list;  // fixable nodes
   const double* val;
   int count, cls, move, N, M;
   double h;
@@ -1550,20 +1596,21 @@ struct MovedLevelSet {
     return on ? (move == 0 ? v + h : v - h) : v;
   }
   __device__ double fixed(long j) const {
-    return node_fixed(raw0[j], phi0[j]) ? val[find_node(list, count, (int)j)] : raw(j);
+    return mark[j] & MARK_FIXABLE ? val[find_node(list, count, (int)j)] : raw(j);
   }
 };
 
-// table[(cls * 2 + move) * count + l] = level set of fixed node l after the fix with the corners of class cls
+// table[(cls * 2 + move) * count + l] = level set of fixable node l after the fix with the corners of class cls
 // moved: one workgroup per class and move repeats k_osc_iter's pass over the list until nothing
 // changes (a node depends on lower ones only, so that is the ordered sweep's result whatever the
 // order of the updates within a pass)
 __global__ void __launch_bounds__(256) k_chain_table(const double* __restrict__ raw0, const double* __restrict__ phi0,
+                                                     const unsigned char* __restrict__ mark,
                                                      const int* __restrict__ list, int count, int N, int M, int K,
                                                      Box box, double h, double* table) {
   const long NM = (long)N * M;
   volatile double* val = table + (long)blockIdx.x * count;
-  const MovedLevelSet f{raw0, phi0, list, table + (long)blockIdx.x * count, count, (int)blockIdx.x / 2,
+  const MovedLevelSet f{raw0, mark, list, table + (long)blockIdx.x * count, count, (int)blockIdx.x / 2,
                         (int)blockIdx.x % 2, N, M, h, box};
   for (int l = threadIdx.x; l < count; l += blockDim.x) val[l] = phi0[list[l]];
   for (;;) {
@@ -1574,7 +1621,7 @@ __global__ void __launch_bounds__(256) k_chain_table(const double* __restrict__ 
       const long j = list[l];
       const int z = (int)(j / NM);
       auto lower = [&](long k) {
-        return node_fixed(raw0[k], phi0[k]) ? (double)val[find_node(list, count, (int)k)] : f.raw(k);
+        return mark[k] & MARK_FIXABLE ? (double)val[find_node(list, count, (int)k)] : f.raw(k);
       };
       double v = f.raw(j);
       check_osc(v, lower(j - 1), f.raw(j + 1));
@@ -1589,20 +1636,21 @@ __global__ void __launch_bounds__(256) k_chain_table(const double* __restrict__ 
   }
 }
 
-// mark the corners whose cells read a fixed node next to a lower fixed one: its cells' rows reach the
-// corners within 4 of it
-__global__ void __launch_bounds__(256) k_chain_mark(const double* __restrict__ raw0, const double* __restrict__ phi0,
-                                                    const int* __restrict__ list, int N, int M, int K, Box box,
-                                                    unsigned char* __restrict__ mark) {
+// mark the corners whose cells read a fixable node next to a lower one: its cells' rows reach the corners
+// within 4 of it (every writer of a byte adds the same bit to the same marks)
+__global__ void __launch_bounds__(256) k_chain_mark(const int* __restrict__ list, int N, int M, int K, Box box,
+                                                    unsigned char* mark) {
   const long NM = (long)N * M, j = list[blockIdx.x];
   int x, y, z;
   decode(j, N, M, &x, &y, &z);
-  auto fixed = [&](long k) { return node_fixed(raw0[k], phi0[k]); };
-  if (!fixed(j - 1) && !fixed(j - N) && !(z > 0 && fixed(j - NM))) return;
+  auto fixable = [&](long k) { return (mark[k] & MARK_FIXABLE) != 0; };
+  if (!fixable(j - 1) && !fixable(j - N) && !(z > 0 && fixable(j - NM))) return;
   for (int q = threadIdx.x; q < 729; q += blockDim.x) {
     const int cx = x + q % 9 - 4, cy = y + q / 9 % 9 - 4, cz = z + q / 81 - 4;
-    if (cx >= 0 && cx < N && cy >= 0 && cy < M && cz >= 0 && cz < K && in_box(cx, cy, box))
-      mark[cx + (long)N * cy + NM * cz] = 1;
+    if (cx >= 0 && cx < N && cy >= 0 && cy < M && cz >= 0 && cz < K && in_box(cx, cy, box)) {
+      unsigned char* m = mark + cx + (long)N * cy + NM * cz;
+      *m = (*m & MARK_FIXABLE) | MARK_CORNER;
+    }
   }
 }
 
@@ -1643,11 +1691,13 @@ struct PatchCell {
 // both moves in turn; the terms of the 216 reached cells are added in index order.  Bound by the
 // latency of its dozen stages.  Without chains the corner's move changes nodes and cells c + [-1, 4]^3 at
 // most and the fix is repeated in LDS (31 KB: four workgroups share a CU); CHAIN: every cell and edge
-// that the rows of the reach read, c + [-4, 4]^3, with the fixed nodes' values from the table.
+// that the rows of the reach read, c + [-4, 4]^3, with the fixable nodes' values from the table.
 template <bool CHAIN>
 __global__ void __launch_bounds__(CHAIN ? 768 : 256) k_corner(GeoBase g, const int* __restrict__ list, int n_active,
-                                                              LagrArgs la, double h, const int* __restrict__ fixed,
-                                                              int n_fixed, const double* __restrict__ table,
+                                                              LagrArgs la, double h,
+                                                              const unsigned char* __restrict__ mark,
+                                                              const int* __restrict__ fixable, int n_fixable,
+                                                              const double* __restrict__ table,
                                                               double* __restrict__ out) {
   constexpr int PA = CHAIN ? 9 : 6, LO = CHAIN ? -4 : -1, CELLS = PA * PA * PA, RA = 6, REACH = RA * RA * RA;
   __shared__ Patch<PA> S[2];
@@ -1707,7 +1757,8 @@ __global__ void __launch_bounds__(CHAIN ? 768 : 256) k_corner(GeoBase g, const i
       for (int m = 0; m < 2; ++m) {
         const PatchCell<PA> q{&S[m], g, lx, ly, lz, i, N, NM};
         const int cls = corner_class(cx, cy, cz);
-        const MovedLevelSet f{g.raw, g.phi, fixed, table + (long)(cls * 2 + m) * n_fixed, n_fixed, cls, m, N, M, h, box};
+        const MovedLevelSet f{g.raw, mark, fixable, table + (long)(cls * 2 + m) * n_fixable, n_fixable, cls, m, N, M, h,
+                              box};
         auto phi = [&](int dx, int dy, int dz) {
           if constexpr (CHAIN)
             return f.fixed(i + dx + (long)N * dy + NM * dz);
@@ -1882,11 +1933,19 @@ void list_nodes(const double* phi_raw, const double* phi, const unsigned char* m
   if (!list) k_active_scan<<<1, 1024, 0, s>>>(count, nb);
 }
 
-void chain_tables(const double* phi_raw, const double* phi, const int* fixed, int n_fixed, int N, int M, int K, Box box,
-                  double h, double* table, unsigned char* mark, hipStream_t s) {
-  (void)hipMemsetAsync(mark, 0, (size_t)N * M * K, s);
-  k_chain_mark<<<n_fixed, 256, 0, s>>>(phi_raw, phi, fixed, N, M, K, box, mark);
-  k_chain_table<<<2 * SG_CLASSES, 256, 0, s>>>(phi_raw, phi, fixed, n_fixed, N, M, K, box, h, table);
+void fixable_first(const double* phi_raw, int N, int M, int K, Box box, double h, unsigned char* mark, hipStream_t s) {
+  k_fixable_first<<<grid_1d((long)N * M * K), 256, 0, s>>>(phi_raw, N, M, K, box, h, mark);
+}
+
+void fixable_next(const double* phi_raw, int N, int M, int K, Box box, double h, const unsigned char* cur,
+                  unsigned char* nxt, int* state, hipStream_t s) {
+  k_fixable_next<<<grid_1d((long)N * M * K), 256, 0, s>>>(phi_raw, N, M, K, box, h, cur, nxt, state);
+}
+
+void chain_tables(const double* phi_raw, const double* phi, const int* fixable, int n_fixable, int N, int M, int K,
+                  Box box, double h, double* table, unsigned char* mark, hipStream_t s) {
+  k_chain_mark<<<n_fixable, 256, 0, s>>>(fixable, N, M, K, box, mark);
+  k_chain_table<<<2 * SG_CLASSES, 256, 0, s>>>(phi_raw, phi, mark, fixable, n_fixable, N, M, K, box, h, table);
 }
 
 static LagrArgs lagr_args(const double* dx, const double* dy, const double* dz, int N, int M, int K, Box box, int pin,
@@ -1896,17 +1955,17 @@ static LagrArgs lagr_args(const double* dx, const double* dy, const double* dz, 
   return LagrArgs{dx, dy, dz, p, lam, N, M, K, pin, objective, rhs ? 1 : 0, box, in, 0.5 / h};
 }
 
-void corner_gradient(const GeoBase& g, const int* list, int count, const int* fixed, int n_fixed, const double* table,
-                     const double* dx, const double* dy, const double* dz, int N, int M, int K, Box box, int pin,
-                     const double* p, const double* lam, int objective, const RhsArgs* rhs, double h, double* out,
-                     hipStream_t s) {
+void corner_gradient(const GeoBase& g, const int* list, int count, const unsigned char* mark, const int* fixable,
+                     int n_fixable, const double* table, const double* dx, const double* dy, const double* dz, int N,
+                     int M, int K, Box box, int pin, const double* p, const double* lam, int objective,
+                     const RhsArgs* rhs, double h, double* out, hipStream_t s) {
   if (count < 1) return;
   const LagrArgs la = lagr_args(dx, dy, dz, N, M, K, box, pin, p, lam, objective, rhs, h);
   const int blocks = count < 4096 ? count : 4096;
   if (table)
-    k_corner<true><<<blocks, 768, 0, s>>>(g, list, count, la, h, fixed, n_fixed, table, out);
+    k_corner<true><<<blocks, 768, 0, s>>>(g, list, count, la, h, mark, fixable, n_fixable, table, out);
   else
-    k_corner<false><<<blocks, 256, 0, s>>>(g, list, count, la, h, nullptr, 0, nullptr, out);
+    k_corner<false><<<blocks, 256, 0, s>>>(g, list, count, la, h, nullptr, nullptr, 0, nullptr, out);
 }
 
 void bezier_chain(const double* g, const int* list, int count, const double* cx, const double* cy, const double* cz,

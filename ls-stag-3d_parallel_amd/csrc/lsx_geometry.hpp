@@ -100,26 +100,32 @@ void drag_noalloc(const int* type, const double* tx, const double* dy, const dou
 // Address of the library's drag scratch array on the current device (looked up once per device
 // with hipGetSymbolAddress); 0, or a negative value when the lookup fails.
 int drag_scratch(double** out);
-// Lists of nodes in index order: AC_FIXED those that the oscillation fix changed, AC_CORNERS the corners
-// that a move by h can change the geometry at and (mark given) the marked ones.  list null: fills
+// Nodes that the oscillation fix can change with some corner moved by h, in marks of one byte a node:
+// fixable_first writes them all, fixable_next (cur to nxt) adds those next to a marked one and sets
+// state[0] if it meets any, state[1] if one was not marked yet.  To be repeated while it does.
+void fixable_first(const double* phi_raw, int N, int M, int K, Box box, double h, unsigned char* mark, hipStream_t s);
+void fixable_next(const double* phi_raw, int N, int M, int K, Box box, double h, const unsigned char* cur,
+                  unsigned char* nxt, int* state, hipStream_t s);
+// Lists of nodes in index order: AC_FIXABLE those, AC_CORNERS the corners that a move by h can change the
+// geometry at and (mark given) those that chain_tables marked.  list null: fills
 // count[0 .. nb) with the offsets of nb = active_blocks(n) blocks of nodes and count[nb] with the
 // number of listed ones; list given (after that): writes them.
-enum { AC_FIXED = 0, AC_CORNERS = 1 };
+enum { AC_FIXABLE = 0, AC_CORNERS = 1 };
 int active_blocks(long n);
 void list_nodes(const double* phi_raw, const double* phi, const unsigned char* mark, int mode, int N, int M, int K,
                 Box box, double h, int* count, int* list, hipStream_t s);
-// Where fixed nodes have read fixed nodes: table gets their values with the corners of each class moved
-// by +h and -h (432 n_fixed doubles), mark (n bytes) the corners whose cells read such a node.
+// Where a fixable node reads another: table gets the listed ones' values with the corners of each class
+// moved by +h and -h (432 n_fixable doubles), mark the corners whose cells read such a node.
 constexpr int CHAIN_MOVES = 432;
-void chain_tables(const double* phi_raw, const double* phi, const int* fixed, int n_fixed, int N, int M, int K, Box box,
-                  double h, double* table, unsigned char* mark, hipStream_t s);
+void chain_tables(const double* phi_raw, const double* phi, const int* fixable, int n_fixable, int N, int M, int K,
+                  Box box, double h, double* table, unsigned char* mark, hipStream_t s);
 // out[c] = sum over the cells c + [-2, 3]^3 of (F_i(+) - F_i(-)) / 2h with F_i = J_i + lambda_i (b_i - (A p)_i), for
 // the count listed corners, moved by +h and -h one by one, or (table given) together with the others of
 // their class; rhs null: b fixed
-void corner_gradient(const GeoBase& g, const int* list, int count, const int* fixed, int n_fixed, const double* table,
-                     const double* dx, const double* dy, const double* dz, int N, int M, int K, Box box, int pin,
-                     const double* p, const double* lam, int objective, const RhsArgs* rhs, double h, double* out,
-                     hipStream_t s);
+void corner_gradient(const GeoBase& g, const int* list, int count, const unsigned char* mark, const int* fixable,
+                     int n_fixable, const double* table, const double* dx, const double* dy, const double* dz, int N,
+                     int M, int K, Box box, int pin, const double* p, const double* lam, int objective,
+                     const RhsArgs* rhs, double h, double* out, hipStream_t s);
 // out[288] = sum over the count listed corners of g dphi/dctrl through the closest point (hf, huv, hw: count,
 // 2 count, 3 count scratch)
 void bezier_chain(const double* g, const int* list, int count, const double* cx, const double* cy, const double* cz,

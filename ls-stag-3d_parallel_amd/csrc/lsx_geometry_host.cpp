@@ -4,7 +4,9 @@
 
 #include "lsx_geometry_host.hpp"
 
+#include <algorithm>
 #include <cmath>
+#include <utility>
 
 namespace lsx {
 
@@ -163,14 +165,16 @@ void Geometry::stage_flow(const double* u, const double* v, const double* w, con
   }
 }
 
-// nodes of a list (geo::AC_*) into `list`, which grows with some room for the next body's; their number
-int Geometry::list_nodes(int mode, const unsigned char* mark, double h, DevBuf<int>& list) {
+// nodes of a list (geo::AC_*) into `list`, which grows with some room for the next body's; their number.
+// state given: receives the two ints behind the counts (geo::fixable_next) in the same copy
+int Geometry::list_nodes(int mode, const unsigned char* mark, double h, DevBuf<int>& list, int* state) {
   const int nb = geo::active_blocks(n());
-  sg_count.alloc(nb + 1);
   geo::list_nodes(phi_raw.p, phi.p, mark, mode, N, M, K, box_, h, sg_count.p, nullptr, stream);
-  int count = 0;
-  LSX_HIP(hipMemcpyAsync(&count, sg_count.p + nb, sizeof(int), hipMemcpyDeviceToHost, stream));
+  int got[3] = {0, 0, 0};
+  LSX_HIP(hipMemcpyAsync(got, sg_count.p + nb, sizeof(got), hipMemcpyDeviceToHost, stream));
   LSX_HIP(hipStreamSynchronize(stream));
+  const int count = got[0];
+  if (state) std::copy(got + 1, got + 3, state);
   if ((size_t)count > list.n) list.alloc((size_t)count + count / 4);
   if (count > 0)
     geo::list_nodes(phi_raw.p, phi.p, mark, mode, N, M, K, box_, h, sg_count.p, list.p, stream);
@@ -276,19 +280,41 @@ void Geometry::shape_gradient(const double* p, const double* lam, int objective,
   }
   sg_g.alloc(nn);
   LSX_HIP(hipMemsetAsync(sg_g.p, 0, nn * sizeof(double), stream));
-  // fixed nodes that have read fixed nodes (a third pass of the fix): corners move by classes
-  int n_fixed = 0;
-  if (osc_passes > 2) {
-    n_fixed = list_nodes(geo::AC_FIXED, nullptr, h, sg_fixed);
-    if ((size_t)n_fixed * geo::CHAIN_MOVES > sg_table.n) sg_table.alloc((size_t)(n_fixed + n_fixed / 4) * geo::CHAIN_MOVES);
-    if (n_fixed > 0)
-      geo::chain_tables(phi_raw.p, phi.p, sg_fixed.p, n_fixed, N, M, K, box_, h, sg_table.p, flag.p, stream);
+  // Where, in some moved geometry, a node that the oscillation fix changes reads another such node, a
+  // corner's move can reach beyond its patch: corners then move by classes, with the fixed values of each
+  // class's moves in a table.  Every body pays the look (two passes over a byte a node, read with the
+  // first list's count): whether the unmoved geometry chains does not say it, a body aligned with the
+  // grid may chain only once a node at 0 has moved.
+  const int nb = geo::active_blocks(nn);
+  sg_count.alloc(nb + 3);
+  sg_mark.alloc(nn);
+  int* const dstate = sg_count.p + nb + 1;
+  unsigned char *cur = flag.p, *nxt = sg_mark.p;
+  auto spread = [&] {
+    LSX_HIP(hipMemsetAsync(dstate, 0, 2 * sizeof(int), stream));
+    geo::fixable_next(phi_raw.p, N, M, K, box_, h, cur, nxt, dstate, stream);
+    std::swap(cur, nxt);
+  };
+  geo::fixable_first(phi_raw.p, N, M, K, box_, h, cur, stream);
+  spread();
+  int state[2], n_fixable = 0;
+  int active = list_nodes(geo::AC_CORNERS, nullptr, h, sg_list, state);
+  const bool chain = state[0] != 0;
+  if (chain) {
+    while (state[1]) {
+      spread();
+      LSX_HIP(hipMemcpyAsync(state, dstate, sizeof(state), hipMemcpyDeviceToHost, stream));
+      LSX_HIP(hipStreamSynchronize(stream));
+    }
+    n_fixable = list_nodes(geo::AC_FIXABLE, cur, h, sg_fixable);
+    if ((size_t)n_fixable * geo::CHAIN_MOVES > sg_table.n)
+      sg_table.alloc((size_t)(n_fixable + n_fixable / 4) * geo::CHAIN_MOVES);
+    geo::chain_tables(phi_raw.p, phi.p, sg_fixable.p, n_fixable, N, M, K, box_, h, sg_table.p, cur, stream);
+    active = list_nodes(geo::AC_CORNERS, cur, h, sg_list);
   }
-  const bool chain = n_fixed > 0;
-  const int active = list_nodes(geo::AC_CORNERS, chain ? flag.p : nullptr, h, sg_list);
   const geo::GeoBase base{phi_raw.p, phi.p, {ax.p, ay.p, az.p}, {tx.p, ty.p, tz.p}, vof.p, type.p};
-  geo::corner_gradient(base, sg_list.p, active, sg_fixed.p, n_fixed, chain ? sg_table.p : nullptr, dx.p, dy.p, dz.p, N, M,
-                       K, box_, pin, dp, dl, objective, rhs, h, sg_g.p, stream);
+  geo::corner_gradient(base, sg_list.p, active, cur, sg_fixable.p, n_fixable, chain ? sg_table.p : nullptr, dx.p, dy.p,
+                       dz.p, N, M, K, box_, pin, dp, dl, objective, rhs, h, sg_g.p, stream);
   LSX_HIP(hipGetLastError());
   if (dJdphi)
     LSX_HIP(hipMemcpyAsync(dJdphi, sg_g.p, nn * sizeof(double),

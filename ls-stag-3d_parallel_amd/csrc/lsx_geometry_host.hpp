@@ -98,11 +98,12 @@ class Geometry {
   DevBuf<double> bez;  // Bezier control values (device)
   geo::Body body_{};
   geo::Box box_{};
-  // shape-gradient work: node lists and their offsets, the fixed nodes' values per class and move, g
-  // per corner, closest points of the listed corners
+  // shape-gradient work: node lists with their offsets, the marks of the fixable nodes (and `flag`), these
+  // nodes' values per class and move, g per corner, closest points of the listed corners
   DevBuf<double> sg_g, sg_uv, sg_w, sg_partial, sg_out, sg_table;
-  DevBuf<int> sg_count, sg_list, sg_fixed, sg_f;
-  int list_nodes(int mode, const unsigned char* mark, double h, DevBuf<int>& list);
+  DevBuf<int> sg_count, sg_list, sg_fixable, sg_f;
+  DevBuf<unsigned char> sg_mark;
+  int list_nodes(int mode, const unsigned char* mark, double h, DevBuf<int>& list, int* state = nullptr);
 };
 
 }  // namespace lsx
