@@ -321,11 +321,10 @@ void Geometry::shape_gradient(const double* p, const double* lam, int objective,
                            mem == LSX_MEM_HOST ? hipMemcpyDeviceToHost : hipMemcpyDeviceToDevice, stream));
   if (dJdctrl) {
     sg_out.alloc(288);
-    if ((size_t)active > sg_f.n) {
-      sg_f.alloc(sg_list.n);
-      sg_uv.alloc(2 * sg_list.n);
-      sg_w.alloc(3 * sg_list.n);
-    }
+    // each by its own size: a call that ran out of memory may have grown some of them
+    if ((size_t)active > sg_f.n) sg_f.alloc(sg_list.n);
+    if (2 * (size_t)active > sg_uv.n) sg_uv.alloc(2 * sg_list.n);
+    if (3 * (size_t)active > sg_w.n) sg_w.alloc(3 * sg_list.n);
     geo::bezier_chain(sg_g.p, sg_list.p, active, cx.p, cy.p, cz.p, N, M, body_, sg_f.p, sg_uv.p, sg_w.p, sg_out.p,
                       stream);
     LSX_HIP(hipGetLastError());

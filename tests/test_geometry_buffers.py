@@ -1,0 +1,73 @@
+"""Host side of the shape gradient on a stand-in runtime: after a call that ran out of memory half way
+through growing its work buffers, a later call with fewer corners has buffers of the sizes it needs."""
+import host_build
+
+PROGRAM = r"""
+#include "host_runtime.hpp"
+#include "lsx_geometry_host.hpp"
+
+using host_runtime::room;
+static int corners = 0;
+
+namespace lsx { namespace geo {
+void level_set(const double*, const double*, const double*, int, int, int, Box, Body, double*, hipStream_t) {}
+int oscillation_fix(const double*, double*, double*, unsigned char*, int*, int, int, int, Box, hipStream_t) { return 1; }
+void alpha(const double*, int, int, int, Box, double*, double*, double*, hipStream_t) {}
+void types(const double*, int, int, int, Box, int*, int*, int*, int*, hipStream_t) {}
+void theta(const double*, const double*, const double*, const int*, const int*, const int*, int, int, int, Box, double*,
+           double*, double*, hipStream_t) {}
+void vof(const int*, const double*, const double*, const double*, const double*, const double*, const double*,
+         const double*, const double*, const double*, int, int, int, double*, hipStream_t) {}
+int active_blocks(long) { return 1; }
+void fixable_first(const double*, int, int, int, Box, double, unsigned char*, hipStream_t) {}
+void fixable_next(const double*, int, int, int, Box, double, const unsigned char*, unsigned char*, int*, hipStream_t) {}
+void list_nodes(const double*, const double*, const unsigned char*, int, int, int, int, Box, double, int* count,
+                int* list, hipStream_t) {
+  if (!list) count[1] = corners;
+  if (list) CHECK(room(list) >= corners * sizeof(int));
+}
+void corner_gradient(const GeoBase&, const int*, int, const unsigned char*, const int*, int, const double*,
+                     const double*, const double*, const double*, int, int, int, Box, int, const double*, const double*,
+                     int, const RhsArgs*, double, double*, hipStream_t) {}
+void bezier_chain(const double*, const int*, int count, const double*, const double*, const double*, int, int, Body,
+                  int* hf, double* huv, double* hw, double* out, hipStream_t) {
+  CHECK(room(hf) >= count * sizeof(int));
+  CHECK(room(huv) >= 2 * count * sizeof(double));
+  CHECK(room(hw) >= 3 * count * sizeof(double));
+  CHECK(room(out) >= 288 * sizeof(double));
+}
+} }
+
+int main() {
+  const int N = 8;
+  const double w[N] = {1, 1, 1, 1, 1, 1, 1, 1};
+  const std::vector<double> v(N * N * N, 1.0), ctrl(288, 0.5);
+  double out[288];
+  const size_t list = 100 + 100 / 4;  // what a list of 100 corners grows to
+  for (size_t size : {list * sizeof(int), 2 * list * sizeof(double), 3 * list * sizeof(double)}) {
+    lsx::Geometry g(N, N, N, w, w, w, 0, 0, 0, nullptr);
+    g.build(lsx::geo::Body{lsx::geo::BODY_BEZIER6, {4, 4, 4}, {1, 1, 1}}, lsx::geo::Box{1, N - 1, 1, N - 1}, ctrl.data());
+    auto gradient = [&](int n) {
+      corners = n;
+      g.shape_gradient(v.data(), v.data(), lsx::geo::OBJ_DRAG_X, nullptr, 1, 1e-7, nullptr, out, LSX_MEM_DEVICE);
+    };
+    gradient(10);
+    host_runtime::fail_size = size;
+    bool failed = false;
+    try {
+      gradient(100);
+    } catch (const lsx::Error&) {
+      failed = true;
+    }
+    CHECK(failed);
+    (void)hipGetLastError();
+    host_runtime::fail_size = 0;
+    for (int n : {50, 10, 100, 0, 101}) gradient(n);
+  }
+  std::printf("ok\n");
+}
+"""
+
+
+def test_buffers_after_a_failed_growth(tmp_path):
+    host_build.run(tmp_path, PROGRAM, ["lsx_geometry_host.cpp"])
