@@ -3,6 +3,7 @@
 
 #include <hip/hip_runtime.h>
 
+#include <algorithm>
 #include <mutex>
 #include <stdexcept>
 #include <string>
@@ -32,14 +33,26 @@ struct Error : std::runtime_error {
 // evaluation of a shape, 2.4 of its 4.9 ms.  Inside a Scope a DevBuf takes a block of exactly its
 // size and gives it back on release; blocks above `bound` and those of other owners go to hipFree as
 // ever.  An owner uses its blocks on its one stream only, which orders a block's next use after
-// its last; blocks not in use are at most `bound` bytes and go with the owner.
+// its last; blocks not in use are at most `bound` bytes and go with the owner, or when any allocation
+// of the library runs out of memory.
 class BlockPool {
  public:
   static constexpr size_t bound = size_t(256) << 20;
-  BlockPool() = default;
+  BlockPool() {
+    Live& l = live();
+    std::lock_guard<std::mutex> lock(l.m);
+    l.pools.push_back(this);
+  }
   BlockPool(const BlockPool&) = delete;
   BlockPool& operator=(const BlockPool&) = delete;
-  ~BlockPool() { drop(); }
+  ~BlockPool() {
+    {
+      Live& l = live();
+      std::lock_guard<std::mutex> lock(l.m);
+      l.pools.erase(std::find(l.pools.begin(), l.pools.end(), this));
+    }
+    drop();
+  }
   class Scope {  // this thread's allocations go through `pool` until the end of the scope
    public:
     explicit Scope(BlockPool& pool) : prev(current()) { current() = &pool; }
@@ -84,12 +97,27 @@ class BlockPool {
     held = 0;
     return any;
   }
+  static bool drop_all() {  // of every handle (hipFree waits for the work that last used a block)
+    Live& l = live();
+    std::lock_guard<std::mutex> lock(l.m);
+    bool any = false;
+    for (BlockPool* p : l.pools) any = p->drop() || any;
+    return any;
+  }
 
  private:
   struct Block {
     void* p;
     size_t bytes;
   };
+  struct Live {  // the pools of the process; outlives every handle
+    std::mutex m;
+    std::vector<BlockPool*> pools;
+  };
+  static Live& live() {
+    static Live* const l = new Live;
+    return *l;
+  }
   std::vector<Block> idle;
   size_t held = 0;
   std::mutex m;
@@ -127,10 +155,11 @@ struct DevBuf {
     if (count && pool) p = static_cast<T*>(pool->take(count * sizeof(T)));
     if (count && !p) {
       hipError_t e = hipMalloc(&p, count * sizeof(T));
-      if (e == hipErrorOutOfMemory && pool && pool->drop()) {  // idle blocks of other sizes
+      if (e == hipErrorOutOfMemory && BlockPool::drop_all()) {  // idle blocks of other sizes and handles
         (void)hipGetLastError();
         e = hipMalloc(&p, count * sizeof(T));
       }
+      if (e != hipSuccess) p = nullptr;
       LSX_HIP(e);
     }
     n = count;

@@ -1,0 +1,66 @@
+"""Device blocks kept for a handle's next call, on a stand-in runtime."""
+import host_build
+
+HEAD = r"""
+#include "host_runtime.hpp"
+#include "lsx_solver.hpp"
+using lsx::BlockPool;
+using lsx::DevBuf;
+namespace hr = host_runtime;
+"""
+
+OUT_OF_MEMORY = HEAD + r"""
+// leaves `count` idle blocks of `bytes` in a pool
+static void fill(BlockPool& pool, int count, size_t bytes) {
+  BlockPool::Scope s(pool);
+  std::vector<DevBuf<char>> b(count);
+  for (auto& q : b) q.alloc(bytes);
+}
+int main() {
+  hr::limit = 1000;
+  {  // an allocation outside any call's scope, as a solve's staging buffers are
+    BlockPool a;
+    fill(a, 3, 300);
+    CHECK(hr::live == 900);
+    DevBuf<char> x;
+    x.alloc(500);
+    CHECK(hr::live == 500 && hipGetLastError() == hipSuccess);
+  }
+  CHECK(hr::live == 0);
+  {  // another handle's call, with blocks of its own and of a third one
+    BlockPool a, b, c;
+    fill(a, 2, 200);
+    fill(b, 1, 100);
+    fill(c, 1, 100);
+    BlockPool::Scope s(b);
+    DevBuf<char> x;
+    x.alloc(900);
+    CHECK(hr::live == 900);
+  }
+  {  // a pool that is gone is not asked
+    BlockPool a;
+    { BlockPool b; fill(b, 1, 600); }
+    fill(a, 1, 600);
+    DevBuf<char> x;
+    x.alloc(1000);
+  }
+  {  // nothing idle: the error is reported
+    BlockPool a;
+    DevBuf<char> x, y;
+    x.alloc(600);
+    bool failed = false;
+    try {
+      y.alloc(600);
+    } catch (const lsx::Error& e) {
+      failed = e.code == LSX_ERR_HIP;
+    }
+    CHECK(failed && !y.p && y.n == 0);
+  }
+  CHECK(hr::live == 0);
+  std::printf("ok\n");
+}
+"""
+
+
+def test_out_of_memory_takes_every_handles_idle_blocks(tmp_path):
+    host_build.run(tmp_path, OUT_OF_MEMORY)
