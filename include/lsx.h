@@ -15,6 +15,12 @@
  * message of the last failure on the calling thread.  A handle is used by one host thread
  * at a time; distinct handles are independent (no global mutable state per handle).
  * Work is ordered on the handle's HIP stream.
+ *
+ * Device memory: a solver keeps the blocks that its set-ups (lsx_set_*, lsx_rebuild) release, and
+ * a geometry those of its calls with host arrays, for their next calls: at most 256 MB of idle
+ * blocks per handle, each freed after 16 such calls that did not need it, all of them with the handle.
+ * An allocation of the library that runs out of memory frees the idle blocks of every handle
+ * and is tried again; other users of the device get them when the handle is destroyed.
  */
 #ifndef LSX_H_
 #define LSX_H_

@@ -30,14 +30,17 @@ struct Error : std::runtime_error {
 
 // Device blocks that an object keeps for its next call.  Setting up a 64^3 hierarchy and staging host
 // arrays made 54 hipMalloc (19 us each) and as many hipFree (27 us, the device drained) per
-// evaluation of a shape, 2.4 of its 4.9 ms.  Inside a Scope a DevBuf takes a block of exactly its
-// size and gives it back on release; blocks above `bound` and those of other owners go to hipFree as
-// ever.  An owner uses its blocks on its one stream only, which orders a block's next use after
-// its last; blocks not in use are at most `bound` bytes and go with the owner, or when any allocation
-// of the library runs out of memory.
+// evaluation of a shape, 2.4 of its 4.9 ms.  Inside a Scope (a call) a DevBuf takes a block of exactly
+// its size and gives it back on release; blocks of other owners go to hipFree as ever.  An owner uses
+// its blocks on its one stream only, which orders a block's next use after its last.  Blocks not in use
+// are at most `bound` bytes; the one idle longest goes when the present call's need room, and each after
+// `idle_calls` calls of the owner that did not ask for it (a cycle of calls, three momentum set-ups and
+// a pressure one, or geometry, right-hand side, correction, drag and gradient, is shorter).  All go with
+// the owner, or when any allocation of the library runs out of memory.
 class BlockPool {
  public:
   static constexpr size_t bound = size_t(256) << 20;
+  static constexpr int idle_calls = 16;
   BlockPool() {
     Live& l = live();
     std::lock_guard<std::mutex> lock(l.m);
@@ -58,7 +61,10 @@ class BlockPool {
     explicit Scope(BlockPool& pool) : prev(current()) { current() = &pool; }
     Scope(const Scope&) = delete;
     Scope& operator=(const Scope&) = delete;
-    ~Scope() { current() = prev; }
+    ~Scope() {
+      if (current() != prev) current()->call_ends();
+      current() = prev;
+    }
 
    private:
     BlockPool* prev;
@@ -69,7 +75,7 @@ class BlockPool {
   }
   void* take(size_t bytes) {
     std::lock_guard<std::mutex> lock(m);
-    for (size_t i = 0; i < idle.size(); ++i)
+    for (size_t i = idle.size(); i-- > 0;)  // the last given first: blocks too many are not asked for
       if (idle[i].bytes == bytes) {
         void* p = idle[i].p;
         idle.erase(idle.begin() + (long)i);
@@ -80,9 +86,11 @@ class BlockPool {
   }
   bool give(void* p, size_t bytes) {
     std::lock_guard<std::mutex> lock(m);
+    if (bytes > bound) return false;
+    while (held + bytes > bound && idle.front().call < calls) free_first();
     if (held + bytes > bound) return false;
     try {
-      idle.push_back({p, bytes});
+      idle.push_back({p, bytes, calls});
     } catch (...) {
       return false;
     }
@@ -109,7 +117,18 @@ class BlockPool {
   struct Block {
     void* p;
     size_t bytes;
+    long call;  // in which it was given back
   };
+  void free_first() {
+    (void)hipFree(idle.front().p);
+    held -= idle.front().bytes;
+    idle.erase(idle.begin());
+  }
+  void call_ends() {
+    std::lock_guard<std::mutex> lock(m);
+    ++calls;
+    while (!idle.empty() && calls - idle.front().call > idle_calls + 1) free_first();
+  }
   struct Live {  // the pools of the process; outlives every handle
     std::mutex m;
     std::vector<BlockPool*> pools;
@@ -118,8 +137,9 @@ class BlockPool {
     static Live* const l = new Live;
     return *l;
   }
-  std::vector<Block> idle;
+  std::vector<Block> idle;  // in the order they were given back
   size_t held = 0;
+  long calls = 0;
   std::mutex m;
 };
 
