@@ -48,6 +48,7 @@ Geometry::Geometry(int N_, int M_, int K_, const double* dx_, const double* dy_,
     LSX_HIP(hipStreamCreate(&stream));
     own_stream = true;
   }
+  spare.stream = stream;
   dx.alloc(N);
   dy.alloc(M);
   dz.alloc(K);

@@ -48,6 +48,7 @@ Solver::Solver(const lsx_options& o, hipStream_t s) : opt(o) {
     LSX_HIP(hipStreamCreate(&stream));  // default priority
     own_stream = true;
   }
+  spare.stream = stream;
   err.alloc(1);
   scalars.alloc(SC_H + 256 * 257 / 2 + 8);
   partial.alloc(2 * RED_BLOCKS_MAX);

@@ -4,6 +4,7 @@
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
+#include <exception>
 #include <mutex>
 #include <stdexcept>
 #include <string>
@@ -56,18 +57,23 @@ class BlockPool {
     }
     drop();
   }
+  hipStream_t stream = nullptr;  // the owner's, set when it has one
   class Scope {  // this thread's allocations go through `pool` until the end of the scope
    public:
-    explicit Scope(BlockPool& pool) : prev(current()) { current() = &pool; }
+    explicit Scope(BlockPool& pool) : prev(current()), errors(std::uncaught_exceptions()) { current() = &pool; }
     Scope(const Scope&) = delete;
     Scope& operator=(const Scope&) = delete;
     ~Scope() {
+      // a call waits for its stream before it returns; one that fails may have copies of the caller's
+      // arrays under way, which the hipFree of their blocks waited for
+      if (std::uncaught_exceptions() > errors) (void)hipStreamSynchronize(current()->stream);
       if (current() != prev) current()->call_ends();
       current() = prev;
     }
 
    private:
     BlockPool* prev;
+    int errors;
   };
   static BlockPool*& current() {
     thread_local BlockPool* c = nullptr;

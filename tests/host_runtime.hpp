@@ -13,6 +13,7 @@ namespace host_runtime {
 inline std::map<const char*, size_t> blocks;  // live blocks by address
 inline size_t live = 0, limit = ~size_t(0), fail_size = 0;
 inline long mallocs = 0, frees = 0, syncs = 0;
+inline long allowed = -1;  // allocations that still succeed (-1: all)
 inline hipError_t last = hipSuccess;
 // bytes from p to the end of its block, 0 if p lies in none
 inline size_t room(const void* p) {
@@ -35,7 +36,8 @@ inline size_t room(const void* p) {
 extern "C" {
 inline __attribute__((used)) hipError_t stand_in_malloc(void** p, size_t n) {
   using namespace host_runtime;
-  if (n == fail_size || live + n > limit) return last = hipErrorOutOfMemory;
+  if (n == fail_size || live + n > limit || allowed == 0) return last = hipErrorOutOfMemory;
+  if (allowed > 0) --allowed;
   *p = std::calloc(1, n);
   blocks[static_cast<char*>(*p)] = n;
   live += n;

@@ -1,8 +1,10 @@
-"""Host side of the shape gradient on a stand-in runtime: after a call that ran out of memory half way
-through growing its work buffers, a later call with fewer corners has buffers of the sizes it needs."""
+"""Host side of the geometry on a stand-in runtime.  After a shape gradient that ran out of memory half
+way through growing its work buffers, a later call with fewer corners has buffers of the sizes it
+needs; and a call that fails with copies of the caller's arrays under way waits for them, as its
+buffers' hipFree did, before it returns."""
 import host_build
 
-PROGRAM = r"""
+HEAD = r"""
 #include "host_runtime.hpp"
 #include "lsx_geometry_host.hpp"
 
@@ -38,6 +40,9 @@ void bezier_chain(const double*, const int*, int count, const double*, const dou
 }
 } }
 
+"""
+
+GROWTH = HEAD + r"""
 int main() {
   const int N = 8;
   const double w[N] = {1, 1, 1, 1, 1, 1, 1, 1};
@@ -68,6 +73,35 @@ int main() {
 }
 """
 
+FAILURE = HEAD + r"""
+int main() {
+  const int N = 8;
+  const double w[N] = {1, 1, 1, 1, 1, 1, 1, 1};
+  std::vector<double> v(N * N * N, 1.0), b(N * N * N);
+  lsx::Geometry g(N, N, N, w, w, w, 0, 0, 0, nullptr);
+  g.build(lsx::geo::Body{lsx::geo::BODY_SPHERE, {4, 4, 4}, {1, 1, 1}}, lsx::geo::Box{1, N - 1, 1, N - 1});
+  lsx_flow_bc bc{};
+  bc.outflow = 1;
+  for (int round = 0; round < 2; ++round) {  // with new blocks, then with kept ones
+    host_runtime::allowed = round == 0 ? 5 : 0;  // u, v, w, west, b; the outflow's copy comes after their copies
+    const long before = host_runtime::syncs;
+    bool failed = false;
+    try {
+      g.pressure_rhs(v.data(), v.data(), v.data(), v.data(), v.data(), bc, b.data(), LSX_MEM_HOST);
+    } catch (const lsx::Error&) {
+      failed = true;
+    }
+    CHECK(failed);
+    CHECK(host_runtime::syncs > before);
+  }
+  std::printf("ok\n");
+}
+"""
+
 
 def test_buffers_after_a_failed_growth(tmp_path):
-    host_build.run(tmp_path, PROGRAM, ["lsx_geometry_host.cpp"])
+    host_build.run(tmp_path, GROWTH, ["lsx_geometry_host.cpp"])
+
+
+def test_failed_call_waits_for_its_copies(tmp_path):
+    host_build.run(tmp_path, FAILURE, ["lsx_geometry_host.cpp"])
