@@ -10,6 +10,7 @@
 
 #include "lsx_kernels.hpp"
 #include "lsx_lu.hpp"
+#include "lsx_rows.hpp"
 
 #include <algorithm>
 #include <cmath>
@@ -53,14 +54,6 @@ __device__ double block_max(double v) {
     for (int w = 0; w < BS / 64; ++w) s = fmax(s, lds[w]);
   __syncthreads();
   return s;
-}
-
-// contiguous chunk of [0, n) owned by block b of nb
-__device__ inline void chunk_of(long n, int b, int nb, long* lo, long* hi) {
-  const long per = (n + nb - 1) / nb;
-  *lo = per * b;
-  long h = *lo + per;
-  *hi = h < n ? h : n;
 }
 
 // ---- stencil geometry helpers -------------------------------------------------------------
@@ -1328,16 +1321,16 @@ __global__ void __launch_bounds__(BS) k_axpy_dot(double* __restrict__ w, const d
   chunk_of(n, blockIdx.x, gridDim.x, &lo, &hi);
   long i = lo + threadIdx.x;
   double vr[R], wr[R], nr[R];
-  auto load = [&] {
+  auto load = [&] {  // of a thread with a row i
 #pragma unroll
     for (int r = 0; r < R; ++r) {
-      const long q = i + r * BS < hi ? i + r * BS : 0;
+      const long q = row_ahead(i, r * BS, hi);
       vr[r] = v[q];
       wr[r] = w[q];
       nr[r] = vnext ? vnext[q] : 0.0;
     }
   };
-  load();
+  if (i < hi) load();
   double p = 0.0;
   const int nb = gridDim.x, per = (nb + BS - 1) / BS, from = threadIdx.x * per;
   for (int k = from; k < from + per && k < nb; ++k) p += pin[k];
