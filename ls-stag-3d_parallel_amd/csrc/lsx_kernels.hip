@@ -102,8 +102,10 @@ __device__ inline int slot_diag(int npts) { return npts == 7 ? 3 : 13; }
 // of the reference matrices: [b,s,w,p,e,n,t] on the fine level, sorted columns on Galerkin
 // levels).  acc starts at the given value; subtract: terms are subtracted.  Straight-line code: an
 // absent neighbour, whose coefficient is stored as 0, reads the cell itself, so that all loads of
-// a row are in flight together (a branch per term would wait for each).
-template <int NPTS>
+// a row are in flight together (a branch per term would wait for each).  ABSENT0: it counts as 0 whatever
+// is there, since 0 times an infinite value is NaN.  The smoother's products go without (1 to 2 % of a
+// cascade application): the line solves make NaN of an infinite correction in any case.
+template <int NPTS, bool ABSENT0 = true>
 __device__ inline double row_apply(const double* __restrict__ coef, long n, int i, int x, int y, int z, int N, int M,
                                    int K, const double* __restrict__ xv, double acc, bool subtract) {
   const int ox[3] = {x > 0 ? -1 : 0, 0, x < N - 1 ? 1 : 0};
@@ -114,6 +116,14 @@ __device__ inline double row_apply(const double* __restrict__ coef, long n, int 
     const int p = NPTS == 27 ? q : (const int[7]){4, 10, 12, 13, 14, 16, 22}[q];
     a[q] = coef[q * n + i];
     v[q] = xv[i + ox[p % 3] + oy[p / 3 % 3] + oz[p / 9]];
+  }
+  if constexpr (ABSENT0) {
+    const bool hx[3] = {x > 0, true, x < N - 1}, hy[3] = {y > 0, true, y < M - 1}, hz[3] = {z > 0, true, z < K - 1};
+#pragma unroll
+    for (int q = 0; q < NPTS; ++q) {
+      const int p = NPTS == 27 ? q : (const int[7]){4, 10, 12, 13, 14, 16, 22}[q];
+      v[q] = hx[p % 3] && hy[p / 3 % 3] && hz[p / 9] ? v[q] : 0.0;
+    }
   }
 #pragma unroll
   for (int q = 0; q < NPTS; ++q) acc = subtract ? acc - a[q] * v[q] : acc + a[q] * v[q];
@@ -794,7 +804,8 @@ __global__ void __launch_bounds__(256) k_stencil(const double* __restrict__ coef
   int xx, yy, zz;
   if (!own_cell(N, M, K, &xx, &yy, &zz)) return;
   const int i = xx + N * (yy + M * zz);
-  const double q = row_apply<NPTS>(coef, (long)N * M * K, i, xx, yy, zz, N, M, K, x, 0.0, false);
+  const double q =
+      row_apply<NPTS, MODE == ST_PROD>(coef, (long)N * M * K, i, xx, yy, zz, N, M, K, x, 0.0, false);
   y[i] = MODE == ST_PROD ? q : y[i] - q;
 }
 
