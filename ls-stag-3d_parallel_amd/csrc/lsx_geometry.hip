@@ -1466,68 +1466,85 @@ __device__ inline bool corner_active(const double* __restrict__ raw, const doubl
 // change in some moved geometry.
 constexpr unsigned char MARK_CORNER = 1, MARK_FIXABLE = 2;
 
-// The fix can change node i in direction `st` only if a move by h (of one node of the three at most: those
-// that move together are 6 apart) can leave it above the threshold between two nodes below 0.  The
-// upper neighbour is read unfixed, the lower one fixed: below 0 by itself or because the fix
-// brought it there.  NaN compares false: such a node is never fixed.
-__device__ inline bool between(const double* __restrict__ raw, long i, long st, double h) {
-  return raw[i] + h > EQ_DOUBLE && raw[i + st] - h < 0;
-}
-
-// marks of the nodes whose neighbours are low enough by themselves, 0 on all others
-__global__ void __launch_bounds__(256) k_fixable_first(const double* __restrict__ raw, int N, int M, int K, Box box,
-                                                       double h, unsigned char* __restrict__ mark) {
-  const long n = (long)N * M * K, NM = (long)N * M;
-  for (long i = blockIdx.x * (long)blockDim.x + threadIdx.x; i < n; i += (long)gridDim.x * blockDim.x) {
-    int x, y, z;
-    decode(i, N, M, &x, &y, &z);
-    bool on = false;
-    if (in_box(x, y, box)) {
-      auto dir = [&](long st) { return between(raw, i, st, h) && raw[i - st] - h < 0; };
-      on = dir(1) || dir(N) || (z > 0 && z < K - 1 && dir(NM));
-    }
-    mark[i] = on ? MARK_FIXABLE : 0;
+// A node of the box and its neighbours along the axes, for what the fix can do to it once one of them has
+// moved by h.  It changes the node in a direction only if it is above the threshold between two nodes
+// below 0: the upper one unfixed (between), the lower one by itself (alone) or because the fix brought it
+// there.  The first such direction decides (check_osc): one that is so by itself whatever moves
+// (decided) leaves nothing for the directions after it to read.  NaN compares false: never fixed.
+struct FixNode {
+  double r, lo[3], up[3], h;
+  __device__ FixNode(const double* __restrict__ raw, long i, int z, int N, long NM, int K, double h_) : h(h_) {
+    const bool mid = z > 0 && z < K - 1;
+    r = raw[i];
+    lo[0] = raw[i - 1];
+    up[0] = raw[i + 1];
+    lo[1] = raw[i - N];
+    up[1] = raw[i + N];
+    const double b = raw[mid ? i - NM : i], t = raw[mid ? i + NM : i];
+    lo[2] = mid ? b : 1.0;
+    up[2] = mid ? t : 1.0 + h;  // never between
   }
-}
-
-// marks of the nodes above a marked one; state[0]: there is such a node (the fix chains in some moved
-// geometry), state[1]: one was not marked yet.  Repeated until none is added.
-__global__ void __launch_bounds__(256) k_fixable_next(const double* __restrict__ raw, int N, int M, int K, Box box,
-                                                      double h, const unsigned char* __restrict__ cur,
-                                                      unsigned char* __restrict__ nxt, int* __restrict__ state) {
-  const long n = (long)N * M * K, NM = (long)N * M;
-  for (long i = blockIdx.x * (long)blockDim.x + threadIdx.x; i < n; i += (long)gridDim.x * blockDim.x) {
-    int x, y, z;
-    decode(i, N, M, &x, &y, &z);
-    bool above = false;
-    if (in_box(x, y, box)) {
-      auto dir = [&](long st) { return cur[i - st] != 0 && between(raw, i, st, h); };
-      above = dir(1) || dir(N) || (z > 0 && z < K - 1 && dir(NM));
-    }
-    if (above) state[0] = 1;
-    if (above && !cur[i]) state[1] = 1;
-    nxt[i] = above ? MARK_FIXABLE : cur[i];
+  __device__ bool between(int d) const { return r + h > EQ_DOUBLE && up[d] - h < 0; }
+  __device__ bool any() const { return between(0) || between(1) || between(2); }
+  __device__ bool alone() const {
+    return (between(0) && lo[0] - h < 0) || (between(1) && lo[1] - h < 0) || (between(2) && lo[2] - h < 0);
   }
+  __device__ bool decided(int d) const { return r - h > EQ_DOUBLE && lo[d] + h < 0 && up[d] + h < 0; }
+};
+// Fixable nodes' marks by one pass: from the level set (cur null: the nodes fixable by themselves and those
+// that read one), or those of a pass before and those that read one of them.  seen: bit 0 there is a
+// node that reads one (the fix chains in some moved geometry), bit 1 it was not marked yet.
+__device__ inline bool fixable_pass(const double* __restrict__ raw, long i, int N, int M, int K, const Box& box, double h,
+                                    const unsigned char* __restrict__ cur, int* seen) {
+  if (!(raw[i] + h > EQ_DOUBLE)) return false;  // as between: most nodes
+  int x, y, z;
+  decode(i, N, M, &x, &y, &z);
+  if (!in_box(x, y, box)) return false;
+  const long NM = (long)N * M;
+  const FixNode f(raw, i, z, N, NM, K, h);
+  if (!f.any()) return false;
+  const bool was = cur ? cur[i] != 0 : f.alone();
+  auto reads = [&](int d) {  // the lower neighbour's mark
+    if (!f.between(d)) return false;
+    const long j = i - (d == 0 ? 1 : (d == 1 ? N : NM));
+    if (cur) return cur[j] != 0;
+    return in_box(x - (d == 0), y - (d == 1), box) && FixNode(raw, j, z - (d == 2), N, NM, K, h).alone();
+  };
+  const bool rd = reads(0) || (!f.decided(0) && (reads(1) || (!f.decided(1) && reads(2))));
+  *seen |= (rd ? 1 : 0) | (rd && !was ? 2 : 0);
+  return was || rd;
 }
 
-// Lists of nodes in index order: AC_FIXABLE the nodes marked so, AC_CORNERS the active corners and those
-// marked.  Blocks of AC_NODES consecutive nodes count theirs
-// (list null), one workgroup turns the counts into offsets and the total (k_active_scan), and the
-// blocks write (ranks within a block by ballots).
+// Lists of nodes in index order.  AC_LOOK: the active corners, with a first pass over the fixable nodes;
+// AC_FIXABLE: the fixable nodes after another pass (cur null: the first); AC_CORNERS: the active
+// corners and those marked in `cur`.  Blocks of AC_NODES consecutive nodes count theirs (list null) and say
+// what the pass saw, one workgroup turns the counts into offsets, the total and what all saw
+// (k_active_scan), and the blocks write (ranks within a block by ballots; AC_FIXABLE: those marked in `cur`).
 constexpr int AC_NODES = 1024;
 __global__ void __launch_bounds__(256) k_active(const double* __restrict__ raw, const double* __restrict__ phi,
-                                                const unsigned char* __restrict__ mark, int mode, int N, int M, int K,
-                                                Box box, double h,
+                                                const unsigned char* __restrict__ cur, unsigned char* __restrict__ nxt,
+                                                int mode, int N, int M, int K, Box box, double h,
                                                 int* __restrict__ count, int* __restrict__ list) {
   __shared__ int waves[4];
   const long n = (long)N * M * K;
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-  int at = list ? count[blockIdx.x] : 0;
+  int at = list ? count[blockIdx.x] : 0, seen = 0;
   for (int q = 0; q < AC_NODES / 256; ++q) {
     const long i = (long)blockIdx.x * AC_NODES + q * 256 + threadIdx.x;
-    const bool on = i < n && (mode == AC_FIXABLE ? (mark[i] & MARK_FIXABLE) != 0
-                                                 : (mark && (mark[i] & MARK_CORNER)) ||
-                                                       corner_active(raw, phi, i, N, M, K, box, h));
+    bool on = false;
+    if (i < n) {
+      bool fixable = false;
+      if (mode != AC_CORNERS) {
+        if (list) {
+          fixable = mode == AC_FIXABLE && cur[i] != 0;
+        } else {
+          fixable = fixable_pass(raw, i, N, M, K, box, h, mode == AC_LOOK ? nullptr : cur, &seen);
+          nxt[i] = fixable ? MARK_FIXABLE : 0;
+        }
+      }
+      on = mode == AC_FIXABLE ? fixable
+                              : (mode == AC_CORNERS && cur[i] & MARK_CORNER) || corner_active(raw, phi, i, N, M, K, box, h);
+    }
     const unsigned long long m = __ballot(on);
     if (lane == 0) waves[wave] = __popcll(m);
     __syncthreads();
@@ -1540,14 +1557,24 @@ __global__ void __launch_bounds__(256) k_active(const double* __restrict__ raw, 
     at += all;
     __syncthreads();
   }
-  if (!list && threadIdx.x == 0) count[blockIdx.x] = at;
+  if (list) return;
+  const int any = __syncthreads_or(seen & 1), fresh = __syncthreads_or(seen & 2);
+  if (threadIdx.x == 0) {
+    count[blockIdx.x] = at;
+    count[gridDim.x + 2 + blockIdx.x] = (any ? 1 : 0) | (fresh ? 2 : 0);
+  }
 }
 
+// count: nb counts (then offsets), total, what all blocks saw, nb blocks' own
 __global__ void __launch_bounds__(1024) k_active_scan(int* __restrict__ count, int nb) {
   __shared__ int sum[1024];
   const int per = (nb + 1023) / 1024, lo = threadIdx.x * per, hi = lo + per < nb ? lo + per : nb;
-  int mine = 0;
-  for (int b = lo; b < hi; ++b) mine += count[b];
+  int mine = 0, seen = 0;
+  for (int b = lo; b < hi; ++b) {
+    mine += count[b];
+    seen |= count[nb + 2 + b];
+  }
+  const int any = __syncthreads_or(seen & 1), fresh = __syncthreads_or(seen & 2);
   sum[threadIdx.x] = mine;
   __syncthreads();
   for (int st = 1; st < 1024; st <<= 1) {
@@ -1562,7 +1589,10 @@ __global__ void __launch_bounds__(1024) k_active_scan(int* __restrict__ count, i
     count[b] = at;
     at += c;
   }
-  if (threadIdx.x == 1023) count[nb] = sum[1023];
+  if (threadIdx.x == 1023) {
+    count[nb] = sum[1023];
+    count[nb + 1] = (any ? 1 : 0) | (fresh ? 2 : 0);
+  }
 }
 
 // Index of node j in the sorted list of fixable nodes.
@@ -1926,24 +1956,22 @@ double drag(const int* type, const double* tx, const double* dy, const double* d
 
 int active_blocks(long n) { return (int)((n + AC_NODES - 1) / AC_NODES); }
 
-void list_nodes(const double* phi_raw, const double* phi, const unsigned char* mark, int mode, int N, int M, int K,
-                Box box, double h, int* count, int* list, hipStream_t s) {
+void count_nodes(const double* phi_raw, const double* phi, const unsigned char* cur, unsigned char* nxt, int mode, int N,
+                 int M, int K, Box box, double h, int* count, hipStream_t s) {
   const int nb = active_blocks((long)N * M * K);
-  k_active<<<nb, 256, 0, s>>>(phi_raw, phi, mark, mode, N, M, K, box, h, count, list);
-  if (!list) k_active_scan<<<1, 1024, 0, s>>>(count, nb);
+  k_active<<<nb, 256, 0, s>>>(phi_raw, phi, cur, nxt, mode, N, M, K, box, h, count, nullptr);
+  k_active_scan<<<1, 1024, 0, s>>>(count, nb);
 }
 
-void fixable_first(const double* phi_raw, int N, int M, int K, Box box, double h, unsigned char* mark, hipStream_t s) {
-  k_fixable_first<<<grid_1d((long)N * M * K), 256, 0, s>>>(phi_raw, N, M, K, box, h, mark);
-}
-
-void fixable_next(const double* phi_raw, int N, int M, int K, Box box, double h, const unsigned char* cur,
-                  unsigned char* nxt, int* state, hipStream_t s) {
-  k_fixable_next<<<grid_1d((long)N * M * K), 256, 0, s>>>(phi_raw, N, M, K, box, h, cur, nxt, state);
+void list_nodes(const double* phi_raw, const double* phi, const unsigned char* cur, int mode, int N, int M, int K, Box box,
+                double h, int* count, int* list, hipStream_t s) {
+  const int nb = active_blocks((long)N * M * K);
+  k_active<<<nb, 256, 0, s>>>(phi_raw, phi, cur, nullptr, mode, N, M, K, box, h, count, list);
 }
 
 void chain_tables(const double* phi_raw, const double* phi, const int* fixable, int n_fixable, int N, int M, int K,
                   Box box, double h, double* table, unsigned char* mark, hipStream_t s) {
+  if (n_fixable < 1) return;
   k_chain_mark<<<n_fixable, 256, 0, s>>>(fixable, N, M, K, box, mark);
   k_chain_table<<<2 * SG_CLASSES, 256, 0, s>>>(phi_raw, phi, mark, fixable, n_fixable, N, M, K, box, h, table);
 }

@@ -100,20 +100,23 @@ void drag_noalloc(const int* type, const double* tx, const double* dy, const dou
 // Address of the library's drag scratch array on the current device (looked up once per device
 // with hipGetSymbolAddress); 0, or a negative value when the lookup fails.
 int drag_scratch(double** out);
-// Nodes that the oscillation fix can change with some corner moved by h, in marks of one byte a node:
-// fixable_first writes them all, fixable_next (cur to nxt) adds those next to a marked one and sets
-// state[0] if it meets any, state[1] if one was not marked yet.  To be repeated while it does.
-void fixable_first(const double* phi_raw, int N, int M, int K, Box box, double h, unsigned char* mark, hipStream_t s);
-void fixable_next(const double* phi_raw, int N, int M, int K, Box box, double h, const unsigned char* cur,
-                  unsigned char* nxt, int* state, hipStream_t s);
-// Lists of nodes in index order: AC_FIXABLE those, AC_CORNERS the corners that a move by h can change the
-// geometry at and (mark given) those that chain_tables marked.  list null: fills
-// count[0 .. nb) with the offsets of nb = active_blocks(n) blocks of nodes and count[nb] with the
-// number of listed ones; list given (after that): writes them.
-enum { AC_FIXABLE = 0, AC_CORNERS = 1 };
+// Lists of nodes in index order: AC_LOOK the corners that a move by h can change the geometry at, with a
+// first look at the nodes that the oscillation fix can change once some corner has moved by h (fixable);
+// AC_FIXABLE those; AC_CORNERS the corners of AC_LOOK and those that chain_tables marked in `cur`.
+// count_nodes: offsets of nb = active_blocks(n) blocks of nodes, the number of listed ones in count[nb],
+// and in count[nb + 1] what the pass saw: SAW_CHAIN a fixable node that reads another, SAW_NEW one
+// that is marked for the first time (count: active_counts(n) ints).  AC_LOOK and AC_FIXABLE write a
+// byte a node to nxt; AC_FIXABLE adds to the marks `cur` (null: to none) those that read one, and is to be
+// repeated on its result while it sees SAW_NEW.  list_nodes, after that, writes the list (AC_FIXABLE:
+// of the nodes marked in `cur`).
+enum { AC_LOOK = 0, AC_FIXABLE = 1, AC_CORNERS = 2 };
+enum { SAW_CHAIN = 1, SAW_NEW = 2 };
 int active_blocks(long n);
-void list_nodes(const double* phi_raw, const double* phi, const unsigned char* mark, int mode, int N, int M, int K,
-                Box box, double h, int* count, int* list, hipStream_t s);
+inline int active_counts(long n) { return 2 * active_blocks(n) + 2; }
+void count_nodes(const double* phi_raw, const double* phi, const unsigned char* cur, unsigned char* nxt, int mode, int N,
+                 int M, int K, Box box, double h, int* count, hipStream_t s);
+void list_nodes(const double* phi_raw, const double* phi, const unsigned char* cur, int mode, int N, int M, int K, Box box,
+                double h, int* count, int* list, hipStream_t s);
 // Where a fixable node reads another: table gets the listed ones' values with the corners of each class
 // moved by +h and -h (432 n_fixable doubles), mark the corners whose cells read such a node.
 constexpr int CHAIN_MOVES = 432;

@@ -4,9 +4,7 @@
 
 #include "lsx_geometry_host.hpp"
 
-#include <algorithm>
 #include <cmath>
-#include <utility>
 
 namespace lsx {
 
@@ -166,20 +164,20 @@ void Geometry::stage_flow(const double* u, const double* v, const double* w, con
   }
 }
 
-// nodes of a list (geo::AC_*) into `list`, which grows with some room for the next body's; their number.
-// state given: receives the two ints behind the counts (geo::fixable_next) in the same copy
-int Geometry::list_nodes(int mode, const unsigned char* mark, double h, DevBuf<int>& list, int* state) {
-  const int nb = geo::active_blocks(n());
-  geo::list_nodes(phi_raw.p, phi.p, mark, mode, N, M, K, box_, h, sg_count.p, nullptr, stream);
-  int got[3] = {0, 0, 0};
-  LSX_HIP(hipMemcpyAsync(got, sg_count.p + nb, sizeof(got), hipMemcpyDeviceToHost, stream));
+// one pass over the nodes of a list (geo::AC_*), and the list, which grows with some room for the next body's
+void Geometry::count_nodes(int mode, const unsigned char* cur, unsigned char* nxt, double h) {
+  geo::count_nodes(phi_raw.p, phi.p, cur, nxt, mode, N, M, K, box_, h, sg_count.p, stream);
+}
+int Geometry::counted(int* saw) {
+  int got[2] = {0, 0};
+  LSX_HIP(hipMemcpyAsync(got, sg_count.p + geo::active_blocks(n()), sizeof(got), hipMemcpyDeviceToHost, stream));
   LSX_HIP(hipStreamSynchronize(stream));
-  const int count = got[0];
-  if (state) std::copy(got + 1, got + 3, state);
+  if (saw) *saw = got[1];
+  return got[0];
+}
+void Geometry::list_nodes(int mode, const unsigned char* cur, double h, int count, DevBuf<int>& list) {
   if ((size_t)count > list.n) list.alloc((size_t)count + count / 4);
-  if (count > 0)
-    geo::list_nodes(phi_raw.p, phi.p, mark, mode, N, M, K, box_, h, sg_count.p, list.p, stream);
-  return count;
+  if (count > 0) geo::list_nodes(phi_raw.p, phi.p, cur, mode, N, M, K, box_, h, sg_count.p, list.p, stream);
 }
 
 double Geometry::drag(const double* p, double* dJdp, int mem) {
@@ -283,35 +281,35 @@ void Geometry::shape_gradient(const double* p, const double* lam, int objective,
   LSX_HIP(hipMemsetAsync(sg_g.p, 0, nn * sizeof(double), stream));
   // Where, in some moved geometry, a node that the oscillation fix changes reads another such node, a
   // corner's move can reach beyond its patch: corners then move by classes, with the fixed values of each
-  // class's moves in a table.  Every body pays the look (two passes over a byte a node, read with the
-  // first list's count): whether the unmoved geometry chains does not say it, a body aligned with the
-  // grid may chain only once a node at 0 has moved.
-  const int nb = geo::active_blocks(nn);
-  sg_count.alloc(nb + 3);
+  // class's moves in a table.  So it is if the unmoved geometry chains (a third pass of its fix); every
+  // other body pays the look, in the pass that counts its corners: one aligned with the grid may chain
+  // only once a node at 0 has moved.
+  sg_count.alloc(geo::active_counts(nn));
   sg_mark.alloc(nn);
-  int* const dstate = sg_count.p + nb + 1;
-  unsigned char *cur = flag.p, *nxt = sg_mark.p;
-  auto spread = [&] {
-    LSX_HIP(hipMemsetAsync(dstate, 0, 2 * sizeof(int), stream));
-    geo::fixable_next(phi_raw.p, N, M, K, box_, h, cur, nxt, dstate, stream);
-    std::swap(cur, nxt);
-  };
-  geo::fixable_first(phi_raw.p, N, M, K, box_, h, cur, stream);
-  spread();
-  int state[2], n_fixable = 0;
-  int active = list_nodes(geo::AC_CORNERS, nullptr, h, sg_list, state);
-  const bool chain = state[0] != 0;
+  unsigned char *cur = nullptr, *nxt = flag.p;
+  int active = 0, n_fixable = 0, saw = 0;
+  bool chain = osc_passes > 2;
+  if (!chain) {
+    count_nodes(geo::AC_LOOK, nullptr, nxt, h);
+    active = counted(&saw);
+    chain = saw & geo::SAW_CHAIN;
+    if (!chain) list_nodes(geo::AC_LOOK, nullptr, h, active, sg_list);
+  }
   if (chain) {
-    while (state[1]) {
-      spread();
-      LSX_HIP(hipMemcpyAsync(state, dstate, sizeof(state), hipMemcpyDeviceToHost, stream));
-      LSX_HIP(hipStreamSynchronize(stream));
+    // as many passes as the unmoved geometry's fix before the first look at what they saw
+    for (int pass = 1; pass < osc_passes || saw & geo::SAW_NEW || pass < 2; ++pass) {
+      count_nodes(geo::AC_FIXABLE, cur, nxt, h);
+      cur = nxt;
+      nxt = cur == flag.p ? sg_mark.p : flag.p;
+      if (pass + 1 >= osc_passes) n_fixable = counted(&saw);
     }
-    n_fixable = list_nodes(geo::AC_FIXABLE, cur, h, sg_fixable);
+    list_nodes(geo::AC_FIXABLE, cur, h, n_fixable, sg_fixable);
     if ((size_t)n_fixable * geo::CHAIN_MOVES > sg_table.n)
       sg_table.alloc((size_t)(n_fixable + n_fixable / 4) * geo::CHAIN_MOVES);
     geo::chain_tables(phi_raw.p, phi.p, sg_fixable.p, n_fixable, N, M, K, box_, h, sg_table.p, cur, stream);
-    active = list_nodes(geo::AC_CORNERS, cur, h, sg_list);
+    count_nodes(geo::AC_CORNERS, cur, nullptr, h);
+    active = counted(nullptr);
+    list_nodes(geo::AC_CORNERS, cur, h, active, sg_list);
   }
   const geo::GeoBase base{phi_raw.p, phi.p, {ax.p, ay.p, az.p}, {tx.p, ty.p, tz.p}, vof.p, type.p};
   geo::corner_gradient(base, sg_list.p, active, cur, sg_fixable.p, n_fixable, chain ? sg_table.p : nullptr, dx.p, dy.p,

@@ -103,7 +103,9 @@ class Geometry {
   DevBuf<double> sg_g, sg_uv, sg_w, sg_partial, sg_out, sg_table;
   DevBuf<int> sg_count, sg_list, sg_fixable, sg_f;
   DevBuf<unsigned char> sg_mark;
-  int list_nodes(int mode, const unsigned char* mark, double h, DevBuf<int>& list, int* state = nullptr);
+  void count_nodes(int mode, const unsigned char* cur, unsigned char* nxt, double h);
+  int counted(int* saw);  // waits for the count
+  void list_nodes(int mode, const unsigned char* cur, double h, int count, DevBuf<int>& list);
 };
 
 }  // namespace lsx

@@ -21,12 +21,15 @@ void theta(const double*, const double*, const double*, const int*, const int*, 
 void vof(const int*, const double*, const double*, const double*, const double*, const double*, const double*,
          const double*, const double*, const double*, int, int, int, double*, hipStream_t) {}
 int active_blocks(long) { return 1; }
-void fixable_first(const double*, int, int, int, Box, double, unsigned char*, hipStream_t) {}
-void fixable_next(const double*, int, int, int, Box, double, const unsigned char*, unsigned char*, int*, hipStream_t) {}
-void list_nodes(const double*, const double*, const unsigned char*, int, int, int, int, Box, double, int* count,
-                int* list, hipStream_t) {
-  if (!list) count[1] = corners;
-  if (list) CHECK(room(list) >= corners * sizeof(int));
+void count_nodes(const double*, const double*, const unsigned char*, unsigned char*, int, int, int, int, Box, double,
+                 int* count, hipStream_t) {
+  CHECK(room(count) >= active_counts(0) * sizeof(int));
+  count[1] = corners;
+  count[2] = 0;
+}
+void list_nodes(const double*, const double*, const unsigned char*, int, int, int, int, Box, double, int*, int* list,
+                hipStream_t) {
+  CHECK(room(list) >= corners * sizeof(int));
 }
 void corner_gradient(const GeoBase&, const int*, int, const unsigned char*, const int*, int, const double*,
                      const double*, const double*, const double*, int, int, int, Box, int, const double*, const double*,
