@@ -1603,6 +1603,24 @@ __global__ void k_zero_empty(const T* __restrict__ s, double* __restrict__ x, lo
 __device__ inline float recip0(float v) { return v != 0.f ? __builtin_amdgcn_rcpf(v) : 0.f; }
 __device__ inline double recip0(double v) { return v != 0.0 ? 1.0 / v : 0.0; }
 
+// a product that no sum is contracted with
+template <class T>
+__device__ inline T rounded(T a, T b) {
+  #pragma clang fp contract(off)
+  return a * b;
+}
+// The four couplings across a line.  Which of the first two products is rounded by itself is said here
+// and not left to the compiler, so that the passes of the small levels in one workgroup and those
+// launched one by one agree bit for bit.  SECOND: the second (x lines, and rows of transposed passes),
+// else the first (segments).  x lines of several cells a lane, which no small level has, keep the
+// compiler's choice: with this sum the FP64 solve of 128^3 took 5.66 ms, with theirs 5.57.
+template <bool SECOND, class T>
+__device__ inline T across(T c0, T x0, T c1, T x1, T c2, T x2, T c3, T x3) {
+  #pragma clang fp contract(fast)
+  if constexpr (SECOND) return c0 * x0 + rounded(c1, x1) + c2 * x2 + c3 * x3;
+  else return rounded(c0, x0) + c1 * x1 + c2 * x2 + c3 * x3;
+}
+
 // Row of cell i on its line of direction DIR: lower (coupling to the previous cell of the line),
 // diag, upper, rhs.  Pinned rows are identity rows; an empty row (1/a_p stored as 0) keeps its
 // value, as in the point smoother.  ZERO: x taken as 0 (not read).  DFF (forward rows only,
@@ -1612,7 +1630,7 @@ __device__ inline void line_row(const T* __restrict__ x, const T* __restrict__ b
                                 const FT* __restrict__ an, const FT* __restrict__ at, const T* __restrict__ s, T fs,
                                 long i, int xx, int yy, int zz, int N, int M, int K, int pin0, int pin1, bool trans,
                                 T& lo, T& dg, T& up, T& rhs, DiagRule<T> dr = DiagRule<T>{-1, -1, (T)0, (T)0}) {
-  #pragma clang fp contract(fast)  // line solves: no bitwise twin to match
+  #pragma clang fp contract(fast)  // line solves (across: the one sum with a choice)
   // Straight-line code: every load is issued unconditionally (absent neighbours read the cell
   // itself and are masked out), so that a caller evaluating many rows can have all their loads
   // in flight at once.
@@ -1637,8 +1655,8 @@ __device__ inline void line_row(const T* __restrict__ x, const T* __restrict__ b
   if constexpr (!ZERO) {
     xi = x[i];
     if constexpr (DIR == 0) off = cs * x[is] + cn * x[in] + cb * x[ib] + ct * x[it];
-    else if constexpr (DIR == 1) off = cw * x[iw] + ce * x[ie] + cb * x[ib] + ct * x[it];
-    else off = cw * x[iw] + ce * x[ie] + cs * x[is] + cn * x[in];
+    else if constexpr (DIR == 1) off = across<true>(cw, x[iw], ce, x[ie], cb, x[ib], ct, x[it]);
+    else off = across<true>(cw, x[iw], ce, x[ie], cs, x[is], cn, x[in]);
   }
   T ap;
   if constexpr (DFF)
@@ -1688,7 +1706,7 @@ __device__ inline void line_rows_x(const T* __restrict__ x, const T* __restrict_
                                    T fs, long i0, int k0, int yy, int zz, int N, int M, int K, int pin0, int pin1,
                                    bool trans, T (&lo)[CPL], T (&dg)[CPL], T (&up)[CPL], T (&rh)[CPL],
                                    DiagRule<T> dr) {
-  #pragma clang fp contract(fast)  // line solves: no bitwise twin to match
+  #pragma clang fp contract(fast)  // line solves (across: the one sum with a choice)
   const long NM = (long)N * M;
   const bool ys = yy > 0, yn = yy < M - 1, zb = zz > 0, zt = zz < K - 1;
   const long is0 = ys ? i0 - N : i0, in0 = yn ? i0 + N : i0, ib0 = zb ? i0 - NM : i0, it0 = zt ? i0 + NM : i0;
@@ -1728,7 +1746,8 @@ __device__ inline void line_rows_x(const T* __restrict__ x, const T* __restrict_
     T off = (T)0, xi = (T)0;
     if constexpr (!ZERO) {
       xi = xv[j];
-      off = cs * xs[j] + cn * xn[j] + cb * xb[j] + ct * xt[j];
+      if constexpr (CPL == 1) off = across<true>(cs, xs[j], cn, xn[j], cb, xb[j], ct, xt[j]);
+      else off = cs * xs[j] + cn * xn[j] + cb * xb[j] + ct * xt[j];
     }
     const T bi = bv[j];
     T ap;
@@ -1757,7 +1776,7 @@ __global__ void __launch_bounds__(256) k_line_x(const T* __restrict__ x_in, T* _
                                                 const FT* __restrict__ an, const FT* __restrict__ at,
                                                 const T* __restrict__ s, T fs, int N, int M, int K, int pin0,
                                                 int pin1, DiagRule<T> dr) {
-  #pragma clang fp contract(fast)  // line solves: no bitwise twin to match
+  #pragma clang fp contract(fast)  // line solves (across: the one sum with a choice)
   static_assert(!(TRANS && DFF), "a_p from the faces is a forward-operator rule");
   const int lane = threadIdx.x & (LANES - 1);
   const long row_t = (long)blockIdx.x * (256 / LANES) + (threadIdx.x / LANES);
@@ -1918,7 +1937,7 @@ struct SegLine {
       return f;
   }
   __device__ inline void row(unsigned i, int kk, bool first, T& fl_carry, T& lo, T& dg, T& up, T& rh) const {
-  #pragma clang fp contract(fast)  // line solves: no bitwise twin to match
+  #pragma clang fp contract(fast)  // line solves (across: the one sum with a choice)
     const bool hl = kk > 0, hu = kk < len - 1;
     T sv = (T)0;
     if constexpr (!DFF) sv = ldo(s, i);
@@ -1939,7 +1958,7 @@ struct SegLine {
       fal = l32 == 0 ? fw0 : fws;
       const T cAl = hAl ? scl(fal) : (T)0, cAu = hAu ? scl(fau) : (T)0;
       const T cBl = hBl ? scl(fbl) : (T)0, cBu = hBu ? scl(fbu) : (T)0;
-      off = cAl * xal + cAu * xau + cBl * xbl + cBu * xbu;
+      off = across<false>(cAl, xal, cAu, xau, cBl, xbl, cBu, xbu);
     } else if constexpr (DFF) {
       const T fw0 = (T)ldo(ae, i + oW0), fws = __shfl_up(fau, 1, LPW);
       fal = l32 == 0 ? fw0 : fws;
@@ -1980,7 +1999,7 @@ __global__ void __launch_bounds__(1024) k_line_seg(const T* __restrict__ x_in, T
                                                    const FT* __restrict__ an, const FT* __restrict__ at,
                                                    const T* __restrict__ s, T fs, int N, int M, int K, int pin0,
                                                    int pin1, int S, DiagRule<T> dr) {
-  #pragma clang fp contract(fast)  // line solves: no bitwise twin to match
+  #pragma clang fp contract(fast)  // line solves (across: the one sum with a choice)
   static_assert(!(TRANS && DFF), "a_p from the faces is a forward-operator rule");
   constexpr int LPW = lpw<T>();
   extern __shared__ unsigned char lds_raw[];
@@ -2230,8 +2249,6 @@ __global__ void __launch_bounds__(1024) k_line_seg(const T* __restrict__ x_in, T
 // One line pass over a level in LDS (x_in, x_out, b, faces in operator units, reciprocals of s), bit
 // for bit as k_line_x<CPL 1> and k_line_seg: the directions differ in strides only.  A: the first
 // direction across the line, B: the second.
-__device__ inline float fma_of(float a, float b, float c) { return __builtin_fmaf(a, b, c); }
-__device__ inline double fma_of(double a, double b, double c) { return __builtin_fma(a, b, c); }
 template <class T>
 struct LineCells {
   const T *e, *n, *t, *ap, *b;
@@ -2266,10 +2283,7 @@ struct SmallLines {
     const T fl = fL[l0 ? i - sL : i], fu = fL[i];
     const T fa = fA[ia0], fc = fA[i], fb = fB[ib0], fd = fB[i];
     const T ca0 = a0 ? fa : (T)0, ca1 = a1 ? fc : (T)0, cb0 = b0 ? fb : (T)0, cb1 = b1 ? fd : (T)0;
-    // the sum as the compiler contracts it in the passes launched one by one: line_row and line_rows_x
-    // round the second product, SegLine::row (FIRST) the first
-    const T first = FIRST ? fma_of(ca1, x[ia1], ca0 * x[ia0]) : fma_of(ca0, x[ia0], ca1 * x[ia1]);
-    const T off = fma_of(cb1, x[ib1], fma_of(cb0, x[ib0], first));
+    const T off = across<!FIRST>(ca0, x[ia0], ca1, x[ia1], cb0, x[ib0], cb1, x[ib1]);
     const bool empty = d == (T)0;
     lo = empty || !l0 ? (T)0 : fl;
     up = empty || !l1 ? (T)0 : fu;
