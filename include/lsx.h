@@ -190,7 +190,11 @@ int lsx_synchronize(lsx_solver* s);
  * profiler.h:53-274).  While enabled, the fine-level launches of each kernel class below are
  * bracketed by HIP events on the handle's stream.  lsx_kernel_stats reports the launch count,
  * the summed device time and the kernel's algorithmic HBM bytes per launch, averaged over the
- * launches (compulsory traffic: each array read or written once). */
+ * launches (compulsory traffic: each array read or written once).  A timed solve launches the
+ * finest level's kernels one by one where an untimed one fuses them: the cascade runs its small levels
+ * in launches of their own (untimed: all of them in one), a red-black finest level of up to 2^18
+ * cells its half-sweeps (untimed: all sweeps of a side in one), and no graph is replayed.  The
+ * results are the same bits; the times are those of the launches made. */
 #define LSX_K_RESIDUAL 0   /* r -= A c inside the smoother                 */
 #define LSX_K_LINE_X 1     /* x-line solve: cascade c = w T^-1 r, ch += c;  */
 #define LSX_K_LINE_Y 2     /*   V-cycle line relaxation, one pass of x, y  */

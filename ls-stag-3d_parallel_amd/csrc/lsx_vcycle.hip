@@ -411,7 +411,8 @@ __global__ void k_rbgs(T* __restrict__ x, const T* __restrict__ b, const FT* __r
 // through LDS, and the 8 children of each of the 32 coarse cells summed by one thread in the
 // order x, then y, then z fastest-first (the order of the one-workgroup coarse cycle, so the two
 // are bit-identical).  On an axis of odd length the last coarse cell has one child: the absent
-// one adds 0.  DFF: a_p rebuilt from the faces (Level::dff), s not read; no bitwise twin then.
+// one adds 0.  DFF: a_p rebuilt from the faces (Level::dff), s not read; k_rb_tile<.., DFF> is its
+// bitwise twin.
 template <class T, class FT, bool DFF>
 __global__ void __launch_bounds__(256) k_resid_restrict_cells(const T* __restrict__ x, const T* __restrict__ b,
                                                               const FT* __restrict__ ae, const FT* __restrict__ an,
